@@ -1156,6 +1156,9 @@ static int one_step(wd2_ctx *c, const wd2_params *P, int *nql, int *nsor, double
     }
     // main.f:735: one iteration without the energy equation
     const int nme = (!therm && O.nmeiter > 0) ? 1 : O.nmeiter;
+    // without the energy equation and the equation of state nothing stands
+    // between the fills after Project and those at the step's end: one launch
+    const bool fills_twice = !therm && O.neqstate != 1 && nme > 0;
     int st;
     for (int l = 1; l <= nme; l++) {
         // main.f:741-747 (the first iteration's us, vs come with the copies above)
@@ -1174,8 +1177,7 @@ static int one_step(wd2_ctx *c, const wd2_params *P, int *nql, int *nsor, double
         // main.f:783-791
         if (O.nfiltu == 1) launch_filter(c->R, c->TH, ld, VU, O.fpu, c->us, c->qh, s);
         if (O.nfiltv == 1) launch_filter(c->R, c->TH, ld, VV, O.fpv, c->vs, c->qh, s);
-        launch_vel_bc<double>(c->R, ld, c->us, c->vs, false, &c->sc->err, s);
-        launch_pres_bc<double>(c->R, ld, c->p, &c->sc->err, s);
+        launch_fills(c->R, ld, c->us, c->vs, c->p, 1, &c->sc->err, s);
         if (xp && l == 1) launch_mg_extrap(nx, ny, ld, c->p, extrap_p1(c), extrap_p2(c, xp), s);
         c->mg_minc = (xp && l == 1) ? mg_min_cycles(P) : 0;
         st = ppe(c, P->lCartesGrid, P->nPpeSolver, P->msorit, P->dk, P->sortol, P->sorrel, c->us, c->vs, c->p, nsor);
@@ -1183,8 +1185,7 @@ static int one_step(wd2_ctx *c, const wd2_params *P, int *nql, int *nsor, double
         if (st) return st;
         launch_pres_bc<double>(c->R, ld, c->p, &c->sc->err, s);
         launch_project(c->R, ld, P->dk, c->M, c->p, c->us, c->vs, s);
-        launch_vel_bc<double>(c->R, ld, c->us, c->vs, false, &c->sc->err, s);
-        launch_pres_bc<double>(c->R, ld, c->p, &c->sc->err, s);
+        launch_fills(c->R, ld, c->us, c->vs, c->p, fills_twice ? 2 : 1, &c->sc->err, s);
         // main.f:840-855
         if (therm)
             launch_therm_energy(c->R, c->TH, ld, P->dk, O.pe, c->M, c->un, c->vn, c->us, c->vs, c->tn, c->ts, c->tt,
@@ -1219,8 +1220,7 @@ static int one_step(wd2_ctx *c, const wd2_params *P, int *nql, int *nsor, double
     }
     // main.f:890-895
     if (therm && O.nfiltt == 1) launch_filter(c->R, c->TH, ld, VT, O.fpt, c->t, c->qh, s);
-    launch_vel_bc<double>(c->R, ld, c->u, c->v, false, &c->sc->err, s);
-    launch_pres_bc<double>(c->R, ld, c->p, &c->sc->err, s);
+    if (!fills_twice) launch_fills(c->R, ld, c->u, c->v, c->p, 1, &c->sc->err, s);
     if (therm) launch_temp_bc(c->R, c->TH, ld, c->t, &c->sc->err, s);
     // main.f:962-965
     launch_max_norm(nx, ny, ld, c->pn, c->p, c->partials, c->sc, 2, s);
@@ -1283,8 +1283,7 @@ static void step_body(wd2_ctx *c, const wd2_params *P, int Q, int C, int xp) {
     }
     if (O.nfiltu == 1) launch_filter(c->R, c->TH, ld, VU, O.fpu, c->us, c->qh, s);
     if (O.nfiltv == 1) launch_filter(c->R, c->TH, ld, VV, O.fpv, c->vs, c->qh, s);
-    launch_vel_bc<double>(c->R, ld, c->us, c->vs, false, &c->sc->err, s);
-    launch_pres_bc<double>(c->R, ld, c->p, &c->sc->err, s);
+    launch_fills(c->R, ld, c->us, c->vs, c->p, 1, &c->sc->err, s);
     if (xp) launch_mg_extrap(nx, ny, ld, c->p, extrap_p1(c), extrap_p2(c, xp), s);
     // Ppe (pressure.f:30) with the multigrid solver
     launch_divergence(nx, ny, ld, 1, c->M, c->us, c->vs, c->div, s);
@@ -1303,12 +1302,10 @@ static void step_body(wd2_ctx *c, const wd2_params *P, int Q, int C, int xp) {
     }
     launch_pres_bc<double>(c->R, ld, c->p, &c->sc->err, s);
     launch_project(c->R, ld, P->dk, c->M, c->p, c->us, c->vs, s);
-    launch_vel_bc<double>(c->R, ld, c->us, c->vs, false, &c->sc->err, s);
-    launch_pres_bc<double>(c->R, ld, c->p, &c->sc->err, s);
     // u = us, v = vs: the host swaps the buffers after the step, so the rest
-    // of the step works on us, vs as the new u, v (main.f:946-965)
-    launch_vel_bc<double>(c->R, ld, c->us, c->vs, false, &c->sc->err, s);
-    launch_pres_bc<double>(c->R, ld, c->p, &c->sc->err, s);
+    // of the step works on us, vs as the new u, v (main.f:946-965); the fills
+    // after Project and those at the step's end are one launch
+    launch_fills(c->R, ld, c->us, c->vs, c->p, 2, &c->sc->err, s);
     launch_max_norm(nx, ny, ld, c->pn, c->p, c->partials, c->sc, 2, s);
     launch_max_norm(nx, ny, ld, c->un, c->us, c->partials + RED_MAX_BLOCKS, c->sc, 3, s);
     launch_max_norm(nx, ny, ld, c->vn, c->vs, c->partials + 2 * RED_MAX_BLOCKS, c->sc, 4, s);

@@ -66,6 +66,8 @@ void launch_vel_bc(const Regions &R, int ld, T *u, T *v, bool outflow_only, int 
                    const int *stop = nullptr);   // stop: as for launch_trid
 template <typename T>
 void launch_pres_bc(const Regions &R, int ld, T *p, int *err, hipStream_t s);
+// VelBoundCond of u, v and PresBoundCond of p, `reps` times, in one launch.
+void launch_fills(const Regions &R, int ld, double *u, double *v, double *p, int reps, int *err, hipStream_t s);
 
 // Device scalars shared by the reductions (one cache line each).
 struct Scalars {
