@@ -1,0 +1,689 @@
+// k_ql.hip -- one q-l iteration's chain solves and update in one launch
+// (momentum.f:159-188: AltTridLU of both splits of XMomentum and YMomentum,
+// then us += dus, vs += dvs and DMaxNorm of the increments).
+//
+// Both splits of a component run over the same x-ordered rows, and the
+// coupling of a row to rows far away decays geometrically, so a workgroup can
+// take a window of consecutive chain rows, solve the first split on it, form
+// the second split's right-hand side (the solution, 0 on identity rows) and
+// solve the second split on the window's inner rows, all in registers.  The
+// two solves run on overlapping windows: the first needs H rows of halo for
+// its rows to be right, the second another H inside those, so a window of N
+// rows keeps N - 4H.  The separate launches read the chains three times
+// (forward, backward, repair), stored the swept rows and both solutions in
+// between and updated the fields in a pass of their own: per row 130 B in
+// FP64 where this kernel moves 80.
+//
+// The kept rows update the other buffer of a pair (us, vs in; us, vs out), so
+// the iteration's input stays whole: if the solve turns out not to be usable
+// (see the two kernels), the fold sets ql_stop = -1, every kernel queued
+// behind returns at entry, and the host repeats the iteration with the
+// solvers of k_trid.hip.
+#include "wd2_trid.hpp"
+
+namespace wd2 {
+
+// ------------------------------------------------------------ common parts
+// Rows of a segment outside [0, n) are uncoupled rows with solution 0.
+template <typename T, typename CT>
+__device__ inline void ql_load(const T *__restrict__ G, long k0, long n, T pad, CT (&r)[TR_S]) {
+    if (k0 >= 0 && k0 + TR_S <= n) {
+        T v[TR_S];
+        seg_load(G, k0, TR_S, v);
+#pragma unroll
+        for (int s = 0; s < TR_S; s++) r[s] = (CT)v[s];
+    } else {
+#pragma unroll
+        for (int s = 0; s < TR_S; s++) r[s] = (CT)((k0 + s >= 0 && k0 + s < n) ? G[k0 + s] : pad);
+    }
+}
+
+// Kinds of a segment's rows, two bits per row (0 interior or outside [0, n),
+// 1 chain start, 2 chain end).
+__device__ inline unsigned ql_kinds(long k0, long n, const Chains &cs) {
+    unsigned m = 0;
+    unsigned L = 1, r = 0;
+    bool have = false;
+#pragma unroll
+    for (int s = 0; s < TR_S; s++) {
+        const long k = k0 + s;
+        if (k >= 0 && k < n) {
+            if (!have || k == cs.n1) {
+                have = true;
+                L = (unsigned)(k < cs.n1 ? cs.L1 : cs.L2);
+                r = (unsigned)(k < cs.n1 ? k : k - cs.n1) % L;
+            } else if (++r == L) {
+                r = 0;
+            }
+            m |= (r == 0 ? 1u : (r == L - 1 ? 2u : 0u)) << (2 * s);
+        }
+    }
+    return m;
+}
+
+// Identity-row flags of a segment, one bit per row.
+__device__ inline unsigned ql_ident(const unsigned char *__restrict__ Z, long k0, long n) {
+    unsigned m = 0;
+    if (k0 >= 0 && k0 + TR_S <= n) {
+        const unsigned long long zb = *reinterpret_cast<const unsigned long long *>(Z + k0);
+#pragma unroll
+        for (int s = 0; s < TR_S; s++) m |= ((zb >> (8 * s)) & 0xffu) ? 1u << s : 0u;
+    } else {
+        for (int s = 0; s < TR_S; s++)
+            if (k0 + s >= 0 && k0 + s < n && Z[k0 + s]) m |= 1u << s;
+    }
+    return m;
+}
+
+// The fields' part of the launch: rows [0, n1) of the chains are the points
+// (i = 1..nx, j = 2..ny) of u, rows [n1, n) the points (i = 2..nx, j = 1..ny)
+// of v, i fastest.
+struct QlFields {
+    int nx, ny, ld;
+    const double *us, *vs;   // the iterate
+    double *uo, *vo;         // the next one
+    double *dus, *dvs;       // stored increments outside the chain rows, and at (5, 5)
+};
+
+// us + dus, vs + dvs of the window rows [lo, hi) from the increments X in LDS
+// (row l at (l / 8) * 9 + l % 8), a row per lane in order (coalesced where
+// the solve's segments are not), and the increments' maxima over the interior
+// into part[2 block ..].  dus, dvs are stored at (5, 5) only, which the fold
+// reads.
+template <int NT, typename T>
+__device__ inline void ql_update(const QlFields &F, const T *X, long w0, int lo, int hi, long n, long n1,
+                                 double *__restrict__ part, double *sh) {
+    const int nx = F.nx, ny = F.ny, ld = F.ld, t = threadIdx.x;
+    double m1 = 0.0, m2 = 0.0;
+    for (int l = lo + t; l < hi; l += NT) {
+        const long k = w0 + l;
+        if (k < 0 || k >= n) continue;
+        const double dx = (double)X[(l >> 3) * TR_P + (l & 7)];
+        const bool isu = k < n1;
+        const unsigned q = (unsigned)(isu ? k : k - n1), w = (unsigned)(isu ? nx : nx - 1);
+        const unsigned row = q / w, col = q - row * w;
+        const int i = (int)col + (isu ? 1 : 2), j = (int)row + (isu ? 2 : 1);
+        const size_t p = WD2_IX(i, j);
+        const double f = (isu ? F.us : F.vs)[p];
+        (isu ? F.uo : F.vo)[p] = f + dx;
+        if (i == 5 && j == 5) (isu ? F.dus : F.dvs)[p] = dx;
+        if (i >= 2 && i <= nx - 1 && j >= 2 && j <= ny - 1) {
+            if (isu)
+                m1 = dmaxf(m1, fabs(dx));
+            else
+                m2 = dmaxf(m2, fabs(dx));
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        m1 = dmaxf(m1, __shfl_xor(m1, off));
+        m2 = dmaxf(m2, __shfl_xor(m2, off));
+    }
+    if ((t & 63) == 0) {
+        sh[2 * (t >> 6)] = m1;
+        sh[2 * (t >> 6) + 1] = m2;
+    }
+    __syncthreads();
+    if (t < 2) {
+        double m = sh[t];
+        for (int w = 1; w < NT / 64; w++) m = dmaxf(m, sh[2 * w + t]);
+        part[2 * blockIdx.x + t] = m;
+    }
+}
+
+// The points no chain row covers, carried to the output buffers (block b of
+// the nb that follow the windows): the ghost lines, u's line j = 1 and v's
+// column i = 1 -- with their stored increments, as momentum.f:171-176 adds
+// them on i = 1..nx, j = 1..ny.
+template <int NT>
+__device__ inline void ql_border(const QlFields &F, int b, int nb) {
+    const int nx = F.nx, ny = F.ny, ld = F.ld;
+    const int nu = 2 * (ny + 2) + 3 * nx, nv = 3 * (ny + 2) + 2 * (nx - 1);
+    for (int q = b * NT + (int)threadIdx.x; q < nu + nv; q += nb * NT) {
+        const bool isu = q < nu;
+        int r = isu ? q : q - nu, i, j;
+        const int ncol = isu ? 2 : 3;
+        if (r < ncol * (ny + 2)) {
+            const int c = r / (ny + 2);
+            j = r % (ny + 2);
+            i = isu ? (c == 0 ? 0 : nx + 1) : (c == 0 ? 0 : (c == 1 ? 1 : nx + 1));
+        } else {
+            r -= ncol * (ny + 2);
+            const int w = isu ? nx : nx - 1, c = r / w;
+            i = r % w + (isu ? 1 : 2);
+            j = isu ? (c == 0 ? 0 : (c == 1 ? 1 : ny + 1)) : (c == 0 ? 0 : ny + 1);
+        }
+        const size_t p = WD2_IX(i, j);
+        const double f = (isu ? F.us : F.vs)[p];
+        const bool add = i >= 1 && i <= nx && j >= 1 && j <= ny;
+        (isu ? F.uo : F.vo)[p] = add ? f + (isu ? F.dus : F.dvs)[p] : f;
+    }
+}
+
+static int ql_border_blocks(int nx, int ny, int nt) { return (5 * (nx + ny) + 8 * nt - 1) / (8 * nt); }
+
+// ------------------------------------------- bit-exact windows (FP64 path)
+// The speculative segmented Thomas sweep of k_trid.hip on a window: each lane
+// runs its 8 rows from the zero state and the fix-up rounds re-run them from
+// the predecessor's end state until nothing changes, so a window's rows are
+// those of a sequential sweep entered at its first row with the zero state.
+// The recurrences contract, so after H rows that sweep has met the chain's
+// own, bit for bit -- which is checked, not assumed: with the windows
+// overlapping by 4H rows, each pair of neighbours computes the same rows, and
+// equality of
+//   (c', b') of the first split H rows into a window with the predecessor's,
+//   x of the first split H rows before its end with the successor's,
+//   (c', b') of the second split 2H rows in with the predecessor's,
+//   x of the second split 2H rows before the end with the successor's
+// makes every kept row the sequential solve's: the first window starts at a
+// chain start, so by induction along the windows each forward state is exact
+// from its checked row on, and backwards from the last window each x is exact
+// up to its checked row.  Each window publishes the eight values it is
+// checked with and checks others with (chk); the fold compares them.
+//
+// H = 48: two runs of a recurrence meet bit for bit within 53 / log2(1/l)
+// rows for a contraction l per row, 48 rows for l <= 0.46, which a row with
+// |a| + |c| <= 0.76 |d| has.  (Halos of 32 and 64 rows keep 1920 and 1792 of
+// 2048 rows; 64 served stiffer chains, 32 failed the check at viscous numbers
+// the configurations use.)
+constexpr int QX_T = 256, QX_HL = 6, QX_H = QX_HL * TR_S, QX_N = QX_T * TR_S, QX_O = QX_N - 4 * QX_H;
+constexpr int QX_CHK = 12;
+
+template <typename T>
+struct QxShared {
+    // lanes' end states (2 x QX_T), neighbours' rows for the rounding-cycle
+    // test (8 x QX_T); at the end the increments
+    T buf[10 * QX_T];
+    unsigned long long ce[QX_T / 64], cyc[QX_T / 64];
+    unsigned char kint[QX_T];
+    int changed;
+    double red[2 * QX_T / 64];
+};
+static_assert(TR_P <= 10, "the increments fit the staging arrays");
+
+// Forward sweep of the workgroup's rows.  dn7: the diagonal of the row after
+// the lane's last (used where that row starts a chain).  After TR_ACC rounds
+// the rounding-cycle shortcut of k_trid.hip takes over.
+template <typename T>
+__device__ inline void qx_forward(unsigned kinds, const T (&a)[TR_S], const T (&d)[TR_S], const T (&c)[TR_S],
+                                  const T (&b)[TR_S], T dn7, T (&cp)[TR_S], T (&bp)[TR_S], QxShared<T> &S) {
+    const int t = threadIdx.x;
+    T *sc = S.buf, *sb = S.buf + QX_T, *pr = S.buf + 2 * QX_T;
+#define DNEXT(s) ((s) + 1 < TR_S ? d[((s) + 1) % TR_S] : dn7)
+    T cpv = T(0), bpv = T(0);
+#pragma unroll
+    for (int s = 0; s < TR_S; s++) {
+        fwd_row<T>(SKIND(kinds, s), a[s], d[s], c[s], b[s], DNEXT(s), cpv, bpv, cp[s], bp[s]);
+        cpv = cp[s];
+        bpv = bp[s];
+    }
+    const bool dep = t > 0 && SKIND(kinds, 0) != 1;
+    bool accel = false, cen = false;
+    int runlo = -1;
+    for (int round = 0; round <= QX_T; round++) {
+        sc[t] = cp[TR_S - 1];
+        sb[t] = bp[TR_S - 1];
+        if (t == 0) S.changed = 0;
+        if (accel) {
+            bool on = false;
+            if (cen) {
+                T c6, b6, c7, b7;
+                fwd_row<T>(0, a[6], d[6], c[6], b[6], T(1), cp[7], bp[7], c6, b6);
+                fwd_row<T>(0, a[7], d[7], c[7], b[7], T(1), c6, b6, c7, b7);
+                on = same(c7, cp[7]) && same(b7, bp[7]);
+            }
+            const unsigned long long m = __ballot(on);
+            if ((t & 63) == 0) S.cyc[t >> 6] = m;
+        }
+        __syncthreads();
+        if (dep) {
+            T sc0 = sc[t - 1], sb0 = sb[t - 1];
+            if (runlo >= 0) {
+                const int v = lowest_bit_in(S.cyc, runlo, t - 2);
+                if (v >= 0) { sc0 = sc[v]; sb0 = sb[v]; }
+            }
+            bool live = true;
+#pragma unroll
+            for (int s = 0; s < TR_S; s++) {
+                if (live) {
+                    T ck, bk;
+                    fwd_row<T>(SKIND(kinds, s), a[s], d[s], c[s], b[s], DNEXT(s), sc0, sb0, ck, bk);
+                    if (same(ck, cp[s]) && same(bk, bp[s])) {
+                        live = false;
+                    } else {
+                        cp[s] = ck; bp[s] = bk; sc0 = ck; sb0 = bk;
+                    }
+                }
+            }
+            if (live) S.changed = 1;
+        }
+        __syncthreads();
+        if (!S.changed) break;
+        if (round == TR_ACC) {
+            pr[t] = a[6]; pr[1 * QX_T + t] = d[6]; pr[2 * QX_T + t] = c[6]; pr[3 * QX_T + t] = b[6];
+            pr[4 * QX_T + t] = a[7]; pr[5 * QX_T + t] = d[7]; pr[6 * QX_T + t] = c[7]; pr[7 * QX_T + t] = b[7];
+            S.kint[t] = SKIND(kinds, 6) == 0 && SKIND(kinds, 7) == 0;
+            __syncthreads();
+            bool ce = kinds == 0u && t > 0 && S.kint[t - (t > 0)];
+#pragma unroll
+            for (int s = 2; s < TR_S; s++)
+                ce = ce && same(a[s], a[s - 2]) && same(d[s], d[s - 2]) && same(c[s], c[s - 2]) &&
+                     same(b[s], b[s - 2]);
+            const int q = t - (t > 0);
+            ce = ce && same(a[0], pr[q]) && same(d[0], pr[1 * QX_T + q]) && same(c[0], pr[2 * QX_T + q]) &&
+                 same(b[0], pr[3 * QX_T + q]) && same(a[1], pr[4 * QX_T + q]) && same(d[1], pr[5 * QX_T + q]) &&
+                 same(c[1], pr[6 * QX_T + q]) && same(b[1], pr[7 * QX_T + q]);
+            const unsigned long long m = __ballot(ce);
+            if ((t & 63) == 0) S.ce[t >> 6] = m;
+            __syncthreads();
+            cen = t + 1 < QX_T && bit_at(S.ce, t + 1);
+            if (t >= 2 && bit_at(S.ce, t - 1)) runlo = max(0, highest_clear_at_or_below(S.ce, t - 1));
+            accel = true;
+        }
+        __syncthreads();
+    }
+#undef DNEXT
+    __syncthreads();
+}
+
+// Back-substitution, with the zero value after the workgroup's last row.
+template <typename T>
+__device__ inline void qx_backward(unsigned kinds, const T (&cp)[TR_S], const T (&bp)[TR_S], T (&x)[TR_S],
+                                   QxShared<T> &S) {
+    const int t = threadIdx.x;
+    T *sc = S.buf, *pr = S.buf + 2 * QX_T;
+    T xn = T(0);
+#pragma unroll
+    for (int s = TR_S - 1; s >= 0; s--) {
+        x[s] = (SKIND(kinds, s) == 2) ? bp[s] : bp[s] - (cp[s] * xn);
+        xn = x[s];
+    }
+    const bool dep = t + 1 < QX_T && SKIND(kinds, TR_S - 1) != 2;
+    bool accel = false, cev = false;
+    int runhi = -1;
+    for (int round = 0; round <= QX_T; round++) {
+        sc[t] = x[0];
+        if (t == 0) S.changed = 0;
+        if (accel) {
+            bool on = false;
+            if (cev) {
+                const T y = bp[1] - (cp[1] * x[0]);
+                on = same(bp[0] - (cp[0] * y), x[0]);
+            }
+            const unsigned long long m = __ballot(on);
+            if ((t & 63) == 0) S.cyc[t >> 6] = m;
+        }
+        __syncthreads();
+        if (dep) {
+            T xv = sc[t + 1];
+            if (runhi >= 0) {
+                const int v = highest_bit_in(S.cyc, t + 2, runhi);
+                if (v >= 0) xv = sc[v];
+            }
+            bool live = true;
+#pragma unroll
+            for (int s = TR_S - 1; s >= 0; s--) {
+                if (live) {
+                    const T xk = (SKIND(kinds, s) == 2) ? bp[s] : bp[s] - (cp[s] * xv);
+                    if (same(xk, x[s])) live = false; else { x[s] = xk; xv = xk; }
+                }
+            }
+            if (live) S.changed = 1;
+        }
+        __syncthreads();
+        if (!S.changed) break;
+        if (round == TR_ACC) {
+            pr[t] = cp[0]; pr[1 * QX_T + t] = bp[0]; pr[2 * QX_T + t] = cp[1]; pr[3 * QX_T + t] = bp[1];
+            S.kint[t] = SKIND(kinds, 0) == 0 && SKIND(kinds, 1) == 0;
+            __syncthreads();
+            const int q = min(t + 1, QX_T - 1);
+            bool ce = kinds == 0u && t + 1 < QX_T && S.kint[q];
+#pragma unroll
+            for (int s = 0; s + 2 < TR_S; s++) ce = ce && same(cp[s], cp[s + 2]) && same(bp[s], bp[s + 2]);
+            ce = ce && same(cp[6], pr[q]) && same(bp[6], pr[1 * QX_T + q]) && same(cp[7], pr[2 * QX_T + q]) &&
+                 same(bp[7], pr[3 * QX_T + q]);
+            const unsigned long long m = __ballot(ce);
+            if ((t & 63) == 0) S.ce[t >> 6] = m;
+            __syncthreads();
+            cev = t >= 1 && bit_at(S.ce, t - 1);
+            if (t + 1 < QX_T && bit_at(S.ce, t + 1))
+                runhi = min(QX_T - 1, lowest_clear_at_or_above(S.ce, t + 1, QX_T));
+            accel = true;
+        }
+        __syncthreads();
+    }
+    __syncthreads();
+}
+
+template <typename T>
+__global__ __launch_bounds__(QX_T) void k_ql_exact(long n, Chains cs, ChainT<T> h1, ChainT<T> h2,
+                                                   const unsigned char *__restrict__ Z, QlFields F,
+                                                   double *__restrict__ part, T *__restrict__ chk, int nwin,
+                                                   const int *stop) {
+    if (*stop) return;
+    if ((int)blockIdx.x >= nwin) {
+        ql_border<QX_T>(F, (int)blockIdx.x - nwin, (int)gridDim.x - nwin);
+        return;
+    }
+    __shared__ QxShared<T> S;
+    const int t = threadIdx.x;
+    const long w0 = (long)blockIdx.x * QX_O - 2 * QX_H, k0 = w0 + (long)t * TR_S;
+    T *ck = chk + (size_t)blockIdx.x * QX_CHK;
+    T a[TR_S], d[TR_S], c[TR_S], b[TR_S], cp[TR_S], bp[TR_S];
+    ql_load(h1.a, k0, n, T(0), a);
+    ql_load(h1.d, k0, n, T(1), d);
+    ql_load(h1.c, k0, n, T(0), c);
+    ql_load(h1.b, k0, n, T(0), b);
+    const unsigned kinds = ql_kinds(k0, n, cs);
+    const unsigned idm = ql_ident(Z, k0, n);
+    const bool s7 = SKIND(kinds, TR_S - 1) == 1;   // a chain starts on the lane's last row
+    qx_forward<T>(kinds, a, d, c, b, s7 ? h1.d[k0 + TR_S] : T(1), cp, bp, S);
+    if (t == QX_HL - 1) { ck[0] = cp[7]; ck[1] = bp[7]; }
+    if (t == QX_T - 3 * QX_HL - 1) { ck[2] = cp[7]; ck[3] = bp[7]; }
+    // the second split's matrix arrives behind the back-substitution; lanes
+    // outside its window hold uncoupled rows
+    const bool in2 = t >= QX_HL && t < QX_T - QX_HL;
+    const long k2 = in2 ? k0 : n;
+    ql_load(h2.a, k2, n, T(0), a);
+    ql_load(h2.d, k2, n, T(1), d);
+    ql_load(h2.c, k2, n, T(0), c);
+    qx_backward<T>(kinds, cp, bp, b, S);
+    if (t == QX_T - QX_HL) ck[4] = b[0];
+    if (t == 3 * QX_HL) ck[5] = b[0];
+#pragma unroll
+    for (int s = 0; s < TR_S; s++)
+        if (!in2 || ((idm >> s) & 1u)) b[s] = T(0);
+    const unsigned kinds2 = in2 ? kinds : 0u;
+    qx_forward<T>(kinds2, a, d, c, b, in2 && s7 ? h2.d[k0 + TR_S] : T(1), cp, bp, S);
+    if (t == 2 * QX_HL - 1) { ck[6] = cp[7]; ck[7] = bp[7]; }
+    if (t == QX_T - 2 * QX_HL - 1) { ck[8] = cp[7]; ck[9] = bp[7]; }
+    qx_backward<T>(kinds2, cp, bp, b, S);
+    if (t == QX_T - 2 * QX_HL) ck[10] = b[0];
+    if (t == 2 * QX_HL) ck[11] = b[0];
+    T *X = S.buf;
+#pragma unroll
+    for (int s = 0; s < TR_S; s++) X[t * TR_P + s] = b[s];
+    __syncthreads();
+    ql_update<QX_T, T>(F, X, w0, 2 * QX_H, QX_N - 2 * QX_H, n, cs.n1, part, S.red);
+}
+
+// ------------------------------------------------ FP32 windows (mixed path)
+// The window solver of k_trid.hip (partitioned Thomas + PCR, halo TW_H) on
+// both splits, in the compute type CT: float for the iterations after the
+// first; double for the first iteration of a step, whose solve is the whole
+// update from time level n and can be the step's result (the chains are the
+// same FP32 rows, so their solve is then at least as accurate as the
+// sequential FP32 sweep's).  A window whose dominance ratio exceeds TW_DOM in
+// either split sets *weak, which the fold turns into a repeat of the
+// iteration with the bit-exact solver.
+template <typename CT>
+__device__ inline CT qrcp(CT x) {
+    if constexpr (std::is_same<CT, float>::value)
+        return wrcp(x);
+    else
+        return CT(1) / x;
+}
+template <typename CT>
+constexpr CT qeps() { return std::is_same<CT, float>::value ? CT(0x1p-48) : CT(0x1p-60); }
+
+template <typename CT, int NT>
+struct QwShared {
+    // interface rows of both PCR parities: sub- and super-diagonal, right-hand
+    // side, reciprocal diagonal (each 2 NT); at the end the increments
+    CT buf[16 * NT];
+    __device__ CT &a(int p, int i) { return buf[(0 + p) * 2 * NT + i]; }
+    __device__ CT &c(int p, int i) { return buf[(2 + p) * 2 * NT + i]; }
+    __device__ CT &b(int p, int i) { return buf[(4 + p) * 2 * NT + i]; }
+    __device__ CT &q(int p, int i) { return buf[(6 + p) * 2 * NT + i]; }
+    double red[2 * NT / 64];
+};
+
+// The window's solution x from its rows (overwritten: x in b).  lo, hi: the
+// lanes of the window; the coupling out of them is dropped.
+template <typename CT, int NT>
+__device__ inline void qw_solve(CT (&a)[TW_S], CT (&d)[TW_S], CT (&c)[TW_S], CT (&b)[TW_S], int lo, int hi,
+                                QwShared<CT, NT> &S) {
+    constexpr int M = 2 * NT;
+    const int t = threadIdx.x;
+    if (t == lo) a[0] = CT(0);
+    if (t == hi) c[TW_S - 1] = CT(0);
+    // interior rows through x0 and x7: y (particular), v (x0 spike), w (x7 spike)
+    CT cp[TW_S], y[TW_S], v[TW_S], w[TW_S];
+    {
+        CT q = qrcp(d[1]);
+        cp[1] = c[1] * q;
+        y[1] = b[1] * q;
+        v[1] = -a[1] * q;
+        w[1] = CT(0);
+#pragma unroll
+        for (int s = 2; s <= TW_S - 2; s++) {
+            q = qrcp(d[s] - a[s] * cp[s - 1]);
+            cp[s] = c[s] * q;
+            y[s] = (b[s] - a[s] * y[s - 1]) * q;
+            v[s] = -a[s] * v[s - 1] * q;
+            w[s] = ((s == TW_S - 2 ? -c[s] : CT(0)) - a[s] * w[s - 1]) * q;
+        }
+#pragma unroll
+        for (int s = TW_S - 3; s >= 1; s--) {
+            y[s] -= cp[s] * y[s + 1];
+            v[s] -= cp[s] * v[s + 1];
+            w[s] -= cp[s] * w[s + 1];
+        }
+    }
+    CT di[2];
+    {
+        const int i0 = 2 * t, i1 = 2 * t + 1;
+        di[0] = d[0] + c[0] * v[1];
+        di[1] = d[TW_S - 1] + a[TW_S - 1] * w[TW_S - 2];
+        S.a(0, i0) = a[0];
+        S.c(0, i0) = c[0] * w[1];
+        S.b(0, i0) = b[0] - c[0] * y[1];
+        S.q(0, i0) = qrcp(di[0]);
+        S.a(0, i1) = a[TW_S - 1] * v[TW_S - 2];
+        S.c(0, i1) = c[TW_S - 1];
+        S.b(0, i1) = b[TW_S - 1] - a[TW_S - 1] * y[TW_S - 2];
+        S.q(0, i1) = qrcp(di[1]);
+    }
+    __syncthreads();
+    int cur = 0;
+    for (int h = 1; h < M; h <<= 1) {
+        bool coupled = false;
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+            const int i = 2 * t + e;
+            const CT ai = S.a(cur, i), ci = S.c(cur, i), bi = S.b(cur, i);
+            CT an = CT(0), dn = di[e], cn = CT(0), bn = bi;
+            if (i - h >= 0) {
+                const CT k1 = ai * S.q(cur, i - h);
+                an = -S.a(cur, i - h) * k1;
+                dn -= S.c(cur, i - h) * k1;
+                bn -= S.b(cur, i - h) * k1;
+            }
+            if (i + h < M) {
+                const CT k2 = ci * S.q(cur, i + h);
+                cn = -S.c(cur, i + h) * k2;
+                dn -= S.a(cur, i + h) * k2;
+                bn -= S.b(cur, i + h) * k2;
+            }
+            di[e] = dn;
+            S.a(cur ^ 1, i) = an;
+            S.c(cur ^ 1, i) = cn;
+            S.b(cur ^ 1, i) = bn;
+            S.q(cur ^ 1, i) = qrcp(dn);
+            coupled |= !(fabs(an) + fabs(cn) <= qeps<CT>() * fabs(dn));
+        }
+        const int more = __syncthreads_or(coupled);
+        cur ^= 1;
+        if (!more) break;
+    }
+    const CT x0 = S.b(cur, 2 * t) * S.q(cur, 2 * t), x7 = S.b(cur, 2 * t + 1) * S.q(cur, 2 * t + 1);
+#pragma unroll
+    for (int s = 0; s < TW_S; s++) b[s] = s == 0 ? x0 : (s == TW_S - 1 ? x7 : y[s] + v[s] * x0 + w[s] * x7);
+    __syncthreads();   // the interface rows may be overwritten
+}
+
+// Chain starts (no sub-diagonal; the first-row quirk on the super-diagonal,
+// dn7 the diagonal of the row after the lane's last) and ends (no
+// super-diagonal), and the dominance test of the rows.
+template <typename CT>
+__device__ inline bool qw_rows(unsigned kinds, CT (&a)[TW_S], const CT (&d)[TW_S], CT (&c)[TW_S], CT dn7) {
+    bool weak = false;
+#pragma unroll
+    for (int s = 0; s < TW_S; s++) {
+        if (SKIND(kinds, s) == 1) {
+            a[s] = CT(0);
+            c[s] = c[s] * d[s] / (s + 1 < TW_S ? d[(s + 1) % TW_S] : dn7);
+        }
+        if (SKIND(kinds, s) == 2) c[s] = CT(0);
+        weak |= !(fabs(a[s]) + fabs(c[s]) <= CT(TW_DOM) * fabs(d[s]));
+    }
+    return weak;
+}
+
+template <typename CT, int NT>
+__global__ __launch_bounds__(NT) void k_ql_window(long n, Chains cs, ChainT<float> h1, ChainT<float> h2,
+                                                  const unsigned char *__restrict__ Z, QlFields F,
+                                                  double *__restrict__ part, int nwin, int *weakf, const int *stop) {
+    if (*stop) return;
+    if ((int)blockIdx.x >= nwin) {
+        ql_border<NT>(F, (int)blockIdx.x - nwin, (int)gridDim.x - nwin);
+        return;
+    }
+    constexpr int N = NT * TW_S, HL = TW_H / TW_S, O = N - 4 * TW_H;
+    __shared__ QwShared<CT, NT> S;
+    const int t = threadIdx.x;
+    const long w0 = (long)blockIdx.x * O - 2 * TW_H, k0 = w0 + (long)t * TW_S;
+    CT a[TW_S], d[TW_S], c[TW_S], b[TW_S];
+    ql_load(h1.a, k0, n, 0.f, a);
+    ql_load(h1.d, k0, n, 1.f, d);
+    ql_load(h1.c, k0, n, 0.f, c);
+    ql_load(h1.b, k0, n, 0.f, b);
+    const unsigned kinds = ql_kinds(k0, n, cs);
+    const unsigned idm = ql_ident(Z, k0, n);
+    // the second split's matrix, in flight during the first solve
+    const bool in2 = t >= HL && t < NT - HL;
+    const long k2 = in2 ? k0 : n;
+    float a2[TW_S], d2[TW_S], c2[TW_S];
+    ql_load(h2.a, k2, n, 0.f, a2);
+    ql_load(h2.d, k2, n, 1.f, d2);
+    ql_load(h2.c, k2, n, 0.f, c2);
+    const bool s7 = SKIND(kinds, TW_S - 1) == 1;
+    bool weak = qw_rows<CT>(kinds, a, d, c, s7 ? (CT)h1.d[k0 + TW_S] : CT(1));
+    qw_solve<CT, NT>(a, d, c, b, 0, NT - 1, S);
+#pragma unroll
+    for (int s = 0; s < TW_S; s++) {
+        a[s] = (CT)a2[s];
+        d[s] = (CT)d2[s];
+        c[s] = (CT)c2[s];
+        if (!in2 || ((idm >> s) & 1u)) b[s] = CT(0);
+    }
+    weak |= qw_rows<CT>(in2 ? kinds : 0u, a, d, c, in2 && s7 ? (CT)h2.d[k0 + TW_S] : CT(1));
+    if (__any(weak)) *weakf = 1;
+    qw_solve<CT, NT>(a, d, c, b, HL, NT - 1 - HL, S);
+    CT *X = S.buf;
+#pragma unroll
+    for (int s = 0; s < TW_S; s++) X[t * TR_P + s] = b[s];
+    __syncthreads();
+    ql_update<NT, CT>(F, X, w0, 2 * TW_H, N - 2 * TW_H, n, cs.n1, part, S.red);
+}
+
+// ------------------------------------------------------- fold, commit, host
+// The iteration's increment norms from the windows' maxima, whether its solve
+// is usable (exact windows: chk, the neighbours' shared rows agree bit for
+// bit; FP32 windows: no weak window), and the stopping test of iteration m
+// (momentum.f:182-188).
+template <typename T>
+__global__ __launch_bounds__(1024) void k_ql_fold_win(int ld, const double *__restrict__ dus,
+                                                      const double *__restrict__ dvs, const double *__restrict__ part,
+                                                      int nwin, const T *__restrict__ chk, int *weakf, Scalars *sc,
+                                                      double qtol, int m) {
+    if (sc->ql_stop) return;
+    __shared__ double sh[1024 / 64];
+    double r1 = 0.0, r2 = 0.0;
+    bool bad = false;
+    for (int w = threadIdx.x; w < nwin; w += 1024) {
+        r1 = dmaxf(r1, part[2 * w]);
+        r2 = dmaxf(r2, part[2 * w + 1]);
+        if (chk && w + 1 < nwin) {
+            const T *p = chk + (size_t)w * QX_CHK, *q = p + QX_CHK;
+            bad |= !(same(q[0], p[2]) && same(q[1], p[3]) && same(p[4], q[5]) && same(q[6], p[8]) &&
+                     same(q[7], p[9]) && same(p[10], q[11]));
+        }
+    }
+    if (!chk) bad = *weakf != 0;
+    const int anybad = __syncthreads_or(bad);
+    r1 = block_max<1024>(r1, sh, threadIdx.x);
+    r2 = block_max<1024>(r2, sh, threadIdx.x);
+    if (threadIdx.x == 0) {
+        if (anybad) {
+            sc->ql_stop = -1;
+            if (!chk) *weakf = 0;
+            return;
+        }
+        const double v0 = dmaxf(fabs(dus[WD2_IX(5, 5)]), r1), v1 = dmaxf(fabs(dvs[WD2_IX(5, 5)]), r2);
+        sc->val[0] = v0;
+        sc->val[1] = v1;
+        const double difmax = v0 > v1 ? v0 : v1;
+        if (difmax <= qtol) sc->ql_stop = m;
+    }
+}
+
+// After a captured loop of Q iterations: the iterate to (us, vs) where the
+// last iteration that ran left it in the other buffers (ua, va).
+__global__ __launch_bounds__(256) void k_ql_commit(int ld, int nx, int ny, int Q, const Scalars *sc,
+                                                   const double *__restrict__ ua, const double *__restrict__ va,
+                                                   double *__restrict__ us, double *__restrict__ vs) {
+    const int m = sc->ql_stop;
+    if (m < 0 || ((m > 0 ? m : Q) & 1) == 0) return;
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i > nx + 1) return;
+    const size_t k = WD2_IX(i, blockIdx.y);
+    us[k] = ua[k];
+    vs[k] = va[k];
+}
+void launch_ql_commit(int nx, int ny, int ld, int Q, const Scalars *sc, const double *ua, const double *va, double *us,
+                      double *vs, hipStream_t s) {
+    hipLaunchKernelGGL(k_ql_commit, dim3((nx + 2 + 255) / 256, ny + 2), dim3(256), 0, s, ld, nx, ny, Q, sc, ua, va, us,
+                       vs);
+}
+
+// Windows of the smallest shape (the most there are), and the doubles the
+// windows' maxima and checks take.
+size_t ql_pair_part(long n) { return 2 * (size_t)((n + 767) / 768); }
+size_t ql_pair_chk(long n) { return QX_CHK * (size_t)((n + QX_O - 1) / QX_O); }
+
+void launch_ql_pair(const QlPair<double> &q, long n, const Chains &cs, const ChainT<double> &h1,
+                    const ChainT<double> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m, hipStream_t s) {
+    const QlFields F{q.nx, q.ny, q.ld, q.us, q.vs, q.uo, q.vo, q.dus, q.dvs};
+    const int nw = (int)((n + QX_O - 1) / QX_O), nb = ql_border_blocks(q.nx, q.ny, QX_T);
+    hipLaunchKernelGGL(k_ql_exact<double>, dim3(nw + nb), dim3(QX_T), 0, s, n, cs, h1, h2, Z, F, q.part, q.chk, nw,
+                       &sc->ql_stop);
+    hipLaunchKernelGGL(k_ql_fold_win<double>, dim3(1), dim3(1024), 0, s, q.ld, q.dus, q.dvs, q.part, nw,
+                       (const double *)q.chk, (int *)nullptr, sc, qtol, m);
+}
+
+template <typename CT, int NT>
+static void ql_window_as(const QlPair<float> &q, long n, const Chains &cs, const ChainT<float> &h1,
+                         const ChainT<float> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m,
+                         hipStream_t s) {
+    constexpr int O = NT * TW_S - 4 * TW_H;
+    const QlFields F{q.nx, q.ny, q.ld, q.us, q.vs, q.uo, q.vo, q.dus, q.dvs};
+    const int nw = (int)((n + O - 1) / O), nb = ql_border_blocks(q.nx, q.ny, NT);
+    hipLaunchKernelGGL((k_ql_window<CT, NT>), dim3(nw + nb), dim3(NT), 0, s, n, cs, h1, h2, Z, F, q.part, nw,
+                       &sc->ql_weak, &sc->ql_stop);
+    hipLaunchKernelGGL(k_ql_fold_win<float>, dim3(1), dim3(1024), 0, s, q.ld, q.dus, q.dvs, q.part, nw,
+                       (const float *)nullptr, &sc->ql_weak, sc, qtol, m);
+}
+void launch_ql_pair(const QlPair<float> &q, long n, const Chains &cs, const ChainT<float> &h1,
+                    const ChainT<float> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m, hipStream_t s) {
+    if (m == 1) {
+        ql_window_as<double, 256>(q, n, cs, h1, h2, Z, sc, qtol, m, s);
+        return;
+    }
+    switch (q.shape) {
+    case 128: ql_window_as<float, 128>(q, n, cs, h1, h2, Z, sc, qtol, m, s); break;
+    case 512: ql_window_as<float, 512>(q, n, cs, h1, h2, Z, sc, qtol, m, s); break;
+    default: ql_window_as<float, 256>(q, n, cs, h1, h2, Z, sc, qtol, m, s); break;
+    }
+}
+
+}  // namespace wd2

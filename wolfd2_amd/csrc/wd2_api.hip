@@ -80,6 +80,13 @@ struct wd2_ctx {
     double *store = nullptr;
     double *u, *v, *p, *un, *vn, *pn, *us, *vs, *dus, *dvs, *d, *dn, *div, *rhs, *beff, *pscr;
     double *t, *tn, *ts, *qh;      // temperature levels and the filter's copy
+    // the q-l loop's other iterate buffers (an iteration's fused solve reads
+    // us, vs and writes ua, va, or the reverse), the windows' maxima and
+    // checks, and the steps for which the loop keeps the separate solvers
+    // after a fused solve was not usable
+    double *ua, *va;
+    double *ql_part = nullptr;
+    int ql_hold = 0;
     // ThermEnergy's face coefficients: buffers of their own, since the mixed
     // path's FP32 momentum temporaries alias the FP64 ones and read the
     // entries they never write as zero
@@ -147,6 +154,8 @@ struct wd2_ctx {
         wd2_params P;
         int epoch;
         int xp, xw;   // the extrapolated start's order (0: plain start) and history slot
+        const double *us;   // u, us and ua share three buffers
+        bool fused;         // the q-l loop's solver
         hipGraphExec_t exec;
     };
     bool graph_on = false;
@@ -239,6 +248,7 @@ static void ctx_free(wd2_ctx *c) {
     if (c->h_sc) (void)hipHostFree(c->h_sc);
     (void)hipFree(c->tw.cp);
     (void)hipFree(c->zm);
+    (void)hipFree(c->ql_part);
     if (c->s) (void)hipStreamDestroy(c->s);
     delete c;
 }
@@ -265,7 +275,7 @@ static int ctx_alloc(wd2_ctx **out, int nx, int ny) {
                              hipHostMallocDefault));
         HIPCHK(hipEventCreateWithFlags(&c->sev[k], hipEventDisableTiming));
     }
-    const int NFIELDS = 16 + 4 + 4 + 5 + 15;
+    const int NFIELDS = 16 + 4 + 2 + 4 + 5 + 15;
     const size_t nchain = chain_rows(nx, ny);
     const size_t total = NFIELDS * c->nf + 10 * nchain;
     HIPCHK(hipMalloc(&c->store, total * sizeof(double)));
@@ -273,7 +283,7 @@ static int ctx_alloc(wd2_ctx **out, int nx, int ny) {
     double *q = c->store;
     auto take = [&](size_t n) { double *r = q; q += n; return r; };
     double **f[] = {&c->u, &c->v, &c->p, &c->un, &c->vn, &c->pn, &c->us, &c->vs, &c->dus, &c->dvs,
-                    &c->d, &c->dn, &c->div, &c->rhs, &c->beff, &c->pscr, &c->t, &c->tn, &c->ts, &c->qh};
+                    &c->d, &c->dn, &c->div, &c->rhs, &c->beff, &c->pscr, &c->t, &c->tn, &c->ts, &c->qh, &c->ua, &c->va};
     for (double **pp : f) *pp = take(c->nf);
     c->tt = ThermTemps{take(c->nf), take(c->nf), take(c->nf), take(c->nf)};
     for (int k = 0; k < 5; k++) c->pc[k] = take(c->nf);
@@ -288,6 +298,7 @@ static int ctx_alloc(wd2_ctx **out, int nx, int ny) {
     c->ch.x = take(nchain);
     c->ch2 = Chain{take(nchain), take(nchain), take(nchain), take(nchain), take(nchain)};
     HIPCHK(hipMalloc(&c->zm, nchain));
+    HIPCHK(hipMalloc(&c->ql_part, (ql_pair_part((long)nchain) + ql_pair_chk((long)nchain)) * sizeof(double)));
     const int nb = trid_blocks((long)nchain) + 2;
     HIPCHK(hipMalloc(&c->tw.cp, (2 * nchain + 4 * nb) * sizeof(double) + 4 * sizeof(int) + 64));
     c->tw.bp = c->tw.cp + nchain;
@@ -613,9 +624,13 @@ static int momentum(wd2_ctx *c, int comp, double dk, double re, double fr, const
 // Iteration m's kernels return at entry once an earlier iteration has met
 // qtol (sc->ql_stop != 0), and its fold sets sc->ql_stop = m when it does, so
 // the host can queue iteration m before it reads iteration m-1's test.
+//
+// uo, vo: where the fused solve and update (launch_ql_pair) leave the next
+// iterate; null: the separate solvers update us, vs in place.
 template <typename T>
 static void momentum_pair(wd2_ctx *c, double dk, double re, double fr, const MomTempsT<T> &t, const ChainT<T> &ch,
-                          const ChainT<T> &ch2, const TridWorkT<T> &tw, int m, double qtol) {
+                          const ChainT<T> &ch2, const TridWorkT<T> &tw, int m, double qtol, double *us, double *vs,
+                          double *uo, double *vo) {
     const bool n_ready = m > 1;
     const int *stop = &c->sc->ql_stop;
     const int nx = c->nx, ny = c->ny, ld = c->ld;
@@ -631,31 +646,38 @@ static void momentum_pair(wd2_ctx *c, double dk, double re, double fr, const Mom
         launch_mom_n<T>(nx, ny, ld, 1, M, c->un, c->vn, t.cnvn, t.difn, s);
         launch_mom_n<T>(nx, ny, ld, 2, M, c->un, c->vn, t2.cnvn, t2.difn, s);
     }
-    launch_mom_asm_pair<T>(c->R, ld, dk, re, fr, M, t, t2, c->us, c->vs, c->un, c->vn, c->d, c->dn, ch, ch2, c->zm,
+    launch_mom_asm_pair<T>(c->R, ld, dk, re, fr, M, t, t2, us, vs, c->un, c->vn, c->d, c->dn, ch, ch2, c->zm,
                            shift(ch, n1), shift(ch2, n1), c->zm + n1, s, &c->sc->err, live, stop);
     const Chains cs{n1, n1, n2};
-    if constexpr (std::is_same<T, float>::value) {
-        // The window solver serves iterations 2.. of the q-l loop.  The first
-        // iteration's solve is the whole update from time level n and may be
-        // the step's result (the test after one iteration can be met, as on
-        // the first step from rest), so it takes the sequential solver.  Per
-        // solve the two have errors of one size, but on a 1024^2 cavity from
-        // rest the window solver in the first iteration leaves v 1.3e-6 from
-        // the FP64 path after two steps (relative L2), against 2.8e-7 this way.
-        if (g_window_chains && m > 1) {
-            launch_trid_window<T>(tw, n1 + n2, cs, ch.a, ch.d, ch.c, ch.b, ch.x, s, ch2.b, c->zm, stop, c->win_wt);
-            launch_trid_window<T>(tw, n1 + n2, cs, ch2.a, ch2.d, ch2.c, ch2.b, ch2.x, s, nullptr, nullptr, stop,
-                                  c->win_wt);
-        } else {
-            launch_trid<T>(tw, n1 + n2, cs, ch.a, ch.d, ch.c, ch.b, ch.x, s, ch2.b, c->zm, stop);
-            launch_trid<T>(tw, n1 + n2, cs, ch2.a, ch2.d, ch2.c, ch2.b, ch2.x, s, nullptr, nullptr, stop);
-        }
-    } else {
-        launch_trid<T>(tw, n1 + n2, cs, ch.a, ch.d, ch.c, ch.b, ch.x, s, ch2.b, c->zm, stop);
-        launch_trid<T>(tw, n1 + n2, cs, ch2.a, ch2.d, ch2.c, ch2.b, ch2.x, s, nullptr, nullptr, stop);
+    if (uo) {
+        const QlPair<T> q{nx,     ny,     ld,         us, vs, uo, vo, c->dus,
+                          c->dvs, c->ql_part, (T *)(c->ql_part + ql_pair_part(n1 + n2)), c->win_wt};
+        launch_ql_pair(q, n1 + n2, cs, ch, ch2, c->zm, c->sc, qtol, m, s);
+        return;
     }
-    launch_scatter_update<T>(nx, ny, ld, ch2.x, ch2.x + n1, c->us, c->vs, c->dus, c->dvs, c->partials, c->sc, qtol,
-                             m, s);
+    launch_trid<T>(tw, n1 + n2, cs, ch.a, ch.d, ch.c, ch.b, ch.x, s, ch2.b, c->zm, stop);
+    launch_trid<T>(tw, n1 + n2, cs, ch2.a, ch2.d, ch2.c, ch2.b, ch2.x, s, nullptr, nullptr, stop);
+    launch_scatter_update<T>(nx, ny, ld, ch2.x, ch2.x + n1, us, vs, c->dus, c->dvs, c->partials, c->sc, qtol, m, s);
+}
+static void momentum_pair(wd2_ctx *c, double dk, double re, double fr, int m, double qtol, double *us, double *vs,
+                          double *uo, double *vo) {
+    if (c->precision == WD2_PREC_MIXED)
+        momentum_pair<float>(c, dk, re, fr, c->Tf, c->chf, c->chf2, c->twf, m, qtol, us, vs, uo, vo);
+    else
+        momentum_pair<double>(c, dk, re, fr, c->T, c->ch, c->ch2, c->tw, m, qtol, us, vs, uo, vo);
+}
+
+// Whether a q-l loop uses the fused solve and update: FP64 always (the same
+// bits), the mixed path unless its window solver is switched off -- and not
+// for the QL_HOLD steps after a step in which it was not usable (weakly
+// dominant chains, or runs that did not meet within the windows' halos): such
+// chains change slowly, and a repeat costs an iteration.
+constexpr int QL_HOLD = 16;
+static bool ql_fused(const wd2_ctx *c) {
+    return c->ql_hold == 0 && (c->precision != WD2_PREC_MIXED || g_window_chains);
+}
+static void ql_step_done(wd2_ctx *c) {
+    if (c->ql_hold > 0) c->ql_hold--;
 }
 
 static int momentum(wd2_ctx *c, int comp, double dk, double re, double fr, const double *us, const double *vs,
@@ -684,24 +706,51 @@ static int naux_momentum(wd2_ctx *c, int mqiter, double dk, double re, double fr
         hipStream_t s = c->s;
         const int *stop = &c->sc->ql_stop;
         launch_ql_reset(c->sc, s);
+        // fused iterations alternate between (us, vs) and (ua, va): iteration
+        // m reads buffer (m - 1) % 2
+        bool fused = ql_fused(c);
+        double *const ub[2] = {c->us, c->ua}, *const vb[2] = {c->vs, c->va};
+        bool filled = false;   // iteration m's outflow fills are already applied
         int m = 1, last = 0;   // last: the iteration whose test was read last
-        for (; m <= mqiter; m++) {
-            if (c->any_outlet) launch_vel_bc<double>(c->R, ld, c->us, c->vs, true, &c->sc->err, s, stop);
-            if (c->precision == WD2_PREC_MIXED)
-                momentum_pair<float>(c, dk, re, fr, c->Tf, c->chf, c->chf2, c->twf, m, qtol);
-            else
-                momentum_pair<double>(c, dk, re, fr, c->T, c->ch, c->ch2, c->tw, m, qtol);
-            HIPCHK(hipMemcpyAsync(&c->h_flag[2 + m % 2], &c->sc->ql_stop, sizeof(int), hipMemcpyDeviceToHost, s));
-            HIPCHK(hipEventRecord(c->qev[m % 2], s));
-            if (m >= 2) {
-                HIPCHK(hipEventSynchronize(c->qev[(m - 1) % 2]));
-                last = m - 1;
-                if (c->h_flag[2 + last % 2]) break;
+        for (;; m++) {
+            for (; m <= mqiter; m++) {
+                const int in = fused ? (m - 1) % 2 : 0;
+                double *const us = fused ? ub[in] : c->us, *const vs = fused ? vb[in] : c->vs;
+                if (c->any_outlet && !filled) launch_vel_bc<double>(c->R, ld, us, vs, true, &c->sc->err, s, stop);
+                filled = false;
+                momentum_pair(c, dk, re, fr, m, qtol, us, vs, fused ? ub[in ^ 1] : nullptr,
+                              fused ? vb[in ^ 1] : nullptr);
+                HIPCHK(hipMemcpyAsync(&c->h_flag[2 + m % 2], &c->sc->ql_stop, sizeof(int), hipMemcpyDeviceToHost, s));
+                HIPCHK(hipEventRecord(c->qev[m % 2], s));
+                if (m >= 2 && last < m - 1) {
+                    HIPCHK(hipEventSynchronize(c->qev[(m - 1) % 2]));
+                    last = m - 1;
+                    if (c->h_flag[2 + last % 2]) break;
+                }
             }
+            if (m > mqiter && last < mqiter) {
+                HIPCHK(hipEventSynchronize(c->qev[mqiter % 2]));
+                last = mqiter;
+            }
+            if (c->h_flag[2 + last % 2] >= 0) break;
+            // iteration `last` is to be repeated on its unchanged input
+            // (whose outflow fills are applied) with the separate solvers,
+            // which the rest of the loop keeps
+            HIPCHK(hipStreamSynchronize(s));
+            launch_ql_reset(c->sc, s);
+            const int in = (last - 1) % 2;
+            c->us = ub[in]; c->ua = ub[in ^ 1];
+            c->vs = vb[in]; c->va = vb[in ^ 1];
+            fused = false;
+            filled = true;
+            c->ql_hold = QL_HOLD + 1;   // this step included
+            m = last - 1;
+            last = m;
         }
-        if (m > mqiter) {
-            HIPCHK(hipEventSynchronize(c->qev[mqiter % 2]));
-            last = mqiter;
+        if (fused) {   // the iterate is where the last iteration that ran left it
+            const int end = last % 2;
+            c->us = ub[end]; c->ua = ub[end ^ 1];
+            c->vs = vb[end]; c->va = vb[end ^ 1];
         }
         if (c->h_flag[2 + last % 2]) *nql = c->h_flag[2 + last % 2];
         return check_err(c);
@@ -1229,6 +1278,7 @@ static int one_step(wd2_ctx *c, const wd2_params *P, int *nql, int *nsor, double
     if (therm) launch_max_norm(nx, ny, ld, c->tn, c->t, c->partials + 3 * RED_MAX_BLOCKS, c->sc, 5, s);
     if (dif) HIPCHK(hipMemcpyAsync(dif, &c->sc->val[2], (therm ? 4 : 3) * sizeof(double), hipMemcpyDeviceToHost, s));
     extrap_advance(c, xp);
+    ql_step_done(c);
     return check_err(c);
 }
 
@@ -1252,7 +1302,7 @@ static bool graph_ok(const wd2_ctx *c, const wd2_params *P) {
 
 // The step's work on the stream (the body of a capture): main.f:690-972 with
 // Q q-l iterations and C V-cycles queued.
-static void step_body(wd2_ctx *c, const wd2_params *P, int Q, int C, int xp) {
+static void step_body(wd2_ctx *c, const wd2_params *P, int Q, int C, int xp, bool fused) {
     const int nx = c->nx, ny = c->ny, ld = c->ld;
     hipStream_t s = c->s;
     const wd2_step_options &O = c->opt;
@@ -1274,13 +1324,14 @@ static void step_body(wd2_ctx *c, const wd2_params *P, int Q, int C, int xp) {
     }
     const int *stop = &c->sc->ql_stop;
     launch_ql_reset(c->sc, s);
+    double *const ub[2] = {c->us, c->ua}, *const vb[2] = {c->vs, c->va};
     for (int m = 1; m <= Q; m++) {
-        if (c->any_outlet) launch_vel_bc<double>(c->R, ld, c->us, c->vs, true, &c->sc->err, s, stop);
-        if (c->precision == WD2_PREC_MIXED)
-            momentum_pair<float>(c, P->dk, P->re, P->fr, c->Tf, c->chf, c->chf2, c->twf, m, P->qtol);
-        else
-            momentum_pair<double>(c, P->dk, P->re, P->fr, c->T, c->ch, c->ch2, c->tw, m, P->qtol);
+        const int in = fused ? (m - 1) % 2 : 0;
+        if (c->any_outlet) launch_vel_bc<double>(c->R, ld, ub[in], vb[in], true, &c->sc->err, s, stop);
+        momentum_pair(c, P->dk, P->re, P->fr, m, P->qtol, ub[in], vb[in], fused ? ub[in ^ 1] : nullptr,
+                      fused ? vb[in ^ 1] : nullptr);
     }
+    if (fused) launch_ql_commit(nx, ny, ld, Q, c->sc, c->ua, c->va, c->us, c->vs, s);
     if (O.nfiltu == 1) launch_filter(c->R, c->TH, ld, VU, O.fpu, c->us, c->qh, s);
     if (O.nfiltv == 1) launch_filter(c->R, c->TH, ld, VV, O.fpv, c->vs, c->qh, s);
     launch_fills(c->R, ld, c->us, c->vs, c->p, 1, &c->sc->err, s);
@@ -1323,15 +1374,16 @@ static int graph_begin(wd2_ctx *c, const wd2_params *P) {
     if (!c->h_sc) HIPCHK(hipHostMalloc((void **)&c->h_sc, sizeof(Scalars), hipHostMallocDefault));
     const int Q = std::min(P->mqiter, c->ql_last + 2);
     const int C = std::min(P->msorit + 1, c->mg_last + 2);
+    const bool fused = ql_fused(c);
     hipGraphExec_t exec = nullptr;
     for (auto &g : c->graphs)
         if (g.q == Q && g.cyc == C && g.u == c->u && g.epoch == g_graph_epoch && g.xp == xp && g.xw == c->xw &&
-            std::memcmp(&g.P, P, sizeof(wd2_params)) == 0)
+            g.us == c->us && g.fused == fused && std::memcmp(&g.P, P, sizeof(wd2_params)) == 0)
             exec = g.exec;
     if (!exec) {
         hipGraph_t graph = nullptr;
         HIPCHK(hipStreamBeginCapture(c->s, hipStreamCaptureModeThreadLocal));
-        step_body(c, P, Q, C, xp);
+        step_body(c, P, Q, C, xp, fused);
         const hipError_t ec = hipStreamEndCapture(c->s, &graph);
         if (ec != hipSuccess) return fail(WD2_ERR_HIP, "step capture: %s", hipGetErrorString(ec));
         const hipError_t ei = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
@@ -1341,7 +1393,7 @@ static int graph_begin(wd2_ctx *c, const wd2_params *P) {
             (void)hipGraphExecDestroy(c->graphs.front().exec);
             c->graphs.erase(c->graphs.begin());
         }
-        c->graphs.push_back({Q, C, c->u, *P, g_graph_epoch, xp, c->xw, exec});
+        c->graphs.push_back({Q, C, c->u, *P, g_graph_epoch, xp, c->xw, c->us, fused, exec});
     }
     HIPCHK(hipGraphLaunch(exec, c->s));
     c->g_q = Q;
@@ -1354,7 +1406,8 @@ static int graph_end(wd2_ctx *c, const wd2_params *P, int *nql, int *nsor, doubl
     HIPCHK(hipStreamSynchronize(c->s));
     const Scalars h = *c->h_sc;
     if (h.err) return check_err(c);
-    const bool ql_short = h.ql_stop == 0 && c->g_q < P->mqiter;
+    // (a fused solve that was not usable counts as a budget that ran out)
+    const bool ql_short = h.ql_stop < 0 || (h.ql_stop == 0 && c->g_q < P->mqiter);
     const bool mg_short = h.mg_done == 0;
     if (ql_short || mg_short) {
         // a budget ran out: restore the step's start and redo it host-driven
@@ -1371,6 +1424,7 @@ static int graph_end(wd2_ctx *c, const wd2_params *P, int *nql, int *nsor, doubl
     std::swap(c->u, c->us);
     std::swap(c->v, c->vs);
     extrap_advance(c, c->g_x);
+    ql_step_done(c);
     *nql = h.ql_stop ? h.ql_stop : -1;
     int nconv = h.mg_nconv;
     c->mg_div = h.val[7];
@@ -2087,6 +2141,7 @@ int wd2_naux_momentum(int nx, int ny, int ld, int mgri, int mgrj, int mqiter, co
     launch_fill(c->ld, 0, nx + 1, 0, ny + 1, 0.0, c->dvs, c->s);
     int nql = -1;
     if ((st = naux_momentum(c, mqiter, dk, re, fr, qtol, &nql))) return st;
+    ql_step_done(c);
     if (nQLiter) *nQLiter = nql;
     if ((st = down(c, c->us, us, ld)) || (st = down(c, c->vs, vs, ld))) return st;
     HIPCHK(hipStreamSynchronize(c->s));

@@ -77,11 +77,12 @@ struct Scalars {
     double sor_dif;
     int err;                       // bad-flag code from a kernel (0 = none)
     int redo_launch, redo_sweeps;  // temporally blocked SOR: launch to redo, sweeps to keep
-    int ql_stop;                   // q-l iteration that met qtol (0 = none yet)
+    int ql_stop;                   // q-l iteration that met qtol (0 = none yet; -1: repeat the iteration)
     int mg_done;                   // multigrid solve stopped
     int mg_nconv;                  // V-cycles applied when it converged, -1 not converged
     int mg_cycles;                 // V-cycles applied so far
-    int pad1[9];
+    int ql_weak;                   // a window of the FP32 chain solve is too weakly dominant
+    int pad1[8];
 };
 
 constexpr int RED_MAX_BLOCKS = 4096;   // partial-maximum slots per reduction
@@ -187,6 +188,31 @@ struct ChainT {
 };
 using MomTemps = MomTempsT<double>;
 using Chain = ChainT<double>;
+// One q-l iteration's chain solves (both splits of both components, k_ql.hip)
+// and its update (us, vs) -> (uo, vo) in one launch, then the fold: DMaxNorm of
+// the increments, and sc->ql_stop = m once they meet qtol or -1 when the solve
+// is not usable (the iteration is then to be repeated with launch_trid on the
+// unchanged us, vs).  h1, h2: the splits' chains as launch_mom_asm_pair leaves
+// them (h2.b unused); part: ql_pair_part(n) doubles; chk (FP64):
+// ql_pair_chk(n); shape (FP32): lanes per window.
+template <typename T>
+struct QlPair {
+    int nx, ny, ld;
+    const double *us, *vs;
+    double *uo, *vo, *dus, *dvs;
+    double *part;
+    T *chk;
+    int shape;
+};
+size_t ql_pair_part(long n);
+size_t ql_pair_chk(long n);
+void launch_ql_pair(const QlPair<double> &q, long n, const Chains &cs, const ChainT<double> &h1,
+                    const ChainT<double> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m, hipStream_t s);
+void launch_ql_pair(const QlPair<float> &q, long n, const Chains &cs, const ChainT<float> &h1,
+                    const ChainT<float> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m, hipStream_t s);
+// us, vs = ua, va if the last of Q captured iterations that ran was odd.
+void launch_ql_commit(int nx, int ny, int ld, int Q, const Scalars *sc, const double *ua, const double *va, double *us,
+                      double *vs, hipStream_t s);
 // metric f of a Metrics m with its box
 #define MARR(m, f) (MArr{(m).f, (m).box[MI_##f]})
 template <typename T>
