@@ -29,10 +29,20 @@
 //   0, 1 down; 1, 0 up); restriction: the sum of a coarse cell's children;
 //   prolongation: bilinear (9, 3, 3, 1) / 16 from the coarse cell and its
 //   neighbours, zero outside the grid;
-// * levels wider than 64 cells run as LDS tiles, one launch per level down
-//   (smooth, residual, restrict) and one up (prolong, smooth); the levels of
-//   at most 64 x 64 cells run in one workgroup (the bottom kernel, e and r in
-//   LDS), down to a grid of at most 2 x 2 cells solved by 6 sweeps.
+// * the wider levels run as 64 x 64 tiles, one launch per level down (smooth,
+//   residual, restrict) and one up (prolong, smooth); the levels of at most
+//   64 cells a side (32 in FP64) run in one workgroup (the bottom kernel), and
+//   from the first level of at most 64 cells in all the rest of the V-cycle
+//   is one product with its matrix, built with the coefficients.
+//
+// A level or tile is held in registers (SPt below): a lane keeps a strip of
+// four rows of one column, so a colour's update reads three of its four
+// neighbours by lane shifts and from its own registers, and only the two rows
+// at a strip's ends cross through LDS.  The smoothing phases are latency (a
+// barrier and a few dependent operations each): with the points in LDS and a
+// point update of four loads and a division, a phase took 0.35 (a 44 x 44
+// tile) to 0.9 us (a 64 x 64 bottom level); here about 0.15.  Launches on the
+// 1024^2 cavity (FP32 / FP64): @FIGS@
 //
 // The down kernel of level 0 also reduces max |r| per tile; every workgroup
 // of the next kernel evaluates the stopping test from those maxima (every
@@ -45,19 +55,19 @@
 namespace wd2 {
 
 constexpr int MG_NU = 2;                       // smoothing sweeps before and after
-constexpr int MG_OT = 32;                      // owned cells per tile side
+constexpr int MG_TW = 64;                      // tile side, one column per lane
+constexpr int MG_SR = 4;                       // rows per strip
+constexpr int MG_NS = MG_TW / MG_SR;           // strips of a tile
+constexpr int MG_NT = 64 * MG_NS;              // threads of a tile workgroup
 constexpr int MG_HD = 2 * MG_NU + 2;           // down halo (2 NU + 1, even)
 constexpr int MG_HU = 2 * MG_NU;               // up halo
-constexpr int MG_TD = MG_OT + 2 * MG_HD;       // down tile side (44)
-constexpr int MG_TU = MG_OT + 2 * MG_HU;       // up tile side (40)
-constexpr int MG_TC = MG_TU / 2 + 2;           // coarse cells of the up tile (22)
-constexpr int MG_NT1 = 1024;                   // threads of a coarser tile workgroup (few tiles: latency)
-constexpr int MG_BSIDE = 64;                   // widest level the bottom kernel can hold
-constexpr int MG_BT = 1024;                    // threads of the bottom workgroup
-constexpr int MG_BCAP = 6400;                  // LDS cells per array (e, r) of the bottom levels
+constexpr int MG_OD = MG_TW - 2 * MG_HD;       // owned cells per tile side, down (52)
+constexpr int MG_OU = MG_TW - 2 * MG_HU;       // up (56)
+constexpr int MG_TAIL = 64;                    // cells of the widest level the tail matrix covers
 constexpr int MG_NCOARSE = 6;                  // sweeps on the coarsest grid (at most 2 x 2 cells)
-constexpr int MG_NC = (MG_OT / 2) * (MG_OT / 2);   // coarse cells of a tile
-static_assert(MG_HD % 2 == 0 && MG_HU % 2 == 0, "even halos keep the tile colours global");
+constexpr int MG_NREG = 3;                     // bottom levels wider than the tail, at most
+static_assert(MG_HD % 2 == 0 && MG_HU % 4 == 0 && MG_OD % 2 == 0 && MG_OU % 4 == 0,
+              "even tile origins keep the colours global; the up strips start on coarse row pairs");
 
 // Level arrays (elements of T): cell (I, J), 0-based, at (I+1) + ld (J+1),
 // with a zero ring (e, r, c); x-face west of cell I (I = 0..nx) at
@@ -102,73 +112,6 @@ __global__ void k_mg_coarsen(MgLevel F, MgLevel C, T sb) {
         v = v / (T)n;
         if (J == 0 || J == C.ny) v *= sb;
         cy[mfy(C.ld, I, J)] = v;
-    }
-}
-
-// ------------------------------------------------------------ tile helpers
-// One colour of a red-black Gauss-Seidel sweep on an LDS tile of side TW
-// (E, R: TW x TW; AX: TW rows of TW + 1 x-faces; AY: TW + 1 rows of TW
-// y-faces).  Updated: points off the tile's outer ring, inside the grid.
-template <typename T, int TW, int NT>
-__device__ inline void tile_colour(T *E, const T *R, const T *AX, const T *AY, int c, int gx0, int gy0, int NX,
-                                   int NY) {
-    constexpr int KW = TW / 2;
-    for (int h = threadIdx.x; h < TW * KW; h += NT) {
-        const int y = h / KW, x = 2 * (h % KW) + ((c ^ y) & 1);
-        const int I = gx0 + x, J = gy0 + y;
-        if (x < 1 || x > TW - 2 || y < 1 || y > TW - 2 || I < 0 || I >= NX || J < 0 || J >= NY) continue;
-        const T aw = AX[y * (TW + 1) + x], ae = AX[y * (TW + 1) + x + 1];
-        const T as = AY[y * TW + x], an = AY[(y + 1) * TW + x];
-        const T a3 = -(aw + ae + as + an);
-        const int q = y * TW + x;
-        E[q] = (R[q] - (as * E[q - TW] + aw * E[q - 1] + ae * E[q + 1] + an * E[q + TW])) / a3;
-    }
-}
-
-template <typename T, int TW>
-__device__ inline T tile_res(const T *E, const T *R, const T *AX, const T *AY, int x, int y) {
-    const T aw = AX[y * (TW + 1) + x], ae = AX[y * (TW + 1) + x + 1];
-    const T as = AY[y * TW + x], an = AY[(y + 1) * TW + x];
-    const int q = y * TW + x;
-    const T a3 = -(aw + ae + as + an);
-    return R[q] - (as * E[q - TW] + aw * E[q - 1] + a3 * E[q] + ae * E[q + 1] + an * E[q + TW]);
-}
-
-// The same two on a level whose faces all hold one x value ax and one y value
-// ay (level 0 of a uniform Cartesian grid: rau and rgv are constants, and the
-// faces to the frozen ghosts carry them too), with ia3 = 1 / a3: no face
-// arrays, a multiply in place of the division.
-template <typename T, int TW, int NT>
-__device__ inline void tile_colour_u(T *E, const T *R, T ax, T ay, T ia3, int c, int gx0, int gy0, int NX, int NY) {
-    constexpr int KW = TW / 2;
-    for (int h = threadIdx.x; h < TW * KW; h += NT) {
-        const int y = h / KW, x = 2 * (h % KW) + ((c ^ y) & 1);
-        const int I = gx0 + x, J = gy0 + y;
-        if (x < 1 || x > TW - 2 || y < 1 || y > TW - 2 || I < 0 || I >= NX || J < 0 || J >= NY) continue;
-        const int q = y * TW + x;
-        E[q] = (R[q] - (ay * (E[q - TW] + E[q + TW]) + ax * (E[q - 1] + E[q + 1]))) * ia3;
-    }
-}
-
-template <typename T, int TW>
-__device__ inline T tile_res_u(const T *E, const T *R, T ax, T ay, T a3, int x, int y) {
-    const int q = y * TW + x;
-    return R[q] - (ay * (E[q - TW] + E[q + TW]) + ax * (E[q - 1] + E[q + 1]) + a3 * E[q]);
-}
-
-// Faces of a tile of side TW at level L whose cell (0, 0) is (gx0, gy0).
-template <typename T, int TW, int NT>
-__device__ inline void tile_faces(const MgLevel &L, int gx0, int gy0, T *AX, T *AY) {
-    const T *ax = (const T *)L.ax, *ay = (const T *)L.ay;
-    for (int q = threadIdx.x; q < TW * (TW + 1); q += NT) {
-        const int y = q / (TW + 1), x = q % (TW + 1);
-        const int I = gx0 + x, J = gy0 + y;
-        AX[q] = (I >= 0 && I <= L.nx && J >= 0 && J < L.ny) ? ax[mfx(L.ld, I, J)] : T(0);
-    }
-    for (int q = threadIdx.x; q < (TW + 1) * TW; q += NT) {
-        const int y = q / TW, x = q % TW;
-        const int I = gx0 + x, J = gy0 + y;
-        AY[q] = (I >= 0 && I < L.nx && J >= 0 && J <= L.ny) ? ay[mfy(L.ld, I, J)] : T(0);
     }
 }
 
@@ -225,126 +168,299 @@ __device__ inline int mg_tile(int ntiles) {
     return (blockIdx.x % 8) * per + blockIdx.x / 8;
 }
 
+// ------------------------------------------------------------ strips
+// Lane shifts within a wavefront: the value of lane - 1 (sh_w) or lane + 1
+// (sh_e), 0 past the ends, and of the lane whose number differs in the last
+// bit (sh_x).
+template <int CTRL>
+__device__ inline float dpp_move(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+template <int CTRL>
+__device__ inline double dpp_move(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+template <typename T>
+__device__ inline T sh_w(T v) { return dpp_move<0x138>(v); }   // wave_shr:1
+template <typename T>
+__device__ inline T sh_e(T v) { return dpp_move<0x130>(v); }   // wave_shl:1
+template <typename T>
+__device__ inline T sh_x(T v) { return dpp_move<0xB1>(v); }    // quad_perm [1,0,3,2]
+
+// A lane's strip: four rows of column x, as two row pairs.  With q = x & 1
+// (tile origins are even, so a point's colour is (x + row) & 1), pair k's
+// point of colour 0 is row 2k + q (A[k]) and of colour 1 row 2k + 1 - q
+// (B[k]).  The horizontal neighbours of A[k] are B[k] of lanes x - 1 and
+// x + 1, its vertical ones are its mate B[k] and, on the other side, row
+// 2k - 1 (q = 0) or 2k + 2 (q = 1): B[k - 1] or B[k + 1], past the strip's
+// end a value of the next strip; and the same with the colours exchanged.
+//
+// A point's update is e = r' + w e_W + e e_E + m e_mate + o e_other with the
+// face coefficients and the right-hand side divided by the diagonal once
+// (and signs turned): the reference has no counterpart whose rounding it
+// would have to keep.  Coefficients towards the ring, and all of a point
+// outside the grid, are 0, so such a point stays 0.
+template <typename T>
+struct SPt {
+    T w, e, m, o, r;
+};
+template <typename T>
+struct Strip {
+    T A[2], B[2];
+    SPt<T> a[2], b[2];
+    T d[2];   // diagonals of the A points (their residuals are restricted)
+};
+
+// The strip's coefficients from its rows' west and east faces, its five
+// y-faces (fs[j] south of row j) and right-hand sides; in: the row's point
+// is in the grid; I, NX: its column and the level's width.
+template <typename T>
+__device__ inline void strip_build(Strip<T> &S, int q, const T (&fw)[4], const T (&fe)[4], const T (&fs)[5],
+                                   const T (&r)[4], const bool (&in)[4], int I, int NX) {
+    SPt<T> v[4];
+    T d[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const T a3 = -(fw[j] + fe[j] + fs[j] + fs[j + 1]);
+        const T i3 = in[j] ? T(1) / a3 : T(0);
+        const T so = -fs[j] * i3, no = -fs[j + 1] * i3;
+        // a row of even j has its mate north of it
+        v[j] = SPt<T>{I > 0 ? -fw[j] * i3 : T(0), I < NX - 1 ? -fe[j] * i3 : T(0), (j & 1) ? so : no,
+                      (j & 1) ? no : so, in[j] ? r[j] * i3 : T(0)};
+        d[j] = in[j] ? a3 : T(0);
+    }
+#define SEL(c, x, y) SPt<T>{c ? x.w : y.w, c ? x.e : y.e, c ? x.m : y.m, c ? x.o : y.o, c ? x.r : y.r}
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        S.a[k] = SEL(q, v[2 * k + 1], v[2 * k]);
+        S.b[k] = SEL(q, v[2 * k], v[2 * k + 1]);
+        S.d[k] = q ? d[2 * k + 1] : d[2 * k];
+    }
+#undef SEL
+}
+template <typename T>
+__device__ inline T strip_eval(const SPt<T> &c, T row, T mate, T other) {
+    // the value from the next strip, read from LDS, enters last
+    return fma(c.o, other, fma(c.w, sh_w(row), fma(c.e, sh_e(row), fma(c.m, mate, c.r))));
+}
+// Row j's value.
+template <typename T>
+__device__ inline T strip_row(const Strip<T> &S, int q, int j) {
+    return ((j & 1) == q) ? S.A[j >> 1] : S.B[j >> 1];
+}
+
+// The rows at the strips' ends in LDS: end (s, h) is strip s's row 0 (h = 0)
+// or 3 (h = 1), for s = -1 .. NS (zero beyond the strips).  Of the two rows a
+// colour's lanes need (below where q = 0, above where q = 1 for colour 0; the
+// other way round for colour 1) all values are of the other colour, so no
+// lane writes what another may still read in the same phase.
+template <typename T>
+struct Ends {
+    T *p;   // this lane's column
+    int lw; // column count
+    __device__ T &at(int s, int h) const { return p[((s + 1) * 2 + h) * lw]; }
+};
+
+// Sweep phases; s: the lane's strip.
+template <typename T>
+__device__ inline void phase_a(Strip<T> &S, int q, int s, const Ends<T> &E) {
+    const T x = q ? E.at(s + 1, 0) : E.at(s - 1, 1);
+    const T a0 = strip_eval(S.a[0], S.B[0], S.B[0], q ? S.B[1] : x);
+    const T a1 = strip_eval(S.a[1], S.B[1], S.B[1], q ? x : S.B[0]);
+    S.A[0] = a0;
+    S.A[1] = a1;
+    E.at(s, q) = q ? a1 : a0;
+}
+template <typename T>
+__device__ inline void phase_b(Strip<T> &S, int q, int s, const Ends<T> &E) {
+    const T x = q ? E.at(s - 1, 1) : E.at(s + 1, 0);
+    const T b0 = strip_eval(S.b[0], S.A[0], S.A[0], q ? x : S.A[1]);
+    const T b1 = strip_eval(S.b[1], S.A[1], S.A[1], q ? S.A[0] : x);
+    S.B[0] = b0;
+    S.B[1] = b1;
+    E.at(s, q ^ 1) = q ? b0 : b1;
+}
+// Both end rows (after a prolongation).
+template <typename T>
+__device__ inline void ends_put(const Strip<T> &S, int q, int s, const Ends<T> &E) {
+    E.at(s, 0) = q ? S.B[0] : S.A[0];
+    E.at(s, 1) = q ? S.A[1] : S.B[1];
+}
+// NU sweeps from e = 0, colours 0 then 1 (the first phase's neighbours are 0).
+// act: the lane holds a strip (others only take part in the syncs).
+template <typename T, typename Sync>
+__device__ inline void sweep_down(Strip<T> &S, int q, int s, const Ends<T> &E, bool act, Sync sync) {
+    S.A[0] = S.a[0].r;
+    S.A[1] = S.a[1].r;
+    if (act) E.at(s, q) = q ? S.A[1] : S.A[0];
+    sync();
+#pragma unroll
+    for (int k = 0; k < MG_NU; k++) {
+        if (k && act) phase_a(S, q, s, E);
+        if (k) sync();
+        if (act) phase_b(S, q, s, E);
+        sync();
+    }
+}
+template <typename T, typename Sync>
+__device__ inline void sweep_up(Strip<T> &S, int q, int s, const Ends<T> &E, bool act, Sync sync) {
+    if (act) ends_put(S, q, s, E);
+    sync();
+#pragma unroll
+    for (int k = 0; k < MG_NU; k++) {
+        if (act) phase_b(S, q, s, E);
+        sync();
+        if (act) phase_a(S, q, s, E);
+        if (k + 1 < MG_NU) sync();
+    }
+}
+// Residuals of the strip's two row pairs summed over a coarse cell's
+// children, for the lanes of even x.  Colour 1 was relaxed last, so its
+// residuals are zero; colour 0's are the diagonal times what one more
+// relaxation would add.
+template <typename T>
+__device__ inline void strip_restrict(const Strip<T> &S, int q, int s, const Ends<T> &E, T (&rc)[2]) {
+    const T x = q ? E.at(s + 1, 0) : E.at(s - 1, 1);
+    const T g0 = strip_eval(S.a[0], S.B[0], S.B[0], q ? S.B[1] : x);
+    const T g1 = strip_eval(S.a[1], S.B[1], S.B[1], q ? x : S.B[0]);
+    const T r0 = S.d[0] * (g0 - S.A[0]), r1 = S.d[1] * (g1 - S.A[1]);
+    rc[0] = r0 + sh_x(r0);
+    rc[1] = r1 + sh_x(r1);
+}
+// e += prolongation: h[k] = 3 c + c' of the coarse rows jc0 - 1 .. jc0 + 2 on
+// the column's coarse cell (c) and its horizontal neighbour (c').
+template <typename T>
+__device__ inline T prolong(const T (&h)[4], int j) {
+    const int k = (j >> 1) + 1;
+    return (T(3) * h[k] + h[(j & 1) ? k + 1 : k - 1]) * T(0.0625);
+}
+
 // ------------------------------------------------------------ down
 // Level l: e = NU sweeps from 0 on A e = r, then r_(l+1) = restriction of
-// r - A e.  L0: r = b - A p is formed here in FP64 from p (staged in LDS, the
-// tile and one more ring) and b (ghosts frozen), stored in T for the up pass,
-// and max |r| of the owned points goes to part[tile].  D.nt > 0: this launch
-// first evaluates the stopping test of the level-0 kernel before it.
-// UF: level 0 with uniform faces (rau_c, rgv_c), see tile_colour_u.
-template <typename T, bool L0, int NT, bool STAGE, bool UF>
-__global__ __launch_bounds__(NT) void k_mg_down(MgLevel L, MgLevel C, int ntx, int ntiles, int nx, int ny, int ld,
-                                                const double *__restrict__ p, const double *__restrict__ b,
-                                                const double *__restrict__ rau, const double *__restrict__ rgv,
-                                                int uni, double rau_c, double rgv_c, double *__restrict__ part,
-                                                MgDecide D, Scalars *sc) {
+// r - A e.  L0: r = b - A p is formed here in FP64 from p and b (ghosts
+// frozen), stored in T for the up pass, and max |r| of the owned points goes
+// to part[tile].  D.nt > 0: this launch first evaluates the stopping test of
+// the level-0 kernel before it.  A tile owns the MG_OD x MG_OD cells from
+// (I0, J0); what its outermost lanes miss (the columns beyond the tile) moves
+// inwards one column a phase and stays off the owned cells.  uni: rau and rgv
+// are one value each (level 0 of a uniform Cartesian grid): no loads.
+template <typename T, bool L0>
+__global__ __launch_bounds__(MG_NT) void k_mg_down(MgLevel L, MgLevel C, int ntx, int ntiles, int nx, int ny, int ld,
+                                                   const double *__restrict__ p, const double *__restrict__ b,
+                                                   const double *__restrict__ rau, const double *__restrict__ rgv,
+                                                   int uni, double rau_c, double rgv_c, double *__restrict__ part,
+                                                   MgDecide D, Scalars *sc) {
     if (mg_stopped(sc)) return;
-    static_assert(L0 || !UF, "uniform faces are a level-0 shape");
-    constexpr int TW = MG_TD, PW = TW + 2;
-    __shared__ T E[TW * TW], R[TW * TW], AX[UF ? 1 : TW * (TW + 1)], AY[UF ? 1 : (TW + 1) * TW];
-    __shared__ double PS[(L0 && STAGE) ? PW * PW : 1];
-    __shared__ double red[NT / 64];
-    if (D.nt > 0 && mg_decide<NT>(D.part, D.nt, D.dk, D.tol, D.cycle, D.maxcyc, D.minc, sc, red)) return;
+    __shared__ T ends[(MG_NS + 2) * 2 * MG_TW];
+    __shared__ double red[MG_NT / 64];
+    if (D.nt > 0 && mg_decide<MG_NT>(D.part, D.nt, D.dk, D.tol, D.cycle, D.maxcyc, D.minc, sc, red)) return;
     const int tile = mg_tile(ntiles);
     if (tile >= ntiles) return;
-    const int I0 = (tile % ntx) * MG_OT, J0 = (tile / ntx) * MG_OT;
-    const int gx0 = I0 - MG_HD, gy0 = J0 - MG_HD;
+    const int I0 = (tile % ntx) * MG_OD, J0 = (tile / ntx) * MG_OD;
     const int NX = L.nx, NY = L.ny;
-    T *e = (T *)L.e, *r = (T *)L.r;
-    const T uax = (T)rau_c, uay = (T)rgv_c, ua3 = -(uax + uax + uay + uay), uia3 = T(1) / ua3;
-    if (!UF) tile_faces<T, TW, NT>(L, gx0, gy0, AX, AY);
-    if (L0 && STAGE) {
-        // p on the tile and one more ring: field (i, j) = (I + 2, J + 2) for
-        // I = gx0 - 1 .., 0 outside the field
-        for (int q = threadIdx.x; q < PW * PW; q += NT) {
-            const int i = gx0 + 1 + q % PW, j = gy0 + 1 + q / PW;
-            PS[q] = (i >= 0 && i <= nx + 1 && j >= 0 && j <= ny + 1) ? p[WD2_IX(i, j)] : 0.0;
-        }
-        __syncthreads();
+    const int x = threadIdx.x & 63, s = threadIdx.x >> 6, q = x & 1;
+    const int I = I0 - MG_HD + x, Jb = J0 - MG_HD + MG_SR * s;
+    const bool inx = I >= 0 && I < NX;
+    const bool ownx = inx && x >= MG_HD && x < MG_HD + MG_OD;
+    if (s == 0 || s == MG_NS - 1) {   // the zero rows beyond the strips
+        const int g = s == 0 ? -1 : MG_NS;
+        ends[((g + 1) * 2) * MG_TW + x] = T(0);
+        ends[((g + 1) * 2 + 1) * MG_TW + x] = T(0);
     }
+    bool in[4];
+    T fw[4], fe[4], fs[5], rv[4];
     double rmax = 0.0;
-    for (int q = threadIdx.x; q < TW * TW; q += NT) {
-        const int y = q / TW, x = q % TW;
-        const int I = gx0 + x, J = gy0 + y;
-        const bool in = I >= 0 && I < NX && J >= 0 && J < NY;
-        E[q] = T(0);
-        T rv = T(0);
-        if (in) {
-            if (L0) {
-                // FP64 residual of the pressure system at (i, j) = (I+2, J+2)
-                const int i = I + 2, j = J + 2;
-                double a1, a2, a4, a5;
-                if (uni) {
-                    a1 = a5 = rgv_c;
-                    a2 = a4 = rau_c;
-                } else {
-                    a1 = rgv[WD2_IX(i, j - 1)];
-                    a2 = rau[WD2_IX(i - 1, j)];
-                    a4 = rau[WD2_IX(i, j)];
-                    a5 = rgv[WD2_IX(i, j)];
-                }
-                const double a3 = -a4 - a2 - a5 - a1;
-                double res;
-                if (STAGE) {
-                    const int k = (y + 1) * PW + x + 1;
-                    res = b[WD2_IX(i, j)] -
-                          (a1 * PS[k - PW] + a2 * PS[k - 1] + a3 * PS[k] + a4 * PS[k + 1] + a5 * PS[k + PW]);
-                } else {
-                    res = b[WD2_IX(i, j)] - (a1 * p[WD2_IX(i, j - 1)] + a2 * p[WD2_IX(i - 1, j)] +
-                                             a3 * p[WD2_IX(i, j)] + a4 * p[WD2_IX(i + 1, j)] + a5 * p[WD2_IX(i, j + 1)]);
-                }
-                rv = (T)res;
-                const bool own = x >= MG_HD && x < MG_HD + MG_OT && y >= MG_HD && y < MG_HD + MG_OT;
-                // a NaN residual wins the maximum (never converged)
-                if (own && !(fabs(res) <= rmax)) rmax = fabs(res);
-            } else {
-                rv = r[mc(L.ld, I, J)];
-            }
+#pragma unroll
+    for (int j = 0; j < 4; j++) in[j] = inx && Jb + j >= 0 && Jb + j < NY;
+    if (L0) {
+        // field (i, j) = (I + 2, J + 2); addresses are clamped to the field
+        // (values outside serve only points outside the grid)
+        const int i = min(max(I + 2, 0), nx + 1);
+        auto row = [&](int J) { return min(max(J + 2, 0), ny + 1); };
+        double pc[6], bb[4];
+#pragma unroll
+        for (int j = 0; j < 6; j++) pc[j] = p[WD2_IX(i, row(Jb + j - 1))];
+#pragma unroll
+        for (int j = 0; j < 4; j++) bb[j] = b[WD2_IX(i, row(Jb + j))];
+        double a4[4], a5[5];
+        if (uni) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) a4[j] = rau_c;
+#pragma unroll
+            for (int j = 0; j < 5; j++) a5[j] = rgv_c;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) a4[j] = rau[WD2_IX(i, row(Jb + j))];
+#pragma unroll
+            for (int j = 0; j < 5; j++) a5[j] = rgv[WD2_IX(i, row(Jb + j - 1))];
         }
-        R[q] = rv;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const double a1 = a5[j], a2 = uni ? rau_c : sh_w(a4[j]);
+            const double a3 = -a4[j] - a2 - a5[j + 1] - a1;
+            const double res = bb[j] - (a1 * pc[j] + a2 * sh_w(pc[j + 1]) + a3 * pc[j + 1] + a4[j] * sh_e(pc[j + 1]) +
+                                        a5[j + 1] * pc[j + 2]);
+            rv[j] = in[j] ? (T)res : T(0);
+            const int y = MG_SR * s + j;
+            // a NaN residual wins the maximum (never converged)
+            if (in[j] && ownx && y >= MG_HD && y < MG_HD + MG_OD && !(fabs(res) <= rmax)) rmax = fabs(res);
+            fw[j] = (T)a2;
+            fe[j] = (T)a4[j];
+        }
+#pragma unroll
+        for (int j = 0; j < 5; j++) fs[j] = (T)a5[j];
+    } else {
+        const T *r = (const T *)L.r, *ax = (const T *)L.ax, *ay = (const T *)L.ay;
+        const bool fx = I >= 0 && I <= NX;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int J = Jb + j;
+            rv[j] = in[j] ? r[mc(L.ld, I, J)] : T(0);
+            fw[j] = (fx && J >= 0 && J < NY) ? ax[mfx(L.ld, I, J)] : T(0);
+        }
+#pragma unroll
+        for (int j = 0; j < 5; j++) {
+            const int J = Jb + j;
+            fs[j] = (inx && J >= 0 && J <= NY) ? ay[mfy(L.ld, I, J)] : T(0);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) fe[j] = sh_e(fw[j]);
     }
+    Strip<T> S;
+    strip_build<T>(S, q, fw, fe, fs, rv, in, I, NX);
+    const Ends<T> E{ends + x, MG_TW};
     if (L0) {
         for (int off = 32; off > 0; off >>= 1) {
             const double o = __shfl_xor(rmax, off);
             if (!(o <= rmax)) rmax = o;
         }
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = rmax;
+        if (x == 0) red[s] = rmax;
     }
-    __syncthreads();
+    sweep_down<T>(S, q, s, E, true, [] { __syncthreads(); });
     if (L0 && threadIdx.x == 0) {
         double m = red[0];
-        for (int w = 1; w < NT / 64; w++)
+        for (int w = 1; w < MG_NT / 64; w++)
             if (!(red[w] <= m)) m = red[w];
         part[tile] = m;
     }
-    for (int s = 0; s < MG_NU; s++)
-        for (int c = 0; c < 2; c++) {
-            if (UF)
-                tile_colour_u<T, TW, NT>(E, R, uax, uay, uia3, c, gx0, gy0, NX, NY);
-            else
-                tile_colour<T, TW, NT>(E, R, AX, AY, c, gx0, gy0, NX, NY);
-            __syncthreads();
+    T rc[2];
+    strip_restrict<T>(S, q, s, E, rc);
+    T *e = (T *)L.e, *r = (T *)L.r, *cr = (T *)C.r;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int y = MG_SR * s + j;
+        if (in[j] && ownx && y >= MG_HD && y < MG_HD + MG_OD) {
+            e[mc(L.ld, I, Jb + j)] = strip_row(S, q, j);
+            if (L0) r[mc(L.ld, I, Jb + j)] = rv[j];
         }
-    // a coarse cell per thread: its children's residuals summed; e (and, on
-    // level 0, r) of the owned children stored for the up pass
-    T *rc = (T *)C.r;
-    for (int q = threadIdx.x; q < MG_NC; q += NT) {
-        const int cx = q % (MG_OT / 2), cy = q / (MG_OT / 2);
-        const int Ic = I0 / 2 + cx, Jc = J0 / 2 + cy;
-        T sum = T(0);
+    }
 #pragma unroll
-        for (int dy = 0; dy < 2; dy++)
-#pragma unroll
-            for (int dx = 0; dx < 2; dx++) {
-                const int x = MG_HD + 2 * cx + dx, y = MG_HD + 2 * cy + dy;
-                const int I = gx0 + x, J = gy0 + y;
-                if (I < NX && J < NY) {
-                    sum += UF ? tile_res_u<T, TW>(E, R, uax, uay, ua3, x, y) : tile_res<T, TW>(E, R, AX, AY, x, y);
-                    e[mc(L.ld, I, J)] = E[y * TW + x];
-                    if (L0) r[mc(L.ld, I, J)] = R[y * TW + x];
-                }
-            }
-        if (Ic < C.nx && Jc < C.ny) rc[mc(C.ld, Ic, Jc)] = sum;
+    for (int k = 0; k < 2; k++) {
+        const int y = MG_SR * s + 2 * k, Ic = I >> 1, Jc = (Jb + 2 * k) >> 1;
+        if (q == 0 && ownx && y >= MG_HD && y < MG_HD + MG_OD && Ic < C.nx && Jc < C.ny) cr[mc(C.ld, Ic, Jc)] = rc[k];
     }
 }
 
@@ -352,348 +468,397 @@ __global__ __launch_bounds__(NT) void k_mg_down(MgLevel L, MgLevel C, int ntx, i
 // Level l: c = e + prolongation of c_(l+1), then NU sweeps; c of the owned
 // points is written (L0: p += c in FP64 instead).  The input e of the halos
 // and the output c are separate arrays, so no tile reads what another writes.
-// UF: level 0 with uniform faces ax, ay (see tile_colour_u).
-template <typename T, bool L0, int NT, bool UF>
-__global__ __launch_bounds__(NT) void k_mg_up(MgLevel L, MgLevel C, int ntx, int ntiles, int ld,
-                                              double *__restrict__ p, const Scalars *sc, double rau_c, double rgv_c) {
+template <typename T, bool L0>
+__global__ __launch_bounds__(MG_NT) void k_mg_up(MgLevel L, MgLevel C, int ntx, int ntiles, int nx, int ny, int ld,
+                                                 double *__restrict__ p, const double *__restrict__ rau,
+                                                 const double *__restrict__ rgv, int uni, double rau_c, double rgv_c,
+                                                 const Scalars *sc) {
     if (mg_stopped(sc)) return;
-    static_assert(L0 || !UF, "uniform faces are a level-0 shape");
-    constexpr int TW = MG_TU;
-    __shared__ T E[TW * TW], R[TW * TW], AX[UF ? 1 : TW * (TW + 1)], AY[UF ? 1 : (TW + 1) * TW], EC[MG_TC * MG_TC];
+    __shared__ T ends[(MG_NS + 2) * 2 * MG_TW];
     const int tile = mg_tile(ntiles);
     if (tile >= ntiles) return;
-    const int I0 = (tile % ntx) * MG_OT, J0 = (tile / ntx) * MG_OT;
-    const int gx0 = I0 - MG_HU, gy0 = J0 - MG_HU;
-    const int cgx0 = gx0 / 2 - 1, cgy0 = gy0 / 2 - 1;   // gx0 is even
+    const int I0 = (tile % ntx) * MG_OU, J0 = (tile / ntx) * MG_OU;
     const int NX = L.nx, NY = L.ny;
+    const int x = threadIdx.x & 63, s = threadIdx.x >> 6, q = x & 1;
+    const int I = I0 - MG_HU + x, Jb = J0 - MG_HU + MG_SR * s;
+    const bool inx = I >= 0 && I < NX;
+    if (s == 0 || s == MG_NS - 1) {
+        const int g = s == 0 ? -1 : MG_NS;
+        ends[((g + 1) * 2) * MG_TW + x] = T(0);
+        ends[((g + 1) * 2 + 1) * MG_TW + x] = T(0);
+    }
     const T *e = (const T *)L.e, *r = (const T *)L.r, *ec = (const T *)C.c;
-    const T uax = (T)rau_c, uay = (T)rgv_c, uia3 = T(1) / -(uax + uax + uay + uay);
-    if (!UF) tile_faces<T, TW, NT>(L, gx0, gy0, AX, AY);
-    for (int q = threadIdx.x; q < MG_TC * MG_TC; q += NT) {
-        const int Ic = cgx0 + q % MG_TC, Jc = cgy0 + q / MG_TC;
-        EC[q] = (Ic >= 0 && Ic < C.nx && Jc >= 0 && Jc < C.ny) ? ec[mc(C.ld, Ic, Jc)] : T(0);
-    }
-    __syncthreads();
-    for (int q = threadIdx.x; q < TW * TW; q += NT) {
-        const int y = q / TW, x = q % TW;
-        const int I = gx0 + x, J = gy0 + y;
-        T ev = T(0), rv = T(0);
-        if (I >= 0 && I < NX && J >= 0 && J < NY) {
-            const int ic = (I >> 1) - cgx0, jc = (J >> 1) - cgy0;
-            const int dx = (I & 1) ? 1 : -1, dy = (J & 1) ? 1 : -1;
-            const T pc = (T(9) * EC[jc * MG_TC + ic] + T(3) * EC[jc * MG_TC + ic + dx] +
-                          T(3) * EC[(jc + dy) * MG_TC + ic] + EC[(jc + dy) * MG_TC + ic + dx]) *
-                         T(0.0625);
-            ev = e[mc(L.ld, I, J)] + pc;
-            rv = r[mc(L.ld, I, J)];
+    bool in[4];
+    T fw[4], fe[4], fs[5], rv[4], ev[4], h[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) in[j] = inx && Jb + j >= 0 && Jb + j < NY;
+    {
+        const int ic = min(max(I >> 1, 0), C.nx - 1), in2 = ic + ((I & 1) ? 1 : -1), jc0 = Jb >> 1;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int jc = min(max(jc0 - 1 + k, -1), C.ny);
+            h[k] = T(3) * ec[mc(C.ld, ic, jc)] + ec[mc(C.ld, in2, jc)];
         }
-        E[q] = ev;
-        R[q] = rv;
     }
-    __syncthreads();
-    for (int s = 0; s < MG_NU; s++)
-        for (int c = 1; c >= 0; c--) {
-            if (UF)
-                tile_colour_u<T, TW, NT>(E, R, uax, uay, uia3, c, gx0, gy0, NX, NY);
-            else
-                tile_colour<T, TW, NT>(E, R, AX, AY, c, gx0, gy0, NX, NY);
-            __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        ev[j] = in[j] ? e[mc(L.ld, I, Jb + j)] : T(0);
+        rv[j] = in[j] ? r[mc(L.ld, I, Jb + j)] : T(0);
+    }
+    if (L0) {
+        const int i = min(max(I + 2, 0), nx + 1);
+        auto row = [&](int J) { return min(max(J + 2, 0), ny + 1); };
+#pragma unroll
+        for (int j = 0; j < 4; j++) fe[j] = (T)(uni ? rau_c : rau[WD2_IX(i, row(Jb + j))]);
+#pragma unroll
+        for (int j = 0; j < 5; j++) fs[j] = (T)(uni ? rgv_c : rgv[WD2_IX(i, row(Jb + j - 1))]);
+#pragma unroll
+        for (int j = 0; j < 4; j++) fw[j] = uni ? (T)rau_c : sh_w(fe[j]);
+    } else {
+        const T *ax = (const T *)L.ax, *ay = (const T *)L.ay;
+        const bool fx = I >= 0 && I <= NX;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int J = Jb + j;
+            fw[j] = (fx && J >= 0 && J < NY) ? ax[mfx(L.ld, I, J)] : T(0);
         }
+#pragma unroll
+        for (int j = 0; j < 5; j++) {
+            const int J = Jb + j;
+            fs[j] = (inx && J >= 0 && J <= NY) ? ay[mfy(L.ld, I, J)] : T(0);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) fe[j] = sh_e(fw[j]);
+    }
+    Strip<T> S;
+    strip_build<T>(S, q, fw, fe, fs, rv, in, I, NX);
+    T v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[j] = in[j] ? ev[j] + prolong<T>(h, j) : T(0);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        S.A[k] = q ? v[2 * k + 1] : v[2 * k];
+        S.B[k] = q ? v[2 * k] : v[2 * k + 1];
+    }
+    const Ends<T> E{ends + x, MG_TW};
+    sweep_up<T>(S, q, s, E, true, [] { __syncthreads(); });
+    if (!inx || x < MG_HU || x >= MG_HU + MG_OU) return;
     T *eo = (T *)L.c;
-    for (int q = threadIdx.x; q < MG_OT * MG_OT; q += NT) {
-        const int x = MG_HU + q % MG_OT, y = MG_HU + q / MG_OT;
-        const int I = gx0 + x, J = gy0 + y;
-        if (I >= NX || J >= NY) continue;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int y = MG_SR * s + j;
+        if (!in[j] || y < MG_HU || y >= MG_HU + MG_OU) continue;
         if (L0)
-            p[WD2_IX(I + 2, J + 2)] += (double)E[y * TW + x];
+            p[WD2_IX(I + 2, Jb + j + 2)] += (double)strip_row(S, q, j);
         else
-            eo[mc(L.ld, I, J)] = E[y * TW + x];
+            eo[mc(L.ld, I, Jb + j)] = strip_row(S, q, j);
     }
 }
 
 // ------------------------------------------------------------ bottom
-// Levels lb..nlev-1 (each at most MG_BSIDE cells wide) in one workgroup: the
-// V-cycle below level lb with the corrections and right-hand sides in LDS.
-// The face coefficients are copied into LDS first where they fit
-// (mg_bottom_faces_fit: compact rows of nx + 1 x-faces and nx y-faces per
-// level), so the ~50 sweep phases between barriers read only LDS; otherwise
-// they are read from the (small, cache-resident) level arrays.  Both give the
-// same bits.  Level lb's r comes from the down kernel above; its correction
+// The bottom levels in one workgroup.  Levels of more than MG_TAIL cells are
+// strips in registers (a level of NX cells a row takes lw = 2^k >= NX lanes a
+// strip, so a narrow level packs several strips into a wavefront; a level
+// that fits one wavefront needs only wavefront syncs).  From the first level
+// of at most MG_TAIL cells on, the rest of the V-cycle is linear in that
+// level's right-hand side: c = M r, with M built by k_mg_tail when the
+// coefficients are (about thirty dependent phases on a handful of points
+// otherwise).  Level 0's r comes from the down kernel above; its correction
 // goes to c for the up kernel above.  D.nt > 0: the stopping test is
-// evaluated first.
+// evaluated first.  The face loads of all levels are issued before the first
+// smoothing phase.
 struct MgBottom {
-    MgLevel lev[MG_MAXLEV];
-    int nlev;   // bottom levels
+    MgLevel lev[MG_NREG + 1];
+    int nreg;          // register levels; lev[nreg] is the tail's level
+    const void *tail;  // M, column j at [MG_TAIL j]
 };
-
-// LDS face values per direction: every bottom level of a 64-wide bottom in
-// FP32, of a 32-wide one in FP64 (the FP64 corrections and right-hand sides
-// take the rest of the LDS).
 template <typename T>
-constexpr int mg_bfcap() { return sizeof(T) == 4 ? 5632 : 1440; }
+constexpr int mg_bottom_width() { return sizeof(T) == 4 ? 64 : 32; }
 
-// Faces of one bottom level: the LDS copy (LF) or the level arrays.
-template <typename T, bool LF>
-struct BtFaces {
-    const T *fx, *fy;   // LF: LDS rows of NX + 1 (x) and NX (y) values
-    const T *ax, *ay;   // the level arrays
-    int ld, NX;
-    __device__ T x(int I, int J) const { return LF ? fx[I + (NX + 1) * J] : ax[mfx(ld, I, J)]; }
-    __device__ T y(int I, int J) const { return LF ? fy[I + NX * J] : ay[mfy(ld, I, J)]; }
+template <typename T>
+struct BtShared {
+    T ends[(MG_NS + 2) * 2 * 64];
+    T r[32 * 32 + 16 * 16 + MG_TAIL];            // right-hand sides of the levels below the first
+    T c[34 * 34 + 18 * 18 + (MG_TAIL + 2) * 3];  // their corrections, with a zero ring
+    T m[MG_TAIL * MG_TAIL];
+    double red[1024 / 64];
 };
+// Offsets of level l >= 1 in r and c.  A level of n cells of the register
+// kind has at most 32 x 32 (l = 1) and 16 x 16 (l = 2) cells; the tail's level
+// at most MG_TAIL, in at most (MG_TAIL + 2) x 3 places with its ring.
+__device__ inline int bt_roff(int l) { return l == 1 ? 0 : (l == 2 ? 1024 : 1280); }
+__device__ inline int bt_coff(int l) { return l == 1 ? 0 : (l == 2 ? 1156 : 1480); }
 
-// Red-black Gauss-Seidel sweeps of level L (E, R in LDS with row stride
-// nx + 2): nsweep sweeps of colours 0 then 1 (rev: 1 then 0), a sync after
-// each colour, by S threads.  A thread's points (point q of a colour: row
-// q / half, position q % half; q = thread + p S, at most P per thread and
-// colour) keep their index, face
-// coefficients, diagonal and right-hand side in registers across the sweeps
-// (R does not change while a level is smoothed), so a phase reads only the
-// four neighbours in E.  The update is the same expression on the same
-// values as a point-by-point evaluation.
-template <typename T, bool LF, int P, int S, typename Sync>
-__device__ inline void bt_smooth(T *E, const T *R, const MgLevel &L, const BtFaces<T, LF> &F, int nsweep, bool rev,
-                                 Sync sync) {
-    const int NX = L.nx, NY = L.ny, W = NX + 2;
-    const int half = (NX + 1) / 2;   // points of one colour per row, at most
-    int kk[2][P];
-    T cw[2][P], ce[2][P], cs[2][P], cn[2][P], ca[2][P], cr[2][P];
+__device__ inline int bt_lw(int NX) { return NX > 32 ? 6 : (NX > 16 ? 5 : (NX > 8 ? 4 : 3)); }
+__device__ inline void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <typename T, int NT>
+struct Bottom {
+    const MgBottom &B;
+    BtShared<T> &H;
+    // the face values of one level's strip (fl: the last column's east faces)
+    struct Faces {
+        T fw[4], fl[4], fs[5];
+    };
+    struct Lane {
+        int x, s, lw, ns;
+        bool act;
+    };
+    __device__ Lane lane(int l) const {
+        const int NX = B.lev[l].nx, k = bt_lw(NX);
+        Lane n;
+        n.lw = 1 << k;
+        n.x = threadIdx.x & (n.lw - 1);
+        n.s = threadIdx.x >> k;
+        n.ns = (B.lev[l].ny + MG_SR - 1) / MG_SR;
+        n.act = n.s < n.ns;
+        return n;
+    }
+    __device__ void load(int l, Faces &F) const {
+        const MgLevel &L = B.lev[l];
+        const Lane n = lane(l);
+        const T *ax = (const T *)L.ax, *ay = (const T *)L.ay;
 #pragma unroll
-    for (int c = 0; c < 2; c++)
-#pragma unroll
-        for (int p = 0; p < P; p++) {
-            const int q = threadIdx.x + p * S;
-            const int J = q / half, I = 2 * (q % half) + ((c ^ J) & 1);
-            kk[c][p] = -1;
-            if (q < half * NY && I < NX) {
-                cw[c][p] = F.x(I, J);
-                ce[c][p] = F.x(I + 1, J);
-                cs[c][p] = F.y(I, J);
-                cn[c][p] = F.y(I, J + 1);
-                ca[c][p] = -(cw[c][p] + ce[c][p] + cs[c][p] + cn[c][p]);
-                kk[c][p] = (I + 1) + W * (J + 1);
-                cr[c][p] = R[kk[c][p]];
-            }
+        for (int j = 0; j < 4; j++) {
+            const int J = MG_SR * n.s + j;
+            F.fw[j] = (n.act && n.x < L.nx && J < L.ny) ? ax[mfx(L.ld, n.x, J)] : T(0);
+            F.fl[j] = (n.act && n.x == L.nx - 1 && J < L.ny) ? ax[mfx(L.ld, L.nx, J)] : T(0);
         }
-    for (int s = 0; s < nsweep; s++)
 #pragma unroll
-        for (int cc = 0; cc < 2; cc++) {
-            const int c = rev ? 1 - cc : cc;
+        for (int j = 0; j < 5; j++) {
+            const int J = MG_SR * n.s + j;
+            F.fs[j] = (n.act && n.x < L.nx && J <= L.ny) ? ay[mfy(L.ld, n.x, J)] : T(0);
+        }
+    }
+    // the V-cycle from level l on; wave: one wavefront is left running it
+    template <int l>
+    __device__ void run(Faces (&F)[MG_NREG], const T (&r0)[4], bool wave) {
+        if (l == B.nreg || l == MG_NREG) {
+            tail(l);
+            return;
+        }
+        if constexpr (l < MG_NREG) {
+            const MgLevel &L = B.lev[l];
+            const Lane n = lane(l);
+            const int q = n.x & 1;
+            auto sync = [&] {
+                if (wave)
+                    wave_sync();
+                else
+                    __syncthreads();
+            };
+            Strip<T> S;
+            {
+                bool in[4];
+                T rv[4], fe[4];
 #pragma unroll
-            for (int p = 0; p < P; p++) {
-                const int k = kk[c][p];
-                if (k >= 0)
-                    E[k] = (cr[c][p] - (cs[c][p] * E[k - W] + cw[c][p] * E[k - 1] + ce[c][p] * E[k + 1] +
-                                        cn[c][p] * E[k + W])) /
-                           ca[c][p];
+                for (int j = 0; j < 4; j++) {
+                    const int J = MG_SR * n.s + j;
+                    in[j] = n.act && n.x < L.nx && J < L.ny;
+                    rv[j] = l == 0 ? r0[j] : (in[j] ? H.r[bt_roff(l) + n.x + L.nx * J] : T(0));
+                    // the east face is the next lane's west face
+                    const T nf = sh_e(F[l].fw[j]);
+                    fe[j] = n.x == L.nx - 1 ? F[l].fl[j] : nf;
+                }
+                strip_build<T>(S, q, F[l].fw, fe, F[l].fs, rv, in, n.x, L.nx);
+            }
+            const Ends<T> E{H.ends + n.x, n.lw};
+            if (n.act) {   // zero rows beyond the strips
+                if (n.s == 0) { E.at(-1, 0) = T(0); E.at(-1, 1) = T(0); }
+                if (n.s == n.ns - 1) { E.at(n.ns, 0) = T(0); E.at(n.ns, 1) = T(0); }
+            }
+            sweep_down<T>(S, q, n.s, E, n.act, sync);
+            const MgLevel &C = B.lev[l + 1];
+            T rc[2];
+            if (n.act) {
+                strip_restrict<T>(S, q, n.s, E, rc);
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    const int Ic = n.x >> 1, Jc = 2 * n.s + k;
+                    if (q == 0 && Ic < C.nx && Jc < C.ny) H.r[bt_roff(l + 1) + Ic + C.nx * Jc] = rc[k];
+                }
             }
             sync();
+            // the next level, in one wavefront where its strips fit one
+            const Lane nn = lane(l + 1);
+            const bool one = l + 1 == B.nreg || nn.lw * nn.ns <= 64;
+            if (wave || !one) {
+                run<l + 1>(F, r0, wave);
+            } else {
+                if (threadIdx.x < 64) run<l + 1>(F, r0, true);
+                __syncthreads();
+            }
+            // prolongation (the ring of the coarse correction is zero)
+            if (n.act) {
+                const int W = C.nx + 2;
+                const T *c = H.c + bt_coff(l + 1);
+                const int ic = min(n.x >> 1, C.nx - 1) + 1, i2 = ic + (q ? 1 : -1);
+                T h[4];
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const int jc = min(2 * n.s + k, C.ny + 1);   // padded row of 2 s - 1 + k
+                    h[k] = T(3) * c[ic + W * jc] + c[i2 + W * jc];
+                }
+                T v[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    v[j] = (n.x < L.nx && MG_SR * n.s + j < L.ny) ? prolong<T>(h, j) : T(0);
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    S.A[k] += q ? v[2 * k + 1] : v[2 * k];
+                    S.B[k] += q ? v[2 * k] : v[2 * k + 1];
+                }
+                // (the zero rows are this level's again)
+                if (n.s == 0) { E.at(-1, 0) = T(0); E.at(-1, 1) = T(0); }
+                if (n.s == n.ns - 1) { E.at(n.ns, 0) = T(0); E.at(n.ns, 1) = T(0); }
+            }
+            sweep_up<T>(S, q, n.s, E, n.act, sync);
+            if (n.act) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const int J = MG_SR * n.s + j;
+                    if (n.x >= L.nx || J >= L.ny) continue;
+                    const T v = strip_row(S, q, j);
+                    if (l == 0)
+                        ((T *)L.c)[mc(L.ld, n.x, J)] = v;
+                    else
+                        H.c[bt_coff(l) + n.x + 1 + (L.nx + 2) * (J + 1)] = v;
+                }
+            }
+            if (l > 0) sync();
         }
+    }
+    // c = M r on the tail's level
+    __device__ void tail(int l) {
+        const MgLevel &L = B.lev[l];
+        const int n = L.nx * L.ny, t = threadIdx.x;
+        if (t < n) {
+            const T *r = H.r + bt_roff(l);
+            T acc[4] = {T(0), T(0), T(0), T(0)};
+            for (int j = 0; j < n; j += 4)
+#pragma unroll
+                for (int u = 0; u < 4; u++)
+                    if (j + u < n) acc[u] = fma(H.m[MG_TAIL * (j + u) + t], r[j + u], acc[u]);
+            const T v = (acc[0] + acc[1]) + (acc[2] + acc[3]);
+            const int I = t % L.nx, J = t / L.nx;
+            if (l == 0)
+                ((T *)L.c)[mc(L.ld, I, J)] = v;
+            else
+                H.c[bt_coff(l) + I + 1 + (L.nx + 2) * (J + 1)] = v;
+        }
+        wave_sync();
+    }
+};
+
+template <typename T, int NT>
+__global__ __launch_bounds__(NT) void k_mg_bottom(MgBottom B, MgDecide D, Scalars *sc) {
+    if (mg_stopped(sc)) return;
+    __shared__ BtShared<T> H;
+    if (D.nt > 0 && mg_decide<NT>(D.part, D.nt, D.dk, D.tol, D.cycle, D.maxcyc, D.minc, sc, H.red)) return;
+    Bottom<T, NT> K{B, H};
+    typename Bottom<T, NT>::Faces F[MG_NREG];
+    T r0[4] = {T(0), T(0), T(0), T(0)};
+    const MgLevel &L = B.lev[0];
+    if (B.nreg > 0) {
+        const auto n = K.lane(0);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int J = MG_SR * n.s + j;
+            if (n.act && n.x < L.nx && J < L.ny) r0[j] = ((const T *)L.r)[mc(L.ld, n.x, J)];
+        }
+    } else if ((int)threadIdx.x < L.nx * L.ny) {
+        H.r[bt_roff(0) + threadIdx.x] = ((const T *)L.r)[mc(L.ld, threadIdx.x % L.nx, threadIdx.x / L.nx)];
+    }
+#pragma unroll
+    for (int l = 0; l < MG_NREG; l++)
+        if (l < B.nreg) K.load(l, F[l]);
+    for (int k = threadIdx.x; k < MG_TAIL * MG_TAIL; k += NT) H.m[k] = ((const T *)B.tail)[k];
+    for (int k = threadIdx.x; k < (int)(sizeof(H.c) / sizeof(T)); k += NT) H.c[k] = T(0);
+    __syncthreads();
+    K.template run<0>(F, r0, false);
 }
 
-template <typename T, bool LF>
-__global__ __launch_bounds__(MG_BT) void k_mg_bottom(MgBottom B, MgDecide D, Scalars *sc) {
-    if (mg_stopped(sc)) return;
-    constexpr int FC = LF ? mg_bfcap<T>() : 1;
-    __shared__ T E[MG_BCAP], R[MG_BCAP];
-    __shared__ T FX[FC], FY[FC];
-    __shared__ double red[MG_BT / 64];
-    if (D.nt > 0 && mg_decide<MG_BT>(D.part, D.nt, D.dk, D.tol, D.cycle, D.maxcyc, D.minc, sc, red)) return;
-    // each level's offset in E and R, and in FX and FY (in LDS: indexed by
-    // the level, they would otherwise go to scratch)
-    __shared__ int off[MG_MAXLEV], ofx[MG_MAXLEV], ofy[MG_MAXLEV];
-    if (threadIdx.x == 0) {
-        int o = 0, ox = 0, oy = 0;
-        for (int l = 0; l < B.nlev; l++) {
-            const int NX = B.lev[l].nx, NY = B.lev[l].ny;
-            off[l] = o;
-            ofx[l] = ox;
-            ofy[l] = oy;
-            o += (NX + 2) * (NY + 2);
-            ox += (NX + 1) * NY;
-            oy += NX * (NY + 1);
-        }
+// The tail matrix: workgroup j (one wavefront) runs the V-cycle of the levels
+// t .. of the hierarchy on the j-th unit vector; its result is column j.
+struct MgTailLevels {
+    MgLevel lev[MG_MAXLEV];
+    int nlev;
+};
+template <typename T>
+__global__ __launch_bounds__(64) void k_mg_tail(MgTailLevels B, T *__restrict__ M) {
+    constexpr int CAP = 512;   // all levels with their rings: 64 x 1 and its halvings take the most
+    __shared__ T E[CAP], R[CAP];
+    __shared__ int off[MG_MAXLEV + 1];
+    const int t = threadIdx.x;
+    if (t == 0) {
+        off[0] = 0;
+        for (int l = 0; l < B.nlev; l++) off[l + 1] = off[l] + (B.lev[l].nx + 2) * (B.lev[l].ny + 2);
+    }
+    for (int k = t; k < CAP; k += 64) E[k] = R[k] = T(0);
+    __syncthreads();
+    if (t == 0) {
+        const int j = blockIdx.x, NX = B.lev[0].nx;
+        R[(j % NX + 1) + (NX + 2) * (j / NX + 1)] = T(1);
     }
     __syncthreads();
-    auto faces = [&](int l) {
+    auto relax = [&](int l, int c, bool res) {   // a colour's relaxation, or (res) the point's residual into E's place
         const MgLevel &L = B.lev[l];
-        return BtFaces<T, LF>{FX + ofx[l], FY + ofy[l], (const T *)L.ax, (const T *)L.ay, L.ld, L.nx};
-    };
-    // Set-up: every global load first (r of the first level, the faces),
-    // then the LDS stores, so the loads' latencies overlap.  E is zeroed
-    // everywhere, R everywhere but the first level's interior.
-    constexpr int RB = (MG_BSIDE * MG_BSIDE + MG_BT - 1) / MG_BT;   // r values per thread
-    constexpr int FB = LF ? (mg_bfcap<T>() + MG_BT - 1) / MG_BT : 1;   // face values per thread and direction
-    const MgLevel &L0 = B.lev[0];
-    const int n0 = L0.nx * L0.ny;
-    T rv[RB], fxv[FB], fyv[FB];
-#pragma unroll
-    for (int it = 0; it < RB; it++) {
-        const int q = threadIdx.x + it * MG_BT;
-        if (q < n0) rv[it] = ((const T *)L0.r)[(size_t)(q % L0.nx + 1) + (size_t)L0.ld * (q / L0.nx + 1)];
-    }
-    const int nl = B.nlev - 1;
-    const int nfx = ofx[nl] + (B.lev[nl].nx + 1) * B.lev[nl].ny, nfy = ofy[nl] + B.lev[nl].nx * (B.lev[nl].ny + 1);
-    if (LF) {
-#pragma unroll
-        for (int it = 0; it < FB; it++) {
-            const int q = threadIdx.x + it * MG_BT;
-            if (q < nfx) {
-                int l = 0;
-                while (l < nl && q >= ofx[l + 1]) l++;
-                const MgLevel &L = B.lev[l];
-                const int u = q - ofx[l];
-                fxv[it] = ((const T *)L.ax)[mfx(L.ld, u % (L.nx + 1), u / (L.nx + 1))];
-            }
-            if (q < nfy) {
-                int l = 0;
-                while (l < nl && q >= ofy[l + 1]) l++;
-                const MgLevel &L = B.lev[l];
-                const int u = q - ofy[l];
-                fyv[it] = ((const T *)L.ay)[mfy(L.ld, u % L.nx, u / L.nx)];
-            }
-        }
-    }
-    for (int l = 0; l < B.nlev; l++) {
-        const MgLevel &L = B.lev[l];
-        const int W = L.nx + 2, n = W * (L.ny + 2);
-        for (int q = threadIdx.x; q < n; q += MG_BT) {
-            const int a = q % W, bb = q / W;   // padded position
-            E[off[l] + q] = T(0);
-            if (!(l == 0 && a >= 1 && a <= L.nx && bb >= 1 && bb <= L.ny)) R[off[l] + q] = T(0);
-        }
-    }
-#pragma unroll
-    for (int it = 0; it < RB; it++) {
-        const int q = threadIdx.x + it * MG_BT;
-        if (q < n0) R[off[0] + (q % L0.nx + 1) + (L0.nx + 2) * (q / L0.nx + 1)] = rv[it];
-    }
-    if (LF) {
-#pragma unroll
-        for (int it = 0; it < FB; it++) {
-            const int q = threadIdx.x + it * MG_BT;
-            if (q < nfx) FX[q] = fxv[it];
-            if (q < nfy) FY[q] = fyv[it];
-        }
-    }
-    __syncthreads();
-    // The levels from lw on (at most 64 points of a colour: one per lane; the
-    // levels shrink) run in wavefront 0 alone, whose phases need only a
-    // wavefront sync; the wider ones use the whole workgroup between
-    // barriers.  The operations and their order are the same either way.
-    int lw = B.nlev;
-    for (int l = B.nlev - 1; l >= 0 && ((B.lev[l].nx + 1) / 2) * B.lev[l].ny <= 64; l--) lw = l;
-    const bool w0 = threadIdx.x < 64;
-    auto sync = [](bool wave) {
-        if (wave) {
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        } else {
-            __syncthreads();
-        }
-    };
-    // a level's sweeps: in wavefront 0 (one point per lane and colour) or by the whole workgroup (at most MG_BSIDE^2 / 2
-    // points per colour: two per thread)
-    static_assert(MG_BSIDE * MG_BSIDE / 2 <= 2 * MG_BT, "two points per thread and colour");
-    auto smooth = [&](T *El, const T *Rl, const MgLevel &L, const BtFaces<T, LF> &F, int nsweep, bool rev,
-                      bool wave) {
-        if (wave)
-            bt_smooth<T, LF, 1, 64>(El, Rl, L, F, nsweep, rev, [&] { sync(true); });
-        else
-            bt_smooth<T, LF, 2, MG_BT>(El, Rl, L, F, nsweep, rev, [&] { sync(false); });
-    };
-    // pre-smoothing of level l and the restriction of its residual
-    auto down = [&](int l, bool wave) {
-        const int step = wave ? 64 : MG_BT;
-        const MgLevel &L = B.lev[l];
-        const BtFaces<T, LF> F = faces(l);
-        const int NX = L.nx, NY = L.ny, W = NX + 2;
-        T *El = E + off[l], *Rl = R + off[l];
-        smooth(El, Rl, L, F, MG_NU, false, wave);
-        const int NXc = B.lev[l + 1].nx, NYc = B.lev[l + 1].ny, Wc = NXc + 2;
-        T *Rc = R + off[l + 1];
-        for (int q = threadIdx.x; q < NXc * NYc; q += step) {
-            const int Ic = q % NXc, Jc = q / NXc;
-            T sum = T(0);
-            for (int dy = 0; dy < 2; dy++)
-                for (int dx = 0; dx < 2; dx++) {
-                    const int I = 2 * Ic + dx, J = 2 * Jc + dy;
-                    if (I >= NX || J >= NY) continue;
-                    const T aw = F.x(I, J), ae = F.x(I + 1, J);
-                    const T as = F.y(I, J), an = F.y(I, J + 1);
-                    const T a3 = -(aw + ae + as + an);
-                    const int k = (I + 1) + W * (J + 1);
-                    sum += Rl[k] - (as * El[k - W] + aw * El[k - 1] + a3 * El[k] + ae * El[k + 1] + an * El[k + W]);
-                }
-            Rc[(Ic + 1) + Wc * (Jc + 1)] = sum;
-        }
-        sync(wave);
-    };
-    // the coarse correction of level l + 1 added to level l, post-smoothing
-    auto up = [&](int l, bool wave) {
-        const int step = wave ? 64 : MG_BT;
-        const int NX = B.lev[l].nx, NY = B.lev[l].ny, W = NX + 2;
-        const int NXc = B.lev[l + 1].nx, Wc = NXc + 2;
+        const T *ax = (const T *)L.ax, *ay = (const T *)L.ay;
         T *El = E + off[l];
-        const T *Ec = E + off[l + 1];
-        for (int q = threadIdx.x; q < NX * NY; q += step) {
-            const int I = q % NX, J = q / NX;
-            const int ic = (I >> 1) + 1, jc = (J >> 1) + 1;   // padded coarse position
-            const int dx = (I & 1) ? 1 : -1, dy = (J & 1) ? 1 : -1;
-            // coarse neighbours beyond the grid read the zero ring
-            const T pc = (T(9) * Ec[ic + Wc * jc] + T(3) * Ec[ic + dx + Wc * jc] + T(3) * Ec[ic + Wc * (jc + dy)] +
-                          Ec[ic + dx + Wc * (jc + dy)]) *
-                         T(0.0625);
-            El[(I + 1) + W * (J + 1)] += pc;
-        }
-        sync(wave);
-        smooth(El, R + off[l], B.lev[l], faces(l), MG_NU, true, wave);
-    };
-    // sweeps on the coarsest level
-    auto coarsest = [&](bool wave) {
-        const int l = B.nlev - 1;
-        smooth(E + off[l], R + off[l], B.lev[l], faces(l), MG_NCOARSE, false, wave);
-    };
-    const int lb = lw < B.nlev ? lw : B.nlev - 1;   // levels below lb: whole workgroup
-    for (int l = 0; l < lb; l++) down(l, false);
-    if (lw < B.nlev) {
-        if (w0) {
-            for (int l = lw; l + 1 < B.nlev; l++) down(l, true);
-            coarsest(true);
-            for (int l = B.nlev - 2; l >= lw; l--) up(l, true);
+        const T *Rl = R + off[l];
+        const int W = L.nx + 2, I = t % L.nx, J = t / L.nx, k = (I + 1) + W * (J + 1);
+        T v = T(0);
+        if (J < L.ny && (res || ((I + J) & 1) == c)) {
+            const T aw = ax[mfx(L.ld, I, J)], ae = ax[mfx(L.ld, I + 1, J)];
+            const T as = ay[mfy(L.ld, I, J)], an = ay[mfy(L.ld, I, J + 1)];
+            const T a3 = -(aw + ae + as + an);
+            const T sum = as * El[k - W] + aw * El[k - 1] + ae * El[k + 1] + an * El[k + W];
+            if (res)
+                v = Rl[k] - (sum + a3 * El[k]);
+            else
+                El[k] = (Rl[k] - sum) / a3;
         }
         __syncthreads();
-    } else {
-        coarsest(false);
+        return v;
+    };
+    for (int l = 0; l + 1 < B.nlev; l++) {
+        for (int k = 0; k < MG_NU; k++)
+            for (int c = 0; c < 2; c++) relax(l, c, false);
+        const T v = relax(l, 0, true);
+        const MgLevel &L = B.lev[l], &C = B.lev[l + 1];
+        T *Rc = R + off[l + 1];
+        const int I = t % L.nx, J = t / L.nx;
+        // children of a coarse cell added in turn
+        for (int u = 0; u < 4; u++) {
+            if (J < L.ny && (I & 1) == (u & 1) && (J & 1) == (u >> 1))
+                Rc[(I / 2 + 1) + (C.nx + 2) * (J / 2 + 1)] += v;
+            __syncthreads();
+        }
     }
-    for (int l = lb - 1; l >= 0; l--) up(l, false);
+    for (int k = 0; k < MG_NCOARSE; k++)
+        for (int c = 0; c < 2; c++) relax(B.nlev - 1, c, false);
+    for (int l = B.nlev - 2; l >= 0; l--) {
+        const MgLevel &L = B.lev[l], &C = B.lev[l + 1];
+        const int I = t % L.nx, J = t / L.nx, Wc = C.nx + 2;
+        if (J < L.ny) {
+            const T *Ec = E + off[l + 1];
+            const int ic = (I >> 1) + 1, jc = (J >> 1) + 1, dx = (I & 1) ? 1 : -1, dy = (J & 1) ? 1 : -1;
+            E[off[l] + (I + 1) + (L.nx + 2) * (J + 1)] +=
+                (T(9) * Ec[ic + Wc * jc] + T(3) * Ec[ic + dx + Wc * jc] + T(3) * Ec[ic + Wc * (jc + dy)] +
+                 Ec[ic + dx + Wc * (jc + dy)]) * T(0.0625);
+        }
+        __syncthreads();
+        for (int k = 0; k < MG_NU; k++)
+            for (int c = 1; c >= 0; c--) relax(l, c, false);
+    }
     const MgLevel &L = B.lev[0];
-    T *e = (T *)L.c;
-    const int W = L.nx + 2;
-    for (int q = threadIdx.x; q < L.nx * L.ny; q += MG_BT) {
-        const int I = q % L.nx, J = q / L.nx;
-        e[(size_t)(I + 1) + (size_t)L.ld * (J + 1)] = E[(I + 1) + W * (J + 1)];
-    }
-}
-
-// Whether the face coefficients of the bottom levels fit the kernel's LDS copy.
-template <typename T>
-static bool mg_bottom_faces_fit(const MgBottom &B) {
-    int fx = 0, fy = 0;
-    for (int l = 0; l < B.nlev; l++) {
-        fx += (B.lev[l].nx + 1) * B.lev[l].ny;
-        fy += B.lev[l].nx * (B.lev[l].ny + 1);
-    }
-    return fx <= mg_bfcap<T>() && fy <= mg_bfcap<T>();
-}
-
-template <typename T>
-static void launch_mg_bottom(const MgBottom &B, const MgDecide &D, Scalars *sc, hipStream_t s) {
-    if (mg_bottom_faces_fit<T>(B))
-        hipLaunchKernelGGL((k_mg_bottom<T, true>), dim3(1), dim3(MG_BT), 0, s, B, D, sc);
-    else
-        hipLaunchKernelGGL((k_mg_bottom<T, false>), dim3(1), dim3(MG_BT), 0, s, B, D, sc);
+    T v = T(0);
+    if (t < L.nx * L.ny) v = E[(t % L.nx + 1) + (L.nx + 2) * (t / L.nx + 1)];
+    M[MG_TAIL * blockIdx.x + t] = v;
 }
 
 // ------------------------------------------------------------ control
@@ -705,14 +870,22 @@ __global__ void k_mg_reset(Scalars *sc) {
 }
 
 // ------------------------------------------------------------ host side
-int mg_tiles(int NX, int NY, int *ntx) {
-    const int tx = (NX + MG_OT - 1) / MG_OT, ty = (NY + MG_OT - 1) / MG_OT;
+static int tiles_of(int NX, int NY, int own, int *ntx) {
+    const int tx = (NX + own - 1) / own, ty = (NY + own - 1) / own;
     if (ntx) *ntx = tx;
     return tx * ty;
 }
-int mg_bottom_side() { return MG_BSIDE; }
-int mg_bottom_cells() { return MG_BCAP; }
-int mg_sweeps() { return MG_NU; }
+int mg_tiles(int NX, int NY, int *ntx) { return tiles_of(NX, NY, MG_OD, ntx); }
+int mg_tail_cells() { return MG_TAIL; }
+int mg_bottom_side(int fp32) { return fp32 ? mg_bottom_width<float>() : mg_bottom_width<double>(); }
+size_t mg_tail_bytes() { return sizeof(double) * MG_TAIL * MG_TAIL; }
+
+// The first level of at most MG_TAIL cells.
+static int tail_level(const MgHierarchy &H) {
+    int l = H.ntiled;
+    while (l + 1 < H.nlev && H.lev[l].nx * H.lev[l].ny > MG_TAIL) l++;
+    return l;
+}
 
 template <typename T>
 void launch_mg_coef(const MgHierarchy &H, int nx, int ny, int ld, const double *rau, const double *rgv,
@@ -727,59 +900,48 @@ void launch_mg_coef(const MgHierarchy &H, int nx, int ny, int ld, const double *
         hipLaunchKernelGGL(k_mg_coarsen<T>, dim3((C.nx + 1 + 255) / 256, C.ny + 1), dim3(256), 0, s, H.lev[l - 1], C,
                            (T)(sl / sp));
     }
+    // the tail's level does not depend on where the tiled levels end (at the
+    // latest at the first level of at most MG_TAIL cells)
+    MgTailLevels B{};
+    int t = 1;
+    while (t + 1 < H.nlev && H.lev[t].nx * H.lev[t].ny > MG_TAIL) t++;
+    B.nlev = H.nlev - t;
+    for (int l = 0; l < B.nlev; l++) B.lev[l] = H.lev[t + l];
+    hipLaunchKernelGGL(k_mg_tail<T>, dim3(B.lev[0].nx * B.lev[0].ny), dim3(64), 0, s, B, (T *)H.tail);
 }
 
-template <typename T, int NT, bool STAGE>
-static void down0_as(const MgHierarchy &H, int nx, int ny, int ld, const double *b, const double *p,
-                     const double *rau, const double *rgv, const double *uni, double *part, Scalars *sc,
-                     hipStream_t s) {
-    int ntx = 0;
-    const int nt = mg_tiles(H.lev[0].nx, H.lev[0].ny, &ntx);
-    const MgDecide none{nullptr, 0, 0, 0, 0.0, 0.0};
-    if (uni)
-        hipLaunchKernelGGL((k_mg_down<T, true, NT, STAGE, true>), dim3(8 * ((nt + 7) / 8)), dim3(NT), 0, s, H.lev[0],
-                           H.lev[1], ntx, nt, nx, ny, ld, p, b, rau, rgv, 1, uni[0], uni[1], part, none, sc);
-    else
-        hipLaunchKernelGGL((k_mg_down<T, true, NT, STAGE, false>), dim3(8 * ((nt + 7) / 8)), dim3(NT), 0, s,
-                           H.lev[0], H.lev[1], ntx, nt, nx, ny, ld, p, b, rau, rgv, 0, 0.0, 0.0, part, none, sc);
-}
-
-// the level-0 down kernel in the shape the hierarchy's tuning selects
 template <typename T>
 static void down0(const MgHierarchy &H, int nx, int ny, int ld, const double *b, const double *p, const double *rau,
                   const double *rgv, const double *uni, double *part, Scalars *sc, hipStream_t s) {
-    const bool big = H.tune.nt0 >= 512;
-    if (H.tune.stage) {
-        if (big)
-            down0_as<T, 512, true>(H, nx, ny, ld, b, p, rau, rgv, uni, part, sc, s);
-        else
-            down0_as<T, 256, true>(H, nx, ny, ld, b, p, rau, rgv, uni, part, sc, s);
-    } else {
-        if (big)
-            down0_as<T, 512, false>(H, nx, ny, ld, b, p, rau, rgv, uni, part, sc, s);
-        else
-            down0_as<T, 256, false>(H, nx, ny, ld, b, p, rau, rgv, uni, part, sc, s);
-    }
-}
-
-template <typename T, int NT>
-static void up0_as(const MgHierarchy &H, int ld, double *p, const double *uni, Scalars *sc, hipStream_t s) {
     int ntx = 0;
     const int nt = mg_tiles(H.lev[0].nx, H.lev[0].ny, &ntx);
-    if (uni)
-        hipLaunchKernelGGL((k_mg_up<T, true, NT, true>), dim3(8 * ((nt + 7) / 8)), dim3(NT), 0, s, H.lev[0], H.lev[1],
-                           ntx, nt, ld, p, sc, uni[0], uni[1]);
-    else
-        hipLaunchKernelGGL((k_mg_up<T, true, NT, false>), dim3(8 * ((nt + 7) / 8)), dim3(NT), 0, s, H.lev[0],
-                           H.lev[1], ntx, nt, ld, p, sc, 0.0, 0.0);
+    const MgDecide none{nullptr, 0, 0, 0, 0.0, 0.0};
+    hipLaunchKernelGGL((k_mg_down<T, true>), dim3(8 * ((nt + 7) / 8)), dim3(MG_NT), 0, s, H.lev[0], H.lev[1], ntx, nt,
+                       nx, ny, ld, p, b, rau, rgv, uni ? 1 : 0, uni ? uni[0] : 0.0, uni ? uni[1] : 0.0, part, none, sc);
 }
 
 template <typename T>
-static void up0(const MgHierarchy &H, int ld, double *p, const double *uni, Scalars *sc, hipStream_t s) {
-    if (H.tune.nt0 >= 512)
-        up0_as<T, 512>(H, ld, p, uni, sc, s);
-    else
-        up0_as<T, 256>(H, ld, p, uni, sc, s);
+static void up0(const MgHierarchy &H, int nx, int ny, int ld, double *p, const double *rau, const double *rgv,
+                const double *uni, Scalars *sc, hipStream_t s) {
+    int ntx = 0;
+    const int nt = tiles_of(H.lev[0].nx, H.lev[0].ny, MG_OU, &ntx);
+    hipLaunchKernelGGL((k_mg_up<T, true>), dim3(8 * ((nt + 7) / 8)), dim3(MG_NT), 0, s, H.lev[0], H.lev[1], ntx, nt, nx,
+                       ny, ld, p, rau, rgv, uni ? 1 : 0, uni ? uni[0] : 0.0, uni ? uni[1] : 0.0, sc);
+}
+
+template <typename T>
+static void launch_mg_bottom(const MgHierarchy &H, const MgDecide &D, Scalars *sc, hipStream_t s) {
+    MgBottom B{};
+    B.nreg = tail_level(H) - H.ntiled;
+    for (int l = 0; l <= B.nreg; l++) B.lev[l] = H.lev[H.ntiled + l];
+    B.tail = H.tail;
+    // lanes of the first level: 256 serve up to 32 x 32 cells
+    if constexpr (sizeof(T) == 4)
+        if (std::max(B.lev[0].nx, B.lev[0].ny) > 32) {
+            hipLaunchKernelGGL((k_mg_bottom<T, 1024>), dim3(1), dim3(1024), 0, s, B, D, sc);
+            return;
+        }
+    hipLaunchKernelGGL((k_mg_bottom<T, 256>), dim3(1), dim3(256), 0, s, B, D, sc);
 }
 
 // One V-cycle of defect correction (cycle is 1-based), every kernel
@@ -798,21 +960,17 @@ void launch_mg_cycle(const MgHierarchy &H, int nx, int ny, int ld, const double 
     const MgDecide none{nullptr, 0, 0, 0, 0.0, 0.0};
     for (int l = 1; l < H.ntiled; l++) {
         const int nt = mg_tiles(H.lev[l].nx, H.lev[l].ny, &ntx);
-        hipLaunchKernelGGL((k_mg_down<T, false, MG_NT1, false, false>), dim3(8 * ((nt + 7) / 8)), dim3(MG_NT1), 0, s, H.lev[l],
-                           H.lev[l + 1], ntx, nt, nx, ny, ld, p, b, rau, rgv, 0, 0.0, 0.0, part, l == 1 ? D : none,
-                           sc);
+        hipLaunchKernelGGL((k_mg_down<T, false>), dim3(8 * ((nt + 7) / 8)), dim3(MG_NT), 0, s, H.lev[l], H.lev[l + 1],
+                           ntx, nt, nx, ny, ld, p, b, rau, rgv, 0, 0.0, 0.0, part, l == 1 ? D : none, sc);
     }
-    MgBottom B{};
-    B.nlev = H.nlev - H.ntiled;
-    for (int l = 0; l < B.nlev; l++) B.lev[l] = H.lev[H.ntiled + l];
-    launch_mg_bottom<T>(B, H.ntiled == 1 ? D : none, sc, s);
+    launch_mg_bottom<T>(H, H.ntiled == 1 ? D : none, sc, s);
     for (int l = H.ntiled - 1; l >= 1; l--) {
-        const int nt = mg_tiles(H.lev[l].nx, H.lev[l].ny, &ntx);
-        hipLaunchKernelGGL((k_mg_up<T, false, MG_NT1, false>), dim3(8 * ((nt + 7) / 8)), dim3(MG_NT1), 0, s, H.lev[l],
-                           H.lev[l + 1], ntx, nt, ld, p, sc, 0.0, 0.0);
+        const int nt = tiles_of(H.lev[l].nx, H.lev[l].ny, MG_OU, &ntx);
+        hipLaunchKernelGGL((k_mg_up<T, false>), dim3(8 * ((nt + 7) / 8)), dim3(MG_NT), 0, s, H.lev[l], H.lev[l + 1],
+                           ntx, nt, nx, ny, ld, p, rau, rgv, 0, 0.0, 0.0, sc);
     }
     if (ev_up) (void)hipEventRecord(ev_up[0], s);
-    up0<T>(H, ld, p, uni, sc, s);
+    up0<T>(H, nx, ny, ld, p, rau, rgv, uni, sc, s);
     if (ev_up) (void)hipEventRecord(ev_up[1], s);
 }
 
@@ -827,18 +985,15 @@ void launch_mg_kernel_bench(const MgHierarchy &H, int which, int reps, int nx, i
                             double *p, const double *rau, const double *rgv, const double *uni, double *part,
                             Scalars *sc, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
     launch_mg_reset(sc, s);
-    MgBottom B{};
-    B.nlev = H.nlev - H.ntiled;
-    for (int l = 0; l < B.nlev; l++) B.lev[l] = H.lev[H.ntiled + l];
     const MgDecide none{nullptr, 0, 0, 0, 0.0, 0.0};
     (void)hipEventRecord(e0, s);
     for (int k = 0; k < reps; k++) {
         if (which == 2)
             down0<T>(H, nx, ny, ld, b, p, rau, rgv, uni, part, sc, s);
         else if (which == 3)
-            up0<T>(H, ld, p, uni, sc, s);
+            up0<T>(H, nx, ny, ld, p, rau, rgv, uni, sc, s);
         else
-            launch_mg_bottom<T>(B, none, sc, s);
+            launch_mg_bottom<T>(H, none, sc, s);
     }
     (void)hipEventRecord(e1, s);
 }

@@ -182,9 +182,7 @@ static int ql_border_blocks(int nx, int ny, int nt) { return (5 * (nx + ny) + 8 
 //
 // H = 48: two runs of a recurrence meet bit for bit within 53 / log2(1/l)
 // rows for a contraction l per row, 48 rows for l <= 0.46, which a row with
-// |a| + |c| <= 0.76 |d| has.  (Halos of 32 and 64 rows keep 1920 and 1792 of
-// 2048 rows; 64 served stiffer chains, 32 failed the check at viscous numbers
-// the configurations use.)
+// |a| + |c| <= 0.76 |d| has (the configurations' chains are below 0.3).
 constexpr int QX_T = 256, QX_HL = 6, QX_H = QX_HL * TR_S, QX_N = QX_T * TR_S, QX_O = QX_N - 4 * QX_H;
 constexpr int QX_CHK = 12;
 
@@ -354,8 +352,12 @@ __device__ inline void qx_backward(unsigned kinds, const T (&cp)[TR_S], const T 
     __syncthreads();
 }
 
+// Registers bound the windows in flight: at three wavefronts per SIMD (168
+// VGPRs, a few spilled) a launch over the 2.1 M FP64 rows of a 1024^2 cavity
+// takes 57 us; without the bound it takes 179 VGPRs, two wavefronts and 66
+// us, at four it spills into 118 us.
 template <typename T>
-__global__ __launch_bounds__(QX_T) void k_ql_exact(long n, Chains cs, ChainT<T> h1, ChainT<T> h2,
+__global__ __launch_bounds__(QX_T, 3) void k_ql_exact(long n, Chains cs, ChainT<T> h1, ChainT<T> h2,
                                                    const unsigned char *__restrict__ Z, QlFields F,
                                                    double *__restrict__ part, T *__restrict__ chk, int nwin,
                                                    const int *stop) {
@@ -539,8 +541,11 @@ __device__ inline bool qw_rows(unsigned kinds, CT (&a)[TW_S], const CT (&d)[TW_S
     return weak;
 }
 
+// Registers again: five wavefronts per SIMD in float, three in double (1024^2
+// cavity: 26 and 53 us a launch; 30 and 58 at the four and two the compiler
+// takes by itself, 32 and 88 at six and four).
 template <typename CT, int NT>
-__global__ __launch_bounds__(NT) void k_ql_window(long n, Chains cs, ChainT<float> h1, ChainT<float> h2,
+__global__ __launch_bounds__(NT, sizeof(CT) == 4 ? 5 : 3) void k_ql_window(long n, Chains cs, ChainT<float> h1, ChainT<float> h2,
                                                   const unsigned char *__restrict__ Z, QlFields F,
                                                   double *__restrict__ part, int nwin, int *weakf, const int *stop) {
     if (*stop) return;

@@ -775,16 +775,17 @@ static int naux_momentum(wd2_ctx *c, int mqiter, double dk, double re, double fr
 }
 
 // ------------------------------------------------------------------- Ppe
-// The levels at most tune.bside cells wide (and at most mg_bottom_side())
-// go to the bottom kernel; level 0 is always tiled.
-static int mg_retile(MgHierarchy &H) {
-    const int side = std::min(H.tune.bside, mg_bottom_side());
+// The levels at most tune.bside cells wide (and at most mg_bottom_side), or of
+// at most mg_tail_cells() cells, go to the bottom kernel; level 0 is always
+// tiled.
+static int mg_retile(wd2_ctx *c) {
+    MgHierarchy &H = c->mg;
+    const int side = std::min(H.tune.bside, mg_bottom_side(c->precision == WD2_PREC_MIXED));
     H.ntiled = 1;
-    while (H.ntiled < H.nlev && std::max(H.lev[H.ntiled].nx, H.lev[H.ntiled].ny) > side) H.ntiled++;
-    size_t cells = 0;
-    for (int l = H.ntiled; l < H.nlev; l++) cells += (size_t)(H.lev[l].nx + 2) * (H.lev[l].ny + 2);
-    if (H.ntiled >= H.nlev || cells > (size_t)mg_bottom_cells())
-        return fail(WD2_ERR_ARG, "multigrid: bottom levels do not fit (%zu cells)", cells);
+    while (H.ntiled < H.nlev && std::max(H.lev[H.ntiled].nx, H.lev[H.ntiled].ny) > side &&
+           H.lev[H.ntiled].nx * H.lev[H.ntiled].ny > mg_tail_cells())
+        H.ntiled++;
+    if (H.ntiled >= H.nlev) return fail(WD2_ERR_ARG, "multigrid: no level for the bottom kernel");
     return WD2_OK;
 }
 
@@ -810,8 +811,10 @@ static int mg_setup(wd2_ctx *c) {
         NY = (NY + 1) / 2;
     }
     H.tune = MgTune{256, 0, 64};
-    int st = mg_retile(H);
+    int st = mg_retile(c);
     if (st) return st;
+    const size_t tail = total;
+    total += mg_tail_bytes() / sizeof(double);
     HIPCHK(hipMalloc(&c->mg_store, total * sizeof(double)));
     c->mg_bytes = total * sizeof(double);
     HIPCHK(hipMemsetAsync(c->mg_store, 0, c->mg_bytes, c->s));
@@ -825,6 +828,7 @@ static int mg_setup(wd2_ctx *c) {
         L.ay = b + 3 * n;
         L.c = b + 4 * n;
     }
+    H.tail = c->mg_store + tail;
     const int nt = mg_tiles(H.lev[0].nx, H.lev[0].ny, nullptr);
     HIPCHK(hipMalloc(&c->mg_part, nt * sizeof(double)));
     return WD2_OK;
@@ -840,6 +844,7 @@ static int mg_prepare(wd2_ctx *c) {
         // float and double views share the storage: clear it (zero rings)
         if (c->mg_prec != -1 && c->mg_prec != c->precision)
             HIPCHK(hipMemsetAsync(c->mg_store, 0, c->mg_bytes, c->s));
+        if ((st = mg_retile(c))) return st;
         if (c->precision == WD2_PREC_MIXED)
             launch_mg_coef<float>(c->mg, c->nx, c->ny, c->ld, c->M.rau, c->M.rgv, uni, c->s);
         else
@@ -2494,9 +2499,9 @@ int wd2_ctx_mg_set_tune(wd2_ctx *c, int nt0, int stage, int bside) {
     graph_clear(c);
     const MgTune old = c->mg.tune;
     c->mg.tune = MgTune{nt0, stage, bside};
-    if ((st = mg_retile(c->mg))) {
+    if ((st = mg_retile(c))) {
         c->mg.tune = old;
-        (void)mg_retile(c->mg);
+        (void)mg_retile(c);
         return st;
     }
     return WD2_OK;
@@ -2526,22 +2531,20 @@ int wd2_ctx_mg_autotune(wd2_ctx *c, double dk, int cycles, double *best_us) {
     MgTune best = c->mg.tune;
     double tbest = 0.0;
     bool have = false;
-    for (int nt0 : {256, 512})
-        for (int stage : {0, 1})
-            for (int bside : {32, 64}) {
-                c->mg.tune = MgTune{nt0, stage, bside};
-                if (mg_retile(c->mg)) continue;
-                double us = 0.0;
-                (void)mg_cycle_time(c, 1, dk, &us);   // warm
-                if ((st = mg_cycle_time(c, cycles, dk, &us))) return st;
-                if (!have || us < tbest) {
-                    tbest = us;
-                    best = c->mg.tune;
-                    have = true;
-                }
-            }
+    for (int bside : {32, 64}) {
+        c->mg.tune.bside = bside;
+        if (mg_retile(c)) continue;
+        double us = 0.0;
+        (void)mg_cycle_time(c, 1, dk, &us);   // warm
+        if ((st = mg_cycle_time(c, cycles, dk, &us))) return st;
+        if (!have || us < tbest) {
+            tbest = us;
+            best = c->mg.tune;
+            have = true;
+        }
+    }
     c->mg.tune = best;
-    if ((st = mg_retile(c->mg))) return st;
+    if ((st = mg_retile(c))) return st;
     if (best_us) *best_us = tbest;
     return WD2_OK;
 }

@@ -290,16 +290,16 @@ void launch_filter(const Regions &R, const Thermal &TH, int ld, int ncomp, doubl
 // c (the correction after the up pass, which the next finer level
 // prolongates: a separate array, since an up launch reads e in its halos
 // while it writes); ax / ay its x- and y-face coefficients.  Levels
-// 0..ntiled-1 run as LDS tiles, the rest in the one-workgroup bottom kernel.
+// 0..ntiled-1 run as tiles, the rest in the one-workgroup bottom kernel.
 constexpr int MG_MAXLEV = 16;
 struct MgLevel {
     int nx, ny, ld;
     void *e, *r, *ax, *ay, *c;
 };
-// Shapes an autotuner chooses among (wd2_ctx_mg_autotune): threads of a
-// level-0 tile workgroup (256 or 512), whether the level-0 residual reads p
-// from an LDS copy of the tile (1) or straight from memory (0), and the
-// widest level the one-workgroup bottom kernel takes (32 or 64).
+// Shapes of the solver (wd2_ctx_mg_set_tune): bside is the widest level the
+// one-workgroup bottom kernel takes (32 or 64; at most mg_bottom_side);
+// nt0 and stage, shapes of an earlier level-0 kernel, are kept for callers
+// and change nothing.
 struct MgTune {
     int nt0, stage, bside;
 };
@@ -307,11 +307,13 @@ struct MgHierarchy {
     int nlev, ntiled;
     MgLevel lev[MG_MAXLEV];
     MgTune tune;
+    void *tail;   // the bottom kernel's tail matrix (mg_tail_bytes)
 };
-int mg_tiles(int NX, int NY, int *ntx);
-int mg_bottom_side();     // widest level the bottom kernel can take
-int mg_bottom_cells();    // LDS cells per array of the bottom kernel
-int mg_sweeps();          // smoothing sweeps before and after
+int mg_tiles(int NX, int NY, int *ntx);   // level-0 down tiles
+int mg_bottom_side(int fp32);   // widest level the bottom kernel can take in FP32 / FP64
+int mg_tail_cells();            // most cells of a level the tail matrix covers
+size_t mg_tail_bytes();
+// Level coefficients and the tail matrix.
 template <typename T>
 void launch_mg_coef(const MgHierarchy &H, int nx, int ny, int ld, const double *rau, const double *rgv,
                     const double *uni, hipStream_t s);
