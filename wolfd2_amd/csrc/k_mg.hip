@@ -31,7 +31,7 @@
 //   neighbours, zero outside the grid;
 // * the wider levels run as 64 x 64 tiles, one launch per level down (smooth,
 //   residual, restrict) and one up (prolong, smooth); the levels of at most
-//   64 cells a side (32 in FP64) run in one workgroup (the bottom kernel), and
+//   64 cells a side run in one workgroup (the bottom kernel), and
 //   from the first level of at most 64 cells in all the rest of the V-cycle
 //   is one product with its matrix, built with the coefficients.
 //
@@ -114,8 +114,6 @@ __global__ void k_mg_coarsen(MgLevel F, MgLevel C, T sb) {
         cy[mfy(C.ld, I, J)] = v;
     }
 }
-
-__device__ inline bool mg_stopped(const Scalars *sc) { return sc->mg_done != 0; }
 
 // The stopping test before V-cycle `cycle` (1-based), evaluated by every
 // workgroup of the first kernel after the level-0 down kernel from that
@@ -218,7 +216,7 @@ struct Strip {
 // y-faces (fs[j] south of row j) and right-hand sides; in: the row's point
 // is in the grid; I, NX: its column and the level's width.
 template <typename T>
-__device__ inline void strip_build(Strip<T> &S, int q, const T (&fw)[4], const T (&fe)[4], const T (&fs)[5],
+__device__ __forceinline__ void strip_build(Strip<T> &S, int q, const T (&fw)[4], const T (&fe)[4], const T (&fs)[5],
                                    const T (&r)[4], const bool (&in)[4], int I, int NX) {
     SPt<T> v[4];
     T d[4];
@@ -241,15 +239,21 @@ __device__ inline void strip_build(Strip<T> &S, int q, const T (&fw)[4], const T
     }
 #undef SEL
 }
+// q ? x : y by value (a conditional of two members would keep the strip in
+// memory).
 template <typename T>
-__device__ inline T strip_eval(const SPt<T> &c, T row, T mate, T other) {
+__device__ __forceinline__ T sel(bool q, T x, T y) {
+    return q ? x : y;
+}
+template <typename T>
+__device__ __forceinline__ T strip_eval(const SPt<T> &c, T row, T mate, T other) {
     // the value from the next strip, read from LDS, enters last
     return fma(c.o, other, fma(c.w, sh_w(row), fma(c.e, sh_e(row), fma(c.m, mate, c.r))));
 }
 // Row j's value.
 template <typename T>
-__device__ inline T strip_row(const Strip<T> &S, int q, int j) {
-    return ((j & 1) == q) ? S.A[j >> 1] : S.B[j >> 1];
+__device__ __forceinline__ T strip_row(const Strip<T> &S, int q, int j) {
+    return sel((j & 1) == q, S.A[j >> 1], S.B[j >> 1]);
 }
 
 // The rows at the strips' ends in LDS: end (s, h) is strip s's row 0 (h = 0)
@@ -266,36 +270,36 @@ struct Ends {
 
 // Sweep phases; s: the lane's strip.
 template <typename T>
-__device__ inline void phase_a(Strip<T> &S, int q, int s, const Ends<T> &E) {
+__device__ __forceinline__ void phase_a(Strip<T> &S, int q, int s, const Ends<T> &E) {
     const T x = q ? E.at(s + 1, 0) : E.at(s - 1, 1);
-    const T a0 = strip_eval(S.a[0], S.B[0], S.B[0], q ? S.B[1] : x);
-    const T a1 = strip_eval(S.a[1], S.B[1], S.B[1], q ? x : S.B[0]);
+    const T a0 = strip_eval(S.a[0], S.B[0], S.B[0], sel(q, S.B[1], x));
+    const T a1 = strip_eval(S.a[1], S.B[1], S.B[1], sel(q, x, S.B[0]));
     S.A[0] = a0;
     S.A[1] = a1;
     E.at(s, q) = q ? a1 : a0;
 }
 template <typename T>
-__device__ inline void phase_b(Strip<T> &S, int q, int s, const Ends<T> &E) {
+__device__ __forceinline__ void phase_b(Strip<T> &S, int q, int s, const Ends<T> &E) {
     const T x = q ? E.at(s - 1, 1) : E.at(s + 1, 0);
-    const T b0 = strip_eval(S.b[0], S.A[0], S.A[0], q ? x : S.A[1]);
-    const T b1 = strip_eval(S.b[1], S.A[1], S.A[1], q ? S.A[0] : x);
+    const T b0 = strip_eval(S.b[0], S.A[0], S.A[0], sel(q, x, S.A[1]));
+    const T b1 = strip_eval(S.b[1], S.A[1], S.A[1], sel(q, S.A[0], x));
     S.B[0] = b0;
     S.B[1] = b1;
     E.at(s, q ^ 1) = q ? b0 : b1;
 }
 // Both end rows (after a prolongation).
 template <typename T>
-__device__ inline void ends_put(const Strip<T> &S, int q, int s, const Ends<T> &E) {
-    E.at(s, 0) = q ? S.B[0] : S.A[0];
-    E.at(s, 1) = q ? S.A[1] : S.B[1];
+__device__ __forceinline__ void ends_put(const Strip<T> &S, int q, int s, const Ends<T> &E) {
+    E.at(s, 0) = sel(q, S.B[0], S.A[0]);
+    E.at(s, 1) = sel(q, S.A[1], S.B[1]);
 }
 // NU sweeps from e = 0, colours 0 then 1 (the first phase's neighbours are 0).
 // act: the lane holds a strip (others only take part in the syncs).
 template <typename T, typename Sync>
-__device__ inline void sweep_down(Strip<T> &S, int q, int s, const Ends<T> &E, bool act, Sync sync) {
+__device__ __forceinline__ void sweep_down(Strip<T> &S, int q, int s, const Ends<T> &E, bool act, Sync sync) {
     S.A[0] = S.a[0].r;
     S.A[1] = S.a[1].r;
-    if (act) E.at(s, q) = q ? S.A[1] : S.A[0];
+    if (act) E.at(s, q) = sel(q, S.A[1], S.A[0]);
     sync();
 #pragma unroll
     for (int k = 0; k < MG_NU; k++) {
@@ -306,7 +310,7 @@ __device__ inline void sweep_down(Strip<T> &S, int q, int s, const Ends<T> &E, b
     }
 }
 template <typename T, typename Sync>
-__device__ inline void sweep_up(Strip<T> &S, int q, int s, const Ends<T> &E, bool act, Sync sync) {
+__device__ __forceinline__ void sweep_up(Strip<T> &S, int q, int s, const Ends<T> &E, bool act, Sync sync) {
     if (act) ends_put(S, q, s, E);
     sync();
 #pragma unroll
@@ -322,10 +326,10 @@ __device__ inline void sweep_up(Strip<T> &S, int q, int s, const Ends<T> &E, boo
 // residuals are zero; colour 0's are the diagonal times what one more
 // relaxation would add.
 template <typename T>
-__device__ inline void strip_restrict(const Strip<T> &S, int q, int s, const Ends<T> &E, T (&rc)[2]) {
+__device__ __forceinline__ void strip_restrict(const Strip<T> &S, int q, int s, const Ends<T> &E, T (&rc)[2]) {
     const T x = q ? E.at(s + 1, 0) : E.at(s - 1, 1);
-    const T g0 = strip_eval(S.a[0], S.B[0], S.B[0], q ? S.B[1] : x);
-    const T g1 = strip_eval(S.a[1], S.B[1], S.B[1], q ? x : S.B[0]);
+    const T g0 = strip_eval(S.a[0], S.B[0], S.B[0], sel(q, S.B[1], x));
+    const T g1 = strip_eval(S.a[1], S.B[1], S.B[1], sel(q, x, S.B[0]));
     const T r0 = S.d[0] * (g0 - S.A[0]), r1 = S.d[1] * (g1 - S.A[1]);
     rc[0] = r0 + sh_x(r0);
     rc[1] = r1 + sh_x(r1);
@@ -333,7 +337,7 @@ __device__ inline void strip_restrict(const Strip<T> &S, int q, int s, const End
 // e += prolongation: h[k] = 3 c + c' of the coarse rows jc0 - 1 .. jc0 + 2 on
 // the column's coarse cell (c) and its horizontal neighbour (c').
 template <typename T>
-__device__ inline T prolong(const T (&h)[4], int j) {
+__device__ __forceinline__ T prolong(const T (&h)[4], int j) {
     const int k = (j >> 1) + 1;
     return (T(3) * h[k] + h[(j & 1) ? k + 1 : k - 1]) * T(0.0625);
 }
@@ -353,10 +357,13 @@ __global__ __launch_bounds__(MG_NT) void k_mg_down(MgLevel L, MgLevel C, int ntx
                                                    const double *__restrict__ rau, const double *__restrict__ rgv,
                                                    int uni, double rau_c, double rgv_c, double *__restrict__ part,
                                                    MgDecide D, Scalars *sc) {
-    if (mg_stopped(sc)) return;
+    // below level 0 the tile's loads are in flight before the flag is looked
+    // at (level 0's would cost a launch that returns here more than it saves
+    // one that runs)
+    const int stopped = sc->mg_done;
+    if (L0 && stopped) return;
     __shared__ T ends[(MG_NS + 2) * 2 * MG_TW];
     __shared__ double red[MG_NT / 64];
-    if (D.nt > 0 && mg_decide<MG_NT>(D.part, D.nt, D.dk, D.tol, D.cycle, D.maxcyc, D.minc, sc, red)) return;
     const int tile = mg_tile(ntiles);
     if (tile >= ntiles) return;
     const int I0 = (tile % ntx) * MG_OD, J0 = (tile / ntx) * MG_OD;
@@ -365,11 +372,6 @@ __global__ __launch_bounds__(MG_NT) void k_mg_down(MgLevel L, MgLevel C, int ntx
     const int I = I0 - MG_HD + x, Jb = J0 - MG_HD + MG_SR * s;
     const bool inx = I >= 0 && I < NX;
     const bool ownx = inx && x >= MG_HD && x < MG_HD + MG_OD;
-    if (s == 0 || s == MG_NS - 1) {   // the zero rows beyond the strips
-        const int g = s == 0 ? -1 : MG_NS;
-        ends[((g + 1) * 2) * MG_TW + x] = T(0);
-        ends[((g + 1) * 2 + 1) * MG_TW + x] = T(0);
-    }
     bool in[4];
     T fw[4], fe[4], fs[5], rv[4];
     double rmax = 0.0;
@@ -414,20 +416,25 @@ __global__ __launch_bounds__(MG_NT) void k_mg_down(MgLevel L, MgLevel C, int ntx
         for (int j = 0; j < 5; j++) fs[j] = (T)a5[j];
     } else {
         const T *r = (const T *)L.r, *ax = (const T *)L.ax, *ay = (const T *)L.ay;
-        const bool fx = I >= 0 && I <= NX;
+        // clamped addresses (values outside serve only points outside)
+        const int Ic = min(max(I, 0), NX - 1), If = min(max(I, 0), NX);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int J = Jb + j;
-            rv[j] = in[j] ? r[mc(L.ld, I, J)] : T(0);
-            fw[j] = (fx && J >= 0 && J < NY) ? ax[mfx(L.ld, I, J)] : T(0);
+            const int J = min(max(Jb + j, 0), NY - 1);
+            rv[j] = r[mc(L.ld, Ic, J)];
+            fw[j] = ax[mfx(L.ld, If, J)];
         }
 #pragma unroll
-        for (int j = 0; j < 5; j++) {
-            const int J = Jb + j;
-            fs[j] = (inx && J >= 0 && J <= NY) ? ay[mfy(L.ld, I, J)] : T(0);
-        }
+        for (int j = 0; j < 5; j++) fs[j] = ay[mfy(L.ld, Ic, min(max(Jb + j, 0), NY))];
 #pragma unroll
         for (int j = 0; j < 4; j++) fe[j] = sh_e(fw[j]);
+    }
+    if (stopped) return;
+    if (D.nt > 0 && mg_decide<MG_NT>(D.part, D.nt, D.dk, D.tol, D.cycle, D.maxcyc, D.minc, sc, red)) return;
+    if (s == 0 || s == MG_NS - 1) {   // the zero rows beyond the strips
+        const int g = s == 0 ? -1 : MG_NS;
+        ends[((g + 1) * 2) * MG_TW + x] = T(0);
+        ends[((g + 1) * 2 + 1) * MG_TW + x] = T(0);
     }
     Strip<T> S;
     strip_build<T>(S, q, fw, fe, fs, rv, in, I, NX);
@@ -473,7 +480,8 @@ __global__ __launch_bounds__(MG_NT) void k_mg_up(MgLevel L, MgLevel C, int ntx, 
                                                  double *__restrict__ p, const double *__restrict__ rau,
                                                  const double *__restrict__ rgv, int uni, double rau_c, double rgv_c,
                                                  const Scalars *sc) {
-    if (mg_stopped(sc)) return;
+    const int stopped = sc->mg_done;
+    if (L0 && stopped) return;
     __shared__ T ends[(MG_NS + 2) * 2 * MG_TW];
     const int tile = mg_tile(ntiles);
     if (tile >= ntiles) return;
@@ -482,11 +490,7 @@ __global__ __launch_bounds__(MG_NT) void k_mg_up(MgLevel L, MgLevel C, int ntx, 
     const int x = threadIdx.x & 63, s = threadIdx.x >> 6, q = x & 1;
     const int I = I0 - MG_HU + x, Jb = J0 - MG_HU + MG_SR * s;
     const bool inx = I >= 0 && I < NX;
-    if (s == 0 || s == MG_NS - 1) {
-        const int g = s == 0 ? -1 : MG_NS;
-        ends[((g + 1) * 2) * MG_TW + x] = T(0);
-        ends[((g + 1) * 2 + 1) * MG_TW + x] = T(0);
-    }
+    const int Ic = min(max(I, 0), NX - 1);   // addresses are clamped to the grid
     const T *e = (const T *)L.e, *r = (const T *)L.r, *ec = (const T *)C.c;
     bool in[4];
     T fw[4], fe[4], fs[5], rv[4], ev[4], h[4];
@@ -502,8 +506,9 @@ __global__ __launch_bounds__(MG_NT) void k_mg_up(MgLevel L, MgLevel C, int ntx, 
     }
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        ev[j] = in[j] ? e[mc(L.ld, I, Jb + j)] : T(0);
-        rv[j] = in[j] ? r[mc(L.ld, I, Jb + j)] : T(0);
+        const int J = min(max(Jb + j, 0), NY - 1);
+        ev[j] = e[mc(L.ld, Ic, J)];
+        rv[j] = r[mc(L.ld, Ic, J)];
     }
     if (L0) {
         const int i = min(max(I + 2, 0), nx + 1);
@@ -516,19 +521,19 @@ __global__ __launch_bounds__(MG_NT) void k_mg_up(MgLevel L, MgLevel C, int ntx, 
         for (int j = 0; j < 4; j++) fw[j] = uni ? (T)rau_c : sh_w(fe[j]);
     } else {
         const T *ax = (const T *)L.ax, *ay = (const T *)L.ay;
-        const bool fx = I >= 0 && I <= NX;
+        const int If = min(max(I, 0), NX);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int J = Jb + j;
-            fw[j] = (fx && J >= 0 && J < NY) ? ax[mfx(L.ld, I, J)] : T(0);
-        }
+        for (int j = 0; j < 4; j++) fw[j] = ax[mfx(L.ld, If, min(max(Jb + j, 0), NY - 1))];
 #pragma unroll
-        for (int j = 0; j < 5; j++) {
-            const int J = Jb + j;
-            fs[j] = (inx && J >= 0 && J <= NY) ? ay[mfy(L.ld, I, J)] : T(0);
-        }
+        for (int j = 0; j < 5; j++) fs[j] = ay[mfy(L.ld, Ic, min(max(Jb + j, 0), NY))];
 #pragma unroll
         for (int j = 0; j < 4; j++) fe[j] = sh_e(fw[j]);
+    }
+    if (stopped) return;
+    if (s == 0 || s == MG_NS - 1) {
+        const int g = s == 0 ? -1 : MG_NS;
+        ends[((g + 1) * 2) * MG_TW + x] = T(0);
+        ends[((g + 1) * 2 + 1) * MG_TW + x] = T(0);
     }
     Strip<T> S;
     strip_build<T>(S, q, fw, fe, fs, rv, in, I, NX);
@@ -559,37 +564,101 @@ __global__ __launch_bounds__(MG_NT) void k_mg_up(MgLevel L, MgLevel C, int ntx, 
 // The bottom levels in one workgroup.  Levels of more than MG_TAIL cells are
 // strips in registers (a level of NX cells a row takes lw = 2^k >= NX lanes a
 // strip, so a narrow level packs several strips into a wavefront; a level
-// that fits one wavefront needs only wavefront syncs).  From the first level
-// of at most MG_TAIL cells on, the rest of the V-cycle is linear in that
-// level's right-hand side: c = M r, with M built by k_mg_tail when the
-// coefficients are (about thirty dependent phases on a handful of points
-// otherwise).  Level 0's r comes from the down kernel above; its correction
-// goes to c for the up kernel above.  D.nt > 0: the stopping test is
-// evaluated first.  The face loads of all levels are issued before the first
-// smoothing phase.
+// that fits one wavefront is run by wavefront 0 alone, between wavefront
+// syncs).  From the first level of at most MG_TAIL cells on, the rest of the
+// V-cycle is linear in that level's right-hand side: c = M r, with M built by
+// k_mg_tail when the coefficients are (about thirty dependent phases on a
+// handful of points otherwise).  Level 0's r comes from the down kernel
+// above; its correction goes to c for the up kernel above.  D.nt > 0: the
+// stopping test is evaluated first.
+//
+// The kernel runs once through its code on one CU, whose instruction cache
+// holds none of it at launch: unrolled over the levels it was 37 KB and took
+// 20 us, most of it instruction fetches.  So the levels are a loop over one
+// copy of each half, their strip coefficients come ready-made from memory
+// (k_mg_pack), loaded one level ahead, and the strips wait in LDS while the
+// coarser levels run.
 struct MgBottom {
     MgLevel lev[MG_NREG + 1];
-    int nreg;          // register levels; lev[nreg] is the tail's level
-    const void *tail;  // M, column j at [MG_TAIL j]
+    const void *pack[MG_NREG];   // the register levels' strip coefficients
+    int nreg;                    // register levels; lev[nreg] is the tail's level
+    const void *tail;            // M, column j at [MG_TAIL j]
 };
+// (FP64 strips of a 64-wide level, with the next level's coefficients in
+// flight, exceed the 128 registers 1024 lanes can have: 26 us a launch
+// against 9 with the 64-wide level as a tile launch down and up of 5 us each)
 template <typename T>
 constexpr int mg_bottom_width() { return sizeof(T) == 4 ? 64 : 32; }
 
+// Lanes of a level's strips.
+struct BtGeo {
+    int k, ns;   // 2^k lanes a strip, ns strips
+    __device__ BtGeo(const MgLevel &L)
+        : k(L.nx > 32 ? 6 : (L.nx > 16 ? 5 : (L.nx > 8 ? 4 : 3))), ns((L.ny + MG_SR - 1) / MG_SR) {}
+    __device__ int lanes() const { return ns << k; }
+    __device__ bool wave() const { return lanes() <= 64; }
+};
+// A lane's coefficients in a pack: value v of lane t at [v lanes + t], the
+// points a[0], a[1], b[0], b[1] with r = 1, then the diagonals d.
+constexpr int BT_PACK = 22;
 template <typename T>
+struct BtCoef {
+    T v[BT_PACK];
+    __device__ SPt<T> pt(int p, T r) const {
+        return SPt<T>{v[5 * p], v[5 * p + 1], v[5 * p + 2], v[5 * p + 3], v[5 * p + 4] * r};
+    }
+};
+
+template <typename T>
+__global__ __launch_bounds__(1024) void k_mg_pack(MgLevel L, T *__restrict__ P) {
+    const BtGeo g(L);
+    const int t = threadIdx.x, x = t & ((1 << g.k) - 1), s = t >> g.k;
+    if (s >= g.ns) return;
+    const T *ax = (const T *)L.ax, *ay = (const T *)L.ay;
+    T fw[4], fe[4], fs[5], one[4];
+    bool in[4];
+    for (int j = 0; j < 5; j++) {
+        const int J = MG_SR * s + j;
+        const bool c = x < L.nx && J < L.ny;
+        fs[j] = (x < L.nx && J <= L.ny) ? ay[mfy(L.ld, x, J)] : T(0);
+        if (j == 4) break;
+        in[j] = c;
+        one[j] = T(1);
+        fw[j] = c ? ax[mfx(L.ld, x, J)] : T(0);
+        fe[j] = c ? ax[mfx(L.ld, x + 1, J)] : T(0);
+    }
+    Strip<T> S;
+    strip_build<T>(S, x & 1, fw, fe, fs, one, in, x, L.nx);
+    for (int p = 0; p < 4; p++) {
+        const SPt<T> &c = p < 2 ? S.a[p & 1] : S.b[p & 1];
+        T *o = P + (size_t)5 * p * g.lanes() + t;
+        o[0] = c.w;
+        o[g.lanes()] = c.e;
+        o[2 * g.lanes()] = c.m;
+        o[3 * g.lanes()] = c.o;
+        o[4 * g.lanes()] = c.r;
+    }
+    P[(size_t)20 * g.lanes() + t] = S.d[0];
+    P[(size_t)21 * g.lanes() + t] = S.d[1];
+}
+
+// LDS of the bottom kernel.  Level l >= 1 has at most 32 x 32 (l = 1), 16 x 16
+// (l = 2) cells and lanes 256, 64; the tail's level at most MG_TAIL cells, in
+// at most (MG_TAIL + 2) x 3 places with its ring.
+template <typename T, int NT>
 struct BtShared {
     T ends[(MG_NS + 2) * 2 * 64];
     T r[32 * 32 + 16 * 16 + MG_TAIL];            // right-hand sides of the levels below the first
     T c[34 * 34 + 18 * 18 + (MG_TAIL + 2) * 3];  // their corrections, with a zero ring
+    T sv[4 * (NT + 256 + 64)];                   // strips of the levels above the running one
     T m[MG_TAIL * MG_TAIL];
     double red[1024 / 64];
 };
-// Offsets of level l >= 1 in r and c.  A level of n cells of the register
-// kind has at most 32 x 32 (l = 1) and 16 x 16 (l = 2) cells; the tail's level
-// at most MG_TAIL, in at most (MG_TAIL + 2) x 3 places with its ring.
 __device__ inline int bt_roff(int l) { return l == 1 ? 0 : (l == 2 ? 1024 : 1280); }
 __device__ inline int bt_coff(int l) { return l == 1 ? 0 : (l == 2 ? 1156 : 1480); }
+template <int NT>
+__device__ inline int bt_soff(int l) { return l == 0 ? 0 : (l == 1 ? 4 * NT : 4 * (NT + 256)); }
 
-__device__ inline int bt_lw(int NX) { return NX > 32 ? 6 : (NX > 16 ? 5 : (NX > 8 ? 4 : 3)); }
 __device__ inline void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -597,189 +666,179 @@ __device__ inline void wave_sync() {
 }
 
 template <typename T, int NT>
-struct Bottom {
-    const MgBottom &B;
-    BtShared<T> &H;
-    // the face values of one level's strip (fl: the last column's east faces)
-    struct Faces {
-        T fw[4], fl[4], fs[5];
+__global__ __launch_bounds__(NT) void k_mg_bottom(MgBottom B, MgDecide D, Scalars *sc) {
+    const int stopped = sc->mg_done;
+    __shared__ BtShared<T, NT> H;
+    const int t = threadIdx.x;
+    auto load = [&](int l) {
+        const int n = BtGeo(B.lev[l]).lanes();
+        const T *P = (const T *)B.pack[l] + min(t, n - 1);
+        BtCoef<T> K;
+#pragma unroll
+        for (int v = 0; v < BT_PACK; v++) K.v[v] = P[(size_t)v * n];
+        return K;
     };
-    struct Lane {
-        int x, s, lw, ns;
-        bool act;
+    // a lane's strip of level l from its coefficients and right-hand sides
+    // (lanes past the level's points have clamped addresses)
+    T r0[4] = {T(0), T(0), T(0), T(0)};   // the first level's right-hand sides
+    auto strip = [&](int l, const MgLevel &L, int x, int s, int q, const BtCoef<T> &K, Strip<T> &S) {
+        T rv[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            rv[j] = l == 0 ? r0[j] : H.r[bt_roff(l) + min(x, L.nx - 1) + L.nx * min(MG_SR * s + j, L.ny - 1)];
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            S.a[k] = K.pt(k, sel(q, rv[2 * k + 1], rv[2 * k]));
+            S.b[k] = K.pt(2 + k, sel(q, rv[2 * k], rv[2 * k + 1]));
+            S.d[k] = K.v[20 + k];
+        }
     };
-    __device__ Lane lane(int l) const {
-        const int NX = B.lev[l].nx, k = bt_lw(NX);
-        Lane n;
-        n.lw = 1 << k;
-        n.x = threadIdx.x & (n.lw - 1);
-        n.s = threadIdx.x >> k;
-        n.ns = (B.lev[l].ny + MG_SR - 1) / MG_SR;
-        n.act = n.s < n.ns;
-        return n;
+    // the first level's right-hand side and coefficients, the tail matrix
+    const MgLevel &L0 = B.lev[0];
+    BtCoef<T> K{};
+    if (B.nreg > 0) {
+        const BtGeo g(L0);
+        const int x = t & ((1 << g.k) - 1), s = t >> g.k;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            r0[j] = ((const T *)L0.r)[mc(L0.ld, min(x, L0.nx - 1), min(MG_SR * s + j, L0.ny - 1))];
+        K = load(0);
     }
-    __device__ void load(int l, Faces &F) const {
-        const MgLevel &L = B.lev[l];
-        const Lane n = lane(l);
-        const T *ax = (const T *)L.ax, *ay = (const T *)L.ay;
+    constexpr int MV = MG_TAIL * MG_TAIL / NT;
+    T mv[MV];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int J = MG_SR * n.s + j;
-            F.fw[j] = (n.act && n.x < L.nx && J < L.ny) ? ax[mfx(L.ld, n.x, J)] : T(0);
-            F.fl[j] = (n.act && n.x == L.nx - 1 && J < L.ny) ? ax[mfx(L.ld, L.nx, J)] : T(0);
-        }
+    for (int k = 0; k < MV; k++) mv[k] = ((const T *)B.tail)[t + NT * k];
+    if (stopped) return;
+    if (D.nt > 0 && mg_decide<NT>(D.part, D.nt, D.dk, D.tol, D.cycle, D.maxcyc, D.minc, sc, H.red)) return;
+    if (B.nreg == 0 && t < L0.nx * L0.ny) H.r[bt_roff(0) + t] = ((const T *)L0.r)[mc(L0.ld, t % L0.nx, t / L0.nx)];
 #pragma unroll
-        for (int j = 0; j < 5; j++) {
-            const int J = MG_SR * n.s + j;
-            F.fs[j] = (n.act && n.x < L.nx && J <= L.ny) ? ay[mfy(L.ld, n.x, J)] : T(0);
-        }
-    }
-    // the V-cycle from level l on; wave: one wavefront is left running it
-    template <int l>
-    __device__ void run(Faces (&F)[MG_NREG], const T (&r0)[4], bool wave) {
-        if (l == B.nreg || l == MG_NREG) {
-            tail(l);
-            return;
-        }
-        if constexpr (l < MG_NREG) {
-            const MgLevel &L = B.lev[l];
-            const Lane n = lane(l);
-            const int q = n.x & 1;
-            auto sync = [&] {
-                if (wave)
-                    wave_sync();
-                else
-                    __syncthreads();
-            };
-            Strip<T> S;
-            {
-                bool in[4];
-                T rv[4], fe[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int J = MG_SR * n.s + j;
-                    in[j] = n.act && n.x < L.nx && J < L.ny;
-                    rv[j] = l == 0 ? r0[j] : (in[j] ? H.r[bt_roff(l) + n.x + L.nx * J] : T(0));
-                    // the east face is the next lane's west face
-                    const T nf = sh_e(F[l].fw[j]);
-                    fe[j] = n.x == L.nx - 1 ? F[l].fl[j] : nf;
-                }
-                strip_build<T>(S, q, F[l].fw, fe, F[l].fs, rv, in, n.x, L.nx);
-            }
-            const Ends<T> E{H.ends + n.x, n.lw};
-            if (n.act) {   // zero rows beyond the strips
-                if (n.s == 0) { E.at(-1, 0) = T(0); E.at(-1, 1) = T(0); }
-                if (n.s == n.ns - 1) { E.at(n.ns, 0) = T(0); E.at(n.ns, 1) = T(0); }
-            }
-            sweep_down<T>(S, q, n.s, E, n.act, sync);
-            const MgLevel &C = B.lev[l + 1];
-            T rc[2];
-            if (n.act) {
-                strip_restrict<T>(S, q, n.s, E, rc);
-#pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    const int Ic = n.x >> 1, Jc = 2 * n.s + k;
-                    if (q == 0 && Ic < C.nx && Jc < C.ny) H.r[bt_roff(l + 1) + Ic + C.nx * Jc] = rc[k];
-                }
-            }
-            sync();
-            // the next level, in one wavefront where its strips fit one
-            const Lane nn = lane(l + 1);
-            const bool one = l + 1 == B.nreg || nn.lw * nn.ns <= 64;
-            if (wave || !one) {
-                run<l + 1>(F, r0, wave);
-            } else {
-                if (threadIdx.x < 64) run<l + 1>(F, r0, true);
+    for (int k = 0; k < MV; k++) H.m[t + NT * k] = mv[k];
+    for (int k = t; k < (int)(sizeof(H.c) / sizeof(T)); k += NT) H.c[k] = T(0);
+    __syncthreads();
+#pragma unroll 1
+    for (int l = 0; l < B.nreg; l++) {
+        const MgLevel &L = B.lev[l], &C = B.lev[l + 1];
+        const BtGeo g(L);
+        const bool wave = g.wave();
+        if (wave && t >= 64) break;
+        const int x = t & ((1 << g.k) - 1), s = t >> g.k, q = x & 1, n = g.lanes();
+        const bool act = s < g.ns;
+        auto sync = [&] {
+            if (wave)
+                wave_sync();
+            else
                 __syncthreads();
+        };
+        BtCoef<T> N{};
+        if (l + 1 < B.nreg) N = load(l + 1);
+        Strip<T> S;
+        strip(l, L, x, s, q, K, S);
+        const Ends<T> E{H.ends + x, 1 << g.k};
+        if (act && s == 0) E.at(-1, 0) = E.at(-1, 1) = T(0);
+        if (act && s == g.ns - 1) E.at(g.ns, 0) = E.at(g.ns, 1) = T(0);
+        sweep_down<T>(S, q, s, E, act, sync);
+        if (act) {
+            T rc[2];
+            strip_restrict<T>(S, q, s, E, rc);
+            T *sv = H.sv + bt_soff<NT>(l) + t;
+#pragma unroll
+            for (int k = 0; k < 2; k++) {
+                const int Ic = x >> 1, Jc = 2 * s + k;
+                if (q == 0 && Ic < C.nx && Jc < C.ny) H.r[bt_roff(l + 1) + Ic + C.nx * Jc] = rc[k];
+                sv[k * n] = S.A[k];
+                sv[(2 + k) * n] = S.B[k];
             }
-            // prolongation (the ring of the coarse correction is zero)
-            if (n.act) {
-                const int W = C.nx + 2;
-                const T *c = H.c + bt_coff(l + 1);
-                const int ic = min(n.x >> 1, C.nx - 1) + 1, i2 = ic + (q ? 1 : -1);
-                T h[4];
-#pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    const int jc = min(2 * n.s + k, C.ny + 1);   // padded row of 2 s - 1 + k
-                    h[k] = T(3) * c[ic + W * jc] + c[i2 + W * jc];
-                }
-                T v[4];
-#pragma unroll
-                for (int j = 0; j < 4; j++)
-                    v[j] = (n.x < L.nx && MG_SR * n.s + j < L.ny) ? prolong<T>(h, j) : T(0);
-#pragma unroll
-                for (int k = 0; k < 2; k++) {
-                    S.A[k] += q ? v[2 * k + 1] : v[2 * k];
-                    S.B[k] += q ? v[2 * k] : v[2 * k + 1];
-                }
-                // (the zero rows are this level's again)
-                if (n.s == 0) { E.at(-1, 0) = T(0); E.at(-1, 1) = T(0); }
-                if (n.s == n.ns - 1) { E.at(n.ns, 0) = T(0); E.at(n.ns, 1) = T(0); }
-            }
-            sweep_up<T>(S, q, n.s, E, n.act, sync);
-            if (n.act) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const int J = MG_SR * n.s + j;
-                    if (n.x >= L.nx || J >= L.ny) continue;
-                    const T v = strip_row(S, q, j);
-                    if (l == 0)
-                        ((T *)L.c)[mc(L.ld, n.x, J)] = v;
-                    else
-                        H.c[bt_coff(l) + n.x + 1 + (L.nx + 2) * (J + 1)] = v;
-                }
-            }
-            if (l > 0) sync();
         }
+        sync();
+        if (l + 1 < B.nreg) K = N;
     }
-    // c = M r on the tail's level
-    __device__ void tail(int l) {
-        const MgLevel &L = B.lev[l];
-        const int n = L.nx * L.ny, t = threadIdx.x;
+    if (t < 64) {   // c = M r on the tail's level
+        const MgLevel &L = B.lev[B.nreg];
+        const int n = L.nx * L.ny;
         if (t < n) {
-            const T *r = H.r + bt_roff(l);
+            const T *r = H.r + bt_roff(B.nreg);
             T acc[4] = {T(0), T(0), T(0), T(0)};
-            for (int j = 0; j < n; j += 4)
+            constexpr int U = 16;   // LDS reads in flight
+            for (int j = 0; j < n; j += U) {
+                T mm[U], rr[U];
 #pragma unroll
-                for (int u = 0; u < 4; u++)
-                    if (j + u < n) acc[u] = fma(H.m[MG_TAIL * (j + u) + t], r[j + u], acc[u]);
+                for (int u = 0; u < U; u++) {
+                    const int c = min(j + u, n - 1);
+                    mm[u] = H.m[MG_TAIL * c + t];
+                    rr[u] = r[c];
+                }
+#pragma unroll
+                for (int u = 0; u < U; u++) acc[u & 3] = fma(mm[u], j + u < n ? rr[u] : T(0), acc[u & 3]);
+            }
             const T v = (acc[0] + acc[1]) + (acc[2] + acc[3]);
             const int I = t % L.nx, J = t / L.nx;
-            if (l == 0)
+            if (B.nreg == 0)
                 ((T *)L.c)[mc(L.ld, I, J)] = v;
             else
-                H.c[bt_coff(l) + I + 1 + (L.nx + 2) * (J + 1)] = v;
+                H.c[bt_coff(B.nreg) + I + 1 + (L.nx + 2) * (J + 1)] = v;
         }
         wave_sync();
     }
-};
-
-template <typename T, int NT>
-__global__ __launch_bounds__(NT) void k_mg_bottom(MgBottom B, MgDecide D, Scalars *sc) {
-    if (mg_stopped(sc)) return;
-    __shared__ BtShared<T> H;
-    if (D.nt > 0 && mg_decide<NT>(D.part, D.nt, D.dk, D.tol, D.cycle, D.maxcyc, D.minc, sc, H.red)) return;
-    Bottom<T, NT> K{B, H};
-    typename Bottom<T, NT>::Faces F[MG_NREG];
-    T r0[4] = {T(0), T(0), T(0), T(0)};
-    const MgLevel &L = B.lev[0];
-    if (B.nreg > 0) {
-        const auto n = K.lane(0);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int J = MG_SR * n.s + j;
-            if (n.act && n.x < L.nx && J < L.ny) r0[j] = ((const T *)L.r)[mc(L.ld, n.x, J)];
+#pragma unroll 1
+    for (int l = B.nreg - 1; l >= 0; l--) {
+        const MgLevel &L = B.lev[l], &C = B.lev[l + 1];
+        const BtGeo g(L);
+        const bool wave = g.wave();
+        // the other wavefronts join where the levels outgrow one
+        if (!wave && (l == B.nreg - 1 || BtGeo(C).wave())) __syncthreads();
+        if (wave && t >= 64) {
+            if (l > 0 && !BtGeo(B.lev[l - 1]).wave()) K = load(l - 1);
+            continue;
         }
-    } else if ((int)threadIdx.x < L.nx * L.ny) {
-        H.r[bt_roff(0) + threadIdx.x] = ((const T *)L.r)[mc(L.ld, threadIdx.x % L.nx, threadIdx.x / L.nx)];
-    }
+        const int x = t & ((1 << g.k) - 1), s = t >> g.k, q = x & 1, n = g.lanes();
+        const bool act = s < g.ns;
+        auto sync = [&] {
+            if (wave)
+                wave_sync();
+            else
+                __syncthreads();
+        };
+        BtCoef<T> N{};
+        if (l > 0) N = load(l - 1);
+        Strip<T> S;
+        strip(l, L, x, s, q, K, S);
+        const T *sv = H.sv + bt_soff<NT>(l) + min(t, n - 1);
+        const int W = C.nx + 2;
+        const T *c = H.c + bt_coff(l + 1);
+        const int ic = min(x >> 1, C.nx - 1) + 1, i2 = ic + (q ? 1 : -1);
+        T h[4], v[4];
 #pragma unroll
-    for (int l = 0; l < MG_NREG; l++)
-        if (l < B.nreg) K.load(l, F[l]);
-    for (int k = threadIdx.x; k < MG_TAIL * MG_TAIL; k += NT) H.m[k] = ((const T *)B.tail)[k];
-    for (int k = threadIdx.x; k < (int)(sizeof(H.c) / sizeof(T)); k += NT) H.c[k] = T(0);
-    __syncthreads();
-    K.template run<0>(F, r0, false);
+        for (int k = 0; k < 4; k++) {
+            const int jc = min(2 * s + k, C.ny + 1);   // padded row of 2 s - 1 + k
+            h[k] = T(3) * c[ic + W * jc] + c[i2 + W * jc];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = (act && x < L.nx && MG_SR * s + j < L.ny) ? prolong<T>(h, j) : T(0);
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            S.A[k] = sv[k * n] + sel(q, v[2 * k + 1], v[2 * k]);
+            S.B[k] = sv[(2 + k) * n] + sel(q, v[2 * k], v[2 * k + 1]);
+        }
+        const Ends<T> E{H.ends + x, 1 << g.k};
+        if (act && s == 0) E.at(-1, 0) = E.at(-1, 1) = T(0);
+        if (act && s == g.ns - 1) E.at(g.ns, 0) = E.at(g.ns, 1) = T(0);
+        sweep_up<T>(S, q, s, E, act, sync);
+        T e[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) e[j] = strip_row(S, q, j);
+        if (l == 0) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (act && x < L.nx && MG_SR * s + j < L.ny) ((T *)L.c)[mc(L.ld, x, MG_SR * s + j)] = e[j];
+        } else {
+            T *o = H.c + bt_coff(l) + x + 1 + (L.nx + 2) * (MG_SR * s + 1);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (act && x < L.nx && MG_SR * s + j < L.ny) o[j * (L.nx + 2)] = e[j];
+        }
+        sync();
+        if (l > 0) K = N;
+    }
 }
 
 // The tail matrix: workgroup j (one wavefront) runs the V-cycle of the levels
@@ -878,13 +937,24 @@ static int tiles_of(int NX, int NY, int own, int *ntx) {
 int mg_tiles(int NX, int NY, int *ntx) { return tiles_of(NX, NY, MG_OD, ntx); }
 int mg_tail_cells() { return MG_TAIL; }
 int mg_bottom_side(int fp32) { return fp32 ? mg_bottom_width<float>() : mg_bottom_width<double>(); }
-size_t mg_tail_bytes() { return sizeof(double) * MG_TAIL * MG_TAIL; }
+size_t mg_tail_bytes() { return sizeof(double) * (MG_TAIL * MG_TAIL + MG_NREG * BT_PACK * 1024); }
 
-// The first level of at most MG_TAIL cells.
+// The tail's level, the first of at most MG_TAIL cells below level 0 (the
+// tiled levels end there at the latest), and the first level the bottom
+// kernel can take: the packs are those of the levels between.
 static int tail_level(const MgHierarchy &H) {
-    int l = H.ntiled;
+    int l = 1;
     while (l + 1 < H.nlev && H.lev[l].nx * H.lev[l].ny > MG_TAIL) l++;
     return l;
+}
+static int pack_level(const MgHierarchy &H) {
+    int l = 1;
+    while (l < tail_level(H) && std::max(H.lev[l].nx, H.lev[l].ny) > mg_bottom_width<float>()) l++;
+    return l;
+}
+template <typename T>
+static T *pack_of(const MgHierarchy &H, int l) {
+    return (T *)H.tail + MG_TAIL * MG_TAIL + (size_t)BT_PACK * 1024 * (l - pack_level(H));
 }
 
 template <typename T>
@@ -900,13 +970,12 @@ void launch_mg_coef(const MgHierarchy &H, int nx, int ny, int ld, const double *
         hipLaunchKernelGGL(k_mg_coarsen<T>, dim3((C.nx + 1 + 255) / 256, C.ny + 1), dim3(256), 0, s, H.lev[l - 1], C,
                            (T)(sl / sp));
     }
-    // the tail's level does not depend on where the tiled levels end (at the
-    // latest at the first level of at most MG_TAIL cells)
     MgTailLevels B{};
-    int t = 1;
-    while (t + 1 < H.nlev && H.lev[t].nx * H.lev[t].ny > MG_TAIL) t++;
+    const int t = tail_level(H);
     B.nlev = H.nlev - t;
     for (int l = 0; l < B.nlev; l++) B.lev[l] = H.lev[t + l];
+    for (int l = pack_level(H); l < t; l++)
+        hipLaunchKernelGGL(k_mg_pack<T>, dim3(1), dim3(1024), 0, s, H.lev[l], pack_of<T>(H, l));
     hipLaunchKernelGGL(k_mg_tail<T>, dim3(B.lev[0].nx * B.lev[0].ny), dim3(64), 0, s, B, (T *)H.tail);
 }
 
@@ -934,9 +1003,10 @@ static void launch_mg_bottom(const MgHierarchy &H, const MgDecide &D, Scalars *s
     MgBottom B{};
     B.nreg = tail_level(H) - H.ntiled;
     for (int l = 0; l <= B.nreg; l++) B.lev[l] = H.lev[H.ntiled + l];
+    for (int l = 0; l < B.nreg; l++) B.pack[l] = pack_of<T>(H, H.ntiled + l);
     B.tail = H.tail;
     // lanes of the first level: 256 serve up to 32 x 32 cells
-    if constexpr (sizeof(T) == 4)
+    if constexpr (mg_bottom_width<T>() > 32)
         if (std::max(B.lev[0].nx, B.lev[0].ny) > 32) {
             hipLaunchKernelGGL((k_mg_bottom<T, 1024>), dim3(1), dim3(1024), 0, s, B, D, sc);
             return;

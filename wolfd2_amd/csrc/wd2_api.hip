@@ -844,7 +844,7 @@ static int mg_prepare(wd2_ctx *c) {
         // float and double views share the storage: clear it (zero rings)
         if (c->mg_prec != -1 && c->mg_prec != c->precision)
             HIPCHK(hipMemsetAsync(c->mg_store, 0, c->mg_bytes, c->s));
-        if ((st = mg_retile(c))) return st;
+        if ((st = mg_retile(c))) return st;   // the bottom's widest level depends on the precision
         if (c->precision == WD2_PREC_MIXED)
             launch_mg_coef<float>(c->mg, c->nx, c->ny, c->ld, c->M.rau, c->M.rgv, uni, c->s);
         else

@@ -307,7 +307,7 @@ struct MgHierarchy {
     int nlev, ntiled;
     MgLevel lev[MG_MAXLEV];
     MgTune tune;
-    void *tail;   // the bottom kernel's tail matrix (mg_tail_bytes)
+    void *tail;   // the bottom kernel's tail matrix and strip coefficients (mg_tail_bytes)
 };
 int mg_tiles(int NX, int NY, int *ntx);   // level-0 down tiles
 int mg_bottom_side(int fp32);   // widest level the bottom kernel can take in FP32 / FP64
