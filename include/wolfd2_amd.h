@@ -41,7 +41,7 @@ const char *wd2_last_error(void);
 /* Number of times the parallel AltTridLU fell back to its sequential path. */
 int wd2_trid_fallbacks(void);
 /* Red-black SOR on Cartesian grids without blockages runs several sweeps per
- * launch on LDS tiles (on by default); 0 selects one launch per colour and
+ * launch on tiles held in registers (on by default); 0 selects one launch per colour and
  * sweep.  Both give the reference's iterates bit for bit.  Returns the
  * previous setting. */
 int wd2_set_tiled_sor(int enable);
@@ -66,8 +66,10 @@ int wd2_set_uniform_coefficients(int enable);
 /* Non-zero (default): print the reference's warnings on standard output
  * (Ppe non-convergence, bad solver flag).  Returns the previous setting. */
 int wd2_set_verbose(int enable);
-/* Red-black SOR sweeps per launch of its dominant kernel (1 when not tiled),
- * FP64 path and mixed-precision path. */
+/* Red-black SOR sweeps per launch of its dominant kernel (1 when not tiled) on
+ * a 1024^2 grid, FP64 path and mixed-precision path.  On other grids the FP64
+ * path runs 4 to 14 sweeps a launch, by the number of tiles, and the whole
+ * solve where one tile holds the grid (up to 64 x 64 cells). */
 int wd2_sor_sweeps_per_launch(void);
 int wd2_sor_mixed_sweeps_per_launch(void);
 

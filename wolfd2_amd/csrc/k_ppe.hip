@@ -1,8 +1,8 @@
 // k_ppe.hip -- the pressure Poisson relaxations of pressure.f (Ppe 30-249).
 //
 //   SorRB / SorRBP (pressure.f:457-656), Cartesian grid without blockages:
-//     k_sor_tiled runs KT sweeps per launch on LDS tiles (temporal blocking,
-//     below), bit for bit the reference's iterates.
+//     k_sor_tiled runs several sweeps per launch on tiles held in registers
+//     (temporal blocking, below), bit for bit the reference's iterates.
 //   SorRB / SorRBP otherwise: two colour kernels per sweep.  Points of one
 //     colour only read points of the other, so every point's arithmetic is
 //     the reference's regardless of order; the unrelaxed |s| is max-reduced
@@ -188,187 +188,307 @@ void launch_sor_rb_check(int nx, int ny, int sweep, double sortol, int msorit, c
 
 // --------------------------------------------- temporally blocked SorRB
 // Cartesian grids without blockages: the right-hand side and the five
-// coefficients do not change during the solve, so a workgroup can run KT
-// sweeps on an LDS tile.  The tile holds TT x TT owned points plus a halo of
-// TH = 2*KT cells: a red-black sweep moves the dependence front by two cells
+// coefficients do not change during the solve, so a workgroup can run many
+// sweeps on a tile it holds.  A tile is ST_W x ST_W points with a halo of
+// 2 * nsweep cells: a red-black sweep moves the dependence front by two cells
 // (black points read red neighbours, red points read the new black ones), so
-// after KT sweeps every owned point has seen exactly the values it sees in
+// after the sweeps every owned point has seen exactly the values it sees in
 // the global sweep order, and its arithmetic is the reference's.  Points of
-// the outermost ring are never updated; points outside the array are never
-// read by an updated point.
+// the outermost ring are never updated.
 //
-// Only p lives in LDS (64 x 64 doubles, stored split by colour).  Each of
-// the 512 lanes owns four horizontal pairs of points, with their right-hand
-// side and coefficients (b, a1 = rgv(i,j-1), a2 = rau(i-1,j), a4 = rau(i,j),
-// a5 = rgv(i,j)) in registers; in each half-sweep a lane updates the point of
-// that colour of each of its pairs.
+// The tile lives in registers: a lane holds a strip of ST_R rows of a pair of
+// columns (32 lanes a strip, 16 strips), with its right-hand side,
+// coefficients and reciprocal diagonals.  A colour takes one point of each
+// row's pair, the same one in every lane, so of its four neighbours one is the
+// lane's own pair mate, two are its own rows above and below, and one comes by
+// a lane shift; only the rows at a strip's ends cross through LDS.  A half
+// sweep is bound by its instructions (about 22 double-precision ones a point,
+// 2048 points over four SIMDs) and one LDS exchange; a launch by those and
+// about 5 us of launch gap, stopping test, loads and stores.  With p in LDS,
+// five LDS reads a point, a plain division and four sweeps a launch, a sweep
+// took 3.1 us on 251 x 243 cells, 6.5 on 1000^2 and, with uniform coefficients,
+// 2.8 on 64^2, 2.9 on 512^2 and 4.2 on 1024^2; here 1.5, 4.5, 0.9, 1.3 and 2.9.
 //
-// The kernel reads p_in and writes the owned points to p_out (tiles read
-// their neighbours' points as halo, so it cannot work in place).  The
+// WHOLE: a grid of at most ST_W x ST_W interior points is one tile without a
+// halo: the ghost cells are constants, and one workgroup runs the sweeps of
+// the whole solve with the stopping test after each (0.9 us a sweep where
+// tiles of 14 sweeps a launch take 1.0).
+//
+// Otherwise the kernel reads p_in and writes the owned points to p_out (tiles
+// read their neighbours' points as halo, so it cannot work in place).  The
 // stopping test of sweep m is max|s| < sortol over the whole grid
 // (pressure.f:534), which holds exactly when it holds on every tile: each tile
 // publishes a bit mask of its sweeps whose owned-point maximum is below
 // sortol, and the test of a launch is the AND of the masks.  Before any work,
 // every workgroup evaluates the previous launch's test; all reach the same
 // decision, so a solve that stopped is never advanced further.
-constexpr int KT = 4, TH = 2 * KT, TW = 64, TT = TW - 2 * TH;   // 48 owned
-constexpr int TP_T = 512;
-constexpr int TP_PAIRS = TW * TW / 2 / TP_T;   // 4
-constexpr int TK = TW / 2;                     // pairs per tile row
+//
+// Division by the fixed diagonal, MODE 0 and 1: with r = 1/d correctly rounded,
+// two steps q += fma(-d, q, x) * r from q = x * r give the correctly rounded
+// x / d (Markstein, IBM J. Res. Dev. 34, 1990: the first makes q faithful, the
+// second rounds it correctly) as long as nothing under- or overflows; d is
+// checked once, and a wavefront that meets a quotient that is tiny, zero or
+// not a number divides instead.  MODE 2: every diagonal is a power of two, so
+// x / d == x * (1 / d) bit for bit.
+constexpr int ST_T = 512, ST_W = 64, ST_R = 4;
+constexpr int ST_L = ST_W / 2;       // lanes of a strip
+constexpr int ST_N = ST_W / ST_R;    // strips
+constexpr double ST_TINY = 0x1p-400, ST_HUGE = 0x1p400;
 
-// RCP: every diagonal a3 of the launch is a power of two (the uniform-grid
-// value, and -1 at points that are not updated), so x / a3 == x * (1 / a3)
-// bit for bit (both are the correctly rounded value of the same real, and
-// 1 / a3 is exact): the sweeps multiply by the reciprocal instead of dividing.
-template <bool RCP>
-__global__ __launch_bounds__(TP_T) void k_sor_tiled(int nx, int ny, int ld, const double *__restrict__ rau,
-                                                    const double *__restrict__ rgv, const double *__restrict__ b,
-                                                    double sorrel, int nsweep, const double *__restrict__ p_in,
-                                                    double *__restrict__ p_out, unsigned *__restrict__ masks,
-                                                    const unsigned *__restrict__ prev_masks, int prev_nsweep,
-                                                    int prev_m0, int prev_launch, double sortol, int msorit,
-                                                    int ntx, int ntiles, Scalars *sc, int force, int uni,
-                                                    double rau_c, double rgv_c) {
-    if (!force && sc->sor_done) return;
-    // p split by colour: PC[c][y*TK + k] is the point of colour c ((i+j) & 1)
-    // in pair k of tile row y, so that the neighbours a colour reads are
-    // unit-stride across the lanes of a wavefront
-    __shared__ double PC[2][TW * TK];
-    __shared__ unsigned sh[TP_T / 64];
-    if (!force && prev_nsweep > 0) {
+template <int CTRL>
+__device__ inline double st_dpp(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+struct StArgs {
+    int nx, ny, ld, nsweep, m0, msorit;
+    int prev_nsweep, prev_m0, prev_launch;
+    int ntx, ntiles, own, force;
+    double sorrel, sortol, rau_c, rgv_c, d_c, rd_c;   // uniform: the diagonal and its reciprocal
+    const double *rau, *rgv, *b, *p_in;
+    double *p_out;
+    unsigned *masks;
+    const unsigned *prev_masks;
+    Scalars *sc;
+};
+
+// One lane's part of a tile.  [r][h]: row r of the strip, column h of the pair.
+template <int MODE>
+struct StTile {
+    double p[ST_R][2], b[ST_R][2];
+    double g[ST_R + 1][2], a[ST_R][2], aw[ST_R], d[ST_R][2], rd[ST_R][2];   // MODE 0
+    bool up[ST_R][2];                  // the point is updated
+    unsigned long long own[ST_R][2];   // lanes whose point is owned
+    bool divide;
+};
+
+// The points of colour C ((i + j) & 1 == C) of one half sweep.  sS, sN: the
+// rows below and above the strip; gw, ge: WHOLE, the west ghosts of a strip's
+// first lane and the east ones of its last.  Returns the lanes that own a
+// point whose |s| is not below sortol (a NaN counts as not converged).
+template <int MODE, bool WHOLE, int C>
+__device__ __forceinline__ unsigned long long st_half(StTile<MODE> &t, double sS, double sN, const double *gw,
+                                                      const double *ge, int l, const StArgs &A) {
+    double x[ST_R], q[ST_R];
+    bool bad = MODE != 2 && t.divide;
+    // the inner rows first, kept there by the empty asm: the end rows'
+    // neighbours are on their way from LDS
+#pragma unroll
+    for (int k = 0; k < ST_R; k++) {
+        const int r = (k + 1) % ST_R, h = (r ^ C) & 1;
+        if (k == ST_R - 2) asm volatile("" : "+v"(sS), "+v"(sN) : "v"(q[1]), "v"(q[2]));
+        double W, E;
+        if (h) {
+            W = t.p[r][0];
+            E = st_dpp<0x130>(t.p[r][0]);   // wave_shl:1
+            if (WHOLE) E = l == ST_L - 1 ? ge[r] : E;
+        } else {
+            W = st_dpp<0x138>(t.p[r][1]);   // wave_shr:1
+            if (WHOLE) W = l == 0 ? gw[r] : W;
+            E = t.p[r][1];
+        }
+        const double S = r > 0 ? t.p[r > 0 ? r - 1 : 0][h] : sS;
+        const double N = r < ST_R - 1 ? t.p[r < ST_R - 1 ? r + 1 : 0][h] : sN;
+        const double a1 = MODE ? A.rgv_c : t.g[r][h], a5 = MODE ? A.rgv_c : t.g[r + 1][h];
+        const double a2 = MODE ? A.rau_c : (h ? t.a[r][0] : t.aw[r]), a4 = MODE ? A.rau_c : t.a[r][h];
+        const double rd = MODE ? A.rd_c : t.rd[r][h], d = MODE ? A.d_c : t.d[r][h];
+        // the reference's order: b - a1 pS - a2 pW - a4 pE - a5 pN
+        x[r] = t.b[r][h] - a1 * S - a2 * W - a4 * E - a5 * N;
+        q[r] = x[r] * rd;
+        if (MODE != 2) {
+            q[r] = __builtin_fma(__builtin_fma(-d, q[r], x[r]), rd, q[r]);
+            q[r] = __builtin_fma(__builtin_fma(-d, q[r], x[r]), rd, q[r]);
+            bad |= t.up[r][h] && !(fabs(q[r]) > ST_TINY);
+        }
+    }
+    if (MODE != 2 && __any(bad)) {
+#pragma unroll
+        for (int r = 0; r < ST_R; r++) q[r] = x[r] / (MODE ? A.d_c : t.d[r][(r ^ C) & 1]);
+    }
+    unsigned long long big = 0;
+#pragma unroll
+    for (int r = 0; r < ST_R; r++) {
+        const int h = (r ^ C) & 1;
+        const double s = q[r] - t.p[r][h];
+        const double pn = t.p[r][h] + A.sorrel * s;
+        t.p[r][h] = t.up[r][h] ? pn : t.p[r][h];
+        big |= __ballot(!(fabs(s) < A.sortol)) & t.own[r][h];
+    }
+    return big;
+}
+
+template <int MODE, bool WHOLE>
+__global__ __launch_bounds__(ST_T, WHOLE ? 2 : 4) void k_sor_tiled(StArgs A) {
+    // the strips' first and last rows by colour; strips 0 and ST_N + 1 are the
+    // rows below and above the tile (WHOLE: the ghost rows)
+    __shared__ double EB[2][ST_N + 2][ST_L], ET[2][ST_N + 2][ST_L];
+    __shared__ unsigned sh[ST_T / 64];
+    __shared__ int more[2];
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), l = tid & (ST_L - 1), st = tid / ST_L;
+    const int nx = A.nx, ny = A.ny, ld = A.ld;
+    // XCD-aware tile order: consecutive workgroups go to different XCDs, so
+    // give each XCD a contiguous band of tiles (their halos then share an L2).
+    const int per = (A.ntiles + 7) / 8;
+    const int tile = WHOLE ? 0 : (blockIdx.x % 8) * per + blockIdx.x / 8;
+    const int halo = WHOLE ? 0 : (ST_W - A.own) / 2;
+    const int TI = tile % A.ntx, TJ = tile / A.ntx;
+    const int i0 = 2 + TI * A.own - halo, j0 = 2 + TJ * A.own - halo;   // tile origin, both even
+    const int x = 2 * l, y = ST_R * st, i = i0 + x, j = j0 + y;
+    // the loads need no answer from the earlier launch: they are in flight
+    // while its stopping test is evaluated
+    StTile<MODE> t;
+#pragma unroll
+    for (int r = 0; r < ST_R; r++) {
+        const double2 pv = load_pair_sel(A.p_in, ld, nx, ny, i, j + r);
+        const double2 bv = load_pair_sel(A.b, ld, nx, ny, i, j + r);
+        t.p[r][0] = pv.x; t.p[r][1] = pv.y;
+        t.b[r][0] = bv.x; t.b[r][1] = bv.y;
+    }
+    if (MODE == 0) {
+#pragma unroll
+        for (int r = 0; r < ST_R; r++) {
+            const double2 gv = load_pair_sel(A.rgv, ld, nx, ny, i, j + r - 1);
+            const double2 av = load_pair_sel(A.rau, ld, nx, ny, i, j + r);
+            t.g[r][0] = gv.x; t.g[r][1] = gv.y;
+            t.a[r][0] = av.x; t.a[r][1] = av.y;
+            t.aw[r] = A.rau[(size_t)min(max(i - 1, 0), ld - 1) + (size_t)ld * (size_t)min(max(j + r, 0), ny + 1)];
+        }
+        const double2 gv = load_pair_sel(A.rgv, ld, nx, ny, i, j + ST_R - 1);
+        t.g[ST_R][0] = gv.x; t.g[ST_R][1] = gv.y;
+    }
+    double gw[ST_R] = {}, ge[ST_R] = {};
+    if (WHOLE) {
+#pragma unroll
+        for (int r = 0; r < ST_R; r++) {
+            gw[r] = load_pair_sel(A.p_in, ld, nx, ny, 0, j + r).y;
+            ge[r] = load_pair_sel(A.p_in, ld, nx, ny, 2 + ST_W, j + r).x;
+        }
+    }
+    if (!A.force && A.sc->sor_done) return;
+    if (!WHOLE && !A.force && A.prev_nsweep > 0) {
         int conv = 0;
-        const int k = tiled_stop(tiled_mask(prev_masks, ntiles, sh), prev_nsweep, prev_m0, msorit, &conv);
+        const int k = tiled_stop(tiled_mask(A.prev_masks, A.ntiles, sh), A.prev_nsweep, A.prev_m0, A.msorit, &conv);
         if (k > 0) {
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-                sc->sor_done = 1;
-                sc->sor_nconv = conv ? prev_m0 + k : 0;
-                sc->sor_m = prev_m0 + k;
-                sc->redo_launch = prev_launch;
-                sc->redo_sweeps = k;
+            if (blockIdx.x == 0 && tid == 0) {
+                A.sc->sor_done = 1;
+                A.sc->sor_nconv = conv ? A.prev_m0 + k : 0;
+                A.sc->sor_m = A.prev_m0 + k;
+                A.sc->redo_launch = A.prev_launch;
+                A.sc->redo_sweeps = k;
             }
             return;
         }
     }
-    // XCD-aware tile order: consecutive workgroups go to different XCDs, so
-    // give each XCD a contiguous band of tiles (their halos then share an L2).
-    const int per = (ntiles + 7) / 8;
-    const int tile = (blockIdx.x % 8) * per + blockIdx.x / 8;
-    if (tile >= ntiles) return;
-    const int TI = tile % ntx, TJ = tile / ntx;
-    const int i0 = 2 + TI * TT - TH, j0 = 2 + TJ * TT - TH;   // tile origin
-    const int t = threadIdx.x;
-    // Per pair r and colour c, everything the sweeps need for the pair's point
-    // of that colour (h = its side, 0 left or 1 right): b and a1, a2, a4, a5
-    // (+0, +0, +0, +0, 1 where the point is not updated, so a3 = -1 there),
-    // a3 = -a4 - a2 - a5 - a1 (the reference's expression, evaluated once),
-    // the LDS offsets of its west and east neighbours (q - 1 + h and q + h)
-    // and of its south and north ones, clamped to the point's own slot where
-    // they would leave the tile (the outer ring is never updated: what such a
-    // point reads is discarded), and whether the point is updated / owned.
-    double cb[TP_PAIRS][2], c1[TP_PAIRS][2], c2[TP_PAIRS][2], c3[TP_PAIRS][2], c4[TP_PAIRS][2], c5[TP_PAIRS][2];
-    int ow[TP_PAIRS][2], oe[TP_PAIRS][2], os[TP_PAIRS], on[TP_PAIRS];
-    bool up[TP_PAIRS][2];
-    unsigned long long ownm[TP_PAIRS][2];
-    int lcs[TP_PAIRS];
-#define PX(r) (2 * ((t + TP_T * (r)) % TK))
-#define PY(r) ((t + TP_T * (r)) / TK)
-#define PB(r) (t + TP_T * (r))   // y*TK + k of the lane's pair r
+    if (tile >= A.ntiles) return;
+    bool divide = false, any_up = false;
 #pragma unroll
-    for (int r = 0; r < TP_PAIRS; r++) {
-        const int x = PX(r), y = PY(r), kk = x / 2;
-        const int i = i0 + x, j = j0 + y;   // i is even: the pair (i, i+1) is 16-byte aligned
-        const double2 pv = load_pair_sel(p_in, ld, nx, ny, i, j);
-        const int lc = (i + j) & 1;   // colour of the left point
-        lcs[r] = lc;
-        PC[lc][PB(r)] = pv.x;
-        PC[lc ^ 1][PB(r)] = pv.y;
-        const bool rowin = j >= 2 && j <= ny && y >= 1 && y <= TW - 2;
-        const bool upd0 = rowin && i >= 2 && i <= nx && x >= 1;
-        const bool upd1 = rowin && i + 1 >= 2 && i + 1 <= nx && x + 1 <= TW - 2;
-        // coefficients as aligned pairs, read from clamped addresses and used
-        // only where a point updates (i >= 2 and i + 1 <= nx + 1 there)
-        const double2 bv = load_pair_sel(b, ld, nx, ny, i, j);
-        double2 g0, g1, av;
-        double aw;
-        if (uni) {   // every rau / rgv entry an updated point reads has this value
-            g0 = g1 = make_double2(rgv_c, rgv_c);
-            av = make_double2(rau_c, rau_c);
-            aw = rau_c;
-        } else {
-            g0 = load_pair_sel(rgv, ld, nx, ny, i, j - 1);
-            g1 = load_pair_sel(rgv, ld, nx, ny, i, j);
-            av = load_pair_sel(rau, ld, nx, ny, i, j);
-            aw = rau[(size_t)min(max(i - 1, 0), ld - 1) + (size_t)ld * (size_t)min(max(j, 0), ny + 1)];
-        }
-        os[r] = y > 0 ? -TK : 0;
-        on[r] = y < TW - 1 ? TK : 0;
+    for (int r = 0; r < ST_R; r++) {
+        const int yy = y + r, jj = j + r;
+        const bool row = jj >= 2 && jj <= ny && (WHOLE || (yy >= 1 && yy <= ST_W - 2));
 #pragma unroll
-        for (int c = 0; c < 2; c++) {
-            const int h = lc ^ c;
-            const bool u = h ? upd1 : upd0;
-            const bool own = u && x + h >= TH && x + h < TH + TT && y >= TH && y < TH + TT;
-            const double bb = u ? (h ? bv.y : bv.x) : 0.0;
-            const double a1 = u ? (h ? g0.y : g0.x) : 0.0;
-            const double a2 = u ? (h ? av.x : aw) : 0.0;
-            const double a4 = u ? (h ? av.y : av.x) : 0.0;
-            const double a5 = u ? (h ? g1.y : g1.x) : 1.0;
-            cb[r][c] = bb; c1[r][c] = a1; c2[r][c] = a2; c4[r][c] = a4; c5[r][c] = a5;
-            c3[r][c] = -a4 - a2 - a5 - a1;
-            if (RCP) c3[r][c] = 1.0 / c3[r][c];
-            ow[r][c] = h ? 0 : (kk > 0 ? -1 : 0);
-            oe[r][c] = h ? (kk < TK - 1 ? 1 : 0) : 0;
-            up[r][c] = u;
-            ownm[r][c] = __ballot(own);
+        for (int h = 0; h < 2; h++) {
+            const int xx = x + h, ii = i + h;
+            const bool u = row && ii >= 2 && ii <= nx && (WHOLE || (xx >= 1 && xx <= ST_W - 2));
+            t.up[r][h] = u;
+            t.own[r][h] =
+                __ballot(u && xx >= halo && xx < ST_W - halo && yy >= halo && yy < ST_W - halo);
+            any_up = any_up || __any(u);
+            if (MODE == 0) {
+                // a3 = -a4 - a2 - a5 - a1, the reference's expression; a point
+                // that is not updated keeps its value whatever it computes
+                const double a2 = h ? t.a[r][0] : t.aw[r];
+                const double d = -t.a[r][h] - a2 - t.g[r + 1][h] - t.g[r][h];
+                t.d[r][h] = u ? d : -1.0;
+                t.rd[r][h] = 1.0 / t.d[r][h];
+                divide |= !(fabs(t.d[r][h]) > ST_TINY && fabs(t.d[r][h]) < ST_HUGE);
+            }
         }
     }
+    t.divide = divide;
+    for (int k = tid; k < 4 * ST_L; k += ST_T) {
+        // rows j0 - 1 (ET of strip 0) and j0 + ST_W (EB of strip ST_N + 1), by colour
+        const int c = (k / ST_L) & 1, top = k / (2 * ST_L), kl = k % ST_L;
+        double v = 0.0;
+        if (WHOLE) {
+            const int jj = top ? 2 + ST_W : 1, h = top ? c : 1 - c, ii = 2 + 2 * kl + h;
+            if (jj <= ny + 1 && ii <= nx + 1) v = A.p_in[WD2_IX(ii, jj)];
+        }
+        if (top) EB[c][ST_N + 1][kl] = v;
+        else ET[c][0][kl] = v;
+    }
+    EB[0][st + 1][l] = t.p[0][0];
+    EB[1][st + 1][l] = t.p[0][1];
+    ET[1][st + 1][l] = t.p[ST_R - 1][0];
+    ET[0][st + 1][l] = t.p[ST_R - 1][1];
+    if (tid < 2) more[tid] = 0;
     __syncthreads();
-    // The sweeps are straight-line code: every point is evaluated and a point
-    // that is not updated keeps its value by a select.  The stopping test
-    // flags an owned point whose |s| is not below sortol (a NaN counts as not
-    // converged), which is max |s| < sortol over the owned points otherwise;
-    // it is gathered per wavefront as ballots.
+    const int lo_w = 8 * w, hi_w = 8 * w + 7;   // the wavefront's rows
     unsigned below = 0;   // bit s: the wavefront's owned max |s| of sweep s is < sortol
-    for (int s = 0; s < nsweep; s++) {
-        unsigned long long big = 0;
-#pragma unroll
-        for (int color = 0; color < 2; color++) {
-            double *__restrict__ dst = PC[color];
-            const double *__restrict__ src = PC[1 - color];
-#pragma unroll
-            for (int r = 0; r < TP_PAIRS; r++) {
-                const int q = PB(r);
-                const double pij = dst[q];
-                // the reference's order: b - a1 pS - a2 pW - a4 pE - a5 pN
-                double sum = cb[r][color] - c1[r][color] * src[q + os[r]] - c2[r][color] * src[q + ow[r][color]] -
-                             c4[r][color] * src[q + oe[r][color]] - c5[r][color] * src[q + on[r]];
-                sum = (RCP ? sum * c3[r][color] : sum / c3[r][color]) - pij;
-                const double pn = pij + sorrel * sum;
-                dst[q] = up[r][color] ? pn : pij;
-                big |= __ballot(!(fabs(sum) < sortol)) & ownm[r][color];
+    for (int s = 0; s < A.nsweep; s++) {
+        // rows that the owned points still depend on: one less a side per half sweep
+        const int rem = 2 * (A.nsweep - 1 - s);
+        const bool act0 = WHOLE ? any_up : (hi_w >= halo - rem - 1 && lo_w <= ST_W - halo + rem);
+        const bool act1 = WHOLE ? any_up : (hi_w >= halo - rem && lo_w <= ST_W - halo - 1 + rem);
+        if (WHOLE && s > 0) {
+            // the test of the sweep before
+            const int m = A.m0 + s;
+            if (m > 1 && !__builtin_amdgcn_readfirstlane(more[(s - 1) & 1])) {
+                if (tid == 0) {
+                    A.sc->sor_done = 1;
+                    A.sc->sor_nconv = A.sc->sor_m = m;
+                }
+                below = 1;
+                break;
             }
-            __syncthreads();
         }
-        if (big == 0) below |= 1u << s;
+        unsigned long long big = 0;
+        if (act0) {
+            big = st_half<MODE, WHOLE, 0>(t, ET[1][st][l], EB[1][st + 2][l], gw, ge, l, A);
+            EB[0][st + 1][l] = t.p[0][0];
+            ET[0][st + 1][l] = t.p[ST_R - 1][1];
+        }
+        __syncthreads();
+        if (WHOLE && tid == 0) more[(s + 1) & 1] = 0;
+        if (act1) {
+            big |= st_half<MODE, WHOLE, 1>(t, ET[0][st][l], EB[0][st + 2][l], gw, ge, l, A);
+            EB[1][st + 1][l] = t.p[0][1];
+            ET[1][st + 1][l] = t.p[ST_R - 1][0];
+        }
+        if (WHOLE) {
+            if (big != 0) more[s & 1] = 1;
+        } else if (big == 0) {
+            below |= 1u << s;
+        }
+        __syncthreads();
     }
-#pragma unroll
-    for (int r = 0; r < TP_PAIRS; r++) {
-#pragma unroll
-        for (int c = 0; c < 2; c++)
-            if ((ownm[r][c] >> (t & 63)) & 1ull) {
-                const int x = PX(r) + (lcs[r] ^ c), y = PY(r);
-                p_out[WD2_IX(i0 + x, j0 + y)] = PC[c][PB(r)];
-            }
+    if (WHOLE && !below && tid == 0) {   // ran all its sweeps: the last one's test
+        const int m = A.m0 + A.nsweep;
+        const bool ok = m > 1 && !more[(A.nsweep - 1) & 1];
+        if (ok || m >= A.msorit) {
+            A.sc->sor_done = 1;
+            A.sc->sor_nconv = ok ? m : 0;
+        }
+        A.sc->sor_m = m;
     }
-#undef PX
-#undef PY
-#undef PB
+    const unsigned long long me = 1ull << (tid & 63);
+#pragma unroll
+    for (int r = 0; r < ST_R; r++) {
+        double *q = A.p_out + WD2_IX(i, j + r);
+        if ((t.own[r][0] & t.own[r][1]) & me) *reinterpret_cast<double2 *>(q) = make_double2(t.p[r][0], t.p[r][1]);
+        else if (t.own[r][0] & me) q[0] = t.p[r][0];
+        else if (t.own[r][1] & me) q[1] = t.p[r][1];
+    }
+    if (WHOLE) return;
     // tile mask = AND over the wavefronts (below is the same in every lane of one)
-    if ((t & 63) == 0) sh[t >> 6] = below;
+    if ((tid & 63) == 0) sh[w] = below;
     __syncthreads();
-    if (t == 0) {
+    if (tid == 0) {
         unsigned r = ~0u;
-        for (int w = 0; w < TP_T / 64; w++) r &= sh[w];
-        masks[tile] = r;
+        for (int k = 0; k < ST_T / 64; k++) r &= sh[k];
+        A.masks[tile] = r;
     }
 }
 
@@ -388,12 +508,47 @@ __global__ __launch_bounds__(RB_T) void k_sor_tiled_check(const unsigned *__rest
     }
 }
 
-int sor_tiled_tiles(int nx, int ny, int *ntx) {
-    const int tx = (nx - 1 + TT - 1) / TT, ty = (ny - 1 + TT - 1) / TT;
+bool sor_whole(int nx, int ny) { return nx - 1 <= ST_W && ny - 1 <= ST_W; }
+
+static int st_tiles(int nx, int ny, int k, int *ntx) {
+    const int own = ST_W - 4 * k, tx = (nx - 1 + own - 1) / own, ty = (ny - 1 + own - 1) / own;
     if (ntx) *ntx = tx;
     return tx * ty;
 }
-int sor_tiled_sweeps() { return KT; }
+// The sweeps of a launch, the fewest microseconds a sweep by a fit to measured
+// launches (251 x 243 to 2048^2, array coefficients): with n tiles on the
+// busiest of 256 CUs a launch of K sweeps takes 3 + 3.4 n + 0.5 (1 + n) K us.
+// Few tiles make long launches pay (up to K = 14, when a tile owns 8 x 8 of
+// its points); with every CU full the halo's work decides (K = 4 or 5).
+int sor_tiled_sweeps(int nx, int ny) {
+    int best = 4;
+    double cost = 1e300;
+    for (int k = 4; k <= 14; k++) {
+        const int nt = st_tiles(nx, ny, k, nullptr);
+        if (k > 8 && nt > 1024) break;   // (the mask buffers hold these)
+        const int n = (nt + 255) / 256;
+        const double c = (3.0 + 3.4 * n) / k + 0.5 * (1 + n);
+        if (c < cost) {
+            cost = c;
+            best = k;
+        }
+    }
+    return best;
+}
+
+int sor_tiled_tiles(int nx, int ny, int *ntx) { return st_tiles(nx, ny, sor_tiled_sweeps(nx, ny), ntx); }
+
+// The uniform coefficients, their diagonal and its reciprocal, and the kernel's MODE.
+static int st_uniform(const double *uni, StArgs &A) {
+    if (!uni) return 0;
+    A.rau_c = uni[0];
+    A.rgv_c = uni[1];
+    A.d_c = -uni[0] - uni[0] - uni[1] - uni[1];   // the kernel's order of operations
+    A.rd_c = 1.0 / A.d_c;
+    int e2 = 0;
+    if (!(std::fabs(A.d_c) > ST_TINY && std::fabs(A.d_c) < ST_HUGE)) return 0;
+    return std::frexp(A.d_c, &e2) == -0.5 ? 2 : 1;
+}
 
 void launch_sor_tiled(int nx, int ny, int ld, const Metrics &m, const double *b, double sorrel, int nsweep,
                       const double *p_in, double *p_out, unsigned *masks, const unsigned *prev_masks,
@@ -401,23 +556,25 @@ void launch_sor_tiled(int nx, int ny, int ld, const Metrics &m, const double *b,
                       int force, const double *uni, hipStream_t s) {
     int ntx = 0;
     const int nt = sor_tiled_tiles(nx, ny, &ntx);
-    const int grid = 8 * ((nt + 7) / 8);
-    // the diagonal of an updated point on the uniform path, in the kernel's
-    // order of operations (-a4 - a2 - a5 - a1); non-updated points have -1
-    bool rcp = false;
-    if (uni) {
-        const double a3 = -uni[0] - uni[0] - uni[1] - uni[1];
-        int e2 = 0;
-        rcp = std::isfinite(a3) && a3 != 0.0 && std::frexp(a3, &e2) == -0.5;
-    }
-    if (rcp)
-        hipLaunchKernelGGL(k_sor_tiled<true>, dim3(grid), dim3(TP_T), 0, s, nx, ny, ld, m.rau, m.rgv, b, sorrel, nsweep,
-                           p_in, p_out, masks, prev_masks, prev_nsweep, prev_m0, prev_launch, sortol, msorit, ntx, nt,
-                           sc, force, 1, uni[0], uni[1]);
-    else
-        hipLaunchKernelGGL(k_sor_tiled<false>, dim3(grid), dim3(TP_T), 0, s, nx, ny, ld, m.rau, m.rgv, b, sorrel,
-                           nsweep, p_in, p_out, masks, prev_masks, prev_nsweep, prev_m0, prev_launch, sortol, msorit,
-                           ntx, nt, sc, force, uni ? 1 : 0, uni ? uni[0] : 0.0, uni ? uni[1] : 0.0);
+    StArgs A{nx, ny, ld, nsweep, 0, msorit, prev_nsweep, prev_m0, prev_launch, ntx, nt, ST_W - 4 * sor_tiled_sweeps(nx, ny), force,
+                   sorrel, sortol, 0.0, 0.0, 0.0, 0.0, m.rau, m.rgv, b, p_in, p_out, masks,
+                   prev_masks, sc};
+    const dim3 g(8 * ((nt + 7) / 8));
+    const int mode = st_uniform(uni, A);
+    if (mode == 2) hipLaunchKernelGGL((k_sor_tiled<2, false>), g, dim3(ST_T), 0, s, A);
+    else if (mode == 1) hipLaunchKernelGGL((k_sor_tiled<1, false>), g, dim3(ST_T), 0, s, A);
+    else hipLaunchKernelGGL((k_sor_tiled<0, false>), g, dim3(ST_T), 0, s, A);
+}
+
+void launch_sor_whole(int nx, int ny, int ld, const Metrics &m, const double *b, double sorrel, int nsweep, int m0,
+                      double *p, double sortol, int msorit, Scalars *sc, const double *uni, hipStream_t s) {
+    StArgs A{nx, ny, ld, nsweep, m0, msorit, 0, 0, 0, 1, 1, ST_W, 0,
+                   sorrel, sortol, 0.0, 0.0, 0.0, 0.0, m.rau, m.rgv, b, p, p, nullptr,
+                   nullptr, sc};
+    const int mode = st_uniform(uni, A);
+    if (mode == 2) hipLaunchKernelGGL((k_sor_tiled<2, true>), dim3(1), dim3(ST_T), 0, s, A);
+    else if (mode == 1) hipLaunchKernelGGL((k_sor_tiled<1, true>), dim3(1), dim3(ST_T), 0, s, A);
+    else hipLaunchKernelGGL((k_sor_tiled<0, true>), dim3(1), dim3(ST_T), 0, s, A);
 }
 
 void launch_sor_tiled_check(int ntiles, int nsweep, int m0, int launch, int msorit, const unsigned *masks,

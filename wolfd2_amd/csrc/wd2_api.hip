@@ -961,6 +961,8 @@ static int ppe_mg(wd2_ctx *c, int cart, int maxcyc, double dk, double tol, doubl
     return WD2_OK;
 }
 
+constexpr int SOR_WHOLE_RUN = 4096;   // sweeps per launch of a one-tile solve (about 3 ms)
+
 static int ppe(wd2_ctx *c, int cart, int solver, int msorit, double dk, double sortol, double sorrel,
                const double *u, const double *v, double *p, int *nconv_out) {
     const int nx = c->nx, ny = c->ny, ld = c->ld;
@@ -992,7 +994,29 @@ static int ppe(wd2_ctx *c, int cart, int solver, int msorit, double dk, double s
         const bool mx = c->precision == WD2_PREC_MIXED;
         auto sweep = mx ? launch_sor_tiled_mx : launch_sor_tiled;
         const double *uni = (g_uniform && c->uni_ok) ? c->uni : nullptr;
-        const int K = mx ? sor_tiled_mx_sweeps() : sor_tiled_sweeps();
+        if (!mx && sor_whole(nx, ny)) {
+            // launches of up to SOR_WHOLE_RUN sweeps, until one has stopped the solve
+            int h[2] = {0, 0};   // sor_done, sor_nconv
+            for (int m0 = 0, k; m0 < msorit && !h[0]; m0 += k) {
+                k = std::min(SOR_WHOLE_RUN, msorit - m0);
+                hipEvent_t *ev = kt_events(c, 1);
+                if (ev) HIPCHK(hipEventRecord(ev[0], s));
+                launch_sor_whole(nx, ny, ld, c->M, b, sorrel, k, m0, p, sortol, msorit, c->sc, uni, s);
+                if (ev) HIPCHK(hipEventRecord(ev[1], s));
+                HIPCHK(hipMemcpyAsync(c->h_flag, &c->sc->sor_done, sizeof(h), hipMemcpyDeviceToHost, s));
+                HIPCHK(hipStreamSynchronize(s));
+                h[0] = c->h_flag[0];
+                h[1] = c->h_flag[1];
+            }
+            if (h[1] < 1) {
+                if (g_verbose)
+                    fprintf(stdout, " Warning: SOR iterations did not converge after %6d iterations.\n", msorit);
+                h[1] = msorit;
+            }
+            *nconv_out = h[1];
+            return WD2_OK;
+        }
+        const int K = mx ? sor_tiled_mx_sweeps() : sor_tiled_sweeps(nx, ny);
         launch_copy(ld, 0, nx + 1, 0, ny + 1, p, c->pscr, s);
         int m0 = 0, L = 0;
         const int nt = mx ? sor_tiled_mx_tiles(nx, ny, nullptr) : sor_tiled_tiles(nx, ny, nullptr);
@@ -1001,15 +1025,15 @@ static int ppe(wd2_ctx *c, int cart, int solver, int msorit, double dk, double s
         // Batches of launches with a stopping check at the end of each, two
         // batches in flight: the host reads batch n's flag (copied to pinned
         // memory) while batch n+1 runs.  A batch issued after the solve
-        // stopped returns at entry in every launch.  Batches grow from 8 to 64
-        // launches, so a short solve is not overrun and a long one rarely
-        // waits; after a solve that ran to msorit they are 128 launches from
+        // stopped returns at entry in every launch.  Batches grow from 32 to
+        // 256 sweeps, so a short solve is not overrun and a long one rarely
+        // waits; after a solve that ran to msorit they are 512 sweeps from
         // the start (fewer checks; a solve that then stops early overruns by
         // at most two batches of launches that return at entry).
         int issued = 0, checked = 0, stop = 0;
         while (!stop) {
             if (m0 < msorit && issued - checked < 2) {
-                const int Q = c->sor_capped ? 128 : std::min(64, 8 << std::min(issued, 3));
+                const int Q = std::max(2, (c->sor_capped ? 512 : std::min(256, 32 << std::min(issued, 3))) / K);
                 // timing: one event pair around the batch's launches (no marker
                 // between two launches, so their durations are not inflated)
                 hipEvent_t *ev = kt_events(c, 1);
@@ -1913,7 +1937,7 @@ extern "C" {
 
 const char *wd2_last_error(void) { return g_err.c_str(); }
 
-int wd2_sor_sweeps_per_launch(void) { return g_tiled_sor ? sor_tiled_sweeps() : 1; }
+int wd2_sor_sweeps_per_launch(void) { return g_tiled_sor ? sor_tiled_sweeps(1024, 1024) : 1; }
 int wd2_sor_mixed_sweeps_per_launch(void) { return sor_tiled_mx_sweeps(); }
 
 int wd2_set_verbose(int enable) {

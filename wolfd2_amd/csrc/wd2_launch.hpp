@@ -130,12 +130,12 @@ void launch_sor_rb_sweep(int nx, int ny, int ld, const Metrics &m, const PpeCoef
 void launch_sor_rb_check(int nx, int ny, int sweep, double sortol, int msorit, const double *partials,
                          Scalars *sc, hipStream_t s);
 void launch_sor_reset(Scalars *sc, hipStream_t s);
-// Temporally blocked SorRB/SorRBP (Cartesian, no blockage): nsweep <= sor_tiled_sweeps()
+// Temporally blocked SorRB/SorRBP (Cartesian, no blockage): nsweep <= sor_tiled_sweeps(nx, ny)
 // sweeps of p_in into p_out; masks receives one stopping-test bit mask per
 // tile.  The launch first applies the stopping test to the previous launch
 // (prev_*; prev_nsweep = 0 for none).
 int sor_tiled_tiles(int nx, int ny, int *ntx);
-int sor_tiled_sweeps();
+int sor_tiled_sweeps(int nx, int ny);
 void launch_sor_tiled(int nx, int ny, int ld, const Metrics &m, const double *b, double sorrel, int nsweep,
                       const double *p_in, double *p_out, unsigned *masks, const unsigned *prev_masks,
                       int prev_nsweep, int prev_m0, int prev_launch, double sortol, int msorit, Scalars *sc,
@@ -143,6 +143,11 @@ void launch_sor_tiled(int nx, int ny, int ld, const Metrics &m, const double *b,
 // uni: null, or {rau, rgv} when every rau entry on i = 1..nx, j = 2..ny and
 // every rgv entry on i = 2..nx, j = 1..ny has that one value (a uniform
 // Cartesian grid): the kernels then use the values instead of loading them.
+// Grids that one tile holds (sor_whole): nsweep sweeps of p after sweep m0 in one
+// workgroup, stopping as the reference does after any of them.
+bool sor_whole(int nx, int ny);
+void launch_sor_whole(int nx, int ny, int ld, const Metrics &m, const double *b, double sorrel, int nsweep, int m0,
+                      double *p, double sortol, int msorit, Scalars *sc, const double *uni, hipStream_t s);
 // Mixed precision (FP64 residual and accumulation, FP32 sweeps), same contract.
 int sor_tiled_mx_tiles(int nx, int ny, int *ntx);
 int sor_tiled_mx_sweeps();

@@ -11,31 +11,35 @@
 
 namespace wd2 {
 
-// AND of the ntiles masks (every thread gets it).
+// AND of the ntiles masks (every thread gets it): a reduction by lane moves
+// within a wavefront, one LDS exchange across them.
 __device__ inline unsigned tiled_mask(const unsigned *__restrict__ masks, int ntiles, unsigned *sh) {
-    unsigned m = ~0u;
-    for (int k = threadIdx.x; k < ntiles; k += blockDim.x) m &= masks[k];
-    for (int off = 32; off > 0; off >>= 1) m &= (unsigned)__shfl_xor((int)m, off);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+    int m = ~0;
+    for (int k = threadIdx.x; k < ntiles; k += blockDim.x) m &= (int)masks[k];
+    m &= __builtin_amdgcn_update_dpp(~0, m, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8
+    m &= __builtin_amdgcn_update_dpp(~0, m, 0x112, 0xf, 0xf, false);
+    m &= __builtin_amdgcn_update_dpp(~0, m, 0x114, 0xf, 0xf, false);
+    m &= __builtin_amdgcn_update_dpp(~0, m, 0x118, 0xf, 0xf, false);
+    m &= __builtin_amdgcn_update_dpp(~0, m, 0x142, 0xa, 0xf, false);   // row_bcast:15
+    m &= __builtin_amdgcn_update_dpp(~0, m, 0x143, 0xc, 0xf, false);   // row_bcast:31
+    if ((threadIdx.x & 63) == 63) sh[threadIdx.x >> 6] = (unsigned)m;
     __syncthreads();
     unsigned r = ~0u;
     for (int w = 0; w < (int)(blockDim.x >> 6); w++) r &= sh[w];
     __syncthreads();
-    return r;
+    return __builtin_amdgcn_readfirstlane(r);
 }
 
-// 1-based sweep of a launch (nsweep sweeps after sweep m0) after which the
-// solve stops, or 0; *conv tells whether it stopped converged.
+// 1-based sweep of a launch (nsweep <= 32 sweeps after sweep m0) after which
+// the solve stops, or 0; *conv tells whether it stopped converged.
 __device__ inline int tiled_stop(unsigned mask, int nsweep, int m0, int msorit, int *conv) {
-    for (int s = 0; s < nsweep; s++) {
-        const int m = m0 + s + 1;
-        const bool ok = m > 1 && ((mask >> s) & 1u);
-        if (ok || m >= msorit) {
-            *conv = ok ? 1 : 0;
-            return s + 1;
-        }
-    }
-    return 0;
+    mask &= nsweep < 32 ? (1u << nsweep) - 1u : ~0u;
+    if (m0 == 0) mask &= ~1u;                    // the first sweep of a solve never stops it
+    const int first = mask ? __ffs(mask) : 33;   // first sweep below the tolerance
+    const int last = max(msorit - m0, 1);        // the sweep that reaches msorit
+    *conv = first <= last;
+    const int k = min(first, last);
+    return k <= nsweep ? k : 0;
 }
 
 }  // namespace wd2
