@@ -45,9 +45,11 @@ int wd2_trid_fallbacks(void);
  * sweep.  Both give the reference's iterates bit for bit.  Returns the
  * previous setting. */
 int wd2_set_tiled_sor(int enable);
-/* Lexicographic Sor (nPpeSolver 1) on grids of up to 512 pressure rows runs
- * as one single-workgroup launch per solve, a grid row per lane (on by
- * default); 0 selects the tiled wavefront, one launch per sweep.  Both give
+/* Lexicographic Sor (nPpeSolver 1) runs as a pipeline of sweeps on the tiles
+ * of the red-black kernel where the grid is Cartesian and has no blockages
+ * (solves of up to 16 sweeps excepted), else, on grids of up to 512 pressure
+ * rows, as one single-workgroup launch per solve, a grid row per lane (on by
+ * default); 0 selects the tiled wavefront, one launch per sweep.  All give
  * the reference's iterates bit for bit.  Returns the previous setting. */
 int wd2_set_lex_rows(int enable);
 /* Mixed precision only: solve the FP32 momentum chains of q-l iterations 2..

@@ -1,5 +1,5 @@
-"""The tiled red-black SOR on the GPU against the oracle, bit for bit, where
-its tiles can go wrong: grids around the one-tile limit (64 interior points a
+"""The tiled red-black and lexicographic SOR (solvers 5 and 1) on the GPU
+against the oracle, bit for bit, where the tiles can go wrong: grids around the one-tile limit (64 interior points a
 side), sides that leave a remainder of every kind after the owned points of
 the larger tiles, sweep counts around a launch's, solves that stop inside one,
 the three forms of the division by the diagonal (array coefficients, one
@@ -40,35 +40,39 @@ def _check(oracle, g, nx, ny, msorit, sortol, seed, scale=1.0, blank=False, solv
     return na
 
 
+@pytest.mark.parametrize("solver", [5, 1])
 @pytest.mark.parametrize("kind", ["uniform", "stretched"])
 @pytest.mark.parametrize("nx,ny", [(5, 5), (65, 65), (65, 7), (64, 66), (66, 65), (73, 74), (75, 130), (257, 40),
                                    (385, 90), (401, 450)])
-def test_tiled_sor_sizes(oracle, kind, nx, ny):
-    print(f"tiled sor {kind} {nx} x {ny}", flush=True)
-    _check(oracle, _grid(kind, nx, ny), nx, ny, 31, 1e-30, nx)
+def test_tiled_sor_sizes(oracle, kind, nx, ny, solver):
+    print(f"tiled sor {solver} {kind} {nx} x {ny}", flush=True)
+    _check(oracle, _grid(kind, nx, ny), nx, ny, 31, 1e-30, nx, solver=solver)
 
 
 @pytest.mark.parametrize("nx", [49, 65, 129])   # one value; one power of two; one power of two over tiles
-@pytest.mark.parametrize("msorit", [1, 2, 13, 14, 15, 28, 29])
-def test_tiled_sor_sweep_counts(oracle, nx, msorit):
-    print(f"tiled sor sweeps {nx} {msorit}", flush=True)
+@pytest.mark.parametrize("solver,msorit", [(5, m) for m in (1, 2, 13, 14, 15, 28, 29)] +
+                         [(1, m) for m in (1, 16, 17, 33, 64, 65, 200)])
+def test_tiled_sor_sweep_counts(oracle, nx, solver, msorit):
+    print(f"tiled sor {solver} sweeps {nx} {msorit}", flush=True)
     g = _grid("uniform", nx, nx)
-    assert _check(oracle, g, nx, nx, msorit, 1e-30, 1) == msorit
-    _check(oracle, g, nx, nx, msorit, 1e30, 2)   # stops at the first sweep that may
+    assert _check(oracle, g, nx, nx, msorit, 1e-30, 1, solver=solver) == msorit
+    _check(oracle, g, nx, nx, msorit, 1e30, 2, solver=solver)   # stops at the first sweep that may
 
 
 @pytest.mark.parametrize("kind", ["uniform", "stretched"])
 @pytest.mark.parametrize("nx", [50, 65, 97])
-def test_tiled_sor_stops_inside_a_launch(oracle, kind, nx):
+@pytest.mark.parametrize("solver", [5, 1])
+def test_tiled_sor_stops_inside_a_launch(oracle, kind, nx, solver):
     g = _grid(kind, nx, nx)
-    stops = {_check(oracle, g, nx, nx, 6000, tol, 3, scale=1e-3) for tol in 10.0 ** -np.arange(1.0, 9.0)}
-    print(f"tiled sor stops {kind} {nx} {sorted(stops)}", flush=True)
+    stops = {_check(oracle, g, nx, nx, 6000, tol, 3, scale=1e-3, solver=solver) for tol in 10.0 ** -np.arange(1.0, 9.0)}
+    print(f"tiled sor {solver} stops {kind} {nx} {sorted(stops)}", flush=True)
     assert len(stops) > 2
 
 
 @pytest.mark.parametrize("kind", ["uniform", "stretched"])
 @pytest.mark.parametrize("nx", [50, 65, 97])
 @pytest.mark.parametrize("scale,blank", [(1.0, True), (0.0, False), (1e-250, False), (1e250, False), (1e308, False)])
-def test_tiled_sor_extreme_quotients(oracle, kind, nx, scale, blank):
-    print(f"tiled sor quotients {kind} {nx} {scale} {blank}", flush=True)
-    _check(oracle, _grid(kind, nx, nx), nx, nx, 17, 1e-300, 4, scale, blank)
+@pytest.mark.parametrize("solver", [5, 1])
+def test_tiled_sor_extreme_quotients(oracle, kind, nx, scale, blank, solver):
+    print(f"tiled sor {solver} quotients {kind} {nx} {scale} {blank}", flush=True)
+    _check(oracle, _grid(kind, nx, nx), nx, nx, 17, 1e-300, 4, scale, blank, solver)

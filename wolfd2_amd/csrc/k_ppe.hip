@@ -7,7 +7,10 @@
 //     colour only read points of the other, so every point's arithmetic is
 //     the reference's regardless of order; the unrelaxed |s| is max-reduced
 //     through per-workgroup partials that the next sweep's kernel folds.
-//   Sor (pressure.f:384-450): lexicographic Gauss-Seidel.  A point needs its
+//   Sor (pressure.f:384-450): lexicographic Gauss-Seidel, on Cartesian grids
+//     without blockages as a pipeline of sweeps on the same tiles (ST_LEX);
+//     otherwise, and for short solves, a row a lane (k_sor_lex_rows) or, past
+//     its rows, tile by tile (k_sor_lex).  There a point needs its
 //     west and south neighbours of this sweep and its east and north neighbours
 //     of the last one, so 64x64 tiles run in wavefront order (each workgroup
 //     takes the next tile in row-major order from an atomic ticket and waits for
@@ -209,12 +212,22 @@ void launch_sor_rb_check(int nx, int ny, int sweep, double sortol, int msorit, c
 // took 3.1 us on 251 x 243 cells, 6.5 on 1000^2 and, with uniform coefficients,
 // 2.8 on 64^2, 2.9 on 512^2 and 4.2 on 1024^2; here 1.5, 4.5, 0.9, 1.3 and 2.9.
 //
-// WHOLE: a grid of at most ST_W x ST_W interior points is one tile without a
+// ST_WHOLE: a grid of at most ST_W x ST_W interior points is one tile without a
 // halo: the ghost cells are constants, and one workgroup runs the sweeps of
 // the whole solve with the stopping test after each (0.9 us a sweep where
 // tiles of 14 sweeps a launch take 1.0).
 //
-// Otherwise the kernel reads p_in and writes the owned points to p_out (tiles
+// ST_LEX: Sor (pressure.f:384-450), the lexicographic sweeps.  A point needs
+// its west and south neighbours of its own sweep and its east and north ones
+// of the sweep before, so at half sweep T every point with i + j of T's parity
+// can run its sweep m = (T - i - j) / 2: a lexicographic solve of M sweeps is
+// a red-black one of (nx + ny) / 2 + M in which a point starts at its first
+// sweep and stops after its last, value for value the reference's.  A sweep's
+// stopping test is known when the last point has run it; the tiles gather it
+// as bits of sweeps with a point not below sortol.  A row a lane, a sweep of
+// 97 x 75 cells took 73 us; here 1.4.
+//
+// With ST_TILES and ST_LEX the kernel reads p_in and writes the owned points to p_out (tiles
 // read their neighbours' points as halo, so it cannot work in place).  The
 // stopping test of sweep m is max|s| < sortol over the whole grid
 // (pressure.f:534), which holds exactly when it holds on every tile: each tile
@@ -235,6 +248,8 @@ constexpr int ST_L = ST_W / 2;       // lanes of a strip
 constexpr int ST_N = ST_W / ST_R;    // strips
 constexpr double ST_TINY = 0x1p-400, ST_HUGE = 0x1p400;
 
+enum { ST_TILES = 0, ST_WHOLE = 1, ST_LEX = 2 };
+
 template <int CTRL>
 __device__ inline double st_dpp(double v) {
     const long long b = __double_as_longlong(v);
@@ -253,6 +268,8 @@ struct StArgs {
     unsigned *masks;
     const unsigned *prev_masks;
     Scalars *sc;
+    int pair, cap;     // ST_LEX: first pair of half sweeps, last sweep
+    unsigned *bits;    // ST_LEX: bit m - 1: some point's |s| in sweep m is not below sortol
 };
 
 // One lane's part of a tile.  [r][h]: row r of the strip, column h of the pair.
@@ -266,12 +283,15 @@ struct StTile {
 };
 
 // The points of colour C ((i + j) & 1 == C) of one half sweep.  sS, sN: the
-// rows below and above the strip; gw, ge: WHOLE, the west ghosts of a strip's
-// first lane and the east ones of its last.  Returns the lanes that own a
-// point whose |s| is not below sortol (a NaN counts as not converged).
-template <int MODE, bool WHOLE, int C>
-__device__ __forceinline__ unsigned long long st_half(StTile<MODE> &t, double sS, double sN, const double *gw,
-                                                      const double *ge, int l, const StArgs &A) {
+// rows below and above the strip; gw, ge: ST_WHOLE, the west ghosts of a
+// strip's first lane and the east ones of its last.  act, ST_LEX: whether the
+// points with (r + h) / 2 = 0, 1, 2 are within their sweeps.  big[] receives
+// the lanes that own a point whose |s| is not below sortol (a NaN counts as
+// not converged), by the same index with ST_LEX, else all in big[0].
+template <int MODE, int KIND, int C>
+__device__ __forceinline__ void st_half(StTile<MODE> &t, double sS, double sN, const double *gw, const double *ge,
+                                        int l, const StArgs &A, const bool *act, unsigned long long *big) {
+    constexpr bool WHOLE = KIND == ST_WHOLE, LEX = KIND == ST_LEX;
     double x[ST_R], q[ST_R];
     bool bad = MODE != 2 && t.divide;
     // the inner rows first, kept there by the empty asm: the end rows'
@@ -301,27 +321,29 @@ __device__ __forceinline__ unsigned long long st_half(StTile<MODE> &t, double sS
         if (MODE != 2) {
             q[r] = __builtin_fma(__builtin_fma(-d, q[r], x[r]), rd, q[r]);
             q[r] = __builtin_fma(__builtin_fma(-d, q[r], x[r]), rd, q[r]);
-            bad |= t.up[r][h] && !(fabs(q[r]) > ST_TINY);
+            bad |= t.up[r][h] && (!LEX || act[(r + h) / 2]) && !(fabs(q[r]) > ST_TINY);
         }
     }
     if (MODE != 2 && __any(bad)) {
 #pragma unroll
         for (int r = 0; r < ST_R; r++) q[r] = x[r] / (MODE ? A.d_c : t.d[r][(r ^ C) & 1]);
     }
-    unsigned long long big = 0;
 #pragma unroll
     for (int r = 0; r < ST_R; r++) {
-        const int h = (r ^ C) & 1;
+        const int h = (r ^ C) & 1, dl = (r + h) / 2;
+        const bool up = t.up[r][h] && (!LEX || act[dl]);
         const double s = q[r] - t.p[r][h];
         const double pn = t.p[r][h] + A.sorrel * s;
-        t.p[r][h] = t.up[r][h] ? pn : t.p[r][h];
-        big |= __ballot(!(fabs(s) < A.sortol)) & t.own[r][h];
+        t.p[r][h] = up ? pn : t.p[r][h];
+        const unsigned long long b = __ballot(!(fabs(s) < A.sortol)) & t.own[r][h];
+        if (LEX) big[dl] |= b & __ballot(act[dl]);
+        else big[0] |= b;
     }
-    return big;
 }
 
-template <int MODE, bool WHOLE>
-__global__ __launch_bounds__(ST_T, WHOLE ? 2 : 4) void k_sor_tiled(StArgs A) {
+template <int MODE, int KIND>
+__global__ __launch_bounds__(ST_T, KIND == ST_WHOLE ? 2 : 4) void k_sor_tiled(StArgs A) {
+    constexpr bool WHOLE = KIND == ST_WHOLE, LEX = KIND == ST_LEX;
     // the strips' first and last rows by colour; strips 0 and ST_N + 1 are the
     // rows below and above the tile (WHOLE: the ghost rows)
     __shared__ double EB[2][ST_N + 2][ST_L], ET[2][ST_N + 2][ST_L];
@@ -368,7 +390,7 @@ __global__ __launch_bounds__(ST_T, WHOLE ? 2 : 4) void k_sor_tiled(StArgs A) {
         }
     }
     if (!A.force && A.sc->sor_done) return;
-    if (!WHOLE && !A.force && A.prev_nsweep > 0) {
+    if (KIND == ST_TILES && !A.force && A.prev_nsweep > 0) {
         int conv = 0;
         const int k = tiled_stop(tiled_mask(A.prev_masks, A.ntiles, sh), A.prev_nsweep, A.prev_m0, A.msorit, &conv);
         if (k > 0) {
@@ -427,6 +449,11 @@ __global__ __launch_bounds__(ST_T, WHOLE ? 2 : 4) void k_sor_tiled(StArgs A) {
     __syncthreads();
     const int lo_w = 8 * w, hi_w = 8 * w + 7;   // the wavefront's rows
     unsigned below = 0;   // bit s: the wavefront's owned max |s| of sweep s is < sortol
+    // ST_LEX: the lane's sweep m - 1 at s = 0, (r + h) / 2 = 0, the
+    // wavefront's first lane's, and the sweeps with a point not below sortol
+    // (bit k: m - 1 = base_w - 35 + k)
+    const int base_w = A.pair - (i0 + j0) / 2 - 1 - 4 * w, base = A.pair - (i0 + j0) / 2 - 1 - l - 2 * st;
+    unsigned long long acc = 0;
     for (int s = 0; s < A.nsweep; s++) {
         // rows that the owned points still depend on: one less a side per half sweep
         const int rem = 2 * (A.nsweep - 1 - s);
@@ -444,22 +471,35 @@ __global__ __launch_bounds__(ST_T, WHOLE ? 2 : 4) void k_sor_tiled(StArgs A) {
                 break;
             }
         }
-        unsigned long long big = 0;
-        if (act0) {
-            big = st_half<MODE, WHOLE, 0>(t, ET[1][st][l], EB[1][st + 2][l], gw, ge, l, A);
+        unsigned long long big[3] = {0, 0, 0};
+        bool act[3] = {true, true, true};
+        bool on = true;   // ST_LEX: some lane's points are within their sweeps
+        if (LEX) {
+#pragma unroll
+            for (int d = 0; d < 3; d++) act[d] = (unsigned)(base + s - d) < (unsigned)A.cap;
+            on = __any(act[0] || act[1] || act[2]);
+        }
+        if (act0 && on) {
+            st_half<MODE, KIND, 0>(t, ET[1][st][l], EB[1][st + 2][l], gw, ge, l, A, act, big);
             EB[0][st + 1][l] = t.p[0][0];
             ET[0][st + 1][l] = t.p[ST_R - 1][1];
         }
         __syncthreads();
         if (WHOLE && tid == 0) more[(s + 1) & 1] = 0;
-        if (act1) {
-            big |= st_half<MODE, WHOLE, 1>(t, ET[0][st][l], EB[0][st + 2][l], gw, ge, l, A);
+        if (act1 && on) {
+            st_half<MODE, KIND, 1>(t, ET[0][st][l], EB[0][st + 2][l], gw, ge, l, A, act, big);
             EB[1][st + 1][l] = t.p[0][1];
             ET[1][st + 1][l] = t.p[ST_R - 1][0];
         }
         if (WHOLE) {
-            if (big != 0) more[s & 1] = 1;
-        } else if (big == 0) {
+            if (big[0] != 0) more[s & 1] = 1;
+        } else if (LEX) {
+#pragma unroll
+            for (int d = 0; d < 3; d++) {
+                const unsigned long long x = __brevll(big[d]);
+                acc |= ((x & 0xffffffffull) | ((x >> 32) << 2)) << (s + 2 - d);
+            }
+        } else if (big[0] == 0) {
             below |= 1u << s;
         }
         __syncthreads();
@@ -482,6 +522,20 @@ __global__ __launch_bounds__(ST_T, WHOLE ? 2 : 4) void k_sor_tiled(StArgs A) {
         else if (t.own[r][1] & me) q[1] = t.p[r][1];
     }
     if (WHOLE) return;
+    if (LEX) {
+        const int lane = tid & 63, b0 = base_w - 35, off = b0 & 31;
+        if (lane < 3) {
+            const unsigned long long lo = acc << off;
+            const unsigned v = lane == 0 ? (unsigned)lo : lane == 1 ? (unsigned)(lo >> 32)
+                                                        : off ? (unsigned)(acc >> (64 - off)) : 0u;
+            // most sweeps' bits are set by the first tile that gets there
+            if (v) {
+                unsigned *q = A.bits + (b0 >> 5) + lane;
+                if ((__hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & v) != v) atomicOr(q, v);
+            }
+        }
+        return;
+    }
     // tile mask = AND over the wavefronts (below is the same in every lane of one)
     if ((tid & 63) == 0) sh[w] = below;
     __syncthreads();
@@ -558,23 +612,88 @@ void launch_sor_tiled(int nx, int ny, int ld, const Metrics &m, const double *b,
     const int nt = sor_tiled_tiles(nx, ny, &ntx);
     StArgs A{nx, ny, ld, nsweep, 0, msorit, prev_nsweep, prev_m0, prev_launch, ntx, nt, ST_W - 4 * sor_tiled_sweeps(nx, ny), force,
                    sorrel, sortol, 0.0, 0.0, 0.0, 0.0, m.rau, m.rgv, b, p_in, p_out, masks,
-                   prev_masks, sc};
+             prev_masks, sc, 0, 0, nullptr};
     const dim3 g(8 * ((nt + 7) / 8));
     const int mode = st_uniform(uni, A);
-    if (mode == 2) hipLaunchKernelGGL((k_sor_tiled<2, false>), g, dim3(ST_T), 0, s, A);
-    else if (mode == 1) hipLaunchKernelGGL((k_sor_tiled<1, false>), g, dim3(ST_T), 0, s, A);
-    else hipLaunchKernelGGL((k_sor_tiled<0, false>), g, dim3(ST_T), 0, s, A);
+    if (mode == 2) hipLaunchKernelGGL((k_sor_tiled<2, ST_TILES>), g, dim3(ST_T), 0, s, A);
+    else if (mode == 1) hipLaunchKernelGGL((k_sor_tiled<1, ST_TILES>), g, dim3(ST_T), 0, s, A);
+    else hipLaunchKernelGGL((k_sor_tiled<0, ST_TILES>), g, dim3(ST_T), 0, s, A);
+}
+
+void launch_sor_lex_tiled(int nx, int ny, int ld, const Metrics &m, const double *b, double sorrel, int npair,
+                          int pair, int cap, const double *p_in, double *p_out, unsigned *bits, double sortol,
+                          Scalars *sc, int force, const double *uni, hipStream_t s) {
+    int ntx = 0;
+    const int nt = sor_tiled_tiles(nx, ny, &ntx);
+    StArgs A{nx, ny, ld, npair, 0, 0, 0, 0, 0, ntx, nt, ST_W - 4 * sor_tiled_sweeps(nx, ny), force,
+             sorrel, sortol, 0.0, 0.0, 0.0, 0.0, m.rau, m.rgv, b, p_in, p_out, nullptr,
+             nullptr, sc, pair, cap, bits};
+    const dim3 g(8 * ((nt + 7) / 8));
+    const int mode = st_uniform(uni, A);
+    if (mode == 2) hipLaunchKernelGGL((k_sor_tiled<2, ST_LEX>), g, dim3(ST_T), 0, s, A);
+    else if (mode == 1) hipLaunchKernelGGL((k_sor_tiled<1, ST_LEX>), g, dim3(ST_T), 0, s, A);
+    else hipLaunchKernelGGL((k_sor_tiled<0, ST_LEX>), g, dim3(ST_T), 0, s, A);
+}
+
+// Start of a solve: the ghost frame of p (which no sweep writes) into the
+// other buffers, and the sweeps' bits cleared.
+__global__ __launch_bounds__(256) void k_lex_begin(int nx, int ny, int ld, const double *p, LexBufs o, unsigned *bits,
+                                                   int nwords) {
+    const int q = blockIdx.x * 256 + threadIdx.x;
+    if (q < nwords) bits[q] = 0;
+    const int nr = 3 * (nx + 2), n = nr + 3 * (ny + 2);
+    if (q >= n) return;
+    const int a = q < nr ? q % (nx + 2) : (q - nr) % (ny + 2), e = q < nr ? q / (nx + 2) : (q - nr) / (ny + 2);
+    const size_t k = q < nr ? WD2_IX(a, e < 2 ? e : ny + 1) : WD2_IX(e < 2 ? e : nx + 1, a);
+    const double v = p[k];
+#pragma unroll
+    for (int c = 0; c < LEX_BUFS; c++) o.b[c][k] = v;
+}
+
+void launch_lex_begin(int nx, int ny, int ld, const double *p, const LexBufs &o, unsigned *bits, int cap,
+                      hipStream_t s) {
+    const int nwords = (cap + 31) / 32, n = std::max(nwords, 3 * (nx + 2) + 3 * (ny + 2));
+    hipLaunchKernelGGL(k_lex_begin, dim3((n + 255) / 256), dim3(256), 0, s, nx, ny, ld, p, o, bits, nwords);
+}
+
+// The stopping test of sweeps m_lo .. m_hi, all complete (one wavefront): the
+// first of them, but not the solve's first sweep, without a point that is not
+// below sortol; cap: the last sweep of the run (m0 sweeps came before it).
+__global__ __launch_bounds__(64) void k_lex_check(const unsigned *bits, int m_lo, int m_hi, int m0, int cap,
+                                                  Scalars *sc) {
+    if (sc->sor_done) return;
+    int best = 0x7fffffff;
+    for (int w = (m_lo - 1) / 32 + threadIdx.x; w <= (m_hi - 1) / 32; w += 64) {
+        unsigned ok = ~bits[w];
+        if (32 * w + 1 < m_lo) ok &= ~0u << (m_lo - 1 - 32 * w);
+        if (32 * w + 32 > m_hi) ok &= ~0u >> (32 * w + 32 - m_hi);
+        if (m0 == 0 && w == 0) ok &= ~1u;
+        if (ok) {
+            best = 32 * w + __ffs(ok);
+            break;
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) best = min(best, __shfl_xor(best, off));
+    if (threadIdx.x == 0 && (best <= m_hi || m_hi >= cap)) {
+        sc->sor_done = 1;
+        sc->sor_nconv = best <= m_hi ? m0 + best : 0;
+        sc->sor_m = best <= m_hi ? best : cap;
+    }
+}
+
+void launch_lex_check(const unsigned *bits, int m_lo, int m_hi, int m0, int cap, Scalars *sc, hipStream_t s) {
+    hipLaunchKernelGGL(k_lex_check, dim3(1), dim3(64), 0, s, bits, m_lo, m_hi, m0, cap, sc);
 }
 
 void launch_sor_whole(int nx, int ny, int ld, const Metrics &m, const double *b, double sorrel, int nsweep, int m0,
                       double *p, double sortol, int msorit, Scalars *sc, const double *uni, hipStream_t s) {
     StArgs A{nx, ny, ld, nsweep, m0, msorit, 0, 0, 0, 1, 1, ST_W, 0,
                    sorrel, sortol, 0.0, 0.0, 0.0, 0.0, m.rau, m.rgv, b, p, p, nullptr,
-                   nullptr, sc};
+             nullptr, sc, 0, 0, nullptr};
     const int mode = st_uniform(uni, A);
-    if (mode == 2) hipLaunchKernelGGL((k_sor_tiled<2, true>), dim3(1), dim3(ST_T), 0, s, A);
-    else if (mode == 1) hipLaunchKernelGGL((k_sor_tiled<1, true>), dim3(1), dim3(ST_T), 0, s, A);
-    else hipLaunchKernelGGL((k_sor_tiled<0, true>), dim3(1), dim3(ST_T), 0, s, A);
+    if (mode == 2) hipLaunchKernelGGL((k_sor_tiled<2, ST_WHOLE>), dim3(1), dim3(ST_T), 0, s, A);
+    else if (mode == 1) hipLaunchKernelGGL((k_sor_tiled<1, ST_WHOLE>), dim3(1), dim3(ST_T), 0, s, A);
+    else hipLaunchKernelGGL((k_sor_tiled<0, ST_WHOLE>), dim3(1), dim3(ST_T), 0, s, A);
 }
 
 void launch_sor_tiled_check(int ntiles, int nsweep, int m0, int launch, int msorit, const unsigned *masks,

@@ -127,6 +127,10 @@ struct wd2_ctx {
     // {rau, rgv} when each is one value over the entries the tiled red-black
     // SOR reads (a uniform Cartesian grid); uni_ok false otherwise
     bool uni_ok = false;
+    // lexicographic Sor on tiles: three kept states (allocated by the first
+    // solve that needs them), and whether the last solve was a short one
+    double *lexbuf = nullptr;
+    bool lex_short = false;
     double uni[2] = {0.0, 0.0};
     // multigrid Poisson solver (nPpeSolver 7): its levels and their storage,
     // the per-tile residual maxima, the precision and metric version its
@@ -238,6 +242,7 @@ static void ctx_free(wd2_ctx *c) {
     (void)hipFree(c->metric_store);
     (void)hipFree(c->store);
     (void)hipFree(c->partials);
+    (void)hipFree(c->lexbuf);
     (void)hipFree(c->sc);
     (void)hipFree(c->tile_flags);
     (void)hipFree(c->mg_store);
@@ -961,6 +966,94 @@ static int ppe_mg(wd2_ctx *c, int cart, int maxcyc, double dk, double tol, doubl
     return WD2_OK;
 }
 
+// Lexicographic Sor as tiled half sweeps (launch_sor_lex_tiled): every point
+// runs up to `msorit - m0` sweeps in a pipeline of (nx + ny) / 2 sweeps, m0
+// sweeps having run already.  A sweep's stopping test is complete only when
+// the last point has run it, when others are up to (nx + ny) / 2 sweeps ahead;
+// a solve that stops is run again from a state before that, with the stopping
+// sweep as everyone's last.  Batches of launches of at least that length, two
+// in flight as for the red-black tiles; the states at the starts of the last
+// three batches are kept (one is always early enough: a stopping sweep found
+// by a batch's test was not complete at the batch's start, and the batch
+// before is a pipeline's length earlier).
+static int ppe_lex(wd2_ctx *c, int msorit, double sortol, double sorrel, int m0, double *p, int *nconv_out) {
+    const int nx = c->nx, ny = c->ny, ld = c->ld;
+    hipStream_t s = c->s;
+    const double *uni = (g_uniform && c->uni_ok) ? c->uni : nullptr;
+    const int K = sor_tiled_sweeps(nx, ny), emax = (nx + ny) / 2, B = std::max(emax, 64);
+    const LexBufs bufs{c->pscr, c->beff, c->lexbuf, c->lexbuf + c->nf, c->lexbuf + 2 * c->nf};
+    unsigned *bits = (unsigned *)c->partials;
+    constexpr int SEG = 1 << 19;   // sweeps whose bits the buffer holds
+    *nconv_out = 0;
+    while (m0 < msorit) {
+        const int cap = std::min(SEG, msorit - m0);
+        launch_lex_begin(nx, ny, ld, p, bufs, bits, cap, s);
+        int P = 3, mlo = 1, flip = 0, issued = 0, checked = 0, stop = 0;
+        const int Pend = cap + emax + 1;
+        const double *cur = p;
+        struct { int P; const double *buf; } start[4];
+        auto run = [&](int &P, int end, int cap, double *last, int force) {   // pairs P .. end - 1
+            int n = 0;
+            while (P < end) {
+                const int k = std::min(K, end - P);
+                double *out = (last && P + k >= end) ? last : bufs.b[flip ^= 1];
+                launch_sor_lex_tiled(nx, ny, ld, c->M, c->rhs, sorrel, k, P, cap, cur, out, bits, sortol, c->sc, force,
+                                     uni, s);
+                cur = out;
+                P += k;
+                n++;
+            }
+            return n;
+        };
+        while (!stop) {
+            if (P < Pend && issued - checked < 2) {
+                start[issued % 4] = {P, cur};
+                hipEvent_t *ev = kt_events(c, 1);
+                if (ev) HIPCHK(hipEventRecord(ev[0], s));
+                const int n = run(P, std::min(Pend, P + (B + K - 1) / K * K), cap, bufs.b[2 + issued % 3], 0);
+                if (ev) {
+                    HIPCHK(hipEventRecord(ev[1], s));
+                    c->kt_cnt.back() = n;
+                }
+                const int mhi = std::min(cap, P - 1 - emax);
+                if (mhi >= mlo) {
+                    launch_lex_check(bits, mlo, mhi, m0, cap, c->sc, s);
+                    mlo = mhi + 1;
+                }
+                HIPCHK(hipMemcpyAsync(&c->h_flag[issued % 2], &c->sc->sor_done, sizeof(int), hipMemcpyDeviceToHost,
+                                      s));
+                HIPCHK(hipEventRecord(c->bev[issued % 2], s));
+                issued++;
+                continue;
+            }
+            if (checked == issued) break;
+            HIPCHK(hipEventSynchronize(c->bev[checked % 2]));
+            stop = c->h_flag[checked % 2];
+            checked++;
+        }
+        Scalars h;
+        HIPCHK(hipMemcpy(&h, c->sc, sizeof(Scalars), hipMemcpyDeviceToHost));
+        *nconv_out = h.sor_nconv;
+        if (h.sor_nconv > 0 && h.sor_m < cap) {
+            // batch checked - 1 found it; its start, or the start before
+            int n = checked - 1;
+            if (n > 0 && start[n % 4].P > h.sor_m + 3) n--;
+            P = start[n % 4].P;
+            cur = start[n % 4].buf;
+            run(P, h.sor_m + emax + 1, h.sor_m, nullptr, 1);
+        }
+        if (cur != p) launch_copy(ld, 2, nx, 2, ny, cur, p, s);
+        if (h.sor_nconv > 0) break;
+        m0 += cap;
+        if (m0 < msorit) launch_sor_reset(c->sc, s);
+    }
+    return WD2_OK;
+}
+
+// Lexicographic solves of up to this many sweeps stay on the row kernel: the
+// tiles' pipeline runs (nx + ny) / 2 sweeps more than the solve's, twice where
+// it stops (128^2 cells: 75 us a sweep by rows, 1.4 by tiles).
+constexpr int LEX_SHORT = 16;
 constexpr int SOR_WHOLE_RUN = 4096;   // sweeps per launch of a one-tile solve (about 3 ms)
 
 static int ppe(wd2_ctx *c, int cart, int solver, int msorit, double dk, double sortol, double sorrel,
@@ -1089,10 +1182,37 @@ static int ppe(wd2_ctx *c, int cart, int solver, int msorit, double dk, double s
     }
     const int batch = (solver == 2) ? 1 : 64;
     int done = 0;
-    if (solver == 1 && g_lex_rows && ny - 1 <= sor_lex_rows_max()) {
-        launch_sor_lex_rows(nx, ny, ld, c->M, coef, c->rhs, c->beff, cart ? 1 : 0, sorrel, sortol, msorit, p, c->sc,
-                            s);
-        done = 1;
+    if (solver == 1 && g_lex_rows) {
+        const bool rows = ny - 1 <= sor_lex_rows_max();
+        bool tiles = cart && !coef && msorit > LEX_SHORT;
+        if (tiles && !c->lexbuf && hipMalloc(&c->lexbuf, 3 * c->nf * sizeof(double)) != hipSuccess) {
+            (void)hipGetLastError();
+            c->lexbuf = nullptr;
+            tiles = false;
+        }
+        // where the last solve was a short one, its length of sweeps by rows first
+        const int nrows = !rows ? 0 : tiles ? (c->lex_short ? LEX_SHORT : 0) : msorit;
+        if (nrows > 0) {
+            launch_sor_lex_rows(nx, ny, ld, c->M, coef, c->rhs, c->beff, cart ? 1 : 0, sorrel, sortol, nrows, p,
+                                c->sc, s);
+            done = 1;
+        }
+        if (tiles) {
+            int nconv = 0;
+            if (nrows > 0) {
+                int h[2];   // sor_done, sor_nconv
+                HIPCHK(hipMemcpyAsync(h, &c->sc->sor_done, sizeof(h), hipMemcpyDeviceToHost, s));
+                HIPCHK(hipStreamSynchronize(s));
+                nconv = h[1];
+                if (nconv < 1) launch_sor_reset(c->sc, s);
+            }
+            if (nconv < 1) {
+                const int st = ppe_lex(c, msorit, sortol, sorrel, nrows, p, &nconv);
+                if (st != WD2_OK) return st;
+            }
+            c->lex_short = nconv > 0 && nconv <= LEX_SHORT;
+            done = 1;
+        }
     }
     for (int it = 0; it < msorit && !done;) {
         for (int q = 0; q < batch && it < msorit; q++, it++) {

@@ -148,6 +148,20 @@ void launch_sor_tiled(int nx, int ny, int ld, const Metrics &m, const double *b,
 bool sor_whole(int nx, int ny);
 void launch_sor_whole(int nx, int ny, int ld, const Metrics &m, const double *b, double sorrel, int nsweep, int m0,
                       double *p, double sortol, int msorit, Scalars *sc, const double *uni, hipStream_t s);
+// Lexicographic Sor on the same tiles (Cartesian, no blockage): half sweeps
+// 2 pair .. 2 (pair + npair) - 1 of p_in into p_out, npair <= sor_tiled_sweeps.
+// A point (i, j) runs sweep pair - (i + j) / 2, from 1 to cap; bit m - 1 of
+// bits is set where a point of sweep m is not below sortol.
+void launch_sor_lex_tiled(int nx, int ny, int ld, const Metrics &m, const double *b, double sorrel, int npair,
+                          int pair, int cap, const double *p_in, double *p_out, unsigned *bits, double sortol,
+                          Scalars *sc, int force, const double *uni, hipStream_t s);
+constexpr int LEX_BUFS = 5;
+struct LexBufs {
+    double *b[LEX_BUFS];   // two the launches alternate between, three that keep a state
+};
+void launch_lex_begin(int nx, int ny, int ld, const double *p, const LexBufs &o, unsigned *bits, int cap,
+                      hipStream_t s);
+void launch_lex_check(const unsigned *bits, int m_lo, int m_hi, int m0, int cap, Scalars *sc, hipStream_t s);
 // Mixed precision (FP64 residual and accumulation, FP32 sweeps), same contract.
 int sor_tiled_mx_tiles(int nx, int ny, int *ntx);
 int sor_tiled_mx_sweeps();
