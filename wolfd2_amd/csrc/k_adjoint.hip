@@ -8,9 +8,9 @@
 // (the convective fluxes, the upwinded chain coefficients) are transposed at
 // the forward state, which the caller recomputes from checkpoints.
 //
-// Scatter-form transposes accumulate with FP64 atomics (the adjoint of a
-// gather is a scatter); the sums are therefore not bit-reproducible, which
-// does not matter to a gradient.
+// Scatter-form transposes accumulate with FP64 atomics, in LDS and between
+// tiles (the adjoint of a gather is a scatter); the sums are therefore not
+// bit-reproducible, which does not matter to a gradient.
 //
 // Pieces and the forward lines they transpose:
 // * chain solves (AltTridLU, momentum.f:1307-1339, with the first-row pivot
@@ -57,61 +57,61 @@ __device__ inline long apos(const Chains &cs, long k, long &L) {
 // S(k-1,k) = C[k-1] (c1 d1 / d2 on a chain's first row), diagonal D[k] and
 // super-diagonal S(k+1,k) = A[k+1]; on a chain's first row the super-diagonal
 // is given as A[k+1] D[k+1] / D[k], which the solver's own first-row quirk
-// turns back into A[k+1].
+// turns back into A[k+1].  *dom (from +0) receives the largest (|sub| +
+// |super|) / |diagonal| of the rows (a NaN wins).
 __global__ __launch_bounds__(AT) void k_adj_tchain(long n, Chains cs, const double *__restrict__ A,
                                                    const double *__restrict__ D, const double *__restrict__ C,
                                                    double *__restrict__ At, double *__restrict__ Dt,
-                                                   double *__restrict__ Ct) {
-    const long k = (long)blockIdx.x * AT + threadIdx.x;
-    if (k >= n) return;
-    long L;
-    const long r = apos(cs, k, L);
-    Dt[k] = D[k];
-    double sub = 0.0, sup = 0.0;
-    if (r > 0) sub = (r - 1 == 0) ? C[k - 1] * D[k - 1] / D[k] : C[k - 1];
-    if (r < L - 1) sup = (r == 0) ? A[k + 1] * D[k + 1] / D[k] : A[k + 1];
-    At[k] = sub;
-    Ct[k] = sup;
+                                                   double *__restrict__ Ct, unsigned long long *dom) {
+    double m = 0.0;
+    for (long k = (long)blockIdx.x * AT + threadIdx.x; k < n; k += (long)gridDim.x * AT) {
+        long L;
+        const long r = apos(cs, k, L);
+        Dt[k] = D[k];
+        double sub = 0.0, sup = 0.0;
+        if (r > 0) sub = (r - 1 == 0) ? C[k - 1] * D[k - 1] / D[k] : C[k - 1];
+        if (r < L - 1) sup = (r == 0) ? A[k + 1] * D[k + 1] / D[k] : A[k + 1];
+        At[k] = sub;
+        Ct[k] = sup;
+        const double q = (fabs(sub) + fabs(sup)) / fabs(D[k]);
+        if (!(q <= m)) m = q;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        const double o = __shfl_xor(m, off);
+        if (!(o <= m)) m = o;
+    }
+    if ((threadIdx.x & 63) == 0) atomicMax(dom, dbits(m));
 }
 
-// Coefficient adjoints -mu_k x_{k-1}, -mu_k x_k, -mu_k x_{k+1} of the
+// Coefficient adjoints -mu_k x_{k-1}, -mu_k x_k, -mu_k x_{k+1} of row k of the
 // matrix S of a solve S x = b (S with the chain solver's first-row quirk
-// S(1,2) = c1 d1 / d2).  Z (optional): rows whose coefficients are constants
-// (identity rows) get none.  XK (optional): x is taken as +0 on the rows not
-// flagged in XK -- at a converged q-l fixed point the first split's x
-// vanishes on every row but the second split's identity rows, and only
-// those rows' columns of S carry a derivative.
-__global__ __launch_bounds__(AT) void k_adj_coef(long n, Chains cs, const double *__restrict__ A,
-                                                 const double *__restrict__ D, const double *__restrict__ C,
-                                                 const double *__restrict__ mu, const double *__restrict__ x,
-                                                 const unsigned char *__restrict__ Z,
-                                                 const unsigned char *__restrict__ XK, double *__restrict__ Ab,
-                                                 double *__restrict__ Db, double *__restrict__ Cb) {
-    const long k = (long)blockIdx.x * AT + threadIdx.x;
-    if (k >= n) return;
+// S(1,2) = c1 d1 / d2).  x is taken as +0 on the rows not flagged in XK -- at
+// a converged q-l fixed point the first split's x vanishes on every row but
+// the second split's identity rows, and only those rows' columns of S carry a
+// derivative.
+struct AdjChain {
+    const double *A, *D, *C, *mu, *x;
+    const unsigned char *XK;
+};
+__device__ inline void adj_coef(const AdjChain &q, const Chains &cs, long k, double m, double &ab, double &db,
+                                double &cb) {
     long L;
     const long r = apos(cs, k, L);
-    auto xv = [&](long q) { return (XK && !XK[q]) ? 0.0 : x[q]; };
-    double ab = 0.0, db = 0.0, cb = 0.0;
-    if (!(Z && Z[k])) {
-        const double m = mu[k];
-        db = -m * xv(k);
-        if (r > 0) ab = -m * xv(k - 1);
-        if (r < L - 1) {
-            const double sb = -m * xv(k + 1);   // adjoint of the entry S(k, k+1)
-            if (r == 0) {   // S(1,2) = c1 d1 / d2
-                cb = sb * D[k] / D[k + 1];
-                db += sb * C[k] / D[k + 1];
-            } else {
-                cb = sb;
-            }
+    auto xv = [&](long o) { return q.XK[o] ? q.x[o] : 0.0; };
+    ab = cb = 0.0;
+    db = -m * xv(k);
+    if (r > 0) ab = -m * xv(k - 1);
+    if (r < L - 1) {
+        const double sb = -m * xv(k + 1);   // adjoint of the entry S(k, k+1)
+        if (r == 0) {   // S(1,2) = c1 d1 / d2
+            cb = sb * q.D[k] / q.D[k + 1];
+            db += sb * q.C[k] / q.D[k + 1];
+        } else {
+            cb = sb;
         }
     }
     // row 2's diagonal also enters S(1,2): d(c1 d1 / d2)/d d2 = -c1 d1 / d2^2
-    if (r == 1 && !(Z && Z[k - 1])) db += mu[k - 1] * xv(k) * C[k - 1] * D[k - 1] / (D[k] * D[k]);
-    Ab[k] = ab;
-    Db[k] = db;
-    Cb[k] = cb;
+    if (r == 1) db += q.mu[k - 1] * xv(k) * q.C[k - 1] * q.D[k - 1] / (q.D[k] * q.D[k]);
 }
 
 // lam in chain order from the adjoints of the increments (X rows i = 1..nx,
@@ -156,21 +156,11 @@ __device__ inline double cj1_x(const Metrics &m, int ld, const double *u, const 
            m.xeu[WD2_IX(i, j)] * (v[WD2_IX(i + 1, j)] + v[WD2_IX(i, j)] + v[WD2_IX(i + 1, j - 1)] + v[WD2_IX(i, j - 1)]) /
                4.0;
 }
-__device__ inline double cj2_x(const Metrics &m, int ld, const double *u, const double *v, int i, int j) {
-    return m.xzu[WD2_IX(i, j)] * (v[WD2_IX(i + 1, j)] + v[WD2_IX(i, j)] + v[WD2_IX(i + 1, j - 1)] + v[WD2_IX(i, j - 1)]) /
-               4.0 -
-           2.0 * m.yzu[WD2_IX(i, j)] * u[WD2_IX(i, j)];
-}
 // ConvCoef case 5 (momentum.f:953-961), djac = 2: written for i = 1..nx, j = 0..ny
 __device__ inline double cj1_y(const Metrics &m, int ld, const double *u, const double *v, int i, int j) {
     return m.yev[WD2_IX(i, j)] * (u[WD2_IX(i, j + 1)] + u[WD2_IX(i - 1, j + 1)] + u[WD2_IX(i, j)] + u[WD2_IX(i - 1, j)]) /
                4.0 -
            2.0 * m.xev[WD2_IX(i, j)] * v[WD2_IX(i, j)];
-}
-__device__ inline double cj2_y(const Metrics &m, int ld, const double *u, const double *v, int i, int j) {
-    return 2.0 * m.xzv[WD2_IX(i, j)] * v[WD2_IX(i, j)] -
-           m.yzv[WD2_IX(i, j)] * (u[WD2_IX(i, j + 1)] + u[WD2_IX(i - 1, j + 1)] + u[WD2_IX(i, j)] + u[WD2_IX(i - 1, j)]) /
-               4.0;
 }
 // ConvCoef case 1 (X, metrics xzn, xec, yzn, yec), djac = 1:
 // c1 written i = 1..nx+1, j = 1..ny+1; c2 written i = 1..nx, j = 1..ny
@@ -197,243 +187,154 @@ __device__ inline double c2_y(const Metrics &m, int ld, const double *u, const d
            0.5;
 }
 
-// DDiffU transposed (momentum.f:1015-1045): d(i,j) += g spreads onto u.
-__device__ inline void ddiff_u_t(const Metrics &m, int ld, double *ub, int i, int j, double g) {
-    const double ac0 = m.rac[WD2_IX(i, j)], ac1 = m.rac[WD2_IX(i + 1, j)];
-    const double bc0 = m.rbc[WD2_IX(i, j)], bc1 = m.rbc[WD2_IX(i + 1, j)];
-    const double bn0 = m.rbn[WD2_IX(i, j)], bnm = m.rbn[WD2_IX(i, j - 1)];
-    const double gn0 = m.rgn[WD2_IX(i, j)], gnm = m.rgn[WD2_IX(i, j - 1)];
-    // s1
-    aadd(&ub[WD2_IX(i + 1, j)], ac1 * g);
-    aadd(&ub[WD2_IX(i, j)], -(ac1 + ac0) * g);
-    aadd(&ub[WD2_IX(i - 1, j)], ac0 * g);
-    aadd(&ub[WD2_IX(i + 1, j + 1)], bc1 * g);
-    aadd(&ub[WD2_IX(i, j + 1)], (bc1 - bc0) * g);
-    aadd(&ub[WD2_IX(i + 1, j - 1)], -bc1 * g);
-    aadd(&ub[WD2_IX(i, j - 1)], (-bc1 + bc0) * g);
-    aadd(&ub[WD2_IX(i - 1, j + 1)], -bc0 * g);
-    aadd(&ub[WD2_IX(i - 1, j - 1)], bc0 * g);
-    // s2
-    aadd(&ub[WD2_IX(i + 1, j + 1)], bn0 * g);
-    aadd(&ub[WD2_IX(i + 1, j)], (bn0 - bnm) * g);
-    aadd(&ub[WD2_IX(i - 1, j + 1)], -bn0 * g);
-    aadd(&ub[WD2_IX(i - 1, j)], (-bn0 + bnm) * g);
-    aadd(&ub[WD2_IX(i + 1, j - 1)], -bnm * g);
-    aadd(&ub[WD2_IX(i - 1, j - 1)], bnm * g);
-    aadd(&ub[WD2_IX(i, j + 1)], gn0 * g);
-    aadd(&ub[WD2_IX(i, j)], -(gn0 + gnm) * g);
-    aadd(&ub[WD2_IX(i, j - 1)], gnm * g);
-}
+// The rows of one component transposed: the adjoints of the first split's
+// chain coefficients and right-hand side (bb = nu) go through the assembly
+// (momentum.f:350-384; 675-754), DConvU/V, DDiffU/V (1015-1045; 1079-1109) and
+// the ConvCoef cases onto the fields us, vs and (with_n) un, vn.  The second
+// split's coefficients need no adjoint: at a converged q-l fixed point they
+// only precondition.  Without porous regions and buoyancy the porosity terms
+// are +0.
+//
+// A workgroup takes GT_X x GT_Y rows and adds their contributions up in LDS: fb
+// to the component's own field, cj, c1, c2 to the ConvCoef outputs.  All of it
+// is linear in the rows, so the tile's ConvCoef adjoints are taken on to the
+// fields at once, in gather form, whether or not a neighbouring tile adds to
+// the same face, and only the fields' sums go to memory: about 3 FP64 atomics
+// a row, where scattering each term took some 40 (five launches,
+// 93 us an iteration on 512^2 cells, bound by the atomics; here 37; tiles of
+// eight rows, 512 lanes at 128 registers, 40).
+constexpr int GT_X = 64, GT_Y = 4, GT_T = GT_X * GT_Y;
+constexpr int GT_W = GT_X + 6, GT_H = GT_Y + 6;   // the rows' reach is 2; a ring of zeros
 
-// DDiffV transposed (momentum.f:1079-1109).
-__device__ inline void ddiff_v_t(const Metrics &m, int ld, double *vb, int i, int j, double g) {
-    const double an0 = m.ran[WD2_IX(i, j)], anm = m.ran[WD2_IX(i - 1, j)];
-    const double bn0 = m.rbn[WD2_IX(i, j)], bnm = m.rbn[WD2_IX(i - 1, j)];
-    const double bc1 = m.rbc[WD2_IX(i, j + 1)], bc0 = m.rbc[WD2_IX(i, j)];
-    const double gc1 = m.rgc[WD2_IX(i, j + 1)], gc0 = m.rgc[WD2_IX(i, j)];
-    // s1
-    aadd(&vb[WD2_IX(i + 1, j)], an0 * g);
-    aadd(&vb[WD2_IX(i, j)], -(an0 + anm) * g);
-    aadd(&vb[WD2_IX(i - 1, j)], anm * g);
-    aadd(&vb[WD2_IX(i + 1, j + 1)], bn0 * g);
-    aadd(&vb[WD2_IX(i, j + 1)], (bn0 - bnm) * g);
-    aadd(&vb[WD2_IX(i + 1, j - 1)], -bn0 * g);
-    aadd(&vb[WD2_IX(i, j - 1)], (-bn0 + bnm) * g);
-    aadd(&vb[WD2_IX(i - 1, j + 1)], -bnm * g);
-    aadd(&vb[WD2_IX(i - 1, j - 1)], bnm * g);
-    // s2
-    aadd(&vb[WD2_IX(i + 1, j + 1)], bc1 * g);
-    aadd(&vb[WD2_IX(i + 1, j)], (bc1 - bc0) * g);
-    aadd(&vb[WD2_IX(i - 1, j + 1)], -bc1 * g);
-    aadd(&vb[WD2_IX(i - 1, j)], (-bc1 + bc0) * g);
-    aadd(&vb[WD2_IX(i + 1, j - 1)], -bc0 * g);
-    aadd(&vb[WD2_IX(i - 1, j - 1)], bc0 * g);
-    aadd(&vb[WD2_IX(i, j + 1)], gc1 * g);
-    aadd(&vb[WD2_IX(i, j)], -(gc1 + gc0) * g);
-    aadd(&vb[WD2_IX(i, j - 1)], gc0 * g);
-}
+struct GtArgs {
+    int nx, ny, ld, with_n;
+    double dk, re;
+    Metrics m;
+    const double *us, *vs, *un, *vn;
+    AdjChain q;
+    Chains cs;
+    double *usb, *vsb, *unb, *vnb;
+};
 
-// XMomentum row (i, j) transposed: the adjoints of the first split's chain
-// coefficients (a1b, d1b, c1b) and right-hand side (bb) go to the fields us,
-// un through the assembly (momentum.f:350-384), DConvU and DDiffU, and to the
-// ConvCoef outputs in A (which k_adj_cc takes on to us, vs, un, vn).  The
-// second split's coefficients need no adjoint: at a converged q-l fixed point
-// they only precondition.  with_n = 0 skips the time-level-n terms.  Without
-// porous regions and buoyancy the porosity terms are +0.
-__global__ __launch_bounds__(AT) void k_adj_asm_x(int nx, int ny, int ld, double dk, double re, Metrics m,
-                                                  const double *__restrict__ us, const double *__restrict__ vs,
-                                                  const double *__restrict__ un, const double *__restrict__ vn,
-                                                  const double *__restrict__ a1b, const double *__restrict__ d1b,
-                                                  const double *__restrict__ c1b, const double *__restrict__ bb,
-                                                  int with_n, double *usb, double *unb, AdjCoefs A) {
-    const long n1 = (long)nx * (ny - 1);
-    const long k = (long)blockIdx.x * AT + threadIdx.x;
-    if (k >= n1) return;
-    const int i = 1 + (int)(k % nx), j = 2 + (int)(k / nx);
-    const double dk2 = dk * 0.5, re1 = 1.0 / re;
-    const double rkj = dk2 * m.dju[WD2_IX(i, j)];
-    // split 1: upwinding on cj1(i,j); cj1(nx+1, j) is never written (+0)
-    if (cj1_x(m, ld, us, vs, i, j) >= 0.0) {
-        aadd(&A.cj1[WD2_IX(i - 1, j)], -rkj * a1b[k]);
-        aadd(&A.cj1[WD2_IX(i, j)], rkj * d1b[k]);
-    } else {
-        aadd(&A.cj1[WD2_IX(i, j)], -rkj * d1b[k]);
-        if (i + 1 <= nx) aadd(&A.cj1[WD2_IX(i + 1, j)], rkj * c1b[k]);
-    }
-    // right-hand side: b = un - us - rkj (cnvs + cnvn) + rkj re1 (difs + difn)
-    const double b = bb[k];
-    if (with_n) aadd(&unb[WD2_IX(i, j)], b);
-    aadd(&usb[WD2_IX(i, j)], -b);
-    const double gc = -rkj * b, gd = rkj * re1 * b;
-    if (b == 0.0) return;
-    // DConvU on (us; c1s, c2s) and (un; c1n, c2n)
-    for (int lev = 0; lev < 1 + with_n; lev++) {
-        const double *u = lev ? un : us, *v = lev ? vn : vs;
-        double *ub = lev ? unb : usb, *c1 = lev ? A.c1n : A.c1s, *c2 = lev ? A.c2n : A.c2s;
-        const double c1w = c1_x(m, ld, u, v, i, j), c1e = c1_x(m, ld, u, v, i + 1, j);
-        const double c2s = c2_x(m, ld, u, v, i, j - 1), c2n = c2_x(m, ld, u, v, i, j);
-        const double u0 = u[WD2_IX(i, j)];
-        aadd(&ub[WD2_IX(i, j - 1)], -c2s * gc);
-        aadd(&ub[WD2_IX(i - 1, j)], -c1w * gc);
-        aadd(&ub[WD2_IX(i, j)], (c1e - c1w + c2n - c2s) * gc);
-        aadd(&ub[WD2_IX(i + 1, j)], c1e * gc);
-        aadd(&ub[WD2_IX(i, j + 1)], c2n * gc);
-        aadd(&c1[WD2_IX(i, j)], (-u[WD2_IX(i - 1, j)] - u0) * gc);
-        aadd(&c1[WD2_IX(i + 1, j)], (u0 + u[WD2_IX(i + 1, j)]) * gc);
-        aadd(&c2[WD2_IX(i, j)], (u0 + u[WD2_IX(i, j + 1)]) * gc);
-        aadd(&c2[WD2_IX(i, j - 1)], (-u[WD2_IX(i, j - 1)] - u0) * gc);
-        ddiff_u_t(m, ld, ub, i, j, gd);
-    }
-}
-
-// YMomentum row (i, j) transposed (momentum.f:675-754 with DConvV, DDiffV).
-__global__ __launch_bounds__(AT) void k_adj_asm_y(int nx, int ny, int ld, double dk, double re, Metrics m,
-                                                  const double *__restrict__ us, const double *__restrict__ vs,
-                                                  const double *__restrict__ un, const double *__restrict__ vn,
-                                                  const double *__restrict__ a1b, const double *__restrict__ d1b,
-                                                  const double *__restrict__ c1b, const double *__restrict__ bb,
-                                                  int with_n, double *vsb, double *vnb, AdjCoefs A) {
-    const long n2 = (long)(nx - 1) * ny;
-    const long k = (long)blockIdx.x * AT + threadIdx.x;
-    if (k >= n2) return;
-    const int i = 2 + (int)(k % (nx - 1)), j = 1 + (int)(k / (nx - 1));
-    const double dk2 = dk * 0.5, re1 = 1.0 / re;
-    const double rkj = dk2 * m.djv[WD2_IX(i, j)];
-    // split 1: cj1(nx+1, j) is never written
-    if (cj1_y(m, ld, us, vs, i, j) >= 0.0) {
-        aadd(&A.cj1[WD2_IX(i - 1, j)], -rkj * a1b[k]);
-        aadd(&A.cj1[WD2_IX(i, j)], rkj * d1b[k]);
-    } else {
-        aadd(&A.cj1[WD2_IX(i, j)], -rkj * d1b[k]);
-        if (i + 1 <= nx) aadd(&A.cj1[WD2_IX(i + 1, j)], rkj * c1b[k]);
-    }
-    const double b = bb[k];
-    if (with_n) aadd(&vnb[WD2_IX(i, j)], b);
-    aadd(&vsb[WD2_IX(i, j)], -b);
-    if (b == 0.0) return;
-    const double gc = -rkj * b, gd = rkj * re1 * b;
-    for (int lev = 0; lev < 1 + with_n; lev++) {
-        const double *u = lev ? un : us, *v = lev ? vn : vs;
-        double *vb = lev ? vnb : vsb, *c1 = lev ? A.c1n : A.c1s, *c2 = lev ? A.c2n : A.c2s;
-        const double c1w = c1_y(m, ld, u, v, i - 1, j), c1e = c1_y(m, ld, u, v, i, j);
-        const double c2s = c2_y(m, ld, u, v, i, j), c2n = c2_y(m, ld, u, v, i, j + 1);
-        const double v0 = v[WD2_IX(i, j)];
-        aadd(&vb[WD2_IX(i, j - 1)], -c2s * gc);
-        aadd(&vb[WD2_IX(i - 1, j)], -c1w * gc);
-        aadd(&vb[WD2_IX(i, j)], (c1e - c1w + c2n - c2s) * gc);
-        aadd(&vb[WD2_IX(i + 1, j)], c1e * gc);
-        aadd(&vb[WD2_IX(i, j + 1)], c2n * gc);
-        aadd(&c1[WD2_IX(i, j)], (v0 + v[WD2_IX(i + 1, j)]) * gc);
-        aadd(&c1[WD2_IX(i - 1, j)], (-v[WD2_IX(i - 1, j)] - v0) * gc);
-        aadd(&c2[WD2_IX(i, j + 1)], (v0 + v[WD2_IX(i, j + 1)]) * gc);
-        aadd(&c2[WD2_IX(i, j)], (-v[WD2_IX(i, j - 1)] - v0) * gc);
-        ddiff_v_t(m, ld, vb, i, j, gd);
-    }
-}
-
-// The ConvCoef outputs' adjoints of one component onto the fields (every
-// point of the written ranges; entries outside them were never written and
-// their adjoints are dropped).  Each thread clears the adjoints it reads, so
-// A is all zero again for the next assembly transpose (with_n = 0: the
-// time-level-n ones are zero and not read).
-__global__ __launch_bounds__(AT) void k_adj_cc(int comp, int nx, int ny, int ld, Metrics m, AdjCoefs A,
-                                               int with_n, double *usb, double *vsb, double *unb, double *vnb) {
-    const int W = nx + 2;
-    const long q = (long)blockIdx.x * AT + threadIdx.x;
-    if (q >= (long)W * (ny + 2)) return;
-    const int i = (int)(q % W), j = (int)(q / W);
+template <int COMP>
+__device__ inline void gt_tile(const GtArgs &A, int tile, double *fb, double *cj, double *c1, double *c2) {
+    const int nx = A.nx, ny = A.ny, ld = A.ld, tid = threadIdx.x;
+    const Metrics &m = A.m;
+    const int ib = COMP == 1 ? 1 : 2, jb = COMP == 1 ? 2 : 1, ni = nx - ib + 1, nj = ny - jb + 1;
+    const int gx = (ni + GT_X - 1) / GT_X;
+    const int I0 = ib + (tile % gx) * GT_X, J0 = jb + (tile / gx) * GT_Y;
+    const int oi = I0 - 3, oj = J0 - 3;
+    auto at = [&](int i, int j) { return (j - oj) * GT_W + (i - oi); };
+    auto add = [&](double *f, int i, int j, double v) { atomicAdd(&f[at(i, j)], v); };
+    const int i = I0 + (tid & (GT_X - 1)), j = J0 + tid / GT_X;
+    const bool row = i <= nx && j <= ny;
     const size_t p = WD2_IX(i, j);
-    const double gj1 = A.cj1[p], gj2 = A.cj2[p];
-    const double gc[2][2] = {{A.c1s[p], A.c2s[p]}, {with_n ? A.c1n[p] : 0.0, with_n ? A.c2n[p] : 0.0}};
-    A.cj1[p] = 0.0;
-    A.cj2[p] = 0.0;
-    A.c1s[p] = 0.0;
-    A.c2s[p] = 0.0;
-    if (with_n) {
-        A.c1n[p] = 0.0;
-        A.c2n[p] = 0.0;
+    double b = 0.0, rkj = 0.0, gc = 0.0, gd = 0.0;
+    if (row) {
+        const long k = (COMP == 1 ? 0 : A.cs.n1) + (long)(j - jb) * ni + (i - ib);
+        b = A.q.mu[k];
+        rkj = A.dk * 0.5 * (COMP == 1 ? m.dju : m.djv)[p];
+        // right-hand side: b = un - us - rkj (cnvs + cnvn) + rkj re1 (difs + difn)
+        gc = -rkj * b;
+        gd = rkj * (1.0 / A.re) * b;
     }
-    if (comp == 1) {
-        // case 4 (i = 0..nx, j = 1..ny): cj1 = 2 yeu u - xeu (4 v)/4, cj2 = xzu (4 v)/4 - 2 yzu u
-        if (i <= nx && j >= 1 && j <= ny) {
-            const double g1 = gj1, g2 = gj2;
-            aadd(&usb[p], 2.0 * m.yeu[p] * g1 - 2.0 * m.yzu[p] * g2);
-            const double gv = (-m.xeu[p] * g1 + m.xzu[p] * g2) / 4.0;
-            if (gv != 0.0) {
-                aadd(&vsb[WD2_IX(i + 1, j)], gv);
-                aadd(&vsb[WD2_IX(i, j)], gv);
-                aadd(&vsb[WD2_IX(i + 1, j - 1)], gv);
-                aadd(&vsb[WD2_IX(i, j - 1)], gv);
+    for (int lev = 0; lev < 1 + A.with_n; lev++) {
+        const double *u = lev ? A.un : A.us, *v = lev ? A.vn : A.vs, *f = COMP == 1 ? u : v;
+        for (int q = tid; q < GT_W * GT_H; q += GT_T) fb[q] = cj[q] = c1[q] = c2[q] = 0.0;
+        __syncthreads();
+        if (row && lev == 0) {
+            // split 1: upwinding on cj1(i,j); cj1(nx+1, j) is never written (+0)
+            const long k = (COMP == 1 ? 0 : A.cs.n1) + (long)(j - jb) * ni + (i - ib);
+            double ab, db, cb;
+            adj_coef(A.q, A.cs, k, b, ab, db, cb);
+            if (ab != 0.0 || db != 0.0 || cb != 0.0) {
+                const double c = COMP == 1 ? cj1_x(m, ld, u, v, i, j) : cj1_y(m, ld, u, v, i, j);
+                if (c >= 0.0) {
+                    add(cj, i - 1, j, -rkj * ab);
+                    add(cj, i, j, rkj * db);
+                } else {
+                    add(cj, i, j, -rkj * db);
+                    if (i + 1 <= nx) add(cj, i + 1, j, rkj * cb);
+                }
             }
         }
-        // case 1: c1 (i = 1..nx+1, j = 1..ny+1), c2 (i = 1..nx, j = 1..ny)
-        for (int lev = 0; lev < 1 + with_n; lev++) {
-            double *ub = lev ? unb : usb, *vb = lev ? vnb : vsb;
-            const double g1 = gc[lev][0], g2 = gc[lev][1];
-            if (i >= 1 && j >= 1) {
-                aadd(&ub[WD2_IX(i, j)], 0.5 * m.yec[p] * g1);
-                aadd(&ub[WD2_IX(i - 1, j)], 0.5 * m.yec[p] * g1);
-                aadd(&vb[WD2_IX(i, j)], -0.5 * m.xec[p] * g1);
-                aadd(&vb[WD2_IX(i, j - 1)], -0.5 * m.xec[p] * g1);
+        if (row && b != 0.0) {
+            double c1w, c1e, c2s, c2n, aW, aE, bW, bE, bS, bN, gS, gN;
+            if (COMP == 1) {
+                c1w = c1_x(m, ld, u, v, i, j), c1e = c1_x(m, ld, u, v, i + 1, j);
+                c2s = c2_x(m, ld, u, v, i, j - 1), c2n = c2_x(m, ld, u, v, i, j);
+                aW = m.rac[p], aE = m.rac[WD2_IX(i + 1, j)];
+                bW = m.rbc[p], bE = m.rbc[WD2_IX(i + 1, j)];
+                bS = m.rbn[WD2_IX(i, j - 1)], bN = m.rbn[p];
+                gS = m.rgn[WD2_IX(i, j - 1)], gN = m.rgn[p];
+            } else {
+                c1w = c1_y(m, ld, u, v, i - 1, j), c1e = c1_y(m, ld, u, v, i, j);
+                c2s = c2_y(m, ld, u, v, i, j), c2n = c2_y(m, ld, u, v, i, j + 1);
+                aW = m.ran[WD2_IX(i - 1, j)], aE = m.ran[p];
+                bW = m.rbn[WD2_IX(i - 1, j)], bE = m.rbn[p];
+                bS = m.rbc[p], bN = m.rbc[WD2_IX(i, j + 1)];
+                gS = m.rgc[p], gN = m.rgc[WD2_IX(i, j + 1)];
             }
-            if (i >= 1 && i <= nx && j >= 1 && j <= ny) {
-                aadd(&vb[WD2_IX(i + 1, j)], 0.5 * m.xzn[p] * g2);
-                aadd(&vb[WD2_IX(i, j)], 0.5 * m.xzn[p] * g2);
-                aadd(&ub[WD2_IX(i, j + 1)], -0.5 * m.yzn[p] * g2);
-                aadd(&ub[WD2_IX(i, j)], -0.5 * m.yzn[p] * g2);
+            add(fb, i, j - 1, (bW - bE + gS) * gd - c2s * gc);
+            add(fb, i - 1, j, (aW - bN + bS) * gd - c1w * gc);
+            add(fb, i, j, -(aE + aW + gN + gS) * gd + (c1e - c1w + c2n - c2s) * gc + (lev ? b : -b));
+            add(fb, i + 1, j, (aE + bN - bS) * gd + c1e * gc);
+            add(fb, i, j + 1, (bE - bW + gN) * gd + c2n * gc);
+            if (bW != 0.0 || bE != 0.0 || bS != 0.0 || bN != 0.0) {   // none on a Cartesian grid
+                add(fb, i - 1, j - 1, (bW + bS) * gd);
+                add(fb, i + 1, j - 1, -(bE + bS) * gd);
+                add(fb, i - 1, j + 1, -(bW + bN) * gd);
+                add(fb, i + 1, j + 1, (bE + bN) * gd);
             }
+            const double f0 = f[p];
+            const int w1 = COMP == 1 ? 0 : 1;   // the west face is c1(i, j) / c1(i-1, j), the south one as well
+            add(c1, i - w1, j, (-f[WD2_IX(i - 1, j)] - f0) * gc);
+            add(c1, i + 1 - w1, j, (f0 + f[WD2_IX(i + 1, j)]) * gc);
+            add(c2, i, j - 1 + w1, (-f[WD2_IX(i, j - 1)] - f0) * gc);
+            add(c2, i, j + w1, (f0 + f[WD2_IX(i, j + 1)]) * gc);
         }
-    } else {
-        // case 5 (i = 1..nx, j = 0..ny): cj1 = yev (4 u)/4 - 2 xev v, cj2 = 2 xzv v - yzv (4 u)/4
-        if (i >= 1 && i <= nx && j <= ny) {
-            const double g1 = gj1, g2 = gj2;
-            aadd(&vsb[p], -2.0 * m.xev[p] * g1 + 2.0 * m.xzv[p] * g2);
-            const double gu = (m.yev[p] * g1 - m.yzv[p] * g2) / 4.0;
-            if (gu != 0.0) {
-                aadd(&usb[WD2_IX(i, j + 1)], gu);
-                aadd(&usb[WD2_IX(i - 1, j + 1)], gu);
-                aadd(&usb[WD2_IX(i, j)], gu);
-                aadd(&usb[WD2_IX(i - 1, j)], gu);
+        __syncthreads();
+        // a face's sum times a metric there (0 where no row of the tile added)
+        auto mv = [&](const double *c, const double *mt, int a, int e) {
+            const double x = c[at(a, e)];
+            return x != 0.0 ? mt[WD2_IX(a, e)] * x : 0.0;
+        };
+        for (int q = tid; q < (GT_W - 2) * (GT_H - 2); q += GT_T) {
+            const int a = oi + 1 + q % (GT_W - 2), e = oj + 1 + q / (GT_W - 2);
+            if (a < 0 || a > nx + 1 || e < 0 || e > ny + 1) continue;
+            double own = fb[at(a, e)], oth;
+            if (COMP == 1) {
+                // case 4: cj1 = 2 yeu u - xeu (4 v) / 4; case 1: c1, c2
+                own += 2.0 * mv(cj, m.yeu, a, e) + 0.5 * (mv(c1, m.yec, a, e) + mv(c1, m.yec, a + 1, e)) -
+                       0.5 * (mv(c2, m.yzn, a, e - 1) + mv(c2, m.yzn, a, e));
+                oth = -0.25 * (mv(cj, m.xeu, a - 1, e) + mv(cj, m.xeu, a, e) + mv(cj, m.xeu, a - 1, e + 1) +
+                               mv(cj, m.xeu, a, e + 1)) -
+                      0.5 * (mv(c1, m.xec, a, e) + mv(c1, m.xec, a, e + 1)) +
+                      0.5 * (mv(c2, m.xzn, a - 1, e) + mv(c2, m.xzn, a, e));
+            } else {
+                // case 5: cj1 = yev (4 u) / 4 - 2 xev v; case 2: c1, c2
+                own += -2.0 * mv(cj, m.xev, a, e) - 0.5 * (mv(c1, m.xen, a - 1, e) + mv(c1, m.xen, a, e)) +
+                       0.5 * (mv(c2, m.xzc, a, e) + mv(c2, m.xzc, a, e + 1));
+                oth = 0.25 * (mv(cj, m.yev, a, e - 1) + mv(cj, m.yev, a + 1, e - 1) + mv(cj, m.yev, a, e) +
+                              mv(cj, m.yev, a + 1, e)) +
+                      0.5 * (mv(c1, m.yen, a, e - 1) + mv(c1, m.yen, a, e)) -
+                      0.5 * (mv(c2, m.yzc, a, e) + mv(c2, m.yzc, a + 1, e));
             }
+            double *ub = lev ? A.unb : A.usb, *vb = lev ? A.vnb : A.vsb;
+            aadd(&(COMP == 1 ? ub : vb)[WD2_IX(a, e)], own);
+            aadd(&(COMP == 1 ? vb : ub)[WD2_IX(a, e)], oth);
         }
-        // case 2: c1 (i = 1..nx, j = 1..ny), c2 (i = 1..nx+1, j = 1..ny+1)
-        for (int lev = 0; lev < 1 + with_n; lev++) {
-            double *ub = lev ? unb : usb, *vb = lev ? vnb : vsb;
-            const double g1 = gc[lev][0], g2 = gc[lev][1];
-            if (i >= 1 && i <= nx && j >= 1 && j <= ny) {
-                aadd(&ub[WD2_IX(i, j + 1)], 0.5 * m.yen[p] * g1);
-                aadd(&ub[WD2_IX(i, j)], 0.5 * m.yen[p] * g1);
-                aadd(&vb[WD2_IX(i + 1, j)], -0.5 * m.xen[p] * g1);
-                aadd(&vb[WD2_IX(i, j)], -0.5 * m.xen[p] * g1);
-            }
-            if (i >= 1 && j >= 1) {
-                aadd(&vb[WD2_IX(i, j)], 0.5 * m.xzc[p] * g2);
-                aadd(&vb[WD2_IX(i, j - 1)], 0.5 * m.xzc[p] * g2);
-                aadd(&ub[WD2_IX(i, j)], -0.5 * m.yzc[p] * g2);
-                aadd(&ub[WD2_IX(i - 1, j)], -0.5 * m.yzc[p] * g2);
-            }
-        }
+        __syncthreads();
     }
+}
+
+// Workgroups [0, t1) take the x-momentum's tiles, the rest the y-momentum's.
+__global__ __launch_bounds__(GT_T, 3) void k_adj_gtrans(GtArgs A, int t1) {
+    __shared__ double fb[GT_W * GT_H], cj[GT_W * GT_H], c1[GT_W * GT_H], c2[GT_W * GT_H];
+    if ((int)blockIdx.x < t1)
+        gt_tile<1>(A, blockIdx.x, fb, cj, c1, c2);
+    else
+        gt_tile<2>(A, (int)blockIdx.x - t1, fb, cj, c1, c2);
 }
 
 // ------------------------------------------------------------ boundary fills
@@ -670,13 +571,10 @@ __global__ __launch_bounds__(AT) void k_adj_maxabs(long n, const double *__restr
 static inline dim3 ag(long n) { return dim3((unsigned)((n + AT - 1) / AT)); }
 
 void launch_adj_tchain(long n, const Chains &cs, const double *A, const double *D, const double *C, double *At,
-                       double *Dt, double *Ct, hipStream_t s) {
-    hipLaunchKernelGGL(k_adj_tchain, ag(n), dim3(AT), 0, s, n, cs, A, D, C, At, Dt, Ct);
-}
-void launch_adj_coef(long n, const Chains &cs, const double *A, const double *D, const double *C, const double *mu,
-                     const double *x, const unsigned char *Z, const unsigned char *XK, double *Ab, double *Db,
-                     double *Cb, hipStream_t s) {
-    hipLaunchKernelGGL(k_adj_coef, ag(n), dim3(AT), 0, s, n, cs, A, D, C, mu, x, Z, XK, Ab, Db, Cb);
+                       double *Dt, double *Ct, unsigned long long *dom, hipStream_t s) {
+    const long nb = std::min<long>(512, (n + AT - 1) / AT);
+    hipLaunchKernelGGL(k_adj_tchain, dim3((unsigned)std::max<long>(nb, 1)), dim3(AT), 0, s, n, cs, A, D, C, At, Dt, Ct,
+                       dom);
 }
 void launch_adj_gather(int nx, int ny, int ld, const double *ub, const double *vb, const unsigned char *Z,
                        double *lam, unsigned long long *red, int slot, hipStream_t s) {
@@ -690,21 +588,15 @@ void launch_adj_update(long n, const double *z, double *nu, unsigned long long *
 void launch_adj_zmask(long n, const unsigned char *Z, const double *in, double *out, hipStream_t s) {
     hipLaunchKernelGGL(k_adj_zmask, ag(n), dim3(AT), 0, s, n, Z, in, out);
 }
-void launch_adj_asm(int comp, int nx, int ny, int ld, double dk, double re, const Metrics &m, const double *us,
-                    const double *vs, const double *un, const double *vn, const double *a1b, const double *d1b,
-                    const double *c1b, const double *bb, int with_n, double *fsb, double *fnb, const AdjCoefs &A,
-                    hipStream_t s) {
-    if (comp == 1)
-        hipLaunchKernelGGL(k_adj_asm_x, ag((long)nx * (ny - 1)), dim3(AT), 0, s, nx, ny, ld, dk, re, m, us, vs, un,
-                           vn, a1b, d1b, c1b, bb, with_n, fsb, fnb, A);
-    else
-        hipLaunchKernelGGL(k_adj_asm_y, ag((long)(nx - 1) * ny), dim3(AT), 0, s, nx, ny, ld, dk, re, m, us, vs, un,
-                           vn, a1b, d1b, c1b, bb, with_n, fsb, fnb, A);
-}
-void launch_adj_cc(int comp, int nx, int ny, int ld, const Metrics &m, const AdjCoefs &A, int with_n, double *usb,
-                   double *vsb, double *unb, double *vnb, hipStream_t s) {
-    hipLaunchKernelGGL(k_adj_cc, ag((long)(nx + 2) * (ny + 2)), dim3(AT), 0, s, comp, nx, ny, ld, m, A, with_n, usb,
-                       vsb, unb, vnb);
+void launch_adj_gtrans(int nx, int ny, int ld, double dk, double re, const Metrics &m, const double *us,
+                       const double *vs, const double *un, const double *vn, const Chain &ch, const Chains &cs,
+                       const double *nu, const unsigned char *XK, int with_n, double *usb, double *vsb, double *unb,
+                       double *vnb, hipStream_t s) {
+    const GtArgs A{nx, ny, ld, with_n, dk, re, m, us, vs, un, vn, AdjChain{ch.a, ch.d, ch.c, nu, ch.x, XK}, cs,
+                   usb, vsb, unb, vnb};
+    auto tiles = [](int ni, int nj) { return ((ni + GT_X - 1) / GT_X) * ((nj + GT_Y - 1) / GT_Y); };
+    const int t1 = tiles(nx, ny - 1), t2 = tiles(nx - 1, ny);
+    hipLaunchKernelGGL(k_adj_gtrans, dim3(t1 + t2), dim3(GT_T), 0, s, A, t1);
 }
 void launch_adj_vbc(const Regions &R, int ld, double *ub, double *vb, double *bcb, hipStream_t s) {
     hipLaunchKernelGGL(k_adj_vbc, dim3(1), dim3(1024), 0, s, R, ld, ub, vb, bcb);

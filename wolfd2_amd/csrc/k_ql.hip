@@ -19,6 +19,8 @@
 // (see the two kernels), the fold sets ql_stop = -1, every kernel queued
 // behind returns at entry, and the host repeats the iteration with the
 // solvers of k_trid.hip.
+#include <cmath>
+
 #include "wd2_trid.hpp"
 
 namespace wd2 {
@@ -163,8 +165,8 @@ static int ql_border_blocks(int nx, int ny, int nt) { return (5 * (nx + ny) + 8 
 
 // ------------------------------------------- bit-exact windows (FP64 path)
 // The speculative segmented Thomas sweep of k_trid.hip on a window: each lane
-// runs its 8 rows from the zero state and the fix-up rounds re-run them from
-// the predecessor's end state until nothing changes, so a window's rows are
+// runs its 8 rows from the zero state and the fix-up rounds (at most `rounds`
+// of them) re-run them from the predecessor's end state until nothing changes, so a window's rows are
 // those of a sequential sweep entered at its first row with the zero state.
 // The recurrences contract, so after H rows that sweep has met the chain's
 // own, bit for bit -- which is checked, not assumed: with the windows
@@ -185,6 +187,7 @@ static int ql_border_blocks(int nx, int ny, int nt) { return (5 * (nx + ny) + 8 
 // |a| + |c| <= 0.76 |d| has (the configurations' chains are below 0.3).
 constexpr int QX_T = 256, QX_HL = 6, QX_H = QX_HL * TR_S, QX_N = QX_T * TR_S, QX_O = QX_N - 4 * QX_H;
 constexpr int QX_CHK = 12;
+constexpr double QX_DOM = 0.45;   // k_adj_window's bound on its rows
 
 template <typename T>
 struct QxShared {
@@ -203,7 +206,8 @@ static_assert(TR_P <= 10, "the increments fit the staging arrays");
 // the rounding-cycle shortcut of k_trid.hip takes over.
 template <typename T>
 __device__ inline void qx_forward(unsigned kinds, const T (&a)[TR_S], const T (&d)[TR_S], const T (&c)[TR_S],
-                                  const T (&b)[TR_S], T dn7, T (&cp)[TR_S], T (&bp)[TR_S], QxShared<T> &S) {
+                                  const T (&b)[TR_S], T dn7, T (&cp)[TR_S], T (&bp)[TR_S], QxShared<T> &S,
+                                  int rounds = QX_T + 1) {
     const int t = threadIdx.x;
     T *sc = S.buf, *sb = S.buf + QX_T, *pr = S.buf + 2 * QX_T;
 #define DNEXT(s) ((s) + 1 < TR_S ? d[((s) + 1) % TR_S] : dn7)
@@ -217,7 +221,7 @@ __device__ inline void qx_forward(unsigned kinds, const T (&a)[TR_S], const T (&
     const bool dep = t > 0 && SKIND(kinds, 0) != 1;
     bool accel = false, cen = false;
     int runlo = -1;
-    for (int round = 0; round <= QX_T; round++) {
+    for (int round = 0; round < rounds; round++) {
         sc[t] = cp[TR_S - 1];
         sb[t] = bp[TR_S - 1];
         if (t == 0) S.changed = 0;
@@ -286,7 +290,7 @@ __device__ inline void qx_forward(unsigned kinds, const T (&a)[TR_S], const T (&
 // Back-substitution, with the zero value after the workgroup's last row.
 template <typename T>
 __device__ inline void qx_backward(unsigned kinds, const T (&cp)[TR_S], const T (&bp)[TR_S], T (&x)[TR_S],
-                                   QxShared<T> &S) {
+                                   QxShared<T> &S, int rounds = QX_T + 1) {
     const int t = threadIdx.x;
     T *sc = S.buf, *pr = S.buf + 2 * QX_T;
     T xn = T(0);
@@ -298,7 +302,7 @@ __device__ inline void qx_backward(unsigned kinds, const T (&cp)[TR_S], const T 
     const bool dep = t + 1 < QX_T && SKIND(kinds, TR_S - 1) != 2;
     bool accel = false, cev = false;
     int runhi = -1;
-    for (int round = 0; round <= QX_T; round++) {
+    for (int round = 0; round < rounds; round++) {
         sc[t] = x[0];
         if (t == 0) S.changed = 0;
         if (accel) {
@@ -406,6 +410,85 @@ __global__ __launch_bounds__(QX_T, 3) void k_ql_exact(long n, Chains cs, ChainT<
     for (int s = 0; s < TR_S; s++) X[t * TR_P + s] = b[s];
     __syncthreads();
     ql_update<QX_T, T>(F, X, w0, 2 * QX_H, QX_N - 2 * QX_H, n, cs.n1, part, S.red);
+}
+
+// The adjoint's preconditioner on the same windows (one fixed-point iteration
+// of the q-l loop's transpose): A2 y = r, y = 0 on identity rows, A1 z = y,
+// nu += z, with part[2 window ..] = max |z|, max |nu| of the kept rows (a NaN
+// wins).  The caller has bounded (|a| + |c|) / |d| of every row of both
+// systems by QX_DOM, so what H rows leave of the entry state is below
+// QX_DOM^48 = 2e-17 of it, and nothing has to be compared; nor have the fix-up
+// rounds to go on after the `rounds` of 8 rows that leave as little (as the
+// update vanishes, the last bits of its decaying tails take many more).  On 512^2 cells the
+// two solves, the mask and the update in launches of their own took 150 us an
+// iteration (the update alone 27, its maxima on two addresses); here 27.
+__global__ __launch_bounds__(QX_T, 3) void k_adj_window(long n, Chains cs, Chain h2, Chain h1,
+                                                      const double *__restrict__ r,
+                                                      const unsigned char *__restrict__ Z, double *__restrict__ nu,
+                                                      double *__restrict__ part, int rounds) {
+    __shared__ QxShared<double> S;
+    const int t = threadIdx.x;
+    const long w0 = (long)blockIdx.x * QX_O - 2 * QX_H, k0 = w0 + (long)t * TR_S;
+    double a[TR_S], d[TR_S], c[TR_S], b[TR_S], cp[TR_S], bp[TR_S];
+    ql_load(h2.a, k0, n, 0.0, a);
+    ql_load(h2.d, k0, n, 1.0, d);
+    ql_load(h2.c, k0, n, 0.0, c);
+    ql_load(r, k0, n, 0.0, b);
+    const unsigned kinds = ql_kinds(k0, n, cs);
+    const unsigned idm = ql_ident(Z, k0, n);
+    const bool s7 = SKIND(kinds, TR_S - 1) == 1;   // a chain starts on the lane's last row
+    qx_forward<double>(kinds, a, d, c, b, s7 ? h2.d[k0 + TR_S] : 1.0, cp, bp, S, rounds);
+    const bool in2 = t >= QX_HL && t < QX_T - QX_HL;
+    const long k2 = in2 ? k0 : n;
+    ql_load(h1.a, k2, n, 0.0, a);
+    ql_load(h1.d, k2, n, 1.0, d);
+    ql_load(h1.c, k2, n, 0.0, c);
+    qx_backward<double>(kinds, cp, bp, b, S, rounds);
+#pragma unroll
+    for (int s = 0; s < TR_S; s++)
+        if (!in2 || ((idm >> s) & 1u)) b[s] = 0.0;
+    const unsigned kinds2 = in2 ? kinds : 0u;
+    qx_forward<double>(kinds2, a, d, c, b, in2 && s7 ? h1.d[k0 + TR_S] : 1.0, cp, bp, S, rounds);
+    qx_backward<double>(kinds2, cp, bp, b, S, rounds);
+    double *X = S.buf;
+#pragma unroll
+    for (int s = 0; s < TR_S; s++) X[t * TR_P + s] = b[s];
+    __syncthreads();
+    double m1 = 0.0, m2 = 0.0;
+    for (int l = 2 * QX_H + t; l < QX_N - 2 * QX_H; l += QX_T) {
+        const long k = w0 + l;
+        if (k < 0 || k >= n) continue;
+        const double z = X[(l >> 3) * TR_P + (l & 7)], v = nu[k] + z;
+        nu[k] = v;
+        if (!(fabs(z) <= m1)) m1 = fabs(z);
+        if (!(fabs(v) <= m2)) m2 = fabs(v);
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        const double q1 = __shfl_xor(m1, off), q2 = __shfl_xor(m2, off);
+        if (!(q1 <= m1)) m1 = q1;
+        if (!(q2 <= m2)) m2 = q2;
+    }
+    if ((t & 63) == 0) {
+        S.red[2 * (t >> 6)] = m1;
+        S.red[2 * (t >> 6) + 1] = m2;
+    }
+    __syncthreads();
+    if (t < 2) {
+        double m = S.red[t];
+        for (int w = 1; w < QX_T / 64; w++)
+            if (!(S.red[2 * w + t] <= m)) m = S.red[2 * w + t];
+        part[2 * blockIdx.x + t] = m;
+    }
+}
+
+double adj_window_dominance() { return QX_DOM; }
+int adj_windows(long n) { return (int)((n + QX_O - 1) / QX_O); }
+void launch_adj_window(long n, const Chains &cs, const Chain &h2, const Chain &h1, const double *r,
+                       const unsigned char *Z, double *nu, double *part, double dom, hipStream_t s) {
+    // rounds of TR_S rows until dom^rows is below 1e-17, at least two
+    int rounds = 2;
+    for (double e = std::pow(dom, 2 * TR_S); e > 1e-17; e *= std::pow(dom, TR_S)) rounds++;
+    hipLaunchKernelGGL(k_adj_window, dim3(adj_windows(n)), dim3(QX_T), 0, s, n, cs, h2, h1, r, Z, nu, part, rounds);
 }
 
 // ------------------------------------------------ FP32 windows (mixed path)

@@ -1629,15 +1629,14 @@ struct wd2_adj {
     double *fin = nullptr;    // (u, v, p) after the run
     // adjoint fields: the state's (ub, vb, pb); scratch tu, tv (w.r.t. us,
     // vs), nub, nvb (w.r.t. un, vn); the Poisson adjoint lam (zero ghosts)
-    // and its right-hand side; the ConvCoef adjoints co (6 fields)
+    // and its right-hand side
     double *fstore = nullptr;
     double *ub, *vb, *pb, *tu, *tv, *nub, *nvb, *lam, *arhs;
-    AdjCoefs co{};
     double *bcb = nullptr;    // 8 x W boundary-value adjoints
     int W = 0;
-    // chain vectors: S1^T and S2^T (A, D, C), nu, r, y, z, coefficient adjoints
+    // chain vectors: S1^T and S2^T (A, D, C), nu, r, y, z
     double *cstore = nullptr;
-    double *At1, *Dt1, *Ct1, *At2, *Dt2, *Ct2, *nu, *r, *y, *z, *a1b, *d1b, *c1b;
+    double *At1, *Dt1, *Ct1, *At2, *Dt2, *Ct2, *nu, *r, *y, *z;
     // tangent-linear pass (wd2_adj_tangent): dual fields us, vs, un, vn, the
     // dual time-level-n terms of both components, the dual chains of both
     // splits; the tangent boundary values (a Regions with zero constants and
@@ -1649,7 +1648,8 @@ struct wd2_adj {
     int *tl_poff = nullptr;
     // maxima of the adjoint q-l updates (two slots per iteration parity) and
     // their pinned copies; qev: the events after each parity's copy
-    unsigned long long *red = nullptr, *h_red = nullptr;
+    unsigned long long *red = nullptr, *h_red = nullptr;   // two iterations' maxima, the chains' dominance
+    double *part = nullptr, *h_part = nullptr;             // two iterations' maxima by window
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     hipEvent_t qev[2] = {nullptr, nullptr};
     wd2_adj_stats st{};
@@ -1668,7 +1668,9 @@ static void adj_free(wd2_adj *a) {
     (void)hipFree(a->tl_pval);
     (void)hipFree(a->tl_poff);
     (void)hipFree(a->red);
+    (void)hipFree(a->part);
     if (a->h_red) (void)hipHostFree(a->h_red);
+    if (a->h_part) (void)hipHostFree(a->h_part);
     for (hipEvent_t e : a->ev)
         if (e) (void)hipEventDestroy(e);
     for (hipEvent_t e : a->qev)
@@ -1700,21 +1702,23 @@ static int adj_alloc(wd2_adj *a) {
     const size_t nf = c->nf, nch = chain_rows(c->nx, c->ny);
     HIPCHK(hipMalloc(&a->tape, 5 * (size_t)a->every * nf * sizeof(double)));
     HIPCHK(hipMalloc(&a->fin, 3 * nf * sizeof(double)));
-    HIPCHK(hipMalloc(&a->fstore, 15 * nf * sizeof(double)));
-    HIPCHK(hipMemsetAsync(a->fstore, 0, 15 * nf * sizeof(double), c->s));
+    HIPCHK(hipMalloc(&a->fstore, 9 * nf * sizeof(double)));
+    HIPCHK(hipMemsetAsync(a->fstore, 0, 9 * nf * sizeof(double), c->s));
     double *f = a->fstore;
     double **fp[9] = {&a->ub, &a->vb, &a->pb, &a->tu, &a->tv, &a->nub, &a->nvb, &a->lam, &a->arhs};
     for (int k = 0; k < 9; k++) *fp[k] = f + k * nf;
-    a->co = AdjCoefs{f + 9 * nf, f + 10 * nf, f + 11 * nf, f + 12 * nf, f + 13 * nf, f + 14 * nf};
     a->W = std::max(c->nx, c->ny) + 2;
     HIPCHK(hipMalloc(&a->bcb, 8 * (size_t)a->W * sizeof(double)));
-    HIPCHK(hipMalloc(&a->cstore, 13 * nch * sizeof(double)));
-    HIPCHK(hipMemsetAsync(a->cstore, 0, 13 * nch * sizeof(double), c->s));
-    double **cp[13] = {&a->At1, &a->Dt1, &a->Ct1, &a->At2, &a->Dt2, &a->Ct2, &a->nu,
-                       &a->r,   &a->y,   &a->z,   &a->a1b, &a->d1b, &a->c1b};
-    for (int k = 0; k < 13; k++) *cp[k] = a->cstore + k * nch;
-    HIPCHK(hipMalloc(&a->red, 4 * sizeof(unsigned long long)));
-    HIPCHK(hipHostMalloc((void **)&a->h_red, 4 * sizeof(unsigned long long), hipHostMallocDefault));
+    HIPCHK(hipMalloc(&a->cstore, 10 * nch * sizeof(double)));
+    HIPCHK(hipMemsetAsync(a->cstore, 0, 10 * nch * sizeof(double), c->s));
+    double **cp[10] = {&a->At1, &a->Dt1, &a->Ct1, &a->At2, &a->Dt2, &a->Ct2, &a->nu,
+                       &a->r,   &a->y,   &a->z};
+    for (int k = 0; k < 10; k++) *cp[k] = a->cstore + k * nch;
+    HIPCHK(hipMalloc(&a->red, 5 * sizeof(unsigned long long)));
+    HIPCHK(hipHostMalloc((void **)&a->h_red, 5 * sizeof(unsigned long long), hipHostMallocDefault));
+    const size_t npart = 4 * (size_t)adj_windows((long)c->nx * (c->ny - 1) + (long)(c->nx - 1) * c->ny);
+    HIPCHK(hipMalloc(&a->part, npart * sizeof(double)));
+    HIPCHK(hipHostMalloc((void **)&a->h_part, npart * sizeof(double), hipHostMallocDefault));
     for (auto &e : a->ev) HIPCHK(hipEventCreate(&e));
     for (auto &e : a->qev) HIPCHK(hipEventCreate(&e));
     return WD2_OK;
@@ -1747,17 +1751,10 @@ static void adj_gtrans(wd2_adj *a, const double *us, const double *vs, const dou
     wd2_ctx *c = a->c;
     const int nx = c->nx, ny = c->ny, ld = c->ld;
     hipStream_t s = c->s;
-    const long n1 = (long)nx * (ny - 1), n2 = (long)(nx - 1) * ny, n = n1 + n2;
+    const long n1 = (long)nx * (ny - 1), n2 = (long)(nx - 1) * ny;
     const Chains cs{n1, n1, n2};
-    launch_adj_coef(n, cs, c->ch.a, c->ch.d, c->ch.c, a->nu, c->ch.x, nullptr, c->zm, a->a1b, a->d1b, a->c1b, s);
-    for (int comp = 1; comp <= 2; comp++) {
-        const long off = comp == 1 ? 0 : n1;
-        // co is all zero here: k_adj_cc clears what it reads
-        launch_adj_asm(comp, nx, ny, ld, a->P.dk, a->P.re, c->M, us, vs, un, vn, a->a1b + off, a->d1b + off,
-                       a->c1b + off, a->nu + off, with_n, comp == 1 ? a->tu : a->tv, comp == 1 ? a->nub : a->nvb,
-                       a->co, s);
-        launch_adj_cc(comp, nx, ny, ld, c->M, a->co, with_n, a->tu, a->tv, a->nub, a->nvb, s);
-    }
+    launch_adj_gtrans(nx, ny, ld, a->P.dk, a->P.re, c->M, us, vs, un, vn, c->ch, cs, a->nu, c->zm, with_n, a->tu,
+                      a->tv, a->nub, a->nvb, s);
 }
 
 // One step backwards: (ub, vb, pb) from the adjoint of the step's end state
@@ -1816,18 +1813,34 @@ static int adj_step(wd2_adj *a, const double *un, const double *vn, const double
     launch_mom_asm_pair<double>(c->R, ld, P.dk, P.re, P.fr, c->M, t, t2, us, vs, un, vn, c->d, c->dn, c->ch, c->ch2,
                                 c->zm, shift(c->ch, n1), shift(c->ch2, n1), c->zm + n1, s, &c->sc->err, 0);
     launch_trid<double>(c->tw, n, cs, c->ch.a, c->ch.d, c->ch.c, c->ch.b, c->ch.x, s);
-    launch_adj_tchain(n, cs, c->ch.a, c->ch.d, c->ch.c, a->At1, a->Dt1, a->Ct1, s);
-    launch_adj_tchain(n, cs, c->ch2.a, c->ch2.d, c->ch2.c, a->At2, a->Dt2, a->Ct2, s);
+    launch_adj_zero(1, (double *)&a->red[4], s);
+    launch_adj_tchain(n, cs, c->ch.a, c->ch.d, c->ch.c, a->At1, a->Dt1, a->Ct1, &a->red[4], s);
+    launch_adj_tchain(n, cs, c->ch2.a, c->ch2.d, c->ch2.c, a->At2, a->Dt2, a->Ct2, &a->red[4], s);
+    HIPCHK(hipMemcpyAsync(&a->h_red[4], &a->red[4], sizeof(unsigned long long), hipMemcpyDeviceToHost, s));
     launch_adj_zero(n, a->nu, s);
     const double *fsrc[2] = {a->ub, a->vb};
     double *fdst[2] = {a->tu, a->tv};
     // Pipelined by one iteration, as the forward q-l loop: iteration m is
     // queued before the host reads iteration m-1's maxima; the extra
     // iteration after the test is met only refines nu.
+    HIPCHK(hipStreamSynchronize(s));
+    double dom;
+    std::memcpy(&dom, &a->h_red[4], sizeof(double));
+    const bool win = dom <= adj_window_dominance();   // false for a NaN
+    const int nwin = adj_windows(n);
+    const Chain t1{a->At1, a->Dt1, a->Ct1, nullptr, nullptr}, t2c{a->At2, a->Dt2, a->Ct2, nullptr, nullptr};
     auto converged = [&](int m) {
-        double zmax, numax;
-        std::memcpy(&zmax, &a->h_red[2 * (m % 2)], sizeof(double));
-        std::memcpy(&numax, &a->h_red[2 * (m % 2) + 1], sizeof(double));
+        double zmax = 0.0, numax = 0.0;
+        if (win) {
+            const double *q = a->h_part + (m % 2) * 2 * (size_t)nwin;
+            for (int w = 0; w < nwin; w++) {   // a NaN wins
+                if (!(q[2 * w] <= zmax)) zmax = q[2 * w];
+                if (!(q[2 * w + 1] <= numax)) numax = q[2 * w + 1];
+            }
+        } else {
+            std::memcpy(&zmax, &a->h_red[2 * (m % 2)], sizeof(double));
+            std::memcpy(&numax, &a->h_red[2 * (m % 2) + 1], sizeof(double));
+        }
         return zmax <= a->fp_tol * numax;
     };
     int m = 1;
@@ -1837,12 +1850,18 @@ static int adj_step(wd2_adj *a, const double *un, const double *vn, const double
         launch_copy_set(ld, 0, nx + 1, 0, ny + 1, fsrc, fdst, 2, s);
         if (m > 1) adj_gtrans(a, us, vs, un, vn, 0);
         launch_adj_gather(nx, ny, ld, a->tu, a->tv, c->zm, a->r, a->red, sl, s);
-        launch_trid<double>(c->tw, n, cs, a->At2, a->Dt2, a->Ct2, a->r, a->y, s);
-        launch_adj_zmask(n, c->zm, a->y, a->y, s);
-        launch_trid<double>(c->tw, n, cs, a->At1, a->Dt1, a->Ct1, a->y, a->z, s);
-        launch_adj_update(n, a->z, a->nu, a->red, sl, s);
-        HIPCHK(hipMemcpyAsync(&a->h_red[sl], &a->red[sl], 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                              s));
+        if (win) {
+            double *part = a->part + sl * (size_t)nwin, *h_part = a->h_part + sl * (size_t)nwin;
+            launch_adj_window(n, cs, t2c, t1, a->r, c->zm, a->nu, part, dom, s);
+            HIPCHK(hipMemcpyAsync(h_part, part, 2 * (size_t)nwin * sizeof(double), hipMemcpyDeviceToHost, s));
+        } else {
+            launch_trid<double>(c->tw, n, cs, a->At2, a->Dt2, a->Ct2, a->r, a->y, s);
+            launch_adj_zmask(n, c->zm, a->y, a->y, s);
+            launch_trid<double>(c->tw, n, cs, a->At1, a->Dt1, a->Ct1, a->y, a->z, s);
+            launch_adj_update(n, a->z, a->nu, a->red, sl, s);
+            HIPCHK(hipMemcpyAsync(&a->h_red[sl], &a->red[sl], 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
+                                  s));
+        }
         HIPCHK(hipEventRecord(a->qev[m % 2], s));
         if (m >= 2) {
             HIPCHK(hipEventSynchronize(a->qev[(m - 1) % 2]));
