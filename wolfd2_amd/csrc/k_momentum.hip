@@ -68,21 +68,45 @@ struct LAcc {
     __device__ T operator()(int i, int j) const { return s[(j - j0) * w + (i - i0)]; }
 };
 // A metric array read only at points inside its constant box (MBox): every
-// read is the box's value, with no test and no load.  mpick<MK_CONST> gives
-// one, mpick<MK_BOX> the array with its box (a load outside the box).
+// read is the box's value, with no test and no load (mpick<MK_CONST>).
 struct MConst {
     double c;
 };
 __device__ inline double mget(const MConst &a, int, int, int) { return a.c; }
-enum { MK_BOX = 0, MK_CONST = 1 };
-template <int MK>
-__device__ inline std::conditional_t<MK == MK_CONST, MConst, MArr> mpick(const double *p, const MBox &b) {
-    if constexpr (MK == MK_CONST)
-        return MConst{b.c};
-    else
-        return MArr{p, b};
+// A metric array on a range of points (mpick<MK_RANGE>): where the range lies
+// in the constant box every read goes to the box's first element, one address
+// that stays in the caches, else to the point's.  Which one is decided once
+// for the range, so the reads have no branch and their loads can all be in
+// flight at once.
+// Offsets are from the range's first point, so that 32 bits hold them and the
+// arrays' addresses stay in scalar registers.
+struct MRange {
+    const char *p;
+    unsigned keep;   // mask of a read's offset: all or nothing
+    int i0, j0;
+};
+__device__ inline double mget(const MRange &a, int ld, int i, int j) {
+    const unsigned off = 8u * ((unsigned)(i - a.i0) + (unsigned)ld * (unsigned)(j - a.j0));
+    return *reinterpret_cast<const double *>(a.p + (size_t)(off & a.keep));
 }
-#define MPICK(m, f) mpick<MK>((m).f, (m).box[MI_##f])
+// Rows i0..i1 x j0..j1 of one component (empty when i0 > i1 or j0 > j1).
+struct AsmRect {
+    int i0, i1, j0, j1;
+};
+enum { MK_RANGE = 0, MK_CONST = 1 };
+// g: the points the reads cover
+template <int MK>
+__device__ inline std::conditional_t<MK == MK_CONST, MConst, MRange> mpick(const double *p, const MBox &b,
+                                                                         const AsmRect &g, int ld) {
+    if constexpr (MK == MK_CONST) {
+        return MConst{b.c};
+    } else {
+        const bool in = g.i0 >= b.i0 && g.i1 <= b.i1 && g.j0 >= b.j0 && g.j1 <= b.j1;
+        const double *q = p + (in ? WD2_IX(b.i0, b.j0) : WD2_IX(g.i0, g.j0));
+        return MRange{reinterpret_cast<const char *>(q), in ? 0u : ~0u, g.i0, g.j0};
+    }
+}
+#define MPICK(m, f) mpick<MK>((m).f, (m).box[MI_##f], grect, ld)
 
 // The centred face coefficients of ConvCoef cases 1 (cc_x1, cc_x2) and 2
 // (cc_y1, cc_y2) at one point (momentum.f:901-925), shared by k_conv_coef and
@@ -624,18 +648,22 @@ template void launch_assemble<float>(const Regions &, int, int, int, double, dou
 // Every value is the same expression as in k_conv_coef / k_conv_diff /
 // k_assemble, so the chains are bit for bit those of the separate kernels.
 //
-// Two kernels share the rows.  A row whose metric reads (i-1..i+1,
-// j-1..j+1) all lie inside their arrays' constant boxes takes the box values
-// as constants -- the same values, with no per-read box test and no load --
-// in k_mom_asm_cb; on a uniform grid that is every row but those next to the
-// ghost points.  Those rows form a rectangle per component (found on the host
-// from the boxes); k_mom_asm_gen takes the rest, up to four strips around it
-// per component, or every row where no metric is constant.  k_mom_asm_cb
-// first copies the us and vs values its rows' stencils read into LDS tiles
-// as T (x-momentum: us on i-1..i+1, j-1..j+1 and vs on i-1..i+2, j-2..j+1
-// around each row point; y-momentum the mirror image), one coalesced load per
-// element in place of about 25 dependent loads per row.  Both kernels serve
-// both components in one launch.
+// A workgroup takes a tile of MX x MY rows of one component.  It first copies
+// the us and vs values its rows' stencils read into LDS as T (x-momentum: us
+// on i-1..i+1, j-1..j+1 and vs on i-1..i+2, j-2..j+1 around each row point;
+// y-momentum the mirror image), one coalesced load per element in place of
+// about 25 dependent loads per row.  Where the metric reads of the tile's rows
+// (i-1..i+1, j-1..j+1) all lie inside their arrays' constant boxes -- on a
+// uniform grid with exact spacings every tile but the outermost -- the metrics
+// are constants (MK_CONST, bound by the chains it writes: 5.7 TB/s on 1024^2
+// cells in FP32).  The other tiles, all of them on most grids, go to a launch
+// of their own (MK_RANGE, which needs half again as many registers): each
+// array is read by point or, where its own box covers the tile (the cross
+// metrics of a Cartesian grid), at one address.  A lane a row, reading fields
+// and boxed metrics (a branch each) from memory, that launch took 13 us for
+// the 1024^2 cavity's strips, 14 for 392 x 256 stretched cells in FP64 and 57
+// for 768^2 in FP32; here 10, 12 and 46.  Both kinds of tile in one launch
+// took 34 us on the 1024^2 cavity (FP32) where the two take 21 and 10.
 
 // One component's outputs: the time-level-n terms it reads, its two chains
 // and its identity-row flags.
@@ -647,12 +675,14 @@ struct AsmOut {
 };
 
 // One chain row: the fused assembly of the row at (i, j), with the us, vs
-// stencils read through U, V and the metrics through mpick<MK>.
+// stencils read through U, V and the metrics through mpick<MK> (grect: the
+// points those reads cover).
 template <int COMP, int MK, typename T, typename E, typename AU, typename AV>
 __device__ inline void mom_asm_row(const Regions &R, int ld, int i, int j, T dk, T dk2, T re1, T fr, const Metrics &m,
                                    const AsmOut<T> &o, const AU &U, const AV &V, const E *__restrict__ us,
                                    const E *__restrict__ vs, const E *__restrict__ un, const E *__restrict__ vn,
-                                   const double *__restrict__ d, const double *__restrict__ dn, int *err, int live) {
+                                   const double *__restrict__ d, const double *__restrict__ dn, int *err, int live,
+                                   const AsmRect &grect) {
     const int nx = R.nx, ny = R.ny;
     const long k = COMP == 1 ? (long)(j - 2) * nx + (i - 1) : (long)(j - 1) * (nx - 1) + (i - 2);
     const T dZero = T(0.0), dOne = T(1.0), dFour = T(4.0);
@@ -713,34 +743,28 @@ __device__ inline void mom_asm_row(const Regions &R, int ld, int i, int j, T dk,
 #undef MM
 }
 
-// Rows i0..i1 x j0..j1 of one component (empty when i0 > i1 or j0 > j1).
-struct AsmRect {
-    int i0, i1, j0, j1;
+// One component's rows (r: i0..i1 x j0..j1) as gx x gy tiles of MX x MY, of
+// which tx0 .. tx0 + ntx - 1 x ty0 .. ty0 + nty - 1 have constant metrics.
+struct AsmTiles {
+    AsmRect r;
+    int gx, gy, tx0, ntx, ty0, nty;
 };
-__host__ __device__ inline int rect_tiles(const AsmRect &r) {
-    return (r.i0 > r.i1 || r.j0 > r.j1) ? 0 : ((r.i1 - r.i0 + MX) / MX) * ((r.j1 - r.j0 + MY) / MY);
-}
 
-// The constant-box rows of one component: its LDS-tiled workgroup, after the
-// us, vs tiles are staged, runs the constant-metric body on its rows inside
-// the rectangle r.  The tiles of r are ordered for the XCDs as xtile does.
-template <int COMP, typename T, typename E>
-__device__ inline void mom_asm_cb_tile(int b, int nb, const AsmRect &r, const Regions &R, int ld, double dk_,
-                                       double dk2_, double re1_, double fr_, const Metrics &m, const AsmOut<T> &o,
-                                       const E *__restrict__ us, const E *__restrict__ vs,
-                                       const E *__restrict__ un, const E *__restrict__ vn,
-                                       const double *__restrict__ d, const double *__restrict__ dn, int *err, int live,
-                                       unsigned char *tu_raw, unsigned char *tv_raw) {
+// Tile (tx, ty) of one component, its us and vs values staged in LDS.
+template <int COMP, int MK, typename T, typename E>
+__device__ inline void mom_asm_tile(int tx, int ty, const AsmRect &r, const Regions &R, int ld, double dk_,
+                                    double dk2_, double re1_, double fr_, const Metrics &m, const AsmOut<T> &o,
+                                    const E *__restrict__ us, const E *__restrict__ vs, const E *__restrict__ un,
+                                    const E *__restrict__ vn, const double *__restrict__ d,
+                                    const double *__restrict__ dn, int *err, int live, unsigned char *tu_raw,
+                                    unsigned char *tv_raw) {
     const int nx = R.nx, ny = R.ny;
-    const int gx = (r.i1 - r.i0 + MX) / MX, nt = gx * ((r.j1 - r.j0 + MY) / MY), per = nb / 8;
-    const int tile = (b % 8) * per + b / 8;
-    if (tile >= nt) return;
     constexpr int NT = MX * MY;
     constexpr int WU = COMP == 1 ? MX + 2 : MX + 3, HU = COMP == 1 ? MY + 2 : MY + 3;
     constexpr int WV = COMP == 1 ? MX + 3 : MX + 2, HV = COMP == 1 ? MY + 3 : MY + 2;
     T *tu = reinterpret_cast<T *>(tu_raw), *tv = reinterpret_cast<T *>(tv_raw);
     // the tile's first row point (I0, J0) and the us, vs tiles around its rows
-    const int I0 = r.i0 + (tile % gx) * MX, J0 = r.j0 + (tile / gx) * MY;
+    const int I0 = r.i0 + tx * MX, J0 = r.j0 + ty * MY;
     const int ui0 = COMP == 1 ? I0 - 1 : I0 - 2, uj0 = J0 - 1;
     const int vi0 = I0 - 1, vj0 = COMP == 1 ? J0 - 2 : J0 - 1;
     {
@@ -775,78 +799,70 @@ __device__ inline void mom_asm_cb_tile(int b, int nb, const AsmRect &r, const Re
     const int i = I0 + threadIdx.x, j = J0 + threadIdx.y;
     if (i > r.i1 || j > r.j1) return;
     const LAcc<T> U{tu, ui0, uj0, WU}, V{tv, vi0, vj0, WV};
-    mom_asm_row<COMP, MK_CONST, T, E>(R, ld, i, j, cv<T>(dk_), cv<T>(dk2_), cv<T>(re1_), cv<T>(fr_), m, o, U, V, us, vs,
-                                  un, vn, d, dn, err, live);
+    const AsmRect g{I0 - 1, min(I0 + MX, r.i1 + 1), J0 - 1, min(J0 + MY, r.j1 + 1)};
+    mom_asm_row<COMP, MK, T, E>(R, ld, i, j, cv<T>(dk_), cv<T>(dk2_), cv<T>(re1_), cv<T>(fr_), m, o, U, V, us, vs, un,
+                                vn, d, dn, err, live, g);
 }
 
-// Workgroups [0, g1) take the x-momentum rectangle r1, the rest the
-// y-momentum rectangle r2 (g1 and the total are multiples of 8, so each part
-// keeps the XCD order).
-template <typename T, typename E>
-__global__ __launch_bounds__(MX *MY) void k_mom_asm_cb(Regions R, int ld, double dk_, double dk2_, double re1_,
-                                                       double fr_, Metrics m, AsmOut<T> o1, AsmOut<T> o2,
-                                                       const E *__restrict__ us, const E *__restrict__ vs,
-                                                       const E *__restrict__ un, const E *__restrict__ vn,
-                                                       const double *__restrict__ d, const double *__restrict__ dn,
-                                                       int *err, int live, const int *stop, AsmRect r1, AsmRect r2,
-                                                       int g1) {
+// Workgroups [0, g1) take x-momentum tiles, the rest y-momentum ones: with
+// MK_CONST those with constant metrics, with MK_RANGE the others (whole tile
+// rows below and above them, then what is left and right).  g1 and the total
+// are multiples of 8; the tiles are ordered for the XCDs as xtile does.
+template <int MK, typename T, typename E>
+__global__ __launch_bounds__(MX *MY) void k_mom_asm(Regions R, int ld, double dk_, double dk2_, double re1_,
+                                                    double fr_, Metrics m, AsmOut<T> o1, AsmOut<T> o2,
+                                                    const E *__restrict__ us, const E *__restrict__ vs,
+                                                    const E *__restrict__ un, const E *__restrict__ vn,
+                                                    const double *__restrict__ d, const double *__restrict__ dn,
+                                                    int *err, int live, const int *stop, AsmTiles w1, AsmTiles w2,
+                                                    int g1) {
     if (stop && *stop) return;
     // raw storage: T may be a type with a constructor (the tangent's Dual)
     constexpr int NU = (MX + 3) * (MY + 3) > (MX + 2) * (MY + 2) ? (MX + 3) * (MY + 3) : (MX + 2) * (MY + 2);
     __shared__ __align__(16) unsigned char tu_raw[NU * sizeof(T)], tv_raw[NU * sizeof(T)];
-    const int b = (int)blockIdx.x;
-    if (b < g1)
-        mom_asm_cb_tile<1, T, E>(b, g1, r1, R, ld, dk_, dk2_, re1_, fr_, m, o1, us, vs, un, vn, d, dn, err, live,
-                                 tu_raw, tv_raw);
+    const bool c1 = (int)blockIdx.x < g1;
+    const AsmTiles w = c1 ? w1 : w2;
+    const int b = c1 ? (int)blockIdx.x : (int)blockIdx.x - g1, nb = c1 ? g1 : (int)gridDim.x - g1;
+    int q = (b % 8) * (nb / 8) + b / 8, tx, ty;
+    if (MK == MK_CONST) {
+        if (q >= w.ntx * w.nty) return;
+        tx = w.tx0 + q % w.ntx;
+        ty = w.ty0 + q / w.ntx;
+    } else {
+        if (q >= w.gx * w.gy - w.ntx * w.nty) return;
+        const int na = w.gx * (w.gy - w.nty);
+        if (q < na) {
+            tx = q % w.gx;
+            ty = q / w.gx;
+            if (ty >= w.ty0) ty += w.nty;
+        } else {
+            q -= na;
+            const int nc = w.gx - w.ntx;
+            tx = q % nc;
+            ty = w.ty0 + q / nc;
+            if (tx >= w.tx0) tx += w.ntx;
+        }
+    }
+    if (c1)
+        mom_asm_tile<1, MK, T, E>(tx, ty, w.r, R, ld, dk_, dk2_, re1_, fr_, m, o1, us, vs, un, vn, d, dn, err, live,
+                                  tu_raw, tv_raw);
     else
-        mom_asm_cb_tile<2, T, E>(b - g1, (int)gridDim.x - g1, r2, R, ld, dk_, dk2_, re1_, fr_, m, o2, us, vs, un, vn, d,
-                                 dn, err, live, tu_raw, tv_raw);
+        mom_asm_tile<2, MK, T, E>(tx, ty, w.r, R, ld, dk_, dk2_, re1_, fr_, m, o2, us, vs, un, vn, d, dn, err, live,
+                                  tu_raw, tv_raw);
 }
 
-// The other rows: up to eight rectangles (at most four per component), one
-// thread per row, reading us, vs and the metrics (through their boxes) from
-// memory.
-struct AsmGen {
-    int n;
-    int comp[8];
-    AsmRect r[8];
-    long start[9];   // first row of each rectangle in the launch; start[n] = the total
-};
-constexpr int AG_T = 256;
-template <typename T, typename E>
-__global__ __launch_bounds__(AG_T) void k_mom_asm_gen(Regions R, int ld, double dk_, double dk2_, double re1_,
-                                                      double fr_, Metrics m, AsmOut<T> o1, AsmOut<T> o2,
-                                                      const E *__restrict__ us, const E *__restrict__ vs,
-                                                      const E *__restrict__ un, const E *__restrict__ vn,
-                                                      const double *__restrict__ d, const double *__restrict__ dn,
-                                                      int *err, int live, const int *stop, AsmGen g) {
-    if (stop && *stop) return;
-    const long q = (long)blockIdx.x * AG_T + threadIdx.x;
-    if (q >= g.start[g.n]) return;
-    int s = 0;
-    while (q >= g.start[s + 1]) s++;
-    const AsmRect &r = g.r[s];
-    const int w = r.i1 - r.i0 + 1;
-    const int i = r.i0 + (int)((q - g.start[s]) % w), j = r.j0 + (int)((q - g.start[s]) / w);
-    const T dk = cv<T>(dk_), dk2 = cv<T>(dk2_), re1 = cv<T>(re1_), fr = cv<T>(fr_);
-    const GAcc<T, E> U{us, ld}, V{vs, ld};
-    if (g.comp[s] == 1)
-        mom_asm_row<1, MK_BOX, T, E>(R, ld, i, j, dk, dk2, re1, fr, m, o1, U, V, us, vs, un, vn, d, dn, err, live);
-    else
-        mom_asm_row<2, MK_BOX, T, E>(R, ld, i, j, dk, dk2, re1, fr, m, o2, U, V, us, vs, un, vn, d, dn, err, live);
-}
-
-// The constant-box rectangle of component comp's rows (x-momentum: i =
-// 1..nx, j = 2..ny; y-momentum: i = 2..nx, j = 1..ny): the rows whose metric
-// reads i-1..i+1, j-1..j+1 lie inside the boxes of every metric the
-// component reads.  The rest of the rows, as up to four strips, go to *g.
-static AsmRect asm_rects(int nx, int ny, const Metrics &m, int comp, AsmGen &g) {
+// The tiles of component comp's rows (x-momentum: i = 1..nx, j = 2..ny;
+// y-momentum: i = 2..nx, j = 1..ny), with as constant ones those whose rows'
+// metric reads i-1..i+1, j-1..j+1 lie inside the boxes of every metric the
+// component reads.
+static AsmTiles asm_tiles(int nx, int ny, const Metrics &m, int comp) {
     static const int u1[13] = {MI_xzu, MI_xeu, MI_yzu, MI_yeu, MI_xec, MI_yec, MI_xzn,
                                MI_yzn, MI_rac, MI_rbc, MI_rbn, MI_rgn, MI_dju};
     static const int u2[13] = {MI_xzv, MI_xev, MI_yzv, MI_yev, MI_xen, MI_yen, MI_xzc,
                                MI_yzc, MI_ran, MI_rbc, MI_rbn, MI_rgc, MI_djv};
-    const AsmRect all = comp == 1 ? AsmRect{1, nx, 2, ny} : AsmRect{2, nx, 1, ny};
-    AsmRect c = all;
+    const AsmRect r = comp == 1 ? AsmRect{1, nx, 2, ny} : AsmRect{2, nx, 1, ny};
+    AsmTiles w{r, (r.i1 - r.i0 + MX) / MX, (r.j1 - r.j0 + MY) / MY, 0, 0, 0, 0};
+    AsmRect c = r;
     for (int q = 0; q < 13; q++) {
         const MBox &b = m.box[comp == 1 ? u1[q] : u2[q]];
         c.i0 = std::max(c.i0, b.i0 + 1);
@@ -854,44 +870,49 @@ static AsmRect asm_rects(int nx, int ny, const Metrics &m, int comp, AsmGen &g) 
         c.j0 = std::max(c.j0, b.j0 + 1);
         c.j1 = std::min(c.j1, b.j1 - 1);
     }
-    auto add = [&](int i0, int i1, int j0, int j1) {
-        if (i0 > i1 || j0 > j1) return;
-        g.comp[g.n] = comp;
-        g.r[g.n] = AsmRect{i0, i1, j0, j1};
-        g.start[g.n + 1] = g.start[g.n] + (long)(i1 - i0 + 1) * (j1 - j0 + 1);
-        g.n++;
-    };
-    if (c.i0 > c.i1 || c.j0 > c.j1) {
-        add(all.i0, all.i1, all.j0, all.j1);
-        return AsmRect{1, 0, 1, 0};
-    }
-    add(all.i0, c.i0 - 1, all.j0, all.j1);   // west strip
-    add(c.i1 + 1, all.i1, all.j0, all.j1);   // east strip
-    add(c.i0, c.i1, all.j0, c.j0 - 1);       // south strip
-    add(c.i0, c.i1, c.j1 + 1, all.j1);       // north strip
-    return c;
+    if (c.i0 > c.i1 || c.j0 > c.j1) return w;
+    const int tx0 = (c.i0 - r.i0 + MX - 1) / MX, tx1 = c.i1 == r.i1 ? w.gx : (c.i1 + 1 - r.i0) / MX;
+    const int ty0 = (c.j0 - r.j0 + MY - 1) / MY, ty1 = c.j1 == r.j1 ? w.gy : (c.j1 + 1 - r.j0) / MY;
+    if (tx0 >= tx1 || ty0 >= ty1) return w;
+    w.tx0 = tx0;
+    w.ntx = tx1 - tx0;
+    w.ty0 = ty0;
+    w.nty = ty1 - ty0;
+    return w;
 }
 
-// Both kernels for the components asked for (o1: x-momentum, o2:
-// y-momentum; a null ch1.a skips a component).
+// Grids of up to this many tiles (two components of about 512^2 rows make
+// 4200) read all metrics, in one launch: with constants in a launch before, a
+// 512^2 cavity in FP64 takes 11.6 + 9.3 us and a launch's gap, without 22.7;
+// a smaller grid's launches are latency, 7 us either way.
+constexpr int ASM_ONE = 2048;
+
+template <int MK, typename T, typename E>
+static void launch_asm_tiles(const Regions &R, int ld, double dk, double re, double fr, const Metrics &m,
+                             const AsmOut<T> &o1, const AsmOut<T> &o2, const E *us, const E *vs, const E *un,
+                             const E *vn, const double *d, const double *dn, hipStream_t s, int *err, int live,
+                             const int *stop, const AsmTiles &w1, const AsmTiles &w2) {
+    auto blocks = [](const AsmTiles &w) {
+        const int nc = w.ntx * w.nty;
+        return 8 * (((MK == MK_CONST ? nc : w.gx * w.gy - nc) + 7) / 8);
+    };
+    const int g1 = blocks(w1), g2 = blocks(w2);
+    if (g1 + g2 > 0)
+        hipLaunchKernelGGL((k_mom_asm<MK, T, E>), dim3(g1 + g2), dim3(MX, MY), 0, s, R, ld, dk, dk * 0.5, 1.0 / re, fr,
+                           m, o1, o2, us, vs, un, vn, d, dn, err, live, stop, w1, w2, g1);
+}
+
+// The kernels for the components asked for (o1: x-momentum, o2: y-momentum; a
+// null ch1.a skips a component).
 template <typename T, typename E>
 static void launch_asm(const Regions &R, int ld, double dk, double re, double fr, const Metrics &m,
                        const AsmOut<T> &o1, const AsmOut<T> &o2, const E *us, const E *vs, const E *un, const E *vn,
                        const double *d, const double *dn, hipStream_t s, int *err, int live, const int *stop) {
-    const double dk2 = dk * 0.5, re1 = 1.0 / re;
-    AsmGen g{};
-    const AsmRect none{1, 0, 1, 0};
-    const AsmRect r1 = o1.ch1.a ? asm_rects(R.nx, R.ny, m, 1, g) : none;
-    const AsmRect r2 = o2.ch1.a ? asm_rects(R.nx, R.ny, m, 2, g) : none;
-    const int g1 = 8 * ((rect_tiles(r1) + 7) / 8), g2 = 8 * ((rect_tiles(r2) + 7) / 8);
-    if (g1 + g2 > 0)
-        hipLaunchKernelGGL((k_mom_asm_cb<T, E>), dim3(g1 + g2), dim3(MX, MY), 0, s, R, ld, dk, dk2, re1, fr, m, o1, o2,
-                           us, vs, un, vn, d, dn, err, live, stop, r1, r2, g1);
-    if (g.n > 0) {
-        const unsigned nb = (unsigned)((g.start[g.n] + AG_T - 1) / AG_T);
-        hipLaunchKernelGGL((k_mom_asm_gen<T, E>), dim3(nb), dim3(AG_T), 0, s, R, ld, dk, dk2, re1, fr, m, o1, o2, us,
-                           vs, un, vn, d, dn, err, live, stop, g);
-    }
+    AsmTiles w1 = o1.ch1.a ? asm_tiles(R.nx, R.ny, m, 1) : AsmTiles{};
+    AsmTiles w2 = o2.ch1.a ? asm_tiles(R.nx, R.ny, m, 2) : AsmTiles{};
+    if (w1.gx * w1.gy + w2.gx * w2.gy <= ASM_ONE) w1.ntx = w1.nty = w2.ntx = w2.nty = 0;
+    launch_asm_tiles<MK_CONST, T, E>(R, ld, dk, re, fr, m, o1, o2, us, vs, un, vn, d, dn, s, err, live, stop, w1, w2);
+    launch_asm_tiles<MK_RANGE, T, E>(R, ld, dk, re, fr, m, o1, o2, us, vs, un, vn, d, dn, s, err, live, stop, w1, w2);
 }
 
 template <typename T>

@@ -247,7 +247,7 @@ template <typename T>
 void launch_conv_diff(int nx, int ny, int ld, int comp, const Metrics &m, const double *us, const double *un,
                       const MomTempsT<T> &t, hipStream_t s);
 // Fused kernels for grids without porous regions: k_mom_n writes cnvn / difn
-// of one component from un, vn; k_mom_asm_cb and k_mom_asm_gen assemble both
+// of one component from un, vn; k_mom_asm assembles both
 // splits of a component from us, vs (ch1: the first split's chain; ch2: the
 // second split's coefficients; zm: its identity rows).
 template <typename T>
