@@ -73,37 +73,15 @@ struct MConst {
     double c;
 };
 __device__ inline double mget(const MConst &a, int, int, int) { return a.c; }
-// A metric array on a range of points (mpick<MK_RANGE>): where the range lies
-// in the constant box every read goes to the box's first element, one address
-// that stays in the caches, else to the point's.  Which one is decided once
-// for the range, so the reads have no branch and their loads can all be in
-// flight at once.
-// Offsets are from the range's first point, so that 32 bits hold them and the
-// arrays' addresses stay in scalar registers.
-struct MRange {
-    const char *p;
-    unsigned keep;   // mask of a read's offset: all or nothing
-    int i0, j0;
-};
-__device__ inline double mget(const MRange &a, int ld, int i, int j) {
-    const unsigned off = 8u * ((unsigned)(i - a.i0) + (unsigned)ld * (unsigned)(j - a.j0));
-    return *reinterpret_cast<const double *>(a.p + (size_t)(off & a.keep));
-}
-// Rows i0..i1 x j0..j1 of one component (empty when i0 > i1 or j0 > j1).
-struct AsmRect {
-    int i0, i1, j0, j1;
-};
 enum { MK_RANGE = 0, MK_CONST = 1 };
 // g: the points the reads cover
 template <int MK>
 __device__ inline std::conditional_t<MK == MK_CONST, MConst, MRange> mpick(const double *p, const MBox &b,
-                                                                         const AsmRect &g, int ld) {
+                                                                         const MRect &g, int ld) {
     if constexpr (MK == MK_CONST) {
         return MConst{b.c};
     } else {
-        const bool in = g.i0 >= b.i0 && g.i1 <= b.i1 && g.j0 >= b.j0 && g.j1 <= b.j1;
-        const double *q = p + (in ? WD2_IX(b.i0, b.j0) : WD2_IX(g.i0, g.j0));
-        return MRange{reinterpret_cast<const char *>(q), in ? 0u : ~0u, g.i0, g.j0};
+        return mrange(p, b, g, ld);
     }
 }
 #define MPICK(m, f) mpick<MK>((m).f, (m).box[MI_##f], grect, ld)
@@ -682,7 +660,7 @@ __device__ inline void mom_asm_row(const Regions &R, int ld, int i, int j, T dk,
                                    const AsmOut<T> &o, const AU &U, const AV &V, const E *__restrict__ us,
                                    const E *__restrict__ vs, const E *__restrict__ un, const E *__restrict__ vn,
                                    const double *__restrict__ d, const double *__restrict__ dn, int *err, int live,
-                                   const AsmRect &grect) {
+                                   const MRect &grect) {
     const int nx = R.nx, ny = R.ny;
     const long k = COMP == 1 ? (long)(j - 2) * nx + (i - 1) : (long)(j - 1) * (nx - 1) + (i - 2);
     const T dZero = T(0.0), dOne = T(1.0), dFour = T(4.0);
@@ -746,13 +724,13 @@ __device__ inline void mom_asm_row(const Regions &R, int ld, int i, int j, T dk,
 // One component's rows (r: i0..i1 x j0..j1) as gx x gy tiles of MX x MY, of
 // which tx0 .. tx0 + ntx - 1 x ty0 .. ty0 + nty - 1 have constant metrics.
 struct AsmTiles {
-    AsmRect r;
+    MRect r;
     int gx, gy, tx0, ntx, ty0, nty;
 };
 
 // Tile (tx, ty) of one component, its us and vs values staged in LDS.
 template <int COMP, int MK, typename T, typename E>
-__device__ inline void mom_asm_tile(int tx, int ty, const AsmRect &r, const Regions &R, int ld, double dk_,
+__device__ inline void mom_asm_tile(int tx, int ty, const MRect &r, const Regions &R, int ld, double dk_,
                                     double dk2_, double re1_, double fr_, const Metrics &m, const AsmOut<T> &o,
                                     const E *__restrict__ us, const E *__restrict__ vs, const E *__restrict__ un,
                                     const E *__restrict__ vn, const double *__restrict__ d,
@@ -799,7 +777,7 @@ __device__ inline void mom_asm_tile(int tx, int ty, const AsmRect &r, const Regi
     const int i = I0 + threadIdx.x, j = J0 + threadIdx.y;
     if (i > r.i1 || j > r.j1) return;
     const LAcc<T> U{tu, ui0, uj0, WU}, V{tv, vi0, vj0, WV};
-    const AsmRect g{I0 - 1, min(I0 + MX, r.i1 + 1), J0 - 1, min(J0 + MY, r.j1 + 1)};
+    const MRect g{I0 - 1, min(I0 + MX, r.i1 + 1), J0 - 1, min(J0 + MY, r.j1 + 1)};
     mom_asm_row<COMP, MK, T, E>(R, ld, i, j, cv<T>(dk_), cv<T>(dk2_), cv<T>(re1_), cv<T>(fr_), m, o, U, V, us, vs, un,
                                 vn, d, dn, err, live, g);
 }
@@ -860,9 +838,9 @@ static AsmTiles asm_tiles(int nx, int ny, const Metrics &m, int comp) {
                                MI_yzn, MI_rac, MI_rbc, MI_rbn, MI_rgn, MI_dju};
     static const int u2[13] = {MI_xzv, MI_xev, MI_yzv, MI_yev, MI_xen, MI_yen, MI_xzc,
                                MI_yzc, MI_ran, MI_rbc, MI_rbn, MI_rgc, MI_djv};
-    const AsmRect r = comp == 1 ? AsmRect{1, nx, 2, ny} : AsmRect{2, nx, 1, ny};
+    const MRect r = comp == 1 ? MRect{1, nx, 2, ny} : MRect{2, nx, 1, ny};
     AsmTiles w{r, (r.i1 - r.i0 + MX) / MX, (r.j1 - r.j0 + MY) / MY, 0, 0, 0, 0};
-    AsmRect c = r;
+    MRect c = r;
     for (int q = 0; q < 13; q++) {
         const MBox &b = m.box[comp == 1 ? u1[q] : u2[q]];
         c.i0 = std::max(c.i0, b.i0 + 1);

@@ -19,6 +19,7 @@
 // (see the two kernels), the fold sets ql_stop = -1, every kernel queued
 // behind returns at entry, and the host repeats the iteration with the
 // solvers of k_trid.hip.
+#include <algorithm>
 #include <cmath>
 
 #include "wd2_trid.hpp"
@@ -679,41 +680,68 @@ __global__ __launch_bounds__(NT, sizeof(CT) == 4 ? 5 : 3) void k_ql_window(long 
 // is usable (exact windows: chk, the neighbours' shared rows agree bit for
 // bit; FP32 windows: no weak window), and the stopping test of iteration m
 // (momentum.f:182-188).
+//
+// One workgroup between every two iterations, all latency: its loads are all
+// in flight before the first is used, and everything is reduced across the
+// wavefronts (as many as there are windows for) with one exchange.  With a
+// reduction after the other in 1024 lanes it took 4.0 us for a few windows and
+// 7.8 for the 1131 of the 1024^2 cavity in FP64; here 3.6 and 5.0.
 template <typename T>
 __global__ __launch_bounds__(1024) void k_ql_fold_win(int ld, const double *__restrict__ dus,
                                                       const double *__restrict__ dvs, const double *__restrict__ part,
                                                       int nwin, const T *__restrict__ chk, int *weakf, Scalars *sc,
                                                       double qtol, int m) {
-    if (sc->ql_stop) return;
-    __shared__ double sh[1024 / 64];
+    __shared__ double sh[2][1024 / 64];
+    __shared__ int shb[1024 / 64];
+    const int t = threadIdx.x, nw = blockDim.x >> 6;
+    const int stopped = sc->ql_stop, weak = chk ? 0 : *weakf;
+    const double d0 = fabs(dus[WD2_IX(5, 5)]), d1 = fabs(dvs[WD2_IX(5, 5)]);
     double r1 = 0.0, r2 = 0.0;
-    bool bad = false;
-    for (int w = threadIdx.x; w < nwin; w += 1024) {
-        r1 = dmaxf(r1, part[2 * w]);
-        r2 = dmaxf(r2, part[2 * w + 1]);
+    bool bad = weak != 0;
+    for (int w = t; w < nwin; w += blockDim.x) {
+        const double2 v = reinterpret_cast<const double2 *>(part)[w];
         if (chk && w + 1 < nwin) {
             const T *p = chk + (size_t)w * QX_CHK, *q = p + QX_CHK;
-            bad |= !(same(q[0], p[2]) && same(q[1], p[3]) && same(p[4], q[5]) && same(q[6], p[8]) &&
-                     same(q[7], p[9]) && same(p[10], q[11]));
+            const bool e0 = same(q[0], p[2]), e1 = same(q[1], p[3]), e2 = same(p[4], q[5]), e3 = same(q[6], p[8]),
+                       e4 = same(q[7], p[9]), e5 = same(p[10], q[11]);
+            bad |= !(e0 & e1 & e2 & e3 & e4 & e5);
         }
+        r1 = dmaxf(r1, v.x);
+        r2 = dmaxf(r2, v.y);
     }
-    if (!chk) bad = *weakf != 0;
-    const int anybad = __syncthreads_or(bad);
-    r1 = block_max<1024>(r1, sh, threadIdx.x);
-    r2 = block_max<1024>(r2, sh, threadIdx.x);
-    if (threadIdx.x == 0) {
+    if (stopped) return;
+    for (int off = 32; off > 0; off >>= 1) {
+        r1 = dmaxf(r1, __shfl_xor(r1, off));
+        r2 = dmaxf(r2, __shfl_xor(r2, off));
+    }
+    const bool wb = __any(bad);
+    if ((t & 63) == 0) {
+        sh[0][t >> 6] = r1;
+        sh[1][t >> 6] = r2;
+        shb[t >> 6] = wb;
+    }
+    __syncthreads();
+    if (t >= 64) return;
+    bool anybad = false;
+    for (int w = 0; w < nw; w++) {
+        r1 = dmaxf(r1, sh[0][w]);
+        r2 = dmaxf(r2, sh[1][w]);
+        anybad |= shb[w] != 0;
+    }
+    if (t == 0) {
         if (anybad) {
             sc->ql_stop = -1;
             if (!chk) *weakf = 0;
             return;
         }
-        const double v0 = dmaxf(fabs(dus[WD2_IX(5, 5)]), r1), v1 = dmaxf(fabs(dvs[WD2_IX(5, 5)]), r2);
+        const double v0 = dmaxf(d0, r1), v1 = dmaxf(d1, r2);
         sc->val[0] = v0;
         sc->val[1] = v1;
         const double difmax = v0 > v1 ? v0 : v1;
         if (difmax <= qtol) sc->ql_stop = m;
     }
 }
+static dim3 fold_lanes(int nwin) { return dim3(std::min(1024, (nwin + 63) / 64 * 64)); }
 
 // After a captured loop of Q iterations: the iterate to (us, vs) where the
 // last iteration that ran left it in the other buffers (ua, va).
@@ -745,7 +773,7 @@ void launch_ql_pair(const QlPair<double> &q, long n, const Chains &cs, const Cha
     const int nw = (int)((n + QX_O - 1) / QX_O), nb = ql_border_blocks(q.nx, q.ny, QX_T);
     hipLaunchKernelGGL(k_ql_exact<double>, dim3(nw + nb), dim3(QX_T), 0, s, n, cs, h1, h2, Z, F, q.part, q.chk, nw,
                        &sc->ql_stop);
-    hipLaunchKernelGGL(k_ql_fold_win<double>, dim3(1), dim3(1024), 0, s, q.ld, q.dus, q.dvs, q.part, nw,
+    hipLaunchKernelGGL(k_ql_fold_win<double>, dim3(1), fold_lanes(nw), 0, s, q.ld, q.dus, q.dvs, q.part, nw,
                        (const double *)q.chk, (int *)nullptr, sc, qtol, m);
 }
 
@@ -758,7 +786,7 @@ static void ql_window_as(const QlPair<float> &q, long n, const Chains &cs, const
     const int nw = (int)((n + O - 1) / O), nb = ql_border_blocks(q.nx, q.ny, NT);
     hipLaunchKernelGGL((k_ql_window<CT, NT>), dim3(nw + nb), dim3(NT), 0, s, n, cs, h1, h2, Z, F, q.part, nw,
                        &sc->ql_weak, &sc->ql_stop);
-    hipLaunchKernelGGL(k_ql_fold_win<float>, dim3(1), dim3(1024), 0, s, q.ld, q.dus, q.dvs, q.part, nw,
+    hipLaunchKernelGGL(k_ql_fold_win<float>, dim3(1), fold_lanes(nw), 0, s, q.ld, q.dus, q.dvs, q.part, nw,
                        (const float *)nullptr, &sc->ql_weak, sc, qtol, m);
 }
 void launch_ql_pair(const QlPair<float> &q, long n, const Chains &cs, const ChainT<float> &h1,

@@ -21,21 +21,27 @@ __global__ __launch_bounds__(SX *SY) void k_project(Regions R, int ld, double dk
     const int i = 1 + blockIdx.x * SX + threadIdx.x, j = 1 + blockIdx.y * SY + threadIdx.y;
     if (i > R.nx || j > R.ny) return;
     const double dFour = 4.0;
+    const int I0 = 1 + blockIdx.x * SX, J0 = 1 + blockIdx.y * SY;
+    const MRect g{I0, min(I0 + SX - 1, R.nx), J0, min(J0 + SY - 1, R.ny)};
+#define MR(f) mrange(m.f, m.box[MI_##f], g, ld)
+    const double dju = mget(MR(dju), ld, i, j), yeu = mget(MR(yeu), ld, i, j), yzu = mget(MR(yzu), ld, i, j);
+    const double djv = mget(MR(djv), ld, i, j), xev = mget(MR(xev), ld, i, j), xzv = mget(MR(xzv), ld, i, j);
+#undef MR
 #define P(a, b) p[WD2_IX(a, b)]
     double uu = u[WD2_IX(i, j)], vv = v[WD2_IX(i, j)];
     bool wu = false, wv = false;
     auto upd_u = [&](void) {
         const double pzi = P(i + 1, j) - P(i, j);
         const double pet = (P(i + 1, j + 1) + P(i, j + 1) - P(i + 1, j - 1) - P(i, j - 1)) / dFour;
-        const double djk = m.dju[WD2_IX(i, j)] * dk;
-        uu = uu - djk * (m.yeu[WD2_IX(i, j)] * pzi - m.yzu[WD2_IX(i, j)] * pet);
+        const double djk = dju * dk;
+        uu = uu - djk * (yeu * pzi - yzu * pet);
         wu = true;
     };
     auto upd_v = [&](void) {
         const double pzi = (P(i + 1, j + 1) + P(i + 1, j) - P(i - 1, j + 1) - P(i - 1, j)) / dFour;
         const double pet = P(i, j + 1) - P(i, j);
-        const double djk = m.djv[WD2_IX(i, j)] * dk;
-        vv = vv - djk * (-m.xev[WD2_IX(i, j)] * pzi + m.xzv[WD2_IX(i, j)] * pet);
+        const double djk = djv * dk;
+        vv = vv - djk * (-xev * pzi + xzv * pet);
         wv = true;
     };
     for (int jr = 1; jr <= R.nj; jr++)
@@ -71,16 +77,28 @@ void launch_project(const Regions &R, int ld, double dk, const Metrics &m, const
 }
 
 // --------------------------------------------------------------- Divergence
-__global__ __launch_bounds__(SX *SY) void k_divergence(int nx, int ny, int ld, int nloc,
-                                                       const double *__restrict__ xet, const double *__restrict__ yet,
-                                                       const double *__restrict__ xzi, const double *__restrict__ yzi,
+// rhs (null: none): also the Ppe right-hand side div / dk on i = 2..nx, j =
+// 2..ny, with blockage rows zeroed (prow != 0 marks them).
+struct DivMetrics {
+    const double *xet, *yet, *xzi, *yzi;
+    MBox bxet, byet, bxzi, byzi;
+};
+__global__ __launch_bounds__(SX *SY) void k_divergence(int nx, int ny, int ld, int nloc, DivMetrics q,
                                                        const double *__restrict__ u, const double *__restrict__ v,
-                                                       double *__restrict__ div) {
+                                                       double *__restrict__ div, double dk,
+                                                       const unsigned char *__restrict__ prow,
+                                                       double *__restrict__ rhs) {
     const int i = 1 + blockIdx.x * SX + threadIdx.x, j = 1 + blockIdx.y * SY + threadIdx.y;
     if (i > nx || j > ny) return;
+    // the metric reads: i-1..i+1, j-1..j+1
+    const int I0 = blockIdx.x * SX, J0 = blockIdx.y * SY;
+    const MRect g{I0, min(I0 + SX, nx) + 1, J0, min(J0 + SY, ny) + 1};
+    const MRange xet = mrange(q.xet, q.bxet, g, ld), yet = mrange(q.yet, q.byet, g, ld);
+    const MRange xzi = mrange(q.xzi, q.bxzi, g, ld), yzi = mrange(q.yzi, q.byzi, g, ld);
 #define U(a, b) u[WD2_IX(a, b)]
 #define V(a, b) v[WD2_IX(a, b)]
-#define M(f, a, b) f[WD2_IX(a, b)]
+#define M(f, a, b) mget(f, ld, a, b)
+    double r;
     if (nloc == 1) {
         const double ucij = M(yet, i, j) * U(i, j) -
                             M(xet, i, j) * (V(i + 1, j) + V(i, j) + V(i + 1, j - 1) + V(i, j - 1)) / 4.0;
@@ -90,7 +108,7 @@ __global__ __launch_bounds__(SX *SY) void k_divergence(int nx, int ny, int ld, i
                             M(yzi, i, j) * (U(i, j + 1) + U(i - 1, j + 1) + U(i, j) + U(i - 1, j)) / 4.0;
         const double vcij1 = M(xzi, i, j - 1) * V(i, j - 1) -
                              M(yzi, i, j - 1) * (U(i, j) + U(i - 1, j) + U(i, j - 1) + U(i - 1, j - 1)) / 4.0;
-        div[WD2_IX(i, j)] = ucij - uci1j + vcij - vcij1;
+        r = ucij - uci1j + vcij - vcij1;
     } else {
         const double uci1j = M(yet, i + 1, j) * (U(i, j + 1) + U(i + 1, j + 1) + U(i, j) + U(i + 1, j)) / 4.0 -
                              M(xet, i + 1, j) * V(i + 1, j);
@@ -100,36 +118,26 @@ __global__ __launch_bounds__(SX *SY) void k_divergence(int nx, int ny, int ld, i
                              M(yzi, i, j + 1) * U(i, j + 1);
         const double vcij = M(xzi, i, j) * (V(i, j) + V(i + 1, j) + V(i, j - 1) + V(i + 1, j - 1)) / 4.0 -
                             M(yzi, i, j) * U(i, j);
-        div[WD2_IX(i, j)] = uci1j - ucij + vcij1 - vcij;
+        r = uci1j - ucij + vcij1 - vcij;
     }
+    const size_t k = WD2_IX(i, j);
+    div[k] = r;
+    if (rhs && i >= 2 && j >= 2) rhs[k] = (prow && prow[k] ? 0.0 : r) / dk;
 #undef U
 #undef V
 #undef M
 }
 
 void launch_divergence(int nx, int ny, int ld, int nloc, const Metrics &m, const double *u, const double *v,
-                       double *div, hipStream_t s) {
-    const double *xet = nloc == 1 ? m.xeu : m.xev, *yet = nloc == 1 ? m.yeu : m.yev;
-    const double *xzi = nloc == 1 ? m.xzv : m.xzu, *yzi = nloc == 1 ? m.yzv : m.yzu;
-    hipLaunchKernelGGL(k_divergence, grid2(nx, ny), dim3(SX, SY), 0, s, nx, ny, ld, nloc, xet, yet, xzi, yzi, u, v,
-                       div);
+                       double *div, hipStream_t s, double dk, const unsigned char *prow, double *rhs) {
+#define MB(f) m.box[MI_##f]
+    const DivMetrics q = nloc == 1 ? DivMetrics{m.xeu, m.yeu, m.xzv, m.yzv, MB(xeu), MB(yeu), MB(xzv), MB(yzv)}
+                                   : DivMetrics{m.xev, m.yev, m.xzu, m.yzu, MB(xev), MB(yev), MB(xzu), MB(yzu)};
+#undef MB
+    hipLaunchKernelGGL(k_divergence, grid2(nx, ny), dim3(SX, SY), 0, s, nx, ny, ld, nloc, q, u, v, div, dk, prow, rhs);
 }
 
 // ------------------------------------------------------------- PPE set-up
-__global__ __launch_bounds__(SX *SY) void k_ppe_rhs(int nx, int ny, int ld, double dk,
-                                                    const double *__restrict__ div,
-                                                    const unsigned char *__restrict__ prow, double *__restrict__ rhs) {
-    const int i = 2 + blockIdx.x * SX + threadIdx.x, j = 2 + blockIdx.y * SY + threadIdx.y;
-    if (i > nx || j > ny) return;
-    const double dv = (prow && prow[WD2_IX(i, j)]) ? 0.0 : div[WD2_IX(i, j)];
-    rhs[WD2_IX(i, j)] = dv / dk;
-}
-
-void launch_ppe_rhs(int nx, int ny, int ld, double dk, const double *div, const unsigned char *prow,
-                    double *rhs, hipStream_t s) {
-    hipLaunchKernelGGL(k_ppe_rhs, grid2(nx - 1, ny - 1), dim3(SX, SY), 0, s, nx, ny, ld, dk, div, prow, rhs);
-}
-
 __global__ __launch_bounds__(SX *SY) void k_rhs_cross(int nx, int ny, int ld, const double *__restrict__ rbu,
                                                       const double *__restrict__ rbv, const double *__restrict__ rhs,
                                                       const double *__restrict__ p, double *__restrict__ beff) {
@@ -180,39 +188,36 @@ void launch_ppe_coef(int nx, int ny, int ld, const Metrics &m, const unsigned ch
 // DiffMaxNorm:          max(|a(2,2)-b(2,2)|, max_{2..nx-1, 2..ny-1} |a-b|)
 // Workgroups publish partial maxima; a one-workgroup kernel folds them with
 // the seed (the kernel boundary orders the two, no device-scope fence).
-__global__ __launch_bounds__(SX *SY) void k_max_norm(int nx, int ny, int ld, const double *__restrict__ a,
-                                                     const double *__restrict__ b, double *__restrict__ partials) {
+// Up to NORM_SET pairs in the two launches, the pair along the grid's z / x.
+__global__ __launch_bounds__(SX *SY) void k_max_norm(int nx, int ny, int ld, NormSet q, double *__restrict__ partials) {
     __shared__ double sh[SX * SY / 64];
     const int tid = threadIdx.x + SX * threadIdx.y;
+    const double *__restrict__ a = q.a[blockIdx.z], *__restrict__ b = q.b[blockIdx.z];
     double mx = 0.0;
     for (int j = 2 + blockIdx.y * SY + threadIdx.y; j <= ny - 1; j += gridDim.y * SY) {
         const int i = 2 + blockIdx.x * SX + threadIdx.x;
         if (i <= nx - 1) mx = dmaxf(mx, b ? fabs(a[WD2_IX(i, j)] - b[WD2_IX(i, j)]) : fabs(a[WD2_IX(i, j)]));
     }
     mx = block_max<SX * SY>(mx, sh, tid);
-    if (tid == 0) partials[blockIdx.x + gridDim.x * blockIdx.y] = mx;
+    if (tid == 0) partials[(size_t)blockIdx.z * RED_MAX_BLOCKS + blockIdx.x + gridDim.x * blockIdx.y] = mx;
 }
 
-__global__ __launch_bounds__(256) void k_max_norm_fold(int ld, const double *__restrict__ a,
-                                                       const double *__restrict__ b,
-                                                       const double *__restrict__ partials, int n, Scalars *sc,
-                                                       int slot) {
+__global__ __launch_bounds__(256) void k_max_norm_fold(int ld, NormSet q, const double *__restrict__ partials, int n,
+                                                       Scalars *sc) {
     __shared__ double sh[4];
+    const double *a = q.a[blockIdx.x], *b = q.b[blockIdx.x], *p = partials + (size_t)blockIdx.x * RED_MAX_BLOCKS;
+    const double seed = b ? fabs(a[WD2_IX(2, 2)] - b[WD2_IX(2, 2)]) : fabs(a[WD2_IX(5, 5)]);
     double r = 0.0;
-    for (int k = threadIdx.x; k < n; k += 256) r = dmaxf(r, partials[k]);
+    for (int k = threadIdx.x; k < n; k += 256) r = dmaxf(r, p[k]);
     r = block_max<256>(r, sh, threadIdx.x);
-    if (threadIdx.x == 0) {
-        const double seed = b ? fabs(a[WD2_IX(2, 2)] - b[WD2_IX(2, 2)]) : fabs(a[WD2_IX(5, 5)]);
-        sc->val[slot] = dmaxf(seed, r);
-    }
+    if (threadIdx.x == 0) sc->val[q.slot[blockIdx.x]] = dmaxf(seed, r);
 }
 
-void launch_max_norm(int nx, int ny, int ld, const double *a, const double *b, double *partials, Scalars *sc,
-                     int slot, hipStream_t s) {
+void launch_max_norms(int nx, int ny, int ld, const NormSet &q, double *partials, Scalars *sc, hipStream_t s) {
     const int gx = (max(nx - 2, 1) + SX - 1) / SX;
     const int gy = min((max(ny - 2, 1) + SY - 1) / SY, max(1, 1024 / gx));
-    hipLaunchKernelGGL(k_max_norm, dim3(gx, gy), dim3(SX, SY), 0, s, nx, ny, ld, a, b, partials);
-    hipLaunchKernelGGL(k_max_norm_fold, dim3(1), dim3(256), 0, s, ld, a, b, partials, gx * gy, sc, slot);
+    hipLaunchKernelGGL(k_max_norm, dim3(gx, gy, q.n), dim3(SX, SY), 0, s, nx, ny, ld, q, partials);
+    hipLaunchKernelGGL(k_max_norm_fold, dim3(q.n), dim3(256), 0, s, ld, q, partials, gx * gy, sc);
 }
 
 // -------------------------------------------------------------- copies

@@ -1066,8 +1066,7 @@ static int ppe(wd2_ctx *c, int cart, int solver, int msorit, double dk, double s
         *nconv_out = msorit;
         return WD2_OK;
     }
-    launch_divergence(nx, ny, ld, 1, c->M, u, v, c->div, s);
-    launch_ppe_rhs(nx, ny, ld, dk, c->div, c->any_blockage ? c->prow : nullptr, c->rhs, s);
+    launch_divergence(nx, ny, ld, 1, c->M, u, v, c->div, s, dk, c->any_blockage ? c->prow : nullptr, c->rhs);
     if (solver == 7) return ppe_mg(c, cart, msorit, dk, sortol, p, nconv_out);
     const PpeCoef cf{c->pc[0], c->pc[1], c->pc[2], c->pc[3], c->pc[4]};
     const PpeCoef *coef = nullptr;
@@ -1396,10 +1395,8 @@ static int one_step(wd2_ctx *c, const wd2_params *P, int *nql, int *nsor, double
         // loop ends either way)
         const bool test = l > 1 && l < nme;
         if (test) {
-            launch_max_norm(nx, ny, ld, c->u, c->us, c->partials, c->sc, 5, s);
-            launch_max_norm(nx, ny, ld, c->v, c->vs, c->partials + RED_MAX_BLOCKS, c->sc, 6, s);
-            launch_max_norm(nx, ny, ld, therm ? c->t : c->u, therm ? c->ts : c->u, c->partials + 2 * RED_MAX_BLOCKS,
-                            c->sc, 7, s);
+            const NormSet q{3, {c->u, c->v, therm ? c->t : c->u}, {c->us, c->vs, therm ? c->ts : c->u}, {5, 6, 7}};
+            launch_max_norms(nx, ny, ld, q, c->partials, c->sc, s);
         }
         // u = us, v = vs, t = ts (swap the buffers: same values)
         std::swap(c->u, c->us);
@@ -1421,10 +1418,8 @@ static int one_step(wd2_ctx *c, const wd2_params *P, int *nql, int *nsor, double
     if (!fills_twice) launch_fills(c->R, ld, c->u, c->v, c->p, 1, &c->sc->err, s);
     if (therm) launch_temp_bc(c->R, c->TH, ld, c->t, &c->sc->err, s);
     // main.f:962-965
-    launch_max_norm(nx, ny, ld, c->pn, c->p, c->partials, c->sc, 2, s);
-    launch_max_norm(nx, ny, ld, c->un, c->u, c->partials + RED_MAX_BLOCKS, c->sc, 3, s);
-    launch_max_norm(nx, ny, ld, c->vn, c->v, c->partials + 2 * RED_MAX_BLOCKS, c->sc, 4, s);
-    if (therm) launch_max_norm(nx, ny, ld, c->tn, c->t, c->partials + 3 * RED_MAX_BLOCKS, c->sc, 5, s);
+    const NormSet q{therm ? 4 : 3, {c->pn, c->un, c->vn, c->tn}, {c->p, c->u, c->v, c->t}, {2, 3, 4, 5}};
+    launch_max_norms(nx, ny, ld, q, c->partials, c->sc, s);
     if (dif) HIPCHK(hipMemcpyAsync(dif, &c->sc->val[2], (therm ? 4 : 3) * sizeof(double), hipMemcpyDeviceToHost, s));
     extrap_advance(c, xp);
     ql_step_done(c);
@@ -1486,8 +1481,7 @@ static void step_body(wd2_ctx *c, const wd2_params *P, int Q, int C, int xp, boo
     launch_fills(c->R, ld, c->us, c->vs, c->p, 1, &c->sc->err, s);
     if (xp) launch_mg_extrap(nx, ny, ld, c->p, extrap_p1(c), extrap_p2(c, xp), s);
     // Ppe (pressure.f:30) with the multigrid solver
-    launch_divergence(nx, ny, ld, 1, c->M, c->us, c->vs, c->div, s);
-    launch_ppe_rhs(nx, ny, ld, P->dk, c->div, nullptr, c->rhs, s);
+    launch_divergence(nx, ny, ld, 1, c->M, c->us, c->vs, c->div, s, P->dk, nullptr, c->rhs);
     const double *uni = (g_uniform && c->uni_ok) ? c->uni : nullptr;
     const double *b = P->lCartesGrid ? c->rhs : c->beff;
     launch_mg_reset(c->sc, s);
@@ -1506,9 +1500,8 @@ static void step_body(wd2_ctx *c, const wd2_params *P, int Q, int C, int xp, boo
     // of the step works on us, vs as the new u, v (main.f:946-965); the fills
     // after Project and those at the step's end are one launch
     launch_fills(c->R, ld, c->us, c->vs, c->p, 2, &c->sc->err, s);
-    launch_max_norm(nx, ny, ld, c->pn, c->p, c->partials, c->sc, 2, s);
-    launch_max_norm(nx, ny, ld, c->un, c->us, c->partials + RED_MAX_BLOCKS, c->sc, 3, s);
-    launch_max_norm(nx, ny, ld, c->vn, c->vs, c->partials + 2 * RED_MAX_BLOCKS, c->sc, 4, s);
+    const NormSet q{3, {c->pn, c->un, c->vn}, {c->p, c->us, c->vs}, {2, 3, 4}};
+    launch_max_norms(nx, ny, ld, q, c->partials, c->sc, s);
     (void)hipMemcpyAsync(c->h_sc, c->sc, sizeof(Scalars), hipMemcpyDeviceToHost, s);
 }
 
@@ -1998,8 +1991,7 @@ static int tl_step(wd2_adj *a, const Regions &Rt, const double *un, const double
     // VelBoundCond, PresBoundCond, then u = us and the step-end fills
     launch_vel_bc<double>(Rt, ld, dus, dvs, false, &c->sc->err, s);
     launch_pres_bc<double>(Rt, ld, dp, &c->sc->err, s);
-    launch_divergence(nx, ny, ld, 1, c->M, dus, dvs, c->div, s);
-    launch_ppe_rhs(nx, ny, ld, P.dk, c->div, nullptr, c->rhs, s);
+    launch_divergence(nx, ny, ld, 1, c->M, dus, dvs, c->div, s, P.dk, nullptr, c->rhs);
     double bmax = 0.0, pmax = 0.0;
     int st = adj_max2(a, nf, c->rhs, dp, &bmax, &pmax);
     if (st) return st;
@@ -2372,7 +2364,7 @@ static int norm_common(int nx, int ny, int ld, const double *a, const double *b,
     if ((st = dropin_ctx(nx, ny, ld))) return st;
     wd2_ctx *c = g_ctx;
     if ((st = up(c, a, ld, c->un)) || (st = up(c, b, ld, c->u))) return st;
-    launch_max_norm(nx, ny, c->ld, c->un, b ? c->u : nullptr, c->partials, c->sc, 2, c->s);
+    launch_max_norms(nx, ny, c->ld, NormSet{1, {c->un}, {b ? c->u : nullptr}, {2}}, c->partials, c->sc, c->s);
     HIPCHK(hipMemcpyAsync(out, &c->sc->val[2], sizeof(double), hipMemcpyDeviceToHost, c->s));
     HIPCHK(hipStreamSynchronize(c->s));
     return WD2_OK;

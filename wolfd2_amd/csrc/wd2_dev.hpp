@@ -124,6 +124,31 @@ __device__ inline double mget(const MArr &a, int ld, int i, int j) { return mget
 
 #define WD2_IX(i, j) ((size_t)(i) + (size_t)ld * (size_t)(j))
 
+// Points i0..i1 x j0..j1 (empty when i0 > i1 or j0 > j1).
+struct MRect {
+    int i0, i1, j0, j1;
+};
+// A metric array on a range of points: where the range lies in the constant
+// box every read goes to the box's first element, one address that stays in
+// the caches, else to the point's.  Which one is decided once for the range,
+// so the reads have no branch and their loads can all be in flight at once.
+// Offsets are from the range's first point, so that 32 bits hold them and the
+// arrays' addresses stay in scalar registers.
+struct MRange {
+    const char *p;
+    unsigned keep;   // mask of a read's offset: all or nothing
+    int i0, j0;
+};
+__device__ inline MRange mrange(const double *p, const MBox &b, const MRect &g, int ld) {
+    const bool in = g.i0 >= b.i0 && g.i1 <= b.i1 && g.j0 >= b.j0 && g.j1 <= b.j1;
+    const double *q = p + (in ? (size_t)b.i0 + (size_t)ld * (size_t)b.j0 : (size_t)g.i0 + (size_t)ld * (size_t)g.j0);
+    return MRange{reinterpret_cast<const char *>(q), in ? 0u : ~0u, g.i0, g.j0};
+}
+__device__ inline double mget(const MRange &a, int ld, int i, int j) {
+    const unsigned off = 8u * ((unsigned)(i - a.i0) + (unsigned)ld * (unsigned)(j - a.j0));
+    return *reinterpret_cast<const double *>(a.p + (size_t)(off & a.keep));
+}
+
 // Non-negative doubles order like their bit patterns read as unsigned integers.
 __device__ inline unsigned long long dbits(double x) { return (unsigned long long)__double_as_longlong(x); }
 __device__ inline double bitsd(unsigned long long b) { return __longlong_as_double((long long)b); }

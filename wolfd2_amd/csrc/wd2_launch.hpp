@@ -92,10 +92,8 @@ void launch_project(const Regions &R, int ld, double dk, const Metrics &m, const
                     double *v, hipStream_t s);
 // pressure.f:Divergence (nloc 1 or 2)
 void launch_divergence(int nx, int ny, int ld, int nloc, const Metrics &m, const double *u, const double *v,
-                       double *div, hipStream_t s);
-// Ppe right-hand side: rhs = div/dk with blockage rows zeroed (prow != 0 marks them).
-void launch_ppe_rhs(int nx, int ny, int ld, double dk, const double *div, const unsigned char *prow,
-                    double *rhs, hipStream_t s);
+                       double *div, hipStream_t s, double dk = 1.0, const unsigned char *prow = nullptr,
+                       double *rhs = nullptr);
 // RhsPpe mixed-derivative terms for curvilinear grids: beff = rhs - cross(p).
 void launch_rhs_cross(int nx, int ny, int ld, const Metrics &m, const double *rhs, const double *p,
                       double *beff, hipStream_t s);
@@ -103,8 +101,13 @@ void launch_rhs_cross(int nx, int ny, int ld, const Metrics &m, const double *rh
 void launch_ppe_coef(int nx, int ny, int ld, const Metrics &m, const unsigned char *prow, double *a1,
                      double *a2, double *a3, double *a4, double *a5, hipStream_t s);
 // utility.f:DMaxNorm / DiffMaxNorm into sc->val[slot] (b may be null for DMaxNorm).
-void launch_max_norm(int nx, int ny, int ld, const double *a, const double *b, double *partials, Scalars *sc,
-                     int slot, hipStream_t s);
+constexpr int NORM_SET = 4;
+struct NormSet {
+    int n;
+    const double *a[NORM_SET], *b[NORM_SET];
+    int slot[NORM_SET];
+};
+void launch_max_norms(int nx, int ny, int ld, const NormSet &q, double *partials, Scalars *sc, hipStream_t s);
 // dst = src on i in [i0,i1], j in [j0,j1]
 void launch_copy(int ld, int i0, int i1, int j0, int j1, const double *src, double *dst, hipStream_t s);
 // dst[q] = src[q] over the same box for q < n (n <= 6), one launch
