@@ -55,8 +55,8 @@ int wd2_set_lex_rows(int enable);
 /* Mixed precision only: solve the FP32 momentum chains of q-l iterations 2..
  * with the windowed partitioned-Thomas/PCR solver (enable = 1, the default;
  * results agree with the bit-exact FP32 solver to FP32 rounding; the first
- * iteration of each step keeps the bit-exact solver) or every chain with the
- * bit-exact speculative solver (0).  Returns the previous setting.  No
+ * iteration of each step solves its FP32 chains on the same windows in FP64
+ * arithmetic) or every chain with the bit-exact speculative solver (0).  Returns the previous setting.  No
  * counterpart in the reference. */
 int wd2_set_window_chains(int enable);
 /* Non-zero (default): on a uniform Cartesian grid, where rau and rgv each hold
@@ -362,14 +362,14 @@ int wd2_ctx_trid_set_window(wd2_ctx *ctx, int window_threads);
  * counterpart in the reference. */
 int wd2_ctx_set_mg_extrapolation(wd2_ctx *ctx, int order);
 int wd2_ctx_trid_autotune(wd2_ctx *ctx, int reps, int *window_threads, double *us);
-/* Kernel shapes of the multigrid solver (no counterpart in the reference;
- * none changes the arithmetic, so results are the same bits): nt0 threads
- * per level-0 tile workgroup (256 or 512), stage 1 to form the level-0
- * residual from an LDS copy of p (0: from memory), bside the widest level
- * the one-workgroup bottom kernel takes (32 or 64). */
+/* Kernel shapes of the multigrid solver (no counterpart in the reference):
+ * bside the widest level the one-workgroup bottom kernel takes (32 or 64; the
+ * FP64 path's takes at most 32).  nt0 (256 or 512) and stage (0 or 1) are
+ * checked and kept for wd2_ctx_mg_get_tune; the level-0 kernels have one
+ * shape. */
 int wd2_ctx_mg_set_tune(wd2_ctx *ctx, int nt0, int stage, int bside);
 int wd2_ctx_mg_get_tune(wd2_ctx *ctx, int *nt0, int *stage, int *bside);
-/* Autotuner: times `cycles` full V-cycles of every shape above on the
+/* Autotuner: times `cycles` full V-cycles with each bside on the
  * context's grid, precision and current right-hand side (p is restored),
  * keeps the fastest and returns its time per V-cycle in *best_us. */
 int wd2_ctx_mg_autotune(wd2_ctx *ctx, double dk, int cycles, double *best_us);
