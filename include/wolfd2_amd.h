@@ -56,8 +56,10 @@ int wd2_set_lex_rows(int enable);
  * with the windowed partitioned-Thomas/PCR solver (enable = 1, the default;
  * results agree with the bit-exact FP32 solver to FP32 rounding; the first
  * iteration of each step solves its FP32 chains on the same windows in FP64
- * arithmetic) or every chain with the bit-exact speculative solver (0).  Returns the previous setting.  No
- * counterpart in the reference. */
+ * arithmetic; an iteration whose chains are not diagonally dominant, or
+ * couple rows 64 apart by more than an FP32 rounding, takes the bit-exact
+ * solver) or every chain with the bit-exact speculative solver (0).  Returns
+ * the previous setting.  No counterpart in the reference. */
 int wd2_set_window_chains(int enable);
 /* Non-zero (default): on a uniform Cartesian grid, where rau and rgv each hold
  * one value over the entries the red-black SOR reads, the tiled SOR kernels

@@ -1,15 +1,15 @@
 """The mixed path's windowed FP32 chain solver (partitioned Thomas + PCR in
 LDS over overlapping windows, wd2_set_window_chains) against the bit-exact
-FP32 speculative solver and the FP64 path.  In a time step the window solver
-serves the q-l iterations after the first; the first keeps the sequential
-solver.
+FP32 speculative solver and the FP64 path.  A time step solves both splits of
+its q-l iterations on such windows, the first iteration in FP64 arithmetic.
 
-* Where every window is diagonally dominant (dominance ratio <= 0.9, the
-  cavities and channels of the measured workloads), the two FP32 solvers agree
-  to FP32 rounding: after tens of steps the two mixed runs differ by less than
-  1e-6 relative L2 (u and v against the norm of the velocity, p against its
-  own), and the window solver's run is no further from FP64 than the exact
-  solver's (within 10 %); on the cavity both are within 1e-6 of FP64.
+* Where every window is usable (dominance ratio <= 0.9 and rows 64 apart
+  coupled by at most 2^-24, the cavities and channels of the measured
+  workloads), the two FP32 solvers agree to FP32 rounding: after tens of steps
+  the two mixed runs differ by less than 1e-6 relative L2 (u and v against the
+  norm of the velocity, p against its own), and the window solver's run is no
+  further from FP64 than the exact solver's (within 10 %); on the cavity both
+  are within 1e-6 of FP64.
 * On random batches of chains the window solver agrees with an FP64 Thomas
   solve of the same matrices (first-row quirk included) to FP32 accuracy.
   Where a window is not dominant enough (ratio 0.95 against the solver's
@@ -200,3 +200,71 @@ def test_window_solver_falls_back_on_weakly_dominant_chains():
     a2, d2, c2, b2 = _chains(rng, 1, 200000, 0.5)
     assert not np.array_equal(_solve32(a2, d2, c2, b2, 0, 1, 200000, True),
                               _solve32(a2, d2, c2, b2, 0, 1, 200000, False))
+
+
+@pytest.mark.parametrize("side", ["sub", "super"])
+@pytest.mark.parametrize("ratio", [0.7, 0.77, 0.8, 0.85, 0.89])
+def test_window_solver_on_one_sided_chains(side, ratio):
+    """Rows coupled to one neighbour only, as upwinding leaves them where
+    convection dominates (ratio C / (1 + C) at a Courant number C), keep
+    ratio^k of a value k rows away.  x is within FP32 rounding of an FP64
+    solve whichever solver takes them: a row adds at most 4 roundings of 2^-24
+    to its neighbour's, which the recurrence sums to 1 / (1 - ratio) of that
+    (twice over: two sweeps)."""
+    rng = np.random.default_rng(int(1000 * ratio))
+    n = 50000
+    d = rng.uniform(1.0, 3.0, n)
+    off, zero = -ratio * d, np.zeros(n)
+    b = rng.uniform(0.5, 1.5, n) * d
+    a, d, c, b = (q.astype(np.float32) for q in ((off, d, zero, b) if side == "sub" else (zero, d, off, b)))
+    ref = _thomas64(a, d, c, b, n)
+    for shape in (128, 256, 512):
+        x = _solve32(a, d, c, b, 0, 1, n, shape)
+        e = (np.abs(x - ref) / np.abs(ref).max()).max()
+        print(f"  one-sided {side} {ratio} ({shape} lanes): {e:.1e}", flush=True)
+        assert e < 8 * 2.0 ** -24 / (1 - ratio)
+
+
+def test_window_solver_keeps_symmetric_rows_of_the_same_ratio():
+    """Ratio 0.89 coupled evenly to both neighbours decays by 0.61 a row: the
+    windows serve it (their bits are not the sequential solver's)."""
+    rng = np.random.default_rng(89)
+    n = 50000
+    d = rng.uniform(1.0, 3.0, n)
+    a, d, c, b = (q.astype(np.float32) for q in (-0.445 * d, d, -0.445 * d, rng.uniform(0.5, 1.5, n) * d))
+    ref = _thomas64(a, d, c, b, n)
+    xe = _solve32(a, d, c, b, 0, 1, n, 0)
+    for shape in (128, 256, 512):
+        x = _solve32(a, d, c, b, 0, 1, n, shape)
+        e = (np.abs(x - ref) / np.abs(ref).max()).max()
+        assert e < 8 * 2.0 ** -24 / (1 - 0.89)
+        assert not np.array_equal(x, xe)
+
+
+@pytest.mark.parametrize("courant", [2.0, 4.0, 6.0, 7.0])
+def test_mixed_first_iteration_of_a_convective_stream(courant):
+    """One q-l iteration (the step's result where mqiter is 1) of a noisy
+    diagonal stream, whose upwinded rows have about the ratio C / (1 + C) in
+    both splits.  The windows leave it no further from the FP64 path than
+    every chain solved whole does, but for the coupling they may drop: 2^-24
+    of the increment in each of the two splits, which their rows sum to
+    1 / (1 - ratio) of that."""
+    nx, ny = 80, 70
+    x, y = case.uniform_nodes(nx, ny, 1.0, (ny - 1) / (nx - 1))
+    g = case.compute_grid(x, y)
+    reg = case.cavity_regions(nx, ny)
+    # (a row's sub-diagonal is -u dt / h, its diagonal 1 + u dt / h)
+    prm = case.Params.from_physical(courant / (nx - 1), 1.0, 1e-6, nPpeSolver=5, msorit=3, mqiter=1)
+    rng = np.random.default_rng(8)
+    f = [1.0 + 0.005 * rng.uniform(-1, 1, (g.ncol, g.ld)) for _ in range(2)]
+    f.append(np.zeros_like(f[0]))
+    fw, _ = _run(g, reg, prm, "mixed", True, 1, f)
+    fe, _ = _run(g, reg, prm, "mixed", False, 1, f)
+    f64, _ = _run(g, reg, prm, "fp64", True, 1, f)
+    S = np.s_[2: ny, 2: nx]
+    ratio = 1.01 * courant / (1 + courant)
+    for k, name in enumerate("uv"):
+        inc = np.abs(f64[k][S] - f[k][S]).max()
+        ew, ee = (np.abs(q[k][S] - f64[k][S]).max() / inc for q in (fw, fe))
+        print(f"  stream C {courant} {name}: windows {ew:.1e}, whole chains {ee:.1e}", flush=True)
+        assert ew <= ee + 2 * 2.0 ** -24 / (1 - ratio), name

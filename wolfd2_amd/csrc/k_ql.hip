@@ -497,10 +497,10 @@ void launch_adj_window(long n, const Chains &cs, const Chain &h2, const Chain &h
 // both splits, in the compute type CT: float for the iterations after the
 // first; double for the first iteration of a step, whose solve is the whole
 // update from time level n and can be the step's result (the chains are the
-// same FP32 rows, so their solve is then at least as accurate as the
-// sequential FP32 sweep's).  A window whose dominance ratio exceeds TW_DOM in
-// either split sets *weak, which the fold turns into a repeat of the
-// iteration with the bit-exact solver.
+// same FP32 rows, and what a window drops is at most an FP32 rounding, so
+// their solve is as accurate as the sequential FP32 sweep's).  A window that
+// is not usable in either split (TW_DOM, TW_REACH) sets *weakf, which the fold
+// turns into a repeat of the iteration with the bit-exact solver.
 template <typename CT>
 __device__ inline CT qrcp(CT x) {
     if constexpr (std::is_same<CT, float>::value)
@@ -524,10 +524,11 @@ struct QwShared {
 };
 
 // The window's solution x from its rows (overwritten: x in b).  lo, hi: the
-// lanes of the window; the coupling out of them is dropped.
+// lanes of the window; the coupling out of them is dropped.  *weakf is set
+// where rows couple further than TW_REACH allows.
 template <typename CT, int NT>
 __device__ inline void qw_solve(CT (&a)[TW_S], CT (&d)[TW_S], CT (&c)[TW_S], CT (&b)[TW_S], int lo, int hi,
-                                QwShared<CT, NT> &S) {
+                                QwShared<CT, NT> &S, int *weakf) {
     constexpr int M = 2 * NT;
     const int t = threadIdx.x;
     if (t == lo) a[0] = CT(0);
@@ -572,7 +573,7 @@ __device__ inline void qw_solve(CT (&a)[TW_S], CT (&d)[TW_S], CT (&c)[TW_S], CT 
     __syncthreads();
     int cur = 0;
     for (int h = 1; h < M; h <<= 1) {
-        bool coupled = false;
+        bool coupled = false, far = false;
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             const int i = 2 * t + e;
@@ -596,7 +597,9 @@ __device__ inline void qw_solve(CT (&a)[TW_S], CT (&d)[TW_S], CT (&c)[TW_S], CT 
             S.b(cur ^ 1, i) = bn;
             S.q(cur ^ 1, i) = qrcp(dn);
             coupled |= !(fabs(an) + fabs(cn) <= qeps<CT>() * fabs(dn));
+            far |= !(fabs(an) + fabs(cn) <= CT(TW_REACH) * fabs(dn));
         }
+        if (h == TW_REACH_LEVEL && __any(far)) *weakf = 1;
         const int more = __syncthreads_or(coupled);
         cur ^= 1;
         if (!more) break;
@@ -657,7 +660,8 @@ __global__ __launch_bounds__(NT, sizeof(CT) == 4 ? 5 : 3) void k_ql_window(long 
     ql_load(h2.c, k2, n, 0.f, c2);
     const bool s7 = SKIND(kinds, TW_S - 1) == 1;
     bool weak = qw_rows<CT>(kinds, a, d, c, s7 ? (CT)h1.d[k0 + TW_S] : CT(1));
-    qw_solve<CT, NT>(a, d, c, b, 0, NT - 1, S);
+    if (__any(weak)) *weakf = 1;
+    qw_solve<CT, NT>(a, d, c, b, 0, NT - 1, S, weakf);
 #pragma unroll
     for (int s = 0; s < TW_S; s++) {
         a[s] = (CT)a2[s];
@@ -665,9 +669,9 @@ __global__ __launch_bounds__(NT, sizeof(CT) == 4 ? 5 : 3) void k_ql_window(long 
         c[s] = (CT)c2[s];
         if (!in2 || ((idm >> s) & 1u)) b[s] = CT(0);
     }
-    weak |= qw_rows<CT>(in2 ? kinds : 0u, a, d, c, in2 && s7 ? (CT)h2.d[k0 + TW_S] : CT(1));
+    weak = qw_rows<CT>(in2 ? kinds : 0u, a, d, c, in2 && s7 ? (CT)h2.d[k0 + TW_S] : CT(1));
     if (__any(weak)) *weakf = 1;
-    qw_solve<CT, NT>(a, d, c, b, HL, NT - 1 - HL, S);
+    qw_solve<CT, NT>(a, d, c, b, HL, NT - 1 - HL, S, weakf);
     CT *X = S.buf;
 #pragma unroll
     for (int s = 0; s < TW_S; s++) X[t * TR_P + s] = b[s];

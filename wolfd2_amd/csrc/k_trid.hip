@@ -456,11 +456,11 @@ __global__ __launch_bounds__(TRF_T) void k_trid_finish(long n, Chains cs, int nb
 // momentum chains are strongly diagonally dominant, so the coupling of a
 // row to rows far away decays geometrically.  Each workgroup solves a window
 // of TW_N rows with the coupling at the window's two edges dropped and keeps
-// the TW_O rows in its middle (TW_H rows from either edge): for a dominance
-// ratio (|a| + |c|) / |d| <= TW_DOM the dropped coupling changes the kept
-// rows by less than about 0.63^TW_H = 1e-13 relative.  The window system is
-// the chain's own matrix, with the first-row quirk (S(1,2) = c1 d1 / d2) and
-// no coupling across chain starts and ends.
+// the TW_O rows in its middle (TW_H rows from either edge); where rows TW_H
+// apart are coupled by at most TW_REACH, the dropped coupling changes the kept
+// rows by less than an FP32 rounding.  The window system is the chain's own
+// matrix, with the first-row quirk (S(1,2) = c1 d1 / d2) and no coupling
+// across chain starts and ends.
 //
 // Inside the window (partitioned Thomas + PCR): each thread holds TW_S rows
 // in registers and expresses its interior rows through its first and last
@@ -469,7 +469,8 @@ __global__ __launch_bounds__(TRF_T) void k_trid_finish(long n, Chains cs, int nb
 // parallel cyclic reduction in LDS solves it (each level l combines a row
 // with the rows 2^l away; at most log2(2 TW_T) levels, fewer once the
 // couplings left are negligible), and the interior rows follow from the
-// interface values.  A window whose dominance ratio exceeds TW_DOM clears
+// interface values.  A window whose rows are not dominant (a ratio
+// (|a| + |c|) / |d| above TW_DOM) or coupled too far (TW_REACH) clears
 // *keep, and the bit-exact speculative solver (launched after this kernel
 // with stop = keep) solves the chains instead.
 // Window shapes: TW_T lanes (128, 256 or 512: windows of 1024, 2048 or
@@ -585,7 +586,7 @@ __global__ __launch_bounds__(TW_T) void k_trid_window(long n, Chains cs, const T
     // dropped terms change x by less than TW_EPS times x 2^l segments away.
     int cur = 0;
     for (int h = 1; h < TW_M; h <<= 1) {
-        bool coupled = false;
+        bool coupled = false, far = false;
 #pragma unroll
         for (int e = 0; e < 2; e++) {
             const int i = 2 * t + e;
@@ -609,7 +610,9 @@ __global__ __launch_bounds__(TW_T) void k_trid_window(long n, Chains cs, const T
             rb[cur ^ 1][i] = bn;
             rq[cur ^ 1][i] = wrcp(dn);
             coupled |= !(fabsf(an) + fabsf(cn) <= TW_EPS * fabsf(dn));
+            far |= !(fabsf(an) + fabsf(cn) <= TW_REACH * fabsf(dn));
         }
+        if (h == TW_REACH_LEVEL && __any(far)) *keep = 0;
         const int more = __syncthreads_or(coupled);
         cur ^= 1;
         if (!more) break;

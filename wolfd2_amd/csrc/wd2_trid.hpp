@@ -170,6 +170,16 @@ struct TwShape {
 };
 constexpr float TW_DOM = 0.9f;
 constexpr float TW_EPS = 0x1p-48f;   // PCR stops once every coupling is below this share of its diagonal
+// A window is usable if its rows couple to those TW_H rows away by at most
+// this share of their diagonal, which PCR has at hand: its level h leaves the
+// interface rows, two a segment of TW_S, coupled to those 2 h interface rows
+// away.  A kept row's error is then at most 2^-24 of what was dropped, as one
+// FP32 rounding.  The rows' ratio (|a| + |c|) / |d| alone does not tell: at
+// 0.89 a value still weighs 0.61^64 = 2e-14 after 64 rows coupled evenly to
+// both sides, but 0.89^64 = 6e-4 after 64 upwinded rows, coupled to one.
+constexpr float TW_REACH = 0x1p-24f;
+constexpr int TW_REACH_LEVEL = TW_H / TW_S;
+static_assert((TW_REACH_LEVEL & (TW_REACH_LEVEL - 1)) == 0, "a PCR level spans the halo");
 
 // Hardware reciprocal (1 ulp) for the window solver, which need not round
 // like the reference.
