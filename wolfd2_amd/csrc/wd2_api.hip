@@ -82,8 +82,8 @@ struct wd2_ctx {
     double *t, *tn, *ts, *qh;      // temperature levels and the filter's copy
     // the q-l loop's other iterate buffers (an iteration's fused solve reads
     // us, vs and writes ua, va, or the reverse), the windows' maxima and
-    // checks, and the steps for which the loop keeps the separate solvers
-    // after a fused solve was not usable
+    // checks, and the steps left of the hold after a fused solve was not
+    // usable (ql_fused)
     double *ua, *va;
     double *ql_part = nullptr;
     int ql_hold = 0;
@@ -672,14 +672,17 @@ static void momentum_pair(wd2_ctx *c, double dk, double re, double fr, int m, do
         momentum_pair<double>(c, dk, re, fr, c->T, c->ch, c->ch2, c->tw, m, qtol, us, vs, uo, vo);
 }
 
-// Whether a q-l loop uses the fused solve and update: FP64 always (the same
-// bits), the mixed path unless its window solver is switched off -- and not
-// for the QL_HOLD steps after a step in which it was not usable (weakly
-// dominant chains, or runs that did not meet within the windows' halos): such
-// chains change slowly, and a repeat costs an iteration.
+// Whether a q-l loop uses the fused solve and update.  FP64: not for the
+// QL_HOLD steps after a step in which it was not usable (weakly dominant
+// chains, or runs that did not meet within the windows' halos), since such
+// chains change slowly and a repeat costs an iteration; both ways give the same
+// bits.  Mixed: they do not, so every step decides by its own chains (unless
+// the window solver is switched off) and its result depends on its fields
+// alone; during the hold steps are only kept from graph replays, which could
+// not repeat the iteration.
 constexpr int QL_HOLD = 16;
 static bool ql_fused(const wd2_ctx *c) {
-    return c->ql_hold == 0 && (c->precision != WD2_PREC_MIXED || g_window_chains);
+    return c->precision == WD2_PREC_MIXED ? g_window_chains : c->ql_hold == 0;
 }
 static void ql_step_done(wd2_ctx *c) {
     if (c->ql_hold > 0) c->ql_hold--;
@@ -1440,6 +1443,7 @@ int noalloc_trid_fallbacks();
 // are the same.  If a budget ran out before its test fired, the step is
 // restored from the copies the graph took first and redone host-driven.
 static bool graph_ok(const wd2_ctx *c, const wd2_params *P) {
+    if (c->precision == WD2_PREC_MIXED && g_window_chains && c->ql_hold > 0) return false;
     return c->graph_on && P->nPpeSolver == 7 && P->mqiter >= 1 && !c->any_porous && !c->any_blockage &&
            c->opt.nthermen != 1 && c->opt.neqstate != 1 && !c->d_live && c->kt_on == 0;
 }
@@ -2485,6 +2489,7 @@ int wd2_ctx_set_fields(wd2_ctx *c, int ld, const double *u, const double *v, con
     int st;
     if ((st = up(c, u, ld, c->u)) || (st = up(c, v, ld, c->v)) || (st = up(c, p, ld, c->p))) return st;
     c->p_hist = c->x_run = 0;
+    c->ql_hold = 0;
     HIPCHK(hipStreamSynchronize(c->s));
     return WD2_OK;
 }
