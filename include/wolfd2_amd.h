@@ -331,22 +331,24 @@ int wd2_ctx_ppe_divergence(wd2_ctx *ctx, double *last, double *max_since, int re
  * between launches); p is restored afterwards.  No counterpart in the
  * reference. */
 int wd2_ctx_mg_kernel_time(wd2_ctx *ctx, int which, int reps, double *avg_us);
-/* Mean time (microseconds) of the chain solver's forward (which = 1) or
- * backward (2) kernel, or of the mixed path's window kernel (3, mixed
- * precision only), over `reps` back-to-back launches on the context's
- * stream, on the first-split chains of the context's last q-l iteration (the
- * X and Y chains as one two-chain batch) in the context's precision.  The
- * chains are solved once more afterwards; fields are unchanged.  No
- * counterpart in the reference (measurement only). */
+/* Mean time (microseconds) of a chain solver's kernel over `reps` back-to-back
+ * launches on the context's stream, on the chains of the context's last q-l
+ * iteration (the X and Y chains as one two-chain batch) in the context's
+ * precision: the q-l loop's windows, both splits and the update in one kernel
+ * (which = 4; on the mixed path those of iterations 2.., and 5 those of the
+ * first, in FP64 arithmetic); and, on the first split's chains, the separate
+ * solver's forward (1) or backward (2) kernel, which the loop falls back to,
+ * or the window kernel of wd2_trid_f32 (3, mixed precision only).  Fields are
+ * unchanged.  No counterpart in the reference (measurement only). */
 int wd2_ctx_trid_kernel_time(wd2_ctx *ctx, int which, int reps, double *avg_us);
 /* The mixed path's window shape (no counterpart in the reference): the
  * lanes of one window's workgroup, 128, 256 (the default) or 512 -- windows
  * of 1024, 2048 or 4096 rows, at most 8, 9 or 10 parallel-cyclic-reduction
  * levels.  The shapes round differently (FP32 results differ in the last
- * bits).  wd2_ctx_trid_autotune times `reps` launches of each on the
- * chains of the context's last q-l iteration (mixed precision, after a
- * step), keeps the fastest and returns it and the three times (us[3], may
- * be NULL); wd2_ctx_trid_set_window sets one. */
+ * bits).  wd2_ctx_trid_autotune times `reps` launches of each (the q-l loop's
+ * windows, which = 4 above) on the chains of the context's last q-l iteration
+ * (mixed precision, after a step), keeps the fastest and returns it and the
+ * three times (us[3], may be NULL); wd2_ctx_trid_set_window sets one. */
 int wd2_ctx_trid_set_window(wd2_ctx *ctx, int window_threads);
 /* Multigrid Poisson solves (nPpeSolver 7) from an extrapolated initial guess
  * on the interior cells, from the pressures p^(n-1), p^(n-2) at the start of

@@ -185,6 +185,36 @@ def test_window_shape_autotune_on_the_cavity():
         assert rel_l2(a[S], b[S]) < 1e-6, name
 
 
+def test_window_shape_autotune_times_the_step_s_kernel():
+    """The shapes' times are those of the kernel that the q-l loop launches
+    (both splits and the update, 26 us here), not of the single split's
+    window solver (10 us), and timing leaves no trace in the run."""
+    g, reg, prm = workloads.cavity(1024, 1000.0, 2e-4, nPpeSolver=7, msorit=100, sortol=1e-8)
+    z = np.zeros((g.ncol, g.ld))
+    out = []
+    for tune in (True, False):
+        sol = api.Solver(g, reg, prm)
+        sol.set_precision("mixed")
+        sol.set_fields(z, z, z)
+        sol.cold_start()
+        sol.step(2)
+        if tune:
+            t = sol.trid_autotune(20)["us"]
+            for shape in (128, 256, 512):
+                sol.set_trid_window(shape)
+                one, step = sol.trid_kernel_time(3, 20), sol.trid_kernel_time(4, 20)
+                print(f"  {shape} lanes: autotune {t[shape]:.2f} us, q-l windows {step:.2f}, one split {one:.2f}, "
+                      f"first iteration {sol.trid_kernel_time(5, 20):.2f}", flush=True)
+                assert one < step
+                assert t[shape] > np.sqrt(one * step)
+            sol.set_trid_window(256)
+        tab = sol.step(2)
+        out.append((tab, *sol.get_fields()))
+        sol.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 def test_window_solver_falls_back_on_weakly_dominant_chains():
     """Dominance ratio 0.95 (above the window solver's 0.9) in one window of a
     long chain: the bit-exact FP32 solver solves the whole batch, so x equals

@@ -262,6 +262,13 @@ class Solver:
         check(lib().wd2_ctx_trid_autotune(self.ctx, reps, C.byref(wt), us))
         return {"window_threads": wt.value, "us": {128: us[0], 256: us[1], 512: us[2]}}
 
+    def trid_kernel_time(self, which: int, reps: int = 20) -> float:
+        """Mean microseconds of a chain solver's kernel on the last q-l
+        iteration's chains (wd2_ctx_trid_kernel_time; 4: the q-l windows)."""
+        us = C.c_double(0)
+        check(lib().wd2_ctx_trid_kernel_time(self.ctx, which, reps, C.byref(us)))
+        return us.value
+
     def set_trid_window(self, window_threads: int) -> None:
         check(lib().wd2_ctx_trid_set_window(self.ctx, window_threads))
 

@@ -1105,7 +1105,7 @@ __global__ __launch_bounds__(256) void k_ql_fold(int ld, const double *__restric
     }
 }
 
-__global__ void k_ql_reset(Scalars *sc) { sc->ql_stop = 0; }
+__global__ void k_ql_reset(Scalars *sc) { sc->ql_stop = sc->ql_weak = 0; }
 void launch_ql_reset(Scalars *sc, hipStream_t s) { hipLaunchKernelGGL(k_ql_reset, dim3(1), dim3(64), 0, s, sc); }
 
 template <typename T>

@@ -771,39 +771,64 @@ void launch_ql_commit(int nx, int ny, int ld, int Q, const Scalars *sc, const do
 size_t ql_pair_part(long n) { return 2 * (size_t)((n + 767) / 768); }
 size_t ql_pair_chk(long n) { return QX_CHK * (size_t)((n + QX_O - 1) / QX_O); }
 
-void launch_ql_pair(const QlPair<double> &q, long n, const Chains &cs, const ChainT<double> &h1,
-                    const ChainT<double> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m, hipStream_t s) {
+// Iteration m's windows; returns their number.
+static int ql_windows(const QlPair<double> &q, long n, const Chains &cs, const ChainT<double> &h1,
+                      const ChainT<double> &h2, const unsigned char *Z, Scalars *sc, int, hipStream_t s) {
     const QlFields F{q.nx, q.ny, q.ld, q.us, q.vs, q.uo, q.vo, q.dus, q.dvs};
     const int nw = (int)((n + QX_O - 1) / QX_O), nb = ql_border_blocks(q.nx, q.ny, QX_T);
     hipLaunchKernelGGL(k_ql_exact<double>, dim3(nw + nb), dim3(QX_T), 0, s, n, cs, h1, h2, Z, F, q.part, q.chk, nw,
                        &sc->ql_stop);
-    hipLaunchKernelGGL(k_ql_fold_win<double>, dim3(1), fold_lanes(nw), 0, s, q.ld, q.dus, q.dvs, q.part, nw,
-                       (const double *)q.chk, (int *)nullptr, sc, qtol, m);
+    return nw;
 }
-
 template <typename CT, int NT>
-static void ql_window_as(const QlPair<float> &q, long n, const Chains &cs, const ChainT<float> &h1,
-                         const ChainT<float> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m,
-                         hipStream_t s) {
+static int ql_windows_as(const QlPair<float> &q, long n, const Chains &cs, const ChainT<float> &h1,
+                         const ChainT<float> &h2, const unsigned char *Z, Scalars *sc, hipStream_t s) {
     constexpr int O = NT * TW_S - 4 * TW_H;
     const QlFields F{q.nx, q.ny, q.ld, q.us, q.vs, q.uo, q.vo, q.dus, q.dvs};
     const int nw = (int)((n + O - 1) / O), nb = ql_border_blocks(q.nx, q.ny, NT);
     hipLaunchKernelGGL((k_ql_window<CT, NT>), dim3(nw + nb), dim3(NT), 0, s, n, cs, h1, h2, Z, F, q.part, nw,
                        &sc->ql_weak, &sc->ql_stop);
+    return nw;
+}
+static int ql_windows(const QlPair<float> &q, long n, const Chains &cs, const ChainT<float> &h1,
+                      const ChainT<float> &h2, const unsigned char *Z, Scalars *sc, int m, hipStream_t s) {
+    if (m == 1) return ql_windows_as<double, 256>(q, n, cs, h1, h2, Z, sc, s);
+    switch (q.shape) {
+    case 128: return ql_windows_as<float, 128>(q, n, cs, h1, h2, Z, sc, s);
+    case 512: return ql_windows_as<float, 512>(q, n, cs, h1, h2, Z, sc, s);
+    default: return ql_windows_as<float, 256>(q, n, cs, h1, h2, Z, sc, s);
+    }
+}
+
+void launch_ql_pair(const QlPair<double> &q, long n, const Chains &cs, const ChainT<double> &h1,
+                    const ChainT<double> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m, hipStream_t s) {
+    const int nw = ql_windows(q, n, cs, h1, h2, Z, sc, m, s);
+    hipLaunchKernelGGL(k_ql_fold_win<double>, dim3(1), fold_lanes(nw), 0, s, q.ld, q.dus, q.dvs, q.part, nw,
+                       (const double *)q.chk, (int *)nullptr, sc, qtol, m);
+}
+
+void launch_ql_pair(const QlPair<float> &q, long n, const Chains &cs, const ChainT<float> &h1,
+                    const ChainT<float> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m, hipStream_t s) {
+    const int nw = ql_windows(q, n, cs, h1, h2, Z, sc, m, s);
     hipLaunchKernelGGL(k_ql_fold_win<float>, dim3(1), fold_lanes(nw), 0, s, q.ld, q.dus, q.dvs, q.part, nw,
                        (const float *)nullptr, &sc->ql_weak, sc, qtol, m);
 }
-void launch_ql_pair(const QlPair<float> &q, long n, const Chains &cs, const ChainT<float> &h1,
-                    const ChainT<float> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m, hipStream_t s) {
-    if (m == 1) {
-        ql_window_as<double, 256>(q, n, cs, h1, h2, Z, sc, qtol, m, s);
-        return;
-    }
-    switch (q.shape) {
-    case 128: ql_window_as<float, 128>(q, n, cs, h1, h2, Z, sc, qtol, m, s); break;
-    case 512: ql_window_as<float, 512>(q, n, cs, h1, h2, Z, sc, qtol, m, s); break;
-    default: ql_window_as<float, 256>(q, n, cs, h1, h2, Z, sc, qtol, m, s); break;
-    }
+
+template <typename T>
+void launch_ql_pair_bench(const QlPair<T> &q, long n, const Chains &cs, const ChainT<T> &h1, const ChainT<T> &h2,
+                          const unsigned char *Z, Scalars *sc, int m, int reps, hipStream_t s, hipEvent_t e0,
+                          hipEvent_t e1) {
+    launch_ql_reset(sc, s);   // the last loop's stop flag ends a window kernel at entry
+    (void)hipEventRecord(e0, s);
+    for (int k = 0; k < reps; k++) ql_windows(q, n, cs, h1, h2, Z, sc, m, s);
+    (void)hipEventRecord(e1, s);
+    launch_ql_reset(sc, s);
 }
+template void launch_ql_pair_bench<double>(const QlPair<double> &, long, const Chains &, const ChainT<double> &,
+                                           const ChainT<double> &, const unsigned char *, Scalars *, int, int,
+                                           hipStream_t, hipEvent_t, hipEvent_t);
+template void launch_ql_pair_bench<float>(const QlPair<float> &, long, const Chains &, const ChainT<float> &,
+                                          const ChainT<float> &, const unsigned char *, Scalars *, int, int,
+                                          hipStream_t, hipEvent_t, hipEvent_t);
 
 }  // namespace wd2

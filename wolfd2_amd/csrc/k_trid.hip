@@ -474,19 +474,15 @@ __global__ __launch_bounds__(TRF_T) void k_trid_finish(long n, Chains cs, int nb
 // *keep, and the bit-exact speculative solver (launched after this kernel
 // with stop = keep) solves the chains instead.
 // Window shapes: TW_T lanes (128, 256 or 512: windows of 1024, 2048 or
-// 4096 rows, at most 8, 9 or 10 PCR levels), chosen by
-// wd2_ctx_trid_autotune; 256 unless tuned.
+// 4096 rows, at most 8, 9 or 10 PCR levels).
 __global__ void k_trid_keep_set(int *keep) { *keep = 1; }
 
 template <typename T, int TW_T>
 __global__ __launch_bounds__(TW_T) void k_trid_window(long n, Chains cs, const T *__restrict__ A,
                                                       const T *__restrict__ D, const T *__restrict__ C,
-                                                      const T *__restrict__ B, T *__restrict__ X, T *__restrict__ B2,
-                                                      const unsigned char *__restrict__ Z, const int *stop,
-                                                      int *keep) {
+                                                      const T *__restrict__ B, T *__restrict__ X, int *keep) {
     static_assert(std::is_same<T, float>::value, "the window solver serves the FP32 chains");
     constexpr int TW_N = TwShape<TW_T>::N, TW_O = TwShape<TW_T>::O, TW_M = TwShape<TW_T>::M;
-    if (stop && *stop) return;
     // interface rows in LDS: sub- and super-diagonal, right-hand side and
     // the reciprocal of the diagonal (each row's diagonal stays with its thread)
     __shared__ T ra[2][TW_M], rc[2][TW_M], rb[2][TW_M], rq[2][TW_M];
@@ -626,63 +622,48 @@ __global__ __launch_bounds__(TW_T) void k_trid_window(long n, Chains cs, const T
     for (int s = 0; s < TW_S; s++) x[s] = s == 0 ? x0 : (s == TW_S - 1 ? x7 : y[s] + v[s] * x0 + w[s] * x7);
     const int len = (int)(n - k0 < TW_S ? n - k0 : TW_S);
     seg_store(X, k0, len, x);
-    if (B2) {
-        unsigned long long zb = 0;   // the segment's identity-row flags, one byte per row
-        if (Z) {
-            if (len == TW_S) {
-                zb = *reinterpret_cast<const unsigned long long *>(Z + k0);
-            } else {
-                for (int q = 0; q < len; q++) zb |= (unsigned long long)Z[k0 + q] << (8 * q);
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < TW_S; q++)
-            if ((zb >> (8 * q)) & 0xffu) x[q] = T(0);
-        seg_store(B2, k0, len, x);
-    }
 }
 
 template <typename T, int TW_T>
 static void launch_window_kernel(long n, const Chains &cs, const T *A, const T *D, const T *C, const T *B, T *X,
-                                 hipStream_t s, T *B2, const unsigned char *Z, const int *stop, int *keep) {
+                                 hipStream_t s, int *keep) {
     const unsigned nb = (unsigned)((n + TwShape<TW_T>::O - 1) / TwShape<TW_T>::O);
-    hipLaunchKernelGGL((k_trid_window<T, TW_T>), dim3(nb), dim3(TW_T), 0, s, n, cs, A, D, C, B, X, B2, Z, stop, keep);
+    hipLaunchKernelGGL((k_trid_window<T, TW_T>), dim3(nb), dim3(TW_T), 0, s, n, cs, A, D, C, B, X, keep);
 }
 template <typename T>
 static void launch_window_shape(int wt, long n, const Chains &cs, const T *A, const T *D, const T *C, const T *B,
-                                T *X, hipStream_t s, T *B2, const unsigned char *Z, const int *stop, int *keep) {
+                                T *X, hipStream_t s, int *keep) {
     if (wt == 128)
-        launch_window_kernel<T, 128>(n, cs, A, D, C, B, X, s, B2, Z, stop, keep);
+        launch_window_kernel<T, 128>(n, cs, A, D, C, B, X, s, keep);
     else if (wt == 512)
-        launch_window_kernel<T, 512>(n, cs, A, D, C, B, X, s, B2, Z, stop, keep);
+        launch_window_kernel<T, 512>(n, cs, A, D, C, B, X, s, keep);
     else
-        launch_window_kernel<T, 256>(n, cs, A, D, C, B, X, s, B2, Z, stop, keep);
+        launch_window_kernel<T, 256>(n, cs, A, D, C, B, X, s, keep);
 }
 int trid_window_shape_ok(int wt) { return wt == 128 || wt == 256 || wt == 512; }
 
 template <typename T>
 void launch_trid_window(const TridWorkT<T> &w, long n, const Chains &cs, const T *A, const T *D, const T *C,
-                        const T *B, T *X, hipStream_t s, T *B2, const unsigned char *Z, const int *stop, int wt) {
+                        const T *B, T *X, hipStream_t s, int wt) {
     // the solver's flag block: fail, nfallback, keep; keep is 1 between solves
     // (set at allocation, and again by each fallback solve that runs)
     int *keep = w.fail + 2;
-    launch_window_shape<T>(wt, n, cs, A, D, C, B, X, s, B2, Z, stop, keep);
-    // the bit-exact solver runs only where a window was too weakly dominant
-    // (keep cleared) and then sets keep again; it also returns at entry once
-    // the q-l loop has stopped, since then the window kernel left keep set
-    launch_trid<T>(w, n, cs, A, D, C, B, X, s, B2, Z, keep, keep);
+    launch_window_shape<T>(wt, n, cs, A, D, C, B, X, s, keep);
+    // the bit-exact solver runs only where a window was not usable (keep
+    // cleared) and then sets keep again
+    launch_trid<T>(w, n, cs, A, D, C, B, X, s, nullptr, nullptr, keep, keep);
 }
 void launch_trid_keep_init(int *fail_block, hipStream_t s) {
     hipLaunchKernelGGL(k_trid_keep_set, dim3(1), dim3(1), 0, s, fail_block + 2);
 }
 // reps back-to-back launches of the window kernel of shape wt between events
-// e0 and e1 (X written; no second right-hand side).
+// e0 and e1 (X written).
 template <typename T>
 void launch_trid_window_bench(const TridWorkT<T> &w, long n, const Chains &cs, const T *A, const T *D, const T *C,
                               const T *B, T *X, int reps, hipStream_t s, hipEvent_t e0, hipEvent_t e1, int wt) {
     int *keep = w.fail + 2;
     (void)hipEventRecord(e0, s);
-    for (int k = 0; k < reps; k++) launch_window_shape<T>(wt, n, cs, A, D, C, B, X, s, nullptr, nullptr, nullptr, keep);
+    for (int k = 0; k < reps; k++) launch_window_shape<T>(wt, n, cs, A, D, C, B, X, s, keep);
     (void)hipEventRecord(e1, s);
     // no fallback runs here: set keep again for the next solve
     hipLaunchKernelGGL(k_trid_keep_set, dim3(1), dim3(1), 0, s, keep);
@@ -691,8 +672,7 @@ template void launch_trid_window_bench<float>(const TridWorkT<float> &, long, co
                                               const float *, const float *, const float *, float *, int, hipStream_t,
                                               hipEvent_t, hipEvent_t, int);
 template void launch_trid_window<float>(const TridWorkT<float> &, long, const Chains &, const float *, const float *,
-                                        const float *, const float *, float *, hipStream_t, float *,
-                                        const unsigned char *, const int *, int);
+                                        const float *, const float *, float *, hipStream_t, int);
 
 int trid_blocks(long n) { return (int)((n + TR_R - 1) / TR_R); }
 

@@ -2354,8 +2354,7 @@ int wd2_trid_f32(long n, long n1, long L1, long L2, const float *a, const float 
     HIPCHK(hipMemcpyAsync(ch.b, b, n * 4, hipMemcpyHostToDevice, c->s));
     const Chains cs{n1, n1 > 0 ? L1 : L2, L2};
     if (window)
-        launch_trid_window<float>(c->twf, n, cs, ch.a, ch.d, ch.c, ch.b, ch.x, c->s, nullptr, nullptr, nullptr,
-                                  window == 1 ? 256 : window);
+        launch_trid_window<float>(c->twf, n, cs, ch.a, ch.d, ch.c, ch.b, ch.x, c->s, window == 1 ? 256 : window);
     else
         launch_trid<float>(c->twf, n, cs, ch.a, ch.d, ch.c, ch.b, ch.x, c->s);
     HIPCHK(hipMemcpyAsync(x, ch.x, n * 4, hipMemcpyDeviceToHost, c->s));
@@ -2735,11 +2734,28 @@ int wd2_ctx_mg_kernel_time(wd2_ctx *c, int which, int reps, double *avg_us) {
     return WD2_OK;
 }
 
+}   // extern "C"
+
+// `reps` launches of the windows of q-l iteration m (shape wt, mixed path) on
+// the context's last chains, between e[0] and e[1]; the iterate goes to the
+// loop's other buffers, the increments' places to the solvers' scratch fields.
+template <typename T>
+static void ql_bench(wd2_ctx *c, const ChainT<T> &ch, const ChainT<T> &ch2, int m, int wt, int reps, hipEvent_t *e) {
+    const long n1 = (long)c->nx * (c->ny - 1), n = n1 + (long)(c->nx - 1) * c->ny;
+    const QlPair<T> q{c->nx,   c->ny,    c->ld,      c->us, c->vs, c->ua, c->va, c->pscr,
+                      c->beff, c->ql_part, (T *)(c->ql_part + ql_pair_part(n)), wt};
+    launch_ql_pair_bench<T>(q, n, Chains{n1, n1, n - n1}, ch, ch2, c->zm, c->sc, m, reps, c->s, e[0], e[1]);
+}
+
+extern "C" {
+
 int wd2_ctx_trid_kernel_time(wd2_ctx *c, int which, int reps, double *avg_us) {
-    if (which < 1 || which > 3 || reps < 1)
-        return fail(WD2_ERR_ARG, "chain solver timing: which %d (1 forward, 2 backward, 3 window), reps %d", which,
-                    reps);
-    if (which == 3 && c->precision != WD2_PREC_MIXED)
+    if (which < 1 || which > 5 || reps < 1)
+        return fail(WD2_ERR_ARG,
+                    "chain solver timing: which %d (1 forward, 2 backward, 3 window, 4 and 5 q-l windows), reps %d",
+                    which, reps);
+    const bool mixed = c->precision == WD2_PREC_MIXED;
+    if ((which == 3 || which == 5) && !mixed)
         return fail(WD2_ERR_ARG, "chain solver timing: the window solver serves the mixed path only");
     if (c->any_porous) return fail(WD2_ERR_UNSUPPORTED, "chain solver timing: the two-chain batches only");
     const long n1 = (long)c->nx * (c->ny - 1), n2 = (long)(c->nx - 1) * c->ny;
@@ -2750,7 +2766,11 @@ int wd2_ctx_trid_kernel_time(wd2_ctx *c, int which, int reps, double *avg_us) {
     if (which == 3)
         launch_trid_window_bench<float>(c->twf, n1 + n2, cs, c->chf.a, c->chf.d, c->chf.c, c->chf.b, c->chf.x, reps,
                                         c->s, e[0], e[1], c->win_wt);
-    else if (c->precision == WD2_PREC_MIXED)
+    else if (which > 3 && mixed)
+        ql_bench<float>(c, c->chf, c->chf2, which == 5 ? 1 : 2, c->win_wt, reps, e);
+    else if (which > 3)
+        ql_bench<double>(c, c->ch, c->ch2, 2, 0, reps, e);
+    else if (mixed)
         launch_trid_kernel_bench<float>(c->twf, n1 + n2, cs, c->chf.a, c->chf.d, c->chf.c, c->chf.b, c->chf.x, which,
                                         reps, c->s, e[0], e[1]);
     else
@@ -2784,8 +2804,6 @@ int wd2_ctx_trid_autotune(wd2_ctx *c, int reps, int *wt_out, double *us_out) {
     if (!c || reps < 1) return fail(WD2_ERR_ARG, "window autotune: reps %d", reps);
     if (c->precision != WD2_PREC_MIXED) return fail(WD2_ERR_ARG, "window autotune: the mixed path only");
     if (c->any_porous) return fail(WD2_ERR_UNSUPPORTED, "window autotune: the two-chain batches only");
-    const long n1 = (long)c->nx * (c->ny - 1), n2 = (long)(c->nx - 1) * c->ny;
-    const Chains cs{n1, n1, n2};
     hipEvent_t e[2];
     HIPCHK(hipEventCreate(&e[0]));
     HIPCHK(hipEventCreate(&e[1]));
@@ -2794,10 +2812,8 @@ int wd2_ctx_trid_autotune(wd2_ctx *c, int reps, int *wt_out, double *us_out) {
     double tbest = 0.0;
     for (int q = 0; q < 3; q++) {
         // one launch first (code load, caches), then the timed ones
-        launch_trid_window_bench<float>(c->twf, n1 + n2, cs, c->chf.a, c->chf.d, c->chf.c, c->chf.b, c->chf.x, 1,
-                                        c->s, e[0], e[1], shapes[q]);
-        launch_trid_window_bench<float>(c->twf, n1 + n2, cs, c->chf.a, c->chf.d, c->chf.c, c->chf.b, c->chf.x, reps,
-                                        c->s, e[0], e[1], shapes[q]);
+        ql_bench<float>(c, c->chf, c->chf2, 2, shapes[q], 1, e);
+        ql_bench<float>(c, c->chf, c->chf2, 2, shapes[q], reps, e);
         HIPCHK(hipStreamSynchronize(c->s));
         float ms = 0.f;
         HIPCHK(hipEventElapsedTime(&ms, e[0], e[1]));

@@ -42,14 +42,12 @@ void launch_trid_keep_init(int *fail_block, hipStream_t s);
 
 // The mixed path's FP32 chain solve (not bit-exact): overlapping windows
 // solved by partitioned Thomas + PCR in LDS, the bit-exact solver as the
-// fallback for a window that is not diagonally dominant enough; same
-// arguments as launch_trid.
+// fallback for a window that is not usable; same arguments as launch_trid.
 // wt: the window shape, the lanes of one window's workgroup (128, 256 or
 // 512: windows of 1024, 2048 or 4096 rows).
 template <typename T>
 void launch_trid_window(const TridWorkT<T> &w, long n, const Chains &cs, const T *A, const T *D, const T *C,
-                        const T *B, T *X, hipStream_t s, T *B2, const unsigned char *Z, const int *stop,
-                        int wt = 256);
+                        const T *B, T *X, hipStream_t s, int wt = 256);
 template <typename T>
 void launch_trid_window_bench(const TridWorkT<T> &w, long n, const Chains &cs, const T *A, const T *D, const T *C,
                               const T *B, T *X, int reps, hipStream_t s, hipEvent_t e0, hipEvent_t e1, int wt = 256);
@@ -232,6 +230,13 @@ void launch_ql_pair(const QlPair<double> &q, long n, const Chains &cs, const Cha
                     const ChainT<double> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m, hipStream_t s);
 void launch_ql_pair(const QlPair<float> &q, long n, const Chains &cs, const ChainT<float> &h1,
                     const ChainT<float> &h2, const unsigned char *Z, Scalars *sc, double qtol, int m, hipStream_t s);
+// reps back-to-back launches of iteration m's solve and update without the
+// fold, between events e0 and e1, on (us, vs) -> (uo, vo); leaves ql_stop and
+// ql_weak clear.
+template <typename T>
+void launch_ql_pair_bench(const QlPair<T> &q, long n, const Chains &cs, const ChainT<T> &h1, const ChainT<T> &h2,
+                          const unsigned char *Z, Scalars *sc, int m, int reps, hipStream_t s, hipEvent_t e0,
+                          hipEvent_t e1);
 // us, vs = ua, va if the last of Q captured iterations that ran was odd.
 void launch_ql_commit(int nx, int ny, int ld, int Q, const Scalars *sc, const double *ua, const double *va, double *us,
                       double *vs, hipStream_t s);
@@ -288,7 +293,7 @@ void launch_update_norms(int nx, int ny, int ld, double *us, double *vs, const d
 template <typename T>
 void launch_scatter_update(int nx, int ny, int ld, const T *x1, const T *x2, double *us, double *vs, double *dus,
                            double *dvs, double *partials, Scalars *sc, double qtol, int m, hipStream_t s);
-// sc->ql_stop = 0 (a kernel, not a memset).
+// sc->ql_stop = sc->ql_weak = 0 (a kernel, not a memset).
 void launch_ql_reset(Scalars *sc, hipStream_t s);
 
 // Thermal energy (k_thermal.hip).  err receives 2000+side for a bad
