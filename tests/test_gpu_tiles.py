@@ -162,6 +162,34 @@ def test_mg_bottom_widths_agree(n):
         assert np.abs(a[S] - b[S]).max() <= 1e-6 * np.abs(b[S]).max(), name
 
 
+@pytest.mark.parametrize("first,other", [("fp64", "mixed"), ("mixed", "fp64")])
+def test_mg_shape_set_between_precisions(first, other):
+    """A bottom width set while the context's precision is not that of the
+    levels' coefficients: the next solve in their precision runs them in its
+    own shape, with the bits of a run that set nothing."""
+    g, reg, prm = workloads.cavity(128, 1000.0, 2e-4, nPpeSolver=7, msorit=100, sortol=1e-10)
+    out = []
+    for change in (True, False):
+        sol = api.Solver(g, reg, prm)
+        sol.set_precision(first)
+        sol.set_mg_tune(256, 0, 64)
+        z = np.zeros((g.ncol, g.ld))
+        sol.set_fields(z, z, z)
+        sol.cold_start()
+        sol.step(2)
+        f = sol.get_fields()
+        if change:
+            sol.set_precision(other)
+            sol.set_mg_tune(256, 0, 64)
+            assert lib().wd2_ctx_mg_kernel_time(sol.ctx, 4, 2, C.byref(C.c_double(0))) == 0
+            sol.set_precision(first)
+        sol.set_fields(*f)
+        out.append((np.asarray(sol.step(2)), *sol.get_fields()))
+        sol.close()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("nx,ny,dt,lid", [(65, 33, 2e-3, 1.0), (73, 41, 2e-3, 1.0), (65, 33, 0.022, 0.05)])
 def test_adjoint_tiles_dot_product(nx, ny, dt, lid):
     """<w, J d> = <J^T w, d> between the tangent-linear pass and the adjoint,

@@ -785,10 +785,11 @@ static int naux_momentum(wd2_ctx *c, int mqiter, double dk, double re, double fr
 // ------------------------------------------------------------------- Ppe
 // The levels at most tune.bside cells wide (and at most mg_bottom_side), or of
 // at most mg_tail_cells() cells, go to the bottom kernel; level 0 is always
-// tiled.
-static int mg_retile(wd2_ctx *c) {
+// tiled.  prec: the arithmetic of the levels' coefficients, whose kernels will
+// run them (the context's own may have changed since they were built).
+static int mg_retile(wd2_ctx *c, int prec) {
     MgHierarchy &H = c->mg;
-    const int side = std::min(H.tune.bside, mg_bottom_side(c->precision == WD2_PREC_MIXED));
+    const int side = std::min(H.tune.bside, mg_bottom_side(prec == WD2_PREC_MIXED));
     H.ntiled = 1;
     while (H.ntiled < H.nlev && std::max(H.lev[H.ntiled].nx, H.lev[H.ntiled].ny) > side &&
            H.lev[H.ntiled].nx * H.lev[H.ntiled].ny > mg_tail_cells())
@@ -819,7 +820,7 @@ static int mg_setup(wd2_ctx *c) {
         NY = (NY + 1) / 2;
     }
     H.tune = MgTune{256, 0, 64};
-    int st = mg_retile(c);
+    int st = mg_retile(c, c->precision);
     if (st) return st;
     const size_t tail = total;
     total += mg_tail_bytes() / sizeof(double);
@@ -852,7 +853,7 @@ static int mg_prepare(wd2_ctx *c) {
         // float and double views share the storage: clear it (zero rings)
         if (c->mg_prec != -1 && c->mg_prec != c->precision)
             HIPCHK(hipMemsetAsync(c->mg_store, 0, c->mg_bytes, c->s));
-        if ((st = mg_retile(c))) return st;   // the bottom's widest level depends on the precision
+        if ((st = mg_retile(c, c->precision))) return st;   // the bottom's widest level depends on it
         if (c->precision == WD2_PREC_MIXED)
             launch_mg_coef<float>(c->mg, c->nx, c->ny, c->ld, c->M.rau, c->M.rgv, uni, c->s);
         else
@@ -2657,10 +2658,11 @@ int wd2_ctx_mg_set_tune(wd2_ctx *c, int nt0, int stage, int bside) {
     if (st) return st;
     graph_clear(c);
     const MgTune old = c->mg.tune;
+    const int prec = c->mg_prec >= 0 ? c->mg_prec : c->precision;
     c->mg.tune = MgTune{nt0, stage, bside};
-    if ((st = mg_retile(c))) {
+    if ((st = mg_retile(c, prec))) {
         c->mg.tune = old;
-        (void)mg_retile(c);
+        (void)mg_retile(c, prec);
         return st;
     }
     return WD2_OK;
@@ -2692,7 +2694,7 @@ int wd2_ctx_mg_autotune(wd2_ctx *c, double dk, int cycles, double *best_us) {
     bool have = false;
     for (int bside : {32, 64}) {
         c->mg.tune.bside = bside;
-        if (mg_retile(c)) continue;
+        if (mg_retile(c, c->precision)) continue;
         double us = 0.0;
         (void)mg_cycle_time(c, 1, dk, &us);   // warm
         if ((st = mg_cycle_time(c, cycles, dk, &us))) return st;
@@ -2703,7 +2705,7 @@ int wd2_ctx_mg_autotune(wd2_ctx *c, double dk, int cycles, double *best_us) {
         }
     }
     c->mg.tune = best;
-    if ((st = mg_retile(c))) return st;
+    if ((st = mg_retile(c, c->precision))) return st;
     if (best_us) *best_us = tbest;
     return WD2_OK;
 }
