@@ -368,14 +368,15 @@ int wd2_ctx_set_mg_extrapolation(wd2_ctx *ctx, int order);
 int wd2_ctx_trid_autotune(wd2_ctx *ctx, int reps, int *window_threads, double *us);
 /* Kernel shapes of the multigrid solver (no counterpart in the reference):
  * bside the widest level the one-workgroup bottom kernel takes (32 or 64; the
- * FP64 path's takes at most 32).  nt0 (256 or 512) and stage (0 or 1) are
- * checked and kept for wd2_ctx_mg_get_tune; the level-0 kernels have one
- * shape. */
+ * FP64 path's takes at most 32, and wd2_ctx_mg_get_tune then returns 32).  nt0
+ * (256 or 512) and stage (0 or 1) select nothing any more: they are checked
+ * and returned as set; the level-0 kernels have one shape. */
 int wd2_ctx_mg_set_tune(wd2_ctx *ctx, int nt0, int stage, int bside);
 int wd2_ctx_mg_get_tune(wd2_ctx *ctx, int *nt0, int *stage, int *bside);
-/* Autotuner: times `cycles` full V-cycles with each bside on the
- * context's grid, precision and current right-hand side (p is restored),
- * keeps the fastest and returns its time per V-cycle in *best_us. */
+/* Autotuner: times `cycles` full V-cycles with each bside that the context's
+ * precision distinguishes on the context's grid and current right-hand side (p
+ * is restored), keeps the fastest and returns its time per V-cycle in
+ * *best_us. */
 int wd2_ctx_mg_autotune(wd2_ctx *ctx, double dk, int cycles, double *best_us);
 /* hipGraph steps (no counterpart in the reference).  enable != 0: each
  * time step of a context on the multigrid path (nPpeSolver 7, no porous

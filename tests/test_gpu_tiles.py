@@ -162,6 +162,24 @@ def test_mg_bottom_widths_agree(n):
         assert np.abs(a[S] - b[S]).max() <= 1e-6 * np.abs(b[S]).max(), name
 
 
+def test_mg_tune_reports_the_width_that_runs():
+    """The FP64 path's bottom kernel holds 32 cells a side, and tuning FP64
+    leaves the mixed path's width as it was set."""
+    g, reg, prm = workloads.cavity(128, 1000.0, 2e-4, nPpeSolver=7, msorit=100, sortol=1e-10)
+    sol = api.Solver(g, reg, prm)
+    z = np.zeros((g.ncol, g.ld))
+    sol.set_fields(z, z, z)
+    for bside in (32, 64):
+        sol.set_mg_tune(256, 0, bside)
+        assert sol.mg_tune()["bside"] == 32
+        assert sol.mg_autotune()["bside"] == 32
+        sol.set_precision("mixed")
+        assert sol.mg_tune()["bside"] == bside
+        assert sol.mg_autotune()["bside"] in (32, 64)
+        sol.set_precision("fp64")
+    sol.close()
+
+
 @pytest.mark.parametrize("first,other", [("fp64", "mixed"), ("mixed", "fp64")])
 def test_mg_shape_set_between_precisions(first, other):
     """A bottom width set while the context's precision is not that of the

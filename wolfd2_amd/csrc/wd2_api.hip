@@ -2673,7 +2673,7 @@ int wd2_ctx_mg_get_tune(wd2_ctx *c, int *nt0, int *stage, int *bside) {
     if (st) return st;
     if (nt0) *nt0 = c->mg.tune.nt0;
     if (stage) *stage = c->mg.tune.stage;
-    if (bside) *bside = c->mg.tune.bside;
+    if (bside) *bside = std::min(c->mg.tune.bside, mg_bottom_side(c->precision == WD2_PREC_MIXED));
     return WD2_OK;
 }
 
@@ -2692,7 +2692,9 @@ int wd2_ctx_mg_autotune(wd2_ctx *c, double dk, int cycles, double *best_us) {
     MgTune best = c->mg.tune;
     double tbest = 0.0;
     bool have = false;
+    const bool one = mg_bottom_side(c->precision == WD2_PREC_MIXED) == 32;   // both widths are the same shape
     for (int bside : {32, 64}) {
+        if (one && bside != best.bside) continue;
         c->mg.tune.bside = bside;
         if (mg_retile(c, c->precision)) continue;
         double us = 0.0;
