@@ -389,6 +389,11 @@ int wd2_ctx_mg_autotune(wd2_ctx *ctx, double dk, int cycles, double *best_us);
  * wd2_ctx_graph_stats: steps replayed and steps redone so far. */
 int wd2_ctx_set_graph(wd2_ctx *ctx, int enable);
 int wd2_ctx_graph_stats(wd2_ctx *ctx, long *steps, long *redos);
+/* Steps so far whose q-l loops began on windows of chain rows (*loops), and
+ * those of them that left the windows for the whole chains (*repeats), where
+ * rows couple further than the windows overlap.  Either pointer may be NULL.
+ * No counterpart in the reference. */
+int wd2_ctx_ql_stats(wd2_ctx *ctx, long *loops, long *repeats);
 
 /* An ensemble of independent contexts (any sizes) advanced together (no
  * counterpart in the reference, which runs one case per process,
@@ -446,6 +451,10 @@ typedef struct {
     double ms_reverse;       /* backward pass: the adjoint steps */
 } wd2_adj_stats;
 int wd2_adj_create(wd2_adj **adj, wd2_ctx *ctx, int checkpoint_every);
+/* Steps of the backward passes so far whose adjoint q-l iterations ran on
+ * windows of chain rows (*windows) and on the whole chains (*chains, where
+ * rows couple too far).  Either pointer may be NULL. */
+int wd2_adj_window_stats(wd2_adj *adj, long *windows, long *chains);
 int wd2_adj_destroy(wd2_adj *adj);
 /* fixed_point_tol: the adjoint q-l loop stops when max|update| <= tol *
  * max|nu| (default 1e-12, at most max_iter iterations, default 200);

@@ -38,6 +38,7 @@ def _step_bitwise(oracle, g, prm, seed):
     sol.set_fields(*f)
     tg = sol.step(1)
     out = sol.get_fields()
+    stats = sol.ql_stats()
     sol.close()
     ref = [a.copy() for a in f]
     to = oracle.run(reg, g, prm, *ref, 1)
@@ -45,6 +46,7 @@ def _step_bitwise(oracle, g, prm, seed):
     S = np.s_[: g.ny + 2, : g.nx + 2]
     for name, a, b in zip("uvp", out, ref):
         assert np.array_equal(a[S], b[S], equal_nan=True), name
+    return stats
 
 
 @pytest.mark.parametrize("kind", ["uniform", "stretched"])
@@ -55,17 +57,18 @@ def test_momentum_tiles_bitwise_vs_oracle(oracle, kind, nx, ny):
     _step_bitwise(oracle, _grid(kind, nx, ny), prm, nx)
 
 
-@pytest.mark.parametrize("dt", [1e-3, 1e-2, 50.0])
-def test_chain_windows_of_weakly_dominant_rows(oracle, dt):
+@pytest.mark.parametrize("dt,repeats", [(1e-4, 0), (1e-3, 1), (1e-2, 1), (50.0, 1)])
+def test_chain_windows_of_weakly_dominant_rows(oracle, dt, repeats):
     """From strong dominance to rows whose coupling outlasts the windows'
     halos, where the iteration is repeated on the whole chains."""
     print(f"chain windows dt {dt}", flush=True)
     prm = case.Params.from_physical(dt, 1.0, 1.0, nPpeSolver=5, msorit=3, mqiter=3)
-    _step_bitwise(oracle, _grid("uniform", 90, 70), prm, 11)
+    stats = _step_bitwise(oracle, _grid("uniform", 90, 70), prm, 11)
+    assert stats == {"loops": 1, "repeats": repeats}
 
 
-@pytest.mark.parametrize("dt", [1e-3, 50.0])
-def test_mixed_chain_windows_against_the_whole_chains(dt):
+@pytest.mark.parametrize("dt,repeats", [(1e-4, 0), (1e-3, 1), (50.0, 1)])
+def test_mixed_chain_windows_against_the_whole_chains(dt, repeats):
     """FP32 windows (and their repeat) against the bit-exact FP32 chains: the
     two differ by FP32 rounding of the iterates, 2^-24 times what three
     unconverged iterations amplify it by (10^2)."""
@@ -81,6 +84,7 @@ def test_mixed_chain_windows_against_the_whole_chains(dt):
             sol.set_fields(*_state(g, 12))
             sol.step(1)
             out.append(sol.get_fields())
+            assert sol.ql_stats() == {"loops": win, "repeats": win * repeats}
             sol.close()
         finally:
             lib().wd2_set_window_chains(old)
@@ -112,6 +116,7 @@ def test_mixed_steps_do_not_depend_on_earlier_runs(graph):
         tab = sol.step(4)
         out.append((np.asarray(tab), *sol.get_fields()))
         if weak_first:
+            assert sol.ql_stats()["repeats"] >= 2   # the first run's steps
             assert (sol.graph_stats()["replayed"] > 0) == graph
         sol.close()
     S = np.s_[: g.ny + 2, : g.nx + 2]
@@ -137,16 +142,18 @@ def test_mg_tile_edges_against_the_sparse_solution(oracle, ncx, ncy):
     assert err < 1e-10
 
 
-@pytest.mark.parametrize("n", [64, 96, 128])
+@pytest.mark.parametrize("n", [80, 96, 128])
 def test_mg_bottom_widths_agree(n):
-    """The bottom kernel from 32 or from 64 cells a side: both V-cycles reach
-    the same solution to the solve's own tolerance."""
+    """The bottom kernel from 32 or from 64 cells a side (a first coarse level
+    of 40 to 64 is a tile launch or the bottom's own): both V-cycles reach the same
+    solution to the solve's own tolerance."""
     g, reg, prm = workloads.cavity(n, 1000.0, 2e-4, nPpeSolver=7, msorit=100, sortol=1e-10)
     out = []
     for bside in (32, 64):
         sol = api.Solver(g, reg, prm)
         sol.set_precision("mixed")
         check(lib().wd2_ctx_mg_set_tune(sol.ctx, 512, 1, bside))
+        assert sol.mg_tune()["bside"] == bside
         z = np.zeros((g.ncol, g.ld))
         sol.set_fields(z, z, z)
         sol.cold_start()
@@ -234,6 +241,8 @@ def test_adjoint_tiles_dot_product(nx, ny, dt, lid):
     tab = adj.forward(2)
     assert np.all(tab[:, 0] > 0)
     r = adj.backward(*w)
+    whole = 2 if lid < 1 else 0   # of its two steps
+    assert adj.window_stats() == {"windows": 2 - whole, "chains": whole}
     t = adj.tangent(*d, np.zeros((4, 2, max(nx, ny) + 2)))
     assert r["stats"]["adj_unconverged"] == 0 and t["stats"]["adj_unconverged"] == 0
     tl = sum(float(np.sum(a * t[k])) for a, k in zip(w, ("duN", "dvN", "dpN")))

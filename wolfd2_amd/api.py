@@ -238,6 +238,13 @@ class Solver:
         check(lib().wd2_ctx_graph_stats(self.ctx, C.byref(a), C.byref(b)))
         return {"replayed": a.value, "redone": b.value}
 
+    def ql_stats(self) -> dict:
+        """Steps whose q-l loops began on the windows, and those that left them
+        for the whole chains (wd2_ctx_ql_stats)."""
+        a, b = C.c_long(), C.c_long()
+        check(lib().wd2_ctx_ql_stats(self.ctx, C.byref(a), C.byref(b)))
+        return {"loops": a.value, "repeats": b.value}
+
     def mg_autotune(self, cycles: int = 5) -> dict:
         """Pick the multigrid solver's fastest kernel shapes for this grid and
         precision (wd2_ctx_mg_autotune); returns the shape and its V-cycle time."""
@@ -388,6 +395,13 @@ class Adjoint:
     def set_tolerances(self, fixed_point_tol: float = 0.0, max_iter: int = 0, poisson_tol: float = 0.0) -> None:
         check(lib().wd2_adj_set_tolerances(self.adj, C.c_double(fixed_point_tol), max_iter,
                                            C.c_double(poisson_tol)))
+
+    def window_stats(self) -> dict:
+        """Steps of the backward passes on windows of chain rows and on the
+        whole chains (wd2_adj_window_stats)."""
+        a, b = C.c_long(), C.c_long()
+        check(lib().wd2_adj_window_stats(self.adj, C.byref(a), C.byref(b)))
+        return {"windows": a.value, "chains": b.value}
 
     def forward(self, nsteps: int) -> np.ndarray:
         """Advance nsteps with checkpoints; rows (ql_iter, ppe_iter)."""

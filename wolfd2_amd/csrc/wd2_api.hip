@@ -87,6 +87,7 @@ struct wd2_ctx {
     double *ua, *va;
     double *ql_part = nullptr;
     int ql_hold = 0;
+    long ql_loops = 0, ql_repeats = 0;   // q-l loops begun on the windows, those that left them
     // ThermEnergy's face coefficients: buffers of their own, since the mixed
     // path's FP32 momentum temporaries alias the FP64 ones and read the
     // entries they never write as zero
@@ -178,6 +179,7 @@ struct wd2_ctx {
     int mg_minc = 0;
     double *phist = nullptr;
     int p_hist = 0, xw = 0, x_run = 0, g_x = 0;
+    bool g_fused = false;   // the queued graph step's q-l solver
     std::vector<GraphEntry> graphs;
     double *gsave = nullptr;
     Scalars *h_sc = nullptr;
@@ -717,6 +719,7 @@ static int naux_momentum(wd2_ctx *c, int mqiter, double dk, double re, double fr
         // fused iterations alternate between (us, vs) and (ua, va): iteration
         // m reads buffer (m - 1) % 2
         bool fused = ql_fused(c);
+        c->ql_loops += fused;
         double *const ub[2] = {c->us, c->ua}, *const vb[2] = {c->vs, c->va};
         bool filled = false;   // iteration m's outflow fills are already applied
         int m = 1, last = 0;   // last: the iteration whose test was read last
@@ -752,6 +755,7 @@ static int naux_momentum(wd2_ctx *c, int mqiter, double dk, double re, double fr
             fused = false;
             filled = true;
             c->ql_hold = QL_HOLD + 1;   // this step included
+            c->ql_repeats++;
             m = last - 1;
             last = m;
         }
@@ -1546,6 +1550,7 @@ static int graph_begin(wd2_ctx *c, const wd2_params *P) {
     c->g_q = Q;
     c->g_c = C;
     c->g_x = xp;
+    c->g_fused = fused;
     return WD2_OK;
 }
 
@@ -1571,6 +1576,7 @@ static int graph_end(wd2_ctx *c, const wd2_params *P, int *nql, int *nsor, doubl
     std::swap(c->u, c->us);
     std::swap(c->v, c->vs);
     extrap_advance(c, c->g_x);
+    c->ql_loops += c->g_fused;
     ql_step_done(c);
     *nql = h.ql_stop ? h.ql_stop : -1;
     int nconv = h.mg_nconv;
@@ -1651,6 +1657,7 @@ struct wd2_adj {
     hipEvent_t ev[3] = {nullptr, nullptr, nullptr};
     hipEvent_t qev[2] = {nullptr, nullptr};
     wd2_adj_stats st{};
+    long win_steps = 0, chain_steps = 0;   // steps of the backward passes by their chain solver
 };
 
 static void adj_free(wd2_adj *a) {
@@ -1825,6 +1832,7 @@ static int adj_step(wd2_adj *a, const double *un, const double *vn, const double
     double dom;
     std::memcpy(&dom, &a->h_red[4], sizeof(double));
     const bool win = dom <= adj_window_dominance();   // false for a NaN
+    (win ? a->win_steps : a->chain_steps)++;
     const int nwin = adj_windows(n);
     const Chain t1{a->At1, a->Dt1, a->Ct1, nullptr, nullptr}, t2c{a->At2, a->Dt2, a->Ct2, nullptr, nullptr};
     auto converged = [&](int m) {
@@ -2847,6 +2855,13 @@ int wd2_ctx_graph_stats(wd2_ctx *c, long *steps, long *redos) {
     return WD2_OK;
 }
 
+int wd2_ctx_ql_stats(wd2_ctx *c, long *loops, long *repeats) {
+    if (!c) return fail(WD2_ERR_ARG, "wd2_ctx_ql_stats: null context");
+    if (loops) *loops = c->ql_loops;
+    if (repeats) *repeats = c->ql_repeats;
+    return WD2_OK;
+}
+
 // ------------------------------------------------------------ ensembles
 struct wd2_ens {
     std::vector<wd2_ctx *> m;
@@ -2950,6 +2965,13 @@ int wd2_adj_create(wd2_adj **out, wd2_ctx *c, int every) {
 
 int wd2_adj_destroy(wd2_adj *a) {
     adj_free(a);
+    return WD2_OK;
+}
+
+int wd2_adj_window_stats(wd2_adj *a, long *windows, long *chains) {
+    if (!a) return fail(WD2_ERR_ARG, "wd2_adj_window_stats: null adjoint");
+    if (windows) *windows = a->win_steps;
+    if (chains) *chains = a->chain_steps;
     return WD2_OK;
 }
 
