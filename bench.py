@@ -177,13 +177,14 @@ def run_path(sol, precision: str, solver: str, fields0, warmup: int, steps: int,
     # shapes round differently, so this comes before the state is recorded)
     wtune = sol.trid_autotune(20) if (precision == "mixed" and warmup) else None
     warm = sol.get_fields()
-    fb0 = L.wd2_trid_fallbacks()
+    fb0, rp0 = L.wd2_trid_fallbacks(), sol.ql_stats()["repeats"]
     L.wd2_ctx_ppe_divergence(sol.ctx, None, None, 1)
     t0 = time.perf_counter()
     tab = sol.step(steps)                 # returns after a device synchronisation
     secs = time.perf_counter() - t0
     div_max = C.c_double(0)
     L.wd2_ctx_ppe_divergence(sol.ctx, None, C.byref(div_max), 1)
+    repeats = sol.ql_stats()["repeats"] - rp0
     fields = sol.get_fields()
     s = 4.0 if precision == "mixed" else 8.0
     roof = {}
@@ -201,26 +202,30 @@ def run_path(sol, precision: str, solver: str, fields0, warmup: int, steps: int,
             us = C.c_double(0)
             L.wd2_ctx_mg_kernel_time(sol.ctx, which, reps, C.byref(us))
             us_cycle, nl = _kernel_time(sol, which, 2)
-            kern = f"k_mg_{name}<{t}, level 0> (2 red-black Gauss-Seidel sweeps on LDS tiles, FP64 pressure)"
+            kern = f"k_mg_{name}<{t}, level 0> (2 red-black Gauss-Seidel sweeps on tiles in registers, FP64 pressure)"
             roof[name] = _roofline(kern, bpl, us.value, reps,
                                    _traffic(f"k_mg_{name}_{precision}_cavity1024_traffic.json"))
             roof[name]["avg_launch_us_in_cycles"] = round(us_cycle, 3)
-        # the chain solver: the forward kernel reads a, d, c, b and writes the
-        # swept super-diagonal and right-hand side (4s in, 2s out per row);
-        # the backward kernel reads those two and writes x (2s in, s out);
-        # rows: the X and Y chains of one q-l iteration as one batch
+        # the chain solves; rows: the X and Y chains of one q-l iteration as
+        # one batch.  The windows, both splits and the update in one kernel,
+        # are what a step runs: both matrices and the first right-hand side
+        # (7s), the identity-row flag, us or vs read and written (the overlap
+        # of the windows is extra traffic).  The separate solver, which the
+        # loop falls back to: its forward kernel reads a, d, c, b and writes
+        # the swept super-diagonal and right-hand side (4s in, 2s out), its
+        # backward kernel reads those two and writes x (2s in, s out).
         rows = sol.g.nx * (sol.g.ny - 1) + (sol.g.nx - 1) * sol.g.ny
-        kinds = [(1, "trid_fwd", 6.0), (2, "trid_bwd", 3.0)]
+        win = "k_ql_window<float>" if precision == "mixed" else "k_ql_exact<double>"
+        kinds = [(4, "ql_windows", f"{win} (chain windows, both splits and the update of a q-l iteration", 7 * s + 17),
+                 (1, "trid_fwd", f"k_trid_fwd<{t}> (parallel AltTridLU, the q-l loop's fallback", 6 * s),
+                 (2, "trid_bwd", f"k_trid_bwd<{t}> (parallel AltTridLU, the q-l loop's fallback", 3 * s)]
         if precision == "mixed":
-            # the mixed path's window solver: a, d, c, b read and x written
-            # per owned row (5s; the overlap of the windows is extra traffic)
-            kinds.append((3, "trid_window", 5.0))
-        for which, name, per in kinds:
+            kinds.append((5, "ql_windows_first", "k_ql_window<double> (the same in a step's first q-l iteration",
+                          7 * s + 17))
+        for which, name, what, per in kinds:
             us = C.c_double(0)
             L.wd2_ctx_trid_kernel_time(sol.ctx, which, reps, C.byref(us))
-            kern = (f"k_{name}<{t}> (" + ("windowed partitioned Thomas + PCR" if which == 3 else "parallel AltTridLU")
-                    + f", {rows} rows: the X and Y chains of one q-l iteration)")
-            roof[name] = _roofline(kern, per * s * rows, us.value, reps,
+            roof[name] = _roofline(f"{what}, {rows} rows)", per * rows, us.value, reps,
                                    _traffic(f"k_{name}_{precision}_cavity1024_traffic.json"))
     else:
         us, nl = _kernel_time(sol, 1, steps)
@@ -243,7 +248,7 @@ def run_path(sol, precision: str, solver: str, fields0, warmup: int, steps: int,
     return {"value": cells * steps / secs / 1e6, "ms_per_step": 1e3 * secs / steps, "fields": fields,
             "warm": warm, "ql": float(np.mean(tab[:, 0])), "ppe": float(np.mean(tab[:, 1])),
             "div_max": div_max.value if solver == "mg" else None, "mg_tune": tune, "window_tune": wtune,
-            "trid_fallbacks": int(L.wd2_trid_fallbacks() - fb0), "roofline": roof}
+            "trid_fallbacks": int(L.wd2_trid_fallbacks() - fb0), "window_repeats": repeats, "roofline": roof}
 
 
 def _errors(a_fields, b_fields, nx, ny) -> dict:
@@ -527,14 +532,17 @@ def main() -> int:
                    "ql_iter_mean": mx["ql"], "vcycles_mean": mx["ppe"],
                    "fp64_ql_iter_mean": f64["ql"], "fp64_vcycles_mean": f64["ppe"],
                    "trid_sequential_fallbacks": {"mixed": mx["trid_fallbacks"], "fp64": f64["trid_fallbacks"]},
+                   "chain_window_repeats": {"mixed": mx["window_repeats"], "fp64": f64["window_repeats"]},
                    "mg_autotuned_shape": {"mixed": mx["mg_tune"], "fp64": f64["mg_tune"]},
                    "window_autotuned_shape": mx["window_tune"]},
-        "roofline": mx["roofline"]["trid_window"],
+        "roofline": mx["roofline"]["ql_windows"],
+        "roofline_ql_windows_first": mx["roofline"]["ql_windows_first"],
         "roofline_trid_fwd": mx["roofline"]["trid_fwd"],
         "roofline_trid_bwd": mx["roofline"]["trid_bwd"],
         "roofline_mg_down": mx["roofline"]["down"],
         "roofline_mg_up": mx["roofline"]["up"],
-        "fp64_roofline": f64["roofline"]["trid_fwd"],
+        "fp64_roofline": f64["roofline"]["ql_windows"],
+        "fp64_roofline_trid_fwd": f64["roofline"]["trid_fwd"],
         "fp64_roofline_trid_bwd": f64["roofline"]["trid_bwd"],
         "fp64_roofline_mg_down": f64["roofline"]["down"],
         "fp64_roofline_mg_up": f64["roofline"]["up"],
