@@ -319,7 +319,9 @@ int wd2_ctx_set_bc_profile(wd2_ctx *ctx, int ireg, int jreg, int side, int var, 
  * launch duration (microseconds: the bracketed time over the launches it
  * holds) and the launch count. */
 int wd2_ctx_kernel_timing(wd2_ctx *ctx, int enable, double *avg_us, long *launches);
-/* The multigrid solver's (nPpeSolver 7) stopping measure: max |dk (b - A p)|
+/* The multigrid solver's (nPpeSolver 7; for grids whose sides are multiples of
+ * 8 cells -- most others converge, but 65, 97, 129 to 131, 257, 258 and 385
+ * cells a side do not) stopping measure: max |dk (b - A p)|
  * over the interior when the last solve stopped (*last) and the largest such
  * value since the last reset (*max_since); reset != 0 then clears the
  * maximum.  No counterpart in the reference. */

@@ -629,8 +629,8 @@ __device__ inline bool qw_rows(unsigned kinds, CT (&a)[TW_S], const CT (&d)[TW_S
 }
 
 // Registers again: five wavefronts per SIMD in float, three in double (1024^2
-// cavity: 26 and 53 us a launch; 30 and 58 at the four and two the compiler
-// takes by itself, 32 and 88 at six and four).
+// cavity, back to back: 27.7 and 44.6 us a launch; 27.9 and 45.4 for bounds of
+// four and two, 28.9 and 49.5 at six and four, which spill).
 template <typename CT, int NT>
 __global__ __launch_bounds__(NT, sizeof(CT) == 4 ? 5 : 3) void k_ql_window(long n, Chains cs, ChainT<float> h1, ChainT<float> h2,
                                                   const unsigned char *__restrict__ Z, QlFields F,
