@@ -52,7 +52,7 @@ int wd2_set_tiled_sor(int enable);
  * default); 0 selects the tiled wavefront, one launch per sweep.  All give
  * the reference's iterates bit for bit.  Returns the previous setting. */
 int wd2_set_lex_rows(int enable);
-/* Mixed precision only: solve the FP32 momentum chains of q-l iterations 2..
+/* Mixed precision only: solve the FP32 momentum chains of the q-l iterations
  * with the windowed partitioned-Thomas/PCR solver (enable = 1, the default;
  * results agree with the bit-exact FP32 solver to FP32 rounding; the first
  * iteration of each step solves its FP32 chains on the same windows in FP64

@@ -42,7 +42,7 @@ void launch_trid_keep_init(int *fail_block, hipStream_t s);
 
 // The mixed path's FP32 chain solve (not bit-exact): overlapping windows
 // solved by partitioned Thomas + PCR in LDS, the bit-exact solver as the
-// fallback for a window that is not usable; same arguments as launch_trid.
+// fallback for a window that is not usable.
 // wt: the window shape, the lanes of one window's workgroup (128, 256 or
 // 512: windows of 1024, 2048 or 4096 rows).
 template <typename T>
@@ -79,7 +79,7 @@ struct Scalars {
     int mg_done;                   // multigrid solve stopped
     int mg_nconv;                  // V-cycles applied when it converged, -1 not converged
     int mg_cycles;                 // V-cycles applied so far
-    int ql_weak;                   // a window of the FP32 chain solve is too weakly dominant
+    int ql_weak;                   // a window of the FP32 chain solve is not usable
     int pad1[8];
 };
 
